@@ -119,41 +119,52 @@ def _rows_per_expert(case, seed):
     return (torch.arange(E) % (rows + 1))[torch.randperm(E, generator=gen)]
 
 
-def prepare(case, seed):
+def _inputs(case, seed):
+    """The tensors that a case's inputs and weights are made of, as its program reads them from its files and its caller."""
     gen = torch.Generator(device="cuda").manual_seed(seed)
     normal = lambda *shape: torch.randn(*shape, device="cuda", generator=gen)  # noqa: E731
     fmt, terms, act, kind = case["fmt"], case["terms"], case["act"], case["kind"]
-    state = {"case": case}
     if kind == "linear":
         K, N, T = case["K"], case["N"], case["T"]
-        stack = [PackedTerm(p[0], s[0]) for p, s in _terms(fmt, terms, 1, N, K, gen)]
-        state["linear"] = TernaryLinear(stack, K, fmt, GROUP, act=act)
-        state["x"] = normal(T, K).bfloat16()
-    elif kind == "grouped":
+        return {"terms": _terms(fmt, terms, 1, N, K, gen), "x": normal(T, K).bfloat16()}
+    if kind == "grouped":
         K, N, E = case["K"], case["N"], case["E"]
         stack = _terms(fmt, terms, E, N, K, gen)
-        state["packed"], state["scale"] = [p for p, _ in stack], [s for _, s in stack]
         counts = _rows_per_expert(case, seed)
-        state["offsets"] = torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]).cuda()
         T = int(counts.sum())
         if act == "int8":
-            state["x"] = torch.randint(-127, 128, (T, K), dtype=torch.int8, device="cuda", generator=gen)
-            state["x_scale"] = 0.01 + 0.02 * torch.rand(T, device="cuda", generator=gen)
+            x = torch.randint(-127, 128, (T, K), dtype=torch.int8, device="cuda", generator=gen)
+            x_scale = 0.01 + 0.02 * torch.rand(T, device="cuda", generator=gen)
         else:
-            state["x"], state["x_scale"] = normal(T, K).bfloat16(), None
+            x, x_scale = normal(T, K).bfloat16(), None
+        return {"terms": stack, "counts": counts, "x": x, "x_scale": x_scale}
+    H, I, E, k = LAYERS[case["layer"]]
+    gate, up = _terms(fmt, terms, E, I, H, gen), _terms(fmt, terms, E, I, H, gen)
+    down = _terms(fmt, terms, E, H, I, gen)
+    x = normal(case["T"], H).bfloat16()
+    logits = 1.5 * normal(case["T"], E)
+    raw = {"gate": gate, "up": up, "down": down, "x": x, "logits": logits}
+    if case["pattern"] == "v4":  # this pattern's router is the caller's: normalised float32 weights of the chosen experts
+        scores, raw["experts"] = torch.topk(torch.softmax(logits, -1), k)
+        raw["weights"] = scores / scores.sum(-1, keepdim=True)
+    return raw
+
+
+def prepare(case, seed):
+    fmt, act, kind, raw = case["fmt"], case["act"], case["kind"], _inputs(case, seed)
+    state = {"case": case, "x": raw["x"]}
+    if kind == "linear":
+        state["linear"] = TernaryLinear([PackedTerm(p[0], s[0]) for p, s in raw["terms"]], case["K"], fmt, GROUP, act=act)
+    elif kind == "grouped":
+        state["packed"], state["scale"] = [p for p, _ in raw["terms"]], [s for _, s in raw["terms"]]
+        state["offsets"] = torch.cat([torch.zeros(1, dtype=torch.int64), raw["counts"].cumsum(0)]).cuda()
+        state["x_scale"] = raw["x_scale"]
     else:
-        H, I, E, k = LAYERS[case["layer"]]
+        H, I, _, k = LAYERS[case["layer"]]
         v4 = case["pattern"] == "v4"
-        gate, up = _terms(fmt, terms, E, I, H, gen), _terms(fmt, terms, E, I, H, gen)
-        down = _terms(fmt, terms, E, H, I, gen)
-        state["moe"] = TernaryMoE(gate, up, down, H, I, k, fmt, GROUP, act=act, pattern=case["pattern"], swiglu_limit=10.0 if v4 else 0.0)
-        state["x"] = normal(case["T"], H).bfloat16()
-        logits = 1.5 * normal(case["T"], E)
-        if v4:  # this pattern's router is the caller's: normalised float32 weights of the chosen experts
-            scores, state["experts"] = torch.topk(torch.softmax(logits, -1), k)
-            state["weights"] = scores / scores.sum(-1, keepdim=True)
-        else:
-            state["logits"] = logits
+        state["moe"] = TernaryMoE(raw["gate"], raw["up"], raw["down"], H, I, k, fmt, GROUP, act=act, pattern=case["pattern"],
+                                  swiglu_limit=10.0 if v4 else 0.0)
+        state.update({name: raw[name] for name in (("experts", "weights") if v4 else ("logits",))})
     return state
 
 
@@ -203,3 +214,58 @@ def tolerance(case):
     if case["kind"] == "linear":
         return {"rel": 4e-4, "max": 0.032}
     return {"rel": 4e-3, "max": 0.12}
+
+
+def _dense(terms, e, K, fmt):
+    """The float64 [N, K] matrix of expert ``e``: the sum of its terms' trits times scales."""
+    total = 0
+    for packed, scale in terms:
+        v = packed[e].int()
+        digits = [v // 3**i % 3 for i in range(5)] if fmt == "tq1" else [v >> 2 * i & 3 for i in range(4)]
+        trits = torch.stack(digits, -1).flatten(1)[:, :K].double() - 1
+        total = total + trits * scale[e].double().repeat_interleave(GROUP, -1)
+    return total
+
+
+def _int8(x):
+    """Rows as whole numbers -127 .. 127 and float32 scales: absmax / 127, halves to even."""
+    scale = (x.float().abs().amax(-1, keepdim=True) / 127).clamp(min=1e-8)
+    return (x.float() / scale).round().clamp(-127, 127).double(), scale.double()
+
+
+def exact(case, seed):
+    """The same products and sums in 64 bits, with the places where the path rounds to bf16 or quantises to int8: a linear's
+    activations, gate, up, hidden and expert rows of a layer. A linear's and a layer's own result are not rounded."""
+    raw, fmt = _inputs(case, seed), case["fmt"]
+    rows = lambda x: _int8(x) if case["act"] == "int8" else (x.double(), 1.0)  # noqa: E731
+    if case["kind"] == "linear":
+        q, scale = rows(raw["x"])
+        return q @ _dense(raw["terms"], 0, case["K"], fmt).T * scale
+    if case["kind"] == "grouped":
+        parts = [x.double() @ _dense(raw["terms"], e, case["K"], fmt).T for e, x in enumerate(raw["x"].split(raw["counts"].tolist())) if len(x)]
+        out = torch.cat(parts)
+        return out if raw["x_scale"] is None else out * raw["x_scale"].double()[:, None]
+    H, I, E, k = LAYERS[case["layer"]]
+    v4 = case["pattern"] == "v4"
+    if v4:
+        weights, experts = raw["weights"], raw["experts"]
+    else:
+        weights, experts = torch.topk(torch.softmax(raw["logits"].double(), -1), k)
+        weights = weights.bfloat16()
+    out = torch.zeros(case["T"], H, dtype=torch.float64, device="cuda")
+    for e in range(E):
+        token, slot = (experts == e).nonzero(as_tuple=True)
+        if not len(token):
+            continue
+        w = weights[token, slot].double()[:, None]
+        q, scale = rows(raw["x"][token])
+        gate, up = ((q @ _dense(raw[n], e, H, fmt).T * scale).bfloat16().double() for n in ("gate", "up"))
+        if v4:
+            gate, up = gate.clamp(max=10.0), up.clamp(-10.0, 10.0)
+            h = (w * (gate * torch.sigmoid(gate) * up)).bfloat16()
+        else:
+            h = ((gate * torch.sigmoid(gate)).bfloat16().double() * up).bfloat16()
+        q, scale = rows(h)
+        y = (q @ _dense(raw["down"], e, I, fmt).T * scale).bfloat16().double()
+        out[token] += y if v4 else (y * w).bfloat16().double()
+    return out
