@@ -89,12 +89,14 @@ extern "C" int bp_set_kernel_policy(int policy) {
 static bool valid_scale_dtype(int d) { return d == BP_F32 || d == BP_F16 || d == BP_BF16; }
 static bool valid_act_dtype(int d) { return d == BP_I8 || d == BP_BF16 || d == BP_F16 || d == BP_F32; }
 
-static int grouped_gemm(float* out, const void* x, int x_dtype, const float* x_scale, const int64_t* offsets,
+// Checks a call and fills its argument block; `empty`: a valid call without work.
+static int check_args(GemmArgs& a, bool& empty, float* out, const void* x, int x_dtype, const float* x_scale, const int64_t* offsets,
                         const int64_t* offsets_host, const uint8_t* const* packed, const void* const* w_scale,
                         int scale_dtype, int n_terms, int64_t T, int64_t N, int64_t K, int64_t Kp, int64_t G, int64_t group,
-                        int64_t E, int fmt, int64_t max_rows, void* workspace, size_t workspace_bytes, void* stream) {
+                        int64_t E, int fmt, int64_t max_rows, void* workspace, size_t workspace_bytes) {
   g_error[0] = 0;
   g_kernel[0] = 0;
+  empty = true;
   if (!valid_act_dtype(x_dtype)) return fail(BP_ERR_ARG, "unexpected ternary GEMM activation dtype");
   if (!valid_scale_dtype(scale_dtype)) return fail(BP_ERR_ARG, "unexpected ternary GEMM scale dtype");
   if (fmt != BP_TQ1 && fmt != BP_TQ2) return fail(BP_ERR_ARG, "fmt must be 1 (TQ1) or 2 (TQ2)");
@@ -129,7 +131,7 @@ static int grouped_gemm(float* out, const void* x, int x_dtype, const float* x_s
   if (!out || !x) return fail(BP_ERR_ARG, "null out or x");
   if (x_dtype == BP_I8 && !x_scale) return fail(BP_ERR_ARG, "int8 activations need x_scale");
 
-  GemmArgs a;
+  empty = false;
   memset(&a, 0, sizeof(a));
   a.out = out; a.x = x; a.x_scale = x_scale; a.offsets = offsets;
   for (int t = 0; t < n_terms; ++t) {
@@ -141,8 +143,19 @@ static int grouped_gemm(float* out, const void* x, int x_dtype, const float* x_s
   a.T = T; a.N = N; a.K = K; a.Kp = Kp; a.G = G; a.group = group; a.E = E; a.max_rows = max_rows;
   a.stage = (unsigned char*)workspace;
   a.stage_bytes = workspace ? (int64_t)workspace_bytes : 0;
+  return BP_OK;
+}
 
-  return run_gemm(a, (hipStream_t)stream);
+static int grouped_gemm(float* out, const void* x, int x_dtype, const float* x_scale, const int64_t* offsets,
+                        const int64_t* offsets_host, const uint8_t* const* packed, const void* const* w_scale,
+                        int scale_dtype, int n_terms, int64_t T, int64_t N, int64_t K, int64_t Kp, int64_t G, int64_t group,
+                        int64_t E, int fmt, int64_t max_rows, void* workspace, size_t workspace_bytes, void* stream) {
+  GemmArgs a;
+  bool empty;
+  if (const int rc = check_args(a, empty, out, x, x_dtype, x_scale, offsets, offsets_host, packed, w_scale, scale_dtype, n_terms, T, N, K, Kp, G,
+                                group, E, fmt, max_rows, workspace, workspace_bytes))
+    return rc;
+  return empty ? BP_OK : run_gemm(a, (hipStream_t)stream);
 }
 
 extern "C" int bp_ternary_grouped_gemm(float* out, const void* x, int x_dtype, const float* x_scale,
@@ -191,6 +204,87 @@ extern "C" int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype
   }
   return grouped_gemm(out, x, x_dtype, x_scale, offsets, offsets_host, packed, w_scale, scale_dtype, n_terms, T, N, K, Kp, G,
                       group, E, fmt, max_rows, workspace, workspace_bytes, stream);
+}
+
+// ---- one dense linear from its float activations to its output rows, in one call: the quantisation to int8 (act_int8),
+// the product, the rounding to bf16. The kernels write bf16 rows themselves where they can (GemmArgs::out16), so that the
+// usual call is one launch, or two with the quantisation; a zero-fill, a product that adds to float32 rows and a rounding
+// pass are left for the calls in which a kernel takes several passes over an output.
+namespace bp {
+namespace {
+struct LinearPlan {  // offsets into the workspace
+  size_t q, q_scale, sums, stage, stage_bytes, bytes;
+};
+LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int fmt, int n_terms) {
+  LinearPlan p;
+  size_t at = 0;
+  auto take = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) & ~(size_t)255; return o; };
+  p.q = take(act_int8 ? (size_t)T * (size_t)K : 0);
+  p.q_scale = take(act_int8 ? 4 * (size_t)T : 0);
+  p.sums = take(out_dtype == BP_F32 ? 0 : 4 * (size_t)T * (size_t)N);
+  p.stage_bytes = bp_grouped_gemm_workspace_bytes(act_int8 ? BP_I8 : x_dtype, T, N, K, 1, fmt, T);
+  p.stage = take(p.stage_bytes);
+  p.bytes = at;
+  return p;
+}
+
+__global__ __launch_bounds__(256) void k_zero4(float* __restrict__ p, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0.f;
+}
+__global__ __launch_bounds__(256) void k_round_bf16(uint16_t* __restrict__ out, const float* __restrict__ in, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) out[i] = f32_to_bf16_bits(in[i]);
+}
+unsigned fill_grid(int64_t n) { return (unsigned)((n + 255) / 256 > 16384 ? 16384 : (n + 255) / 256); }
+}  // namespace
+}  // namespace bp
+
+extern "C" size_t bp_ternary_linear_workspace_bytes(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int fmt, int n_terms) {
+  if (T <= 0 || N <= 0 || K <= 0 || n_terms < 1 || n_terms > BP_MAX_TERMS) return 0;
+  return linear_plan(x_dtype, act_int8, out_dtype, T, N, K, fmt, n_terms).bytes;
+}
+
+extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_dtype, int act_int8, const int64_t* offsets,
+                                 const uint8_t* const* packed, const void* const* w_scale, int scale_dtype, int n_terms,
+                                 int64_t T, int64_t N, int64_t K, int64_t Kp, int64_t G, int64_t group, int fmt, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
+  g_error[0] = 0;
+  g_kernel[0] = 0;
+  if (out_dtype != BP_F32 && out_dtype != BP_BF16) return fail(BP_ERR_ARG, "a linear's output is float32 or bf16");
+  if (x_dtype != BP_BF16 && x_dtype != BP_F16 && x_dtype != BP_F32) return fail(BP_ERR_ARG, "activation dtype must be bf16, f16 or f32");
+  if (workspace && ((uintptr_t)workspace & 255) != 0) return fail(BP_ERR_ARG, "workspace must be 256-byte aligned");
+  const hipStream_t s = (hipStream_t)stream;
+  unsigned char* ws = (unsigned char*)workspace;
+  LinearPlan p = {};
+  if (T > 0 && N > 0 && K > 0 && n_terms >= 1 && n_terms <= BP_MAX_TERMS) p = linear_plan(x_dtype, act_int8, out_dtype, T, N, K, fmt, n_terms);
+  if (p.bytes && (!ws || workspace_bytes < p.bytes)) return fail(BP_ERR_ARG, "the workspace must hold bp_ternary_linear_workspace_bytes() = %zu bytes", p.bytes);
+  GemmArgs a;
+  bool empty;
+  // (the argument checks of the grouped call; int8 activations and their scales are still to be written)
+  if (const int rc = check_args(a, empty, (float*)out, x, act_int8 ? BP_I8 : x_dtype, act_int8 ? (const float*)(ws + p.q_scale) : nullptr, offsets, nullptr,
+                                packed, w_scale, scale_dtype, n_terms, T, N, K, Kp, G, group, 1, fmt, T, p.stage_bytes ? ws + p.stage : nullptr,
+                                p.stage_bytes))
+    return rc;
+  if (empty) return BP_OK;
+  uint16_t* out16 = out_dtype == BP_BF16 ? (uint16_t*)out : nullptr;
+  if (act_int8) {
+    if (const int rc = bp_quant_act_int8((int8_t*)(ws + p.q), (float*)(ws + p.q_scale), x, x_dtype, T, K, stream)) return rc;
+    a.x = ws + p.q;
+  }
+  if (out16) {
+    a.out16 = out16;
+    a.overwrite = 1;
+    const int rc = run_gemm(a, s);
+    if (rc != ERR_NO_OUT16) return rc;
+    a.out16 = nullptr;
+    a.overwrite = 0;
+    a.out = (float*)(ws + p.sums);
+  }
+  hipLaunchKernelGGL(k_zero4, dim3(fill_grid(T * N)), dim3(256), 0, s, a.out, T * N);
+  if (const int rc = check_launch("zero")) return rc;
+  if (const int rc = run_gemm(a, s)) return rc;
+  if (!out16) return BP_OK;
+  hipLaunchKernelGGL(k_round_bf16, dim3(fill_grid(T * N)), dim3(256), 0, s, out16, a.out, T * N);
+  return check_launch("round_bf16");
 }
 
 namespace bp {
@@ -243,6 +337,7 @@ size_t split_bytes(int64_t T, int64_t K) { return ((size_t)T * (size_t)K * 2 + 2
 }  // namespace
 
 int run_gemm(const GemmArgs& a, hipStream_t s) {
+  if (a.out16 && g_policy != 1 && a.stage && split_applies(a)) return ERR_NO_OUT16;  // (two products added up)
   if (g_policy != 1 && a.stage && split_applies(a) && (size_t)a.stage_bytes >= 2 * split_bytes(a.T, a.K)) {
     const size_t part = split_bytes(a.T, a.K);
     uint16_t* hi = (uint16_t*)a.stage;
@@ -269,6 +364,7 @@ int run_gemm(const GemmArgs& a, hipStream_t s) {
   }
   if (a.tiles) return fail(BP_ERR_UNSUPPORTED, "tile-list mode needs one of the 32-token-tile kernels");
   if (g_policy == 2) return fail(BP_ERR_UNSUPPORTED, "shape is outside the tuned kernels (policy 2 forbids the general kernel)");
+  if (a.out16) return ERR_NO_OUT16;
   return launch_general(a, s);
 }
 }  // namespace bp

@@ -45,7 +45,9 @@ struct GemmArgs {
   // x_index[r] / x_div of x, which has x_rows rows (the routed copy of the activations is never materialised).
   const int64_t* x_index;
   int64_t x_div, x_rows;
-  uint16_t* out16;  // (the same kernel, tile-list mode with overwrite) bf16 out16[T, N] is written instead of float32 `out`
+  // bf16 out16[T, N] is written instead of float32 `out` (one launch that covers all of K and all terms; a kernel that
+  // takes several passes over an output returns ERR_NO_OUT16 instead).
+  uint16_t* out16;
   uint16_t* glu_h;
   int glu_v4;
   float glu_limit;
@@ -56,11 +58,12 @@ struct GemmArgs {
 
 __device__ __forceinline__ int64_t clamp_i64(int64_t v, int64_t lo, int64_t hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-// Which token tile of 32 rows a workgroup takes: `slot` is its expert (list entry in tile-list mode), z its token tile.
+// Which token tile of ROWS rows a workgroup takes: `slot` is its expert (list entry in tile-list mode), z its token tile.
 struct TileRef {
   int64_t e, tok0, o1;
   bool live;
 };
+template <int ROWS = 32>
 __device__ __forceinline__ TileRef tile_ref(const GemmArgs& a, int64_t slot, unsigned z) {
   TileRef r = {0, 0, 0, false};
   if (a.tiles) {
@@ -72,13 +75,13 @@ __device__ __forceinline__ TileRef tile_ref(const GemmArgs& a, int64_t slot, uns
     if (slot >= a.E) return r;
     r.e = slot;
     r.o1 = clamp_i64(a.offsets[slot + 1], 0, a.T);
-    r.tok0 = clamp_i64(a.offsets[slot], 0, a.T) + (int64_t)z * 32;
+    r.tok0 = clamp_i64(a.offsets[slot], 0, a.T) + (int64_t)z * ROWS;
   }
   r.live = r.tok0 < r.o1;
   return r;
 }
 
-// Which token tile and which block of output rows a workgroup of a 32-token-tile kernel takes, from its linear index.
+// Which token tile and which block of output rows a workgroup of a token-tile kernel takes, from its linear index.
 // Workgroups are dealt to the 8 XCDs round-robin by linear index and each XCD has its own L2. The row blocks of a token
 // tile read the same activations and the token tiles of an expert the same weights, so an XCD takes its experts one after
 // the other, an expert's token tiles one after the other and a tile's row blocks one after the other: the workgroups
@@ -88,27 +91,29 @@ __device__ __forceinline__ TileRef tile_ref(const GemmArgs& a, int64_t slot, uns
 // dense call (one expert) ran on a single XCD - a linear of 777 tokens x 4096 x 2048, TQ1 in two terms, 389 us against
 // 115, 8192 x 2048 x 6144 int8 on the 32-token tiles 2877 against 441.
 constexpr int TILE_RUN = 4;
+template <int ROWS = 32>
 __device__ __forceinline__ TileRef tile_of_workgroup(const GemmArgs& a, unsigned linear, int row_blocks, int& row_block) {
   const unsigned xcd = linear & 7;
   unsigned q = linear >> 3;
   if (a.tiles) {
     row_block = (int)(q % (unsigned)row_blocks);
     q /= (unsigned)row_blocks;
-    return tile_ref(a, (int64_t)(q / TILE_RUN) * (8 * TILE_RUN) + xcd * TILE_RUN + q % TILE_RUN, 0);
+    return tile_ref<ROWS>(a, (int64_t)(q / TILE_RUN) * (8 * TILE_RUN) + xcd * TILE_RUN + q % TILE_RUN, 0);
   }
-  const unsigned tiles_per_expert = (unsigned)((a.max_rows + 31) / 32);
+  const unsigned tiles_per_expert = (unsigned)((a.max_rows + ROWS - 1) / ROWS);
   const unsigned item = xcd * (gridDim.x >> 3) + q;  // (the grid is a multiple of 8: tile_workgroups; items past the experts are not live)
   row_block = (int)(item % (unsigned)row_blocks);
   const unsigned tile = item / (unsigned)row_blocks;
-  return tile_ref(a, tile / tiles_per_expert, tile % tiles_per_expert);
+  return tile_ref<ROWS>(a, tile / tiles_per_expert, tile % tiles_per_expert);
 }
 // Workgroups of such a launch (-1: more than a grid's x extent holds).
+template <int ROWS = 32>
 inline int64_t tile_workgroups(const GemmArgs& a, int64_t row_blocks) {
   if (a.tiles) {
     const int64_t rounds = (a.tile_cap + 8 * TILE_RUN - 1) / (8 * TILE_RUN);
     return rounds > 0x7fffffff / (row_blocks * 8 * TILE_RUN) ? -1 : row_blocks * 8 * TILE_RUN * rounds;
   }
-  const int64_t z = (a.max_rows + 31) / 32;
+  const int64_t z = (a.max_rows + ROWS - 1) / ROWS;
   if (z > 0x7ffffff8 / row_blocks || a.E > 0x7ffffff8 / (row_blocks * z)) return -1;
   return (a.E * z * row_blocks + 7) & ~(int64_t)7;
 }
@@ -145,6 +150,10 @@ int raise_lds_limit(int bytes) {
   return BP_OK;
 }
 
+// Internal result of a launcher whose kernel cannot write GemmArgs::out16 for this call: the caller takes float32 sums of
+// the whole call and rounds them in a pass of its own.
+constexpr int ERR_NO_OUT16 = -100;
+
 // Kernel selection for a validated argument block (the body of bp_ternary_grouped_gemm after its checks).
 int run_gemm(const GemmArgs& a, hipStream_t s);
 // True when a launch in tile-list mode would run on one of the 32-token-tile kernels (which honour tiles / overwrite).
@@ -161,10 +170,9 @@ bool mfma_supports(const GemmArgs& a);
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
 
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {  // round to nearest even, NaN kept quiet
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x0040u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+  const uint32_t u = __float_as_uint(f);
+  const uint32_t rounded = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16, quiet = (u >> 16) | 0x0040u;
+  return (uint16_t)(f != f ? quiet : rounded);  // (a select: epilogues convert dozens of values per lane)
 }
 
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t b) {
@@ -176,6 +184,12 @@ __device__ __forceinline__ float load_scale(const void* p, int dtype, int64_t i)
   if (dtype == BP_F32) return ((const float*)p)[i];
   const uint16_t b = ((const uint16_t*)p)[i];
   return dtype == BP_F16 ? f16_bits_to_f32(b) : bf16_bits_to_f32(b);
+}
+
+// One finished output: bf16 in place of the float32 one, or the float32 one replaced or added to.
+__device__ __forceinline__ void store_out(const GemmArgs& a, int64_t i, float v) {
+  if (a.out16) a.out16[i] = f32_to_bf16_bits(v);
+  else a.out[i] = (a.overwrite ? 0.f : a.out[i]) + v;
 }
 
 __device__ __forceinline__ float load_act_f32(const void* p, int dtype, int64_t i) {

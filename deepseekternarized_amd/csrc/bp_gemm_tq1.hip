@@ -443,8 +443,7 @@ __global__ __launch_bounds__(Q_THREADS, 2) void k_gemm_tq1(GemmArgs a) {
           for (int r = 0; r < Q_RT; ++r) {
             const int64_t row = n_wave + 16 * r;
             if (row < a.N) {
-              float* o = a.out + tok * a.N + row + r16;
-              *o = (a.overwrite ? 0.f : *o) + total[r][t][i] * xs;
+              store_out(a, tok * a.N + row + r16, total[r][t][i] * xs);
             }
           }
         }

@@ -396,8 +396,7 @@ __global__ __launch_bounds__(GTHREADS, 2) void k_gemm_tq2(GemmArgs a) {
 #pragma unroll
         for (int r = 0; r < GR; ++r) {
           if (rows_valid[r]) {
-            float* o = a.out + tok * a.N + n0 + 16 * r + r16;
-            *o = (a.overwrite ? 0.f : *o) + total[r][mt][q] * xs;
+            store_out(a, tok * a.N + n0 + 16 * r + r16, total[r][mt][q] * xs);
           }
         }
       }

@@ -644,20 +644,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a) {
           for (int q = 0; q < 2; ++q) {
             const int64_t col = tile_row(wave, q);
             if (col < 0) continue;
-            float g = bf16_bits_to_f32(f32_to_bf16_bits(total[q][t][i])), u = bf16_bits_to_f32(f32_to_bf16_bits(total[q + 2][t][i]));
-            float v;
-            if (a.glu_v4) {
-              if (a.glu_limit > 0.f) {  // torch.clamp: a NaN stays a NaN
-                u = u < -a.glu_limit ? -a.glu_limit : (u > a.glu_limit ? a.glu_limit : u);
-                g = g > a.glu_limit ? a.glu_limit : g;
-              }
-              v = (g / (1.0f + expf(-g))) * u;
-              if (a.glu_weights) v = w * v;
-            } else {
-              const float sg = bf16_bits_to_f32(f32_to_bf16_bits(g / (1.0f + expf(-g))));
-              v = sg * u;
-            }
-            a.glu_h[tok * NH + col + r16] = f32_to_bf16_bits(v);
+            a.glu_h[tok * NH + col + r16] = swiglu_value(a, total[q][t][i], total[q + 2][t][i], w);
           }
         }
       }
@@ -674,12 +661,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a) {
           for (int r = 0; r < F_RT; ++r) {
             const int64_t row = tile_row(wave, r);
             if (row >= 0) {
-              if (a.out16) {
-                a.out16[tok * a.N + row + r16] = f32_to_bf16_bits(total[r][t][i]);
-              } else {
-                float* o = a.out + tok * a.N + row + r16;
-                *o = (a.overwrite ? 0.f : *o) + total[r][t][i];
-              }
+              store_out(a, tok * a.N + row + r16, total[r][t][i]);
             }
           }
         }
@@ -732,7 +714,6 @@ size_t gemm_tq2f_workspace_bytes(int64_t T, int64_t K, int64_t E) {
 int gemm_tq2f_applies(const GemmArgs& a) {
   if (a.x_dtype != BP_BF16 || !a.stage || ((uintptr_t)a.stage & 15) != 0) return BP_ERR_UNSUPPORTED;
   if (a.glu_h && (!a.tiles || !a.overwrite || a.N % 32 != 0)) return BP_ERR_UNSUPPORTED;  // (whole row tiles of either half, one launch for all of K)
-  if (a.out16 && (!a.tiles || !a.overwrite)) return BP_ERR_UNSUPPORTED;
   if ((size_t)a.stage_bytes < gemm_tq2f_workspace_bytes(a.T, a.K, a.E) || gemm_tq2f_workspace_bytes(a.T, a.K, a.E) == 0) return BP_ERR_UNSUPPORTED;
   if (a.K > ((int64_t)1 << 24) || a.N * a.Kp > ((int64_t)1 << 31) - 4096) return BP_ERR_UNSUPPORTED;
   if (a.fmt == BP_TQ2 && tuning().tq2g != 'f') {  // (development: BP_TUNE_TQ2G=fp4 runs this kernel wherever it can)

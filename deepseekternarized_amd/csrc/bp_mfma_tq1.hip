@@ -337,8 +337,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq1(GemmArgs a, int CPT 
   for (int q = 0; q < NQ; ++q) {
     const int t = 4 * b + q;
     if (t < ntok && wave_live) {
-      float* o = a.out + (tok0 + t) * a.N + n0 + r16;
-      *o += x_i8 ? total[q] * a.x_scale[tok0 + t] : total[q];
+      store_out(a, (tok0 + t) * a.N + n0 + r16, x_i8 ? total[q] * a.x_scale[tok0 + t] : total[q]);
     }
   }
 }

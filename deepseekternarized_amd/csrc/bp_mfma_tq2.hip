@@ -310,8 +310,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq2(GemmArgs a, int KC, 
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           if (rows_valid[r]) {
-            float* o = a.out + tok * a.N + n0 + 16 * r + r16;
-            *o += total[r][mt][q] * xs;
+            store_out(a, tok * a.N + n0 + 16 * r + r16, total[r][mt][q] * xs);
           }
         }
       }

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(CW_WAVES * 64) void k_tq1_gemv_cw(GemmArgs a, int n
 #pragma unroll
   for (int u = 0; u < CW_STAGE_PER_THREAD; ++u) {
     const int o = (int)threadIdx.x + u * THREADS;
-    was[u] = o < n_stage && ((o >> 4) % NTOK) < ntok ? a.out[out_index(o)] : 0.f;
+    was[u] = !a.out16 && o < n_stage && ((o >> 4) % NTOK) < ntok ? a.out[out_index(o)] : 0.f;
   }
 
   // ---- loaders: state of the current term (the expert's rows and scales as buffers of their own: a tile past N reads
@@ -436,8 +436,12 @@ __global__ __launch_bounds__(CW_WAVES * 64) void k_tq1_gemv_cw(GemmArgs a, int n
       const int64_t tile = tile_of(t);
 #pragma unroll
       for (int tt = 0; tt < NTOK; ++tt) {
-        if (tt % lpg == lidx && tile < tile_end && tt < ntok)
-          a.out[(tok + tt) * a.N + tile * 16 + r16] = __uint_as_float(*(const lds_u32*)(stage + (unsigned)((((int)(tile - tile0) * NTOK + tt) * 16 + r16) * 4)));
+        if (tt % lpg == lidx && tile < tile_end && tt < ntok) {
+          const int64_t at = (tok + tt) * a.N + tile * 16 + r16;
+          const float v = __uint_as_float(*(const lds_u32*)(stage + (unsigned)((((int)(tile - tile0) * NTOK + tt) * 16 + r16) * 4)));
+          if (a.out16) a.out16[at] = f32_to_bf16_bits(v);
+          else a.out[at] = v;
+        }
       }
     }
   }

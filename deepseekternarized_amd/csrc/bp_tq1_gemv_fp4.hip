@@ -196,7 +196,7 @@ __global__ __launch_bounds__(WAVES * 64, KS ? 2 : 4) void k_tq1_gemv_fp4(GemmArg
       total[s] = 0.f;
       const int tile = NTOK > 1 ? 0 : s, tt = NTOK > 1 ? s : 0;
       before[s] = 0.f;
-      if (EARLY && kb == 0 && wave_live && n0 + 16 * tile < a.N && tt < ntok && (!KS || wave == 0))
+      if (EARLY && !a.out16 && kb == 0 && wave_live && n0 + 16 * tile < a.N && tt < ntok && (!KS || wave == 0))
         before[s] = __hip_atomic_load(a.out + (tok + tt) * a.N + n0 + 16 * tile + r16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // chunk c of this block, or (c >= nchunks, chained) chunk c - nchunks of the next one: row offset (scalar) and chunk
@@ -496,9 +496,15 @@ __global__ __launch_bounds__(WAVES * 64, KS ? 2 : 4) void k_tq1_gemv_fp4(GemmArg
       if (wave != 0) continue;
     }
     if (kb == 0 && wave_live && n0 + 16 * tile < a.N && tt < ntok) {
-      float* o = a.out + (tok + tt) * a.N + n0 + 16 * tile + r16;
+      const int64_t at = (tok + tt) * a.N + n0 + 16 * tile + r16;
+      const float v = a.x_dtype == BP_I8 ? t * xsc[tt] : t;
+      if (a.out16) {  // (one term, all of K in this launch)
+        a.out16[at] = f32_to_bf16_bits(v);
+        continue;
+      }
+      float* o = a.out + at;
       const float was = EARLY ? before[s] : __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *o = was + (a.x_dtype == BP_I8 ? t * xsc[tt] : t);
+      *o = was + v;
     }
   }
   }  // pass
@@ -511,6 +517,8 @@ __global__ __launch_bounds__(WAVES * 64, KS ? 2 : 4) void k_tq1_gemv_fp4(GemmArg
 }
 template <int SDT, int WAVES, int ABL = 0, int NTOK = 1, int SR = 0, int KS = 0>
 int launch_f4_k(const GemmArgs& a, hipStream_t s, const char* name, int nchunks, size_t lds, int seg_chunks = 0 /* chunks per launch (0: all) */, int first_row = 0) {
+  // (the kernel adds a term's sums, and a segment's, to the output)
+  if (a.out16 && (a.n_terms > 1 || (seg_chunks > 0 && seg_chunks < nchunks))) return ERR_NO_OUT16;
   if (const int rc = raise_lds_limit<k_tq1_gemv_fp4<SDT, WAVES, ABL, NTOK, SR, KS>>(F4_LDS_MAX)) return rc;
   if (SR) lds += (size_t)WAVES * F4_SCALE_SLOT;
   if (KS) lds += (size_t)WAVES * 64;  // the waves' partial sums

@@ -98,8 +98,8 @@ class _HipTernary:
             need = 0
             if max_rows > _DECODE_ROWS or xdt in (_lib.BP_F16, _lib.BP_F32):
                 need = self.lib.bp_grouped_gemm_workspace_bytes(xdt, T, N, int(K), E, int(fmt), int(max_rows))
-                if need > _WORKSPACE_CAP:  # (about 2.1 bytes per activation: a call this large keeps its memory and runs the kernels without one)
-                    need = 0
+            if need > _WORKSPACE_CAP:  # (up to 2.1 bytes per activation: a call this large keeps its memory and runs the kernels without one)
+                need = 0
             head = (out.data_ptr(), x.data_ptr(), xdt, x_scale.data_ptr() if x_scale is not None else None, offsets.data_ptr(), host,
                     C.cast(pk, C.c_void_p), C.cast(sc, C.c_void_p), _lib.dtype_code(sdt), len(packed_l),
                     T, N, int(K), Kp, G, int(group), E, int(fmt), int(max_rows))
@@ -113,6 +113,44 @@ class _HipTernary:
                 torch.cuda.set_device(prev)
         if rc:
             _lib.check(rc)
+
+    def ternary_linear(self, x, packed, w_scale, K, group, fmt, act_int8, out_dtype):
+        """One dense linear in one library call (``bp_ternary_linear``): ``x`` [T, K] bf16 / f16 / f32 contiguous, quantised
+        per row to int8 with ``act_int8``; ``packed`` / ``w_scale`` lists of [1, N, Kp] / [1, N, G] -> [T, N] ``out_dtype``."""
+        if len(packed) != len(w_scale) or not 1 <= len(packed) <= _lib.BP_MAX_TERMS:
+            raise RuntimeError("packed and w_scale must hold the same number of terms (1..4)")
+        dev = x.device
+        p0, s0 = packed[0], w_scale[0]
+        _, N, Kp = p0.shape
+        G, sdt = s0.shape[2], s0.dtype
+        for p, s in zip(packed, w_scale):
+            if p.device != dev or s.device != dev or not (p.is_contiguous() and s.is_contiguous()):
+                raise RuntimeError("ternary GEMM tensors must share one device")
+            if p.dtype != torch.uint8 or s.dtype != sdt:
+                raise RuntimeError("unexpected ternary GEMM dtype")
+            if p.shape != p0.shape or s.shape != s0.shape or s.shape[1] != N:
+                raise RuntimeError("inconsistent ternary GEMM shapes")
+        T = x.shape[0]
+        n = len(packed)
+        pk, sc = (C.c_void_p * n)(*[p.data_ptr() for p in packed]), (C.c_void_p * n)(*[s.data_ptr() for s in w_scale])
+        xdt, odt, sdc = _lib.dtype_code(x.dtype), _lib.dtype_code(out_dtype), _lib.dtype_code(sdt)
+        offsets = dense_offsets(dev, T)
+        out = torch.empty(T, N, dtype=out_dtype, device=dev)
+        need = self.lib.bp_ternary_linear_workspace_bytes(xdt, act_int8, odt, T, N, K, fmt, n)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+        prev = torch.cuda.current_device()
+        index = dev.index if dev.index is not None else prev
+        if prev != index:
+            torch.cuda.set_device(index)
+        try:
+            rc = self.lib.bp_ternary_linear(out.data_ptr(), odt, x.data_ptr(), xdt, act_int8, offsets.data_ptr(), pk, sc, sdc, n, T, N, K, Kp, G, group,
+                                            fmt, ws.data_ptr() if need else None, need, torch._C._cuda_getCurrentRawStream(index))
+        finally:
+            if prev != index:
+                torch.cuda.set_device(prev)
+        if rc:
+            _lib.check(rc)
+        return out
 
     def last_kernel(self) -> str:
         return self.lib.bp_last_kernel().decode()

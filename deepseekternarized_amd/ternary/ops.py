@@ -83,8 +83,14 @@ class TernaryLinear:
     def __call__(self, x: torch.Tensor, out_dtype=torch.bfloat16) -> torch.Tensor:
         shape = x.shape
         x2 = x.reshape(-1, self.K)
-        _need_ext(x2)
+        e = _need_ext(x2)
         terms = self._on(x2.device)
+        if self.backend in ("auto", "cuda", "hip") and out_dtype in (torch.bfloat16, torch.float32):
+            if x2.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+                x2 = x2.float()
+            out = e.ternary_linear(x2.contiguous(), [p for p, _ in terms], [sc for _, sc in terms], self.K, self.group, _fmt_code(self.fmt),
+                                   int(self.act == "int8"), out_dtype)
+            return out.view(*shape[:-1], -1)
         if self.act == "int8":
             q, s = quant_act_int8(x2)
         else:

@@ -102,6 +102,21 @@ int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype, const flo
                                int64_t group, int64_t E, int fmt, int64_t max_rows, void* workspace,
                                size_t workspace_bytes, void* stream);
 
+/* One dense linear (TernaryLinear.__call__, boilerplate/ternary/ops.py:60-86) from its float activations to its output rows:
+ * out[t, :] = the product of bp_ternary_grouped_gemm with one expert, rounded to bf16 or as float32; it replaces what
+ * `out` holds. act_int8: the rows are quantised first, as by bp_quant_act_int8. The same sums and roundings as those
+ * calls one after the other, without their float32 rows and launches between them where a kernel can do without.
+ *   out      device [T, N] of out_dtype BP_BF16 or BP_F32
+ *   x        device [T, K] of x_dtype BP_BF16, BP_F16 or BP_F32
+ *   offsets  device i64 {0, T}
+ *   packed[t] device u8 [N, Kp], w_scale[t] device [N, G]; n_terms stacked terms
+ *   workspace device memory, 256-byte aligned, at least bp_ternary_linear_workspace_bytes(...) bytes (NULL if that is 0) */
+size_t bp_ternary_linear_workspace_bytes(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int fmt, int n_terms);
+int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_dtype, int act_int8, const int64_t* offsets,
+                      const uint8_t* const* packed, const void* const* w_scale, int scale_dtype, int n_terms,
+                      int64_t T, int64_t N, int64_t K, int64_t Kp, int64_t G, int64_t group, int fmt, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
 /* Selects the kernel family for bp_ternary_grouped_gemm on the calling thread:
  *   0 = automatic (tuned kernels where the shape allows, general kernel otherwise)
  *   1 = general kernel only (any K, group, format; int8 path bit-identical to

@@ -1,0 +1,49 @@
+"""``TernaryLinear`` as one library call (``bp_ternary_linear``) against the calls that it stands for: the quantisation, the
+grouped product with one expert, the rounding to the output type - the same kernels, so the same bits."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(fmt, N, K, group, terms, sdt, seed=3):
+    import deepseekternarized_amd as bp
+
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return [bp.PackedTerm(bp.pack(torch.randint(-1, 2, (N, K), dtype=torch.int8, device="cuda", generator=gen), fmt),
+                          (0.02 * torch.rand(N, -(-K // group), device="cuda", generator=gen)).to(sdt)) for _ in range(terms)], gen
+
+
+def _steps(x, terms, K, group, fmt, act, out_dtype):
+    import deepseekternarized_amd as bp
+    from deepseekternarized_amd.kernels.ternary_hip import dense_offsets
+
+    q, s = bp.quant_act_int8(x) if act == "int8" else (x, None)
+    out = bp.grouped_ternary_gemm(q, s, dense_offsets(x.device, x.size(0)), [t.packed[None] for t in terms], [t.scale[None] for t in terms],
+                                  K, group, fmt, max_rows=x.size(0))
+    return out.to(out_dtype)
+
+
+# every decode and small-batch kernel (1 .. 16 rows), a token tile of 32 and its remainder; the general kernel (groups of 64)
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 6, 8, 9, 16, 40, 130])
+@pytest.mark.parametrize("fmt", ["tq1", "tq2"])
+@pytest.mark.parametrize("act,xdt", [("bf16", torch.bfloat16), ("int8", torch.bfloat16), ("bf16", torch.float32), ("int8", torch.float16)])
+@pytest.mark.parametrize("N,K,group,terms", [(528, 2048, 128, 1), (2048, 7168, 128, 2), (48, 200, 64, 1)])
+def test_linear_call_equals_its_steps(T, fmt, act, xdt, N, K, group, terms):
+    import deepseekternarized_amd as bp
+
+    weights, gen = _weights(fmt, N, K, group, terms, torch.float16)
+    x = torch.randn(T, K, device="cuda", generator=gen).to(xdt)
+    lin = bp.TernaryLinear(weights, K, fmt, group, act=act)
+    for out_dtype in (torch.bfloat16, torch.float32):
+        assert torch.equal(lin(x, out_dtype), _steps(x, weights, K, group, fmt, act, out_dtype)), out_dtype
+
+
+def test_linear_call_with_leading_dimensions():
+    import deepseekternarized_amd as bp
+
+    weights, gen = _weights("tq2", 256, 1024, 128, 1, torch.float16)
+    lin = bp.TernaryLinear(weights, 1024, "tq2", 128)
+    x = torch.randn(2, 3, 1024, device="cuda", generator=gen).bfloat16()
+    assert torch.equal(lin(x), lin(x.view(6, 1024)).view(2, 3, 256))
