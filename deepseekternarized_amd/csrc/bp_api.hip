@@ -183,6 +183,11 @@ extern "C" size_t bp_grouped_gemm_workspace_bytes(int x_dtype, int64_t T, int64_
   return staged_workspace_bytes(T, N, K, E, fmt, max_rows);
 }
 
+extern "C" size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows) {
+  if (fmt != BP_TQ2 || T <= 0 || E <= 0 || N <= 0 || K <= 0 || max_rows <= 16 || tuning().tq2g == 'b') return 0;
+  return tuning().tq2g == 'f' || i8w_pays(T, N, E) ? gemm_i8w_workspace_bytes(T, K, E) : 0;
+}
+
 static size_t staged_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows) {
   if (tuning().tq2g == 'b') return 0;
   // (the launcher's own thresholds, so that a call it would turn down does not make its caller allocate)
@@ -222,7 +227,7 @@ LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int6
   p.q = take(act_int8 ? (size_t)T * (size_t)K : 0);
   p.q_scale = take(act_int8 ? 4 * (size_t)T : 0);
   p.sums = take(out_dtype == BP_F32 ? 0 : 4 * (size_t)T * (size_t)N);
-  p.stage_bytes = bp_grouped_gemm_workspace_bytes(act_int8 ? BP_I8 : x_dtype, T, N, K, 1, fmt, T);
+  p.stage_bytes = act_int8 ? bp_grouped_gemm_int8_workspace_bytes(T, N, K, 1, fmt, T) : bp_grouped_gemm_workspace_bytes(x_dtype, T, N, K, 1, fmt, T);
   p.stage = take(p.stage_bytes);
   p.bytes = at;
   return p;
@@ -266,6 +271,14 @@ extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_
     return rc;
   if (empty) return BP_OK;
   uint16_t* out16 = out_dtype == BP_BF16 ? (uint16_t*)out : nullptr;
+  if (act_int8 && x_dtype == BP_BF16 && a.stage && g_policy != 1) {  // token tiles of 128: the conversion pass quantises the rows
+    GemmArgs w = a;
+    w.x_dtype = BP_BF16;
+    w.quant = 1;
+    w.overwrite = 1;
+    w.out16 = out16;
+    if (mfma_supports(a) && gemm_i8w_applies(w) == BP_OK) return launch_gemm_i8w(w, s);
+  }
   if (act_int8) {
     if (const int rc = bp_quant_act_int8((int8_t*)(ws + p.q), (float*)(ws + p.q_scale), x, x_dtype, T, K, stream)) return rc;
     a.x = ws + p.q;

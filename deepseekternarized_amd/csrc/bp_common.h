@@ -45,6 +45,7 @@ struct GemmArgs {
   // x_index[r] / x_div of x, which has x_rows rows (the routed copy of the activations is never materialised).
   const int64_t* x_index;
   int64_t x_div, x_rows;
+  int quant;  // x is bf16 and the conversion pass of the int8 kernel for 128-token tiles quantises its rows (x_scale unused)
   // bf16 out16[T, N] is written instead of float32 `out` (one launch that covers all of K and all terms; a kernel that
   // takes several passes over an output returns ERR_NO_OUT16 instead).
   uint16_t* out16;
@@ -160,6 +161,8 @@ int run_gemm(const GemmArgs& a, hipStream_t s);
 bool gemm_tiles_supported(const GemmArgs& a);
 // Workspace bytes of the TQ2 grouped GEMM over converted activations (GemmArgs::stage) for T rows in all; 0: not available.
 size_t gemm_tq2f_workspace_bytes(int64_t T, int64_t K, int64_t E);
+// ... of the int8 GEMM over token tiles of 128 rows.
+size_t gemm_i8w_workspace_bytes(int64_t T, int64_t K, int64_t E);
 int launch_general(const GemmArgs& a, hipStream_t s);
 // Returns BP_ERR_UNSUPPORTED (without setting an error message) when the shape is outside the
 // tuned kernels' preconditions.

@@ -26,6 +26,14 @@ int launch_mfma_tq1(const GemmArgs& a, hipStream_t s, int waves);
 int launch_gemm_tq2(const GemmArgs& a, hipStream_t s);
 int launch_gemm_tq2f(const GemmArgs& a, hipStream_t s);
 int gemm_tq2f_applies(const GemmArgs& a);  // BP_OK where launch_gemm_tq2f takes the call (nothing is launched)
+// bp_gemm_i8w.hip: TQ2 with int8 activations (or bf16 ones that it quantises: GemmArgs::quant) and token tiles of 128
+constexpr int I8W_TOK = 128;
+int launch_gemm_i8w(const GemmArgs& a, hipStream_t s);
+int gemm_i8w_applies(const GemmArgs& a);  // BP_OK where launch_gemm_i8w takes the call (nothing is launched)
+// Calls that run on it when the caller brings a workspace.
+inline bool i8w_pays(int64_t T, int64_t N, int64_t E) {
+  return T >= 64 * E && (T + I8W_TOK - 1) / I8W_TOK * ((N + 255) / 256) >= 192;
+}
 // bp_gemm_tq1.hip: TQ1 with token tiles of 32 on the fp8 x fp4 matrix instruction (experts with more than 8 token rows);
 // BP_ERR_UNSUPPORTED without a message when the call is outside its preconditions
 int launch_gemm_tq1(const GemmArgs& a, hipStream_t s);

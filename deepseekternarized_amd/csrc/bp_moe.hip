@@ -26,10 +26,10 @@ namespace {
 
 constexpr int TILE_ROWS = 32;  // token tile of k_gemm_tq1 / k_gemm_tq2
 
-// (expert, first row) of every 32-row token tile, in expert order; count[0] = their number. One workgroup; experts in
+// (expert, first row) of every token tile of `tile_rows` rows, in expert order; count[0] = their number. One workgroup; experts in
 // chunks of 1024 with a running total.
 __global__ __launch_bounds__(1024) void k_tile_list(int32_t* __restrict__ tiles, int32_t* __restrict__ count, const int64_t* __restrict__ offsets,
-                                                    int64_t E, int64_t T, int64_t cap) {
+                                                    int64_t E, int64_t T, int64_t cap, int tile_rows) {
   __shared__ int part[16];
   __shared__ int carry;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -43,7 +43,7 @@ __global__ __launch_bounds__(1024) void k_tile_list(int32_t* __restrict__ tiles,
       const int64_t o1 = clamp_i64(offsets[e + 1], 0, T);
       rows = o1 > o0 ? o1 - o0 : 0;
     }
-    const int mine = (int)((rows + TILE_ROWS - 1) / TILE_ROWS);
+    const int mine = (int)((rows + tile_rows - 1) / tile_rows);
     int incl = mine;  // inclusive prefix sum within the wave
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(1024) void k_tile_list(int32_t* __restrict__ tiles,
     for (int j = 0; j < mine; ++j, ++at) {
       if (at < cap) {
         tiles[2 * at] = (int32_t)e;
-        tiles[2 * at + 1] = (int32_t)(o0 + (int64_t)j * TILE_ROWS);
+        tiles[2 * at + 1] = (int32_t)(o0 + (int64_t)j * tile_rows);
       }
     }
     __syncthreads();
@@ -175,6 +175,10 @@ __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __
   for (int64_t w = gtid; w < z1_16; w += gsz) z1[w] = u32x4{0u, 0u, 0u, 0u};
 }
 
+// Layers whose two GEMMs run on the int8 kernel for token tiles of 128: int8 activations, TQ2, 128 rows per expert on average (the
+// tiles of an expert mostly full; below, the kernel for tiles of 32 computes less padding).
+bool moe_wide(int act, int fmt, int64_t n, int64_t T, int64_t E) { return act == BP_I8 && fmt == BP_TQ2 && T > 64 && n >= 128 * E; }
+
 struct Carve {
   unsigned char* base;
   size_t used;
@@ -222,6 +226,10 @@ Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k
   p.h = c.take(2 * (size_t)n * I);
   p.y = (float*)c.take(4 * (size_t)n * H);
   p.stage_bytes = 0;
+  if (moe_wide(act, fmt, n, T, E)) {
+    const size_t a = gemm_i8w_workspace_bytes(n, H, E), b = gemm_i8w_workspace_bytes(n, I, E);
+    p.stage_bytes = a > b ? a : b;
+  }
   if (act == BP_BF16) {
     const size_t a = gemm_tq2f_workspace_bytes(n, H, E), b = gemm_tq2f_workspace_bytes(n, I, E);
     p.stage_bytes = a > b ? a : b;
@@ -310,6 +318,32 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     }
     fuse = gemm_tiles_supported(a) && gemm_tq2f_applies(a) == BP_OK;
   }
+  // The same for int8 activations where experts have many rows each: the token rows are quantised once and the conversion
+  // pass of either GEMM gathers or quantises its rows; gate | up applies SwiGLU and the down projection writes bf16 rows.
+  GemmArgs wide_gu, wide_down;
+  bool wide = false;
+  if (moe_wide(act, fmt, n, T, E) && tiles && !small && aligned16 && kernel_policy() != 1 && tuning().glu != 'n' && tuning().tq2g != 'b') {
+    memset(&wide_gu, 0, sizeof(wide_gu));
+    GemmArgs& a = wide_gu;
+    a.offsets = p.offsets; a.x_dtype = BP_I8; a.scale_dtype = scale_dtype; a.n_terms = n_terms; a.fmt = fmt; a.group = group;
+    a.T = n; a.E = E; a.max_rows = I8W_TOK; a.overwrite = 1;
+    a.stage = p.stage; a.stage_bytes = (int64_t)p.stage_bytes;
+    a.tiles = p.tiles; a.tile_count = p.tile_count; a.tile_cap = (n + I8W_TOK - 1) / I8W_TOK + E;
+    wide_down = a;
+    for (int t = 0; t < n_terms; ++t) { a.packed[t] = gate_up_packed[t]; a.w_scale[t] = gate_up_scale[t]; }
+    a.x = p.q; a.x_scale = p.q_scale; a.x_index = p.order; a.x_div = k; a.x_rows = T;
+    a.N = 2 * I; a.K = H; a.Kp = (H + per - 1) / per; a.G = (H + group - 1) / group;
+    a.glu_h = (uint16_t*)p.h; a.glu_v4 = v4 ? 1 : 0; a.glu_limit = limit;
+    a.glu_weights = v4 ? (const float*)weights : nullptr; a.glu_order = p.order; a.glu_pairs = n;
+    GemmArgs& d = wide_down;
+    for (int t = 0; t < n_terms; ++t) { d.packed[t] = down_packed[t]; d.w_scale[t] = down_scale[t]; }
+    d.x = p.h; d.x_dtype = BP_BF16; d.quant = 1;
+    d.N = H; d.K = I; d.Kp = (I + per - 1) / per; d.G = (I + group - 1) / group;
+    d.out16 = (uint16_t*)p.y;
+    GemmArgs probe = d;  // (mfma_supports knows the product's own activation type)
+    probe.x_dtype = BP_I8;
+    wide = mfma_supports(a) && mfma_supports(probe) && gemm_i8w_applies(a) == BP_OK && gemm_i8w_applies(d) == BP_OK;
+  }
   if (small) {
     const int64_t z0 = prezeroed ? (int64_t)(4 * (size_t)n * 2 * I / 16) : 0, z1 = prezeroed ? (int64_t)(4 * (size_t)n * H / 16) : 0;
     const int64_t row16 = fuse && fused.x_index ? 0 : H / 8;  // (no rows to copy where the gate | up launch reads them through `order`)
@@ -321,7 +355,9 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     if ((rc = check_launch("route_small")) != BP_OK) return rc;
   } else {
     if ((rc = sort_with_inverse(p.order, p.offsets, p.inv, experts, n, E, p.sort_ws, bad, s)) != BP_OK) return rc;
-    if (fuse && fused.x_index) {
+    if (wide) {
+      if ((rc = bp_quant_act_int8(p.q, p.q_scale, x, BP_BF16, T, H, s)) != BP_OK) return rc;
+    } else if (fuse && fused.x_index) {
       // (no routed copy of the activations: the gate | up launch's conversion pass reads them through `order`)
     } else if (aligned16) {
       const int64_t z0 = prezeroed ? (int64_t)(4 * (size_t)n * 2 * I / 16) : 0, z1 = prezeroed ? (int64_t)(4 * (size_t)n * H / 16) : 0;
@@ -379,8 +415,14 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     return run_gemm(a, s);
   };
   if (tiles && !small) {
-    hipLaunchKernelGGL(k_tile_list, dim3(1), dim3(1024), 0, s, p.tiles, p.tile_count, p.offsets, E, n, p.tile_cap);
+    hipLaunchKernelGGL(k_tile_list, dim3(1), dim3(1024), 0, s, p.tiles, p.tile_count, p.offsets, E, n, p.tile_cap, wide ? I8W_TOK : TILE_ROWS);
     if ((rc = check_launch("tile_list")) != BP_OK) return rc;
+  }
+  if (wide) {
+    if ((rc = launch_gemm_i8w(wide_gu, s)) != BP_OK || (rc = launch_gemm_i8w(wide_down, s)) != BP_OK) return rc;
+    note_kernel_suffix("+glu+gather+y16");
+    if (v4) return moe_combine_v4(out, out_dtype, p.y, true, p.inv, experts, T, k, H, s);
+    return moe_combine(out, p.y, true, p.inv, weights, experts, T, k, H, s);
   }
   if (fuse) {
     rc = launch_gemm_tq2f(fused, s);

@@ -96,7 +96,9 @@ class _HipTernary:
             # fp16 activations run on the bf16 kernels as a pair. The size query answers 0 where the launch would not use
             # one (small calls, a loose max_rows); decode-sized bf16 / int8 calls never do and skip the query.
             need = 0
-            if max_rows > _DECODE_ROWS or xdt in (_lib.BP_F16, _lib.BP_F32):
+            if max_rows > 16 and xdt == _lib.BP_I8:
+                need = self.lib.bp_grouped_gemm_int8_workspace_bytes(T, N, int(K), E, int(fmt), int(max_rows))
+            elif xdt != _lib.BP_I8 and (max_rows > _DECODE_ROWS or xdt != _lib.BP_BF16):
                 need = self.lib.bp_grouped_gemm_workspace_bytes(xdt, T, N, int(K), E, int(fmt), int(max_rows))
             if need > _WORKSPACE_CAP:  # (up to 2.1 bytes per activation: a call this large keeps its memory and runs the kernels without one)
                 need = 0

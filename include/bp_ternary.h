@@ -95,6 +95,9 @@ int bp_ternary_grouped_gemm(float* out, const void* x, int x_dtype, const float*
  * runs on them as well: the activations are split into a bf16 pair x = hi + lo (exact for fp16, to 2^-17 |x| for float32)
  * and both products are added into out. Without one they run on the general kernel. */
 size_t bp_grouped_gemm_workspace_bytes(int x_dtype, int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows);
+/* The same for int8 activations and TQ2: the workspace of the kernel for token tiles of 128 rows (large calls with at least
+ * 64 rows per expert on average), 0 where bp_ternary_grouped_gemm_ws would not use one. */
+size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows);
 int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype, const float* x_scale,
                                const int64_t* offsets, const int64_t* offsets_host,
                                const uint8_t* const* packed, const void* const* w_scale, int scale_dtype,
