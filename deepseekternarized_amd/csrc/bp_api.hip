@@ -218,10 +218,16 @@ extern "C" int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype
 namespace bp {
 namespace {
 struct LinearPlan {  // offsets into the workspace
-  size_t q, q_scale, sums, stage, stage_bytes, bytes;
+  size_t q, q_scale, sums, stage, stage_bytes, repacked, bytes;
+  bool repack;  // TQ1 weights are rewritten as TQ2 ones first
 };
+// TQ1 linears of this many tokens and more rewrite their weights as TQ2 ones, which the token-tile kernels decode faster.
+constexpr int64_t REPACK_TOKENS = 256;
+size_t repacked_bytes(int64_t N, int64_t K) { return ((size_t)N * (size_t)(K / 4) + 255) & ~(size_t)255; }
 LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int fmt, int n_terms) {
   LinearPlan p;
+  p.repack = fmt == BP_TQ1 && T >= REPACK_TOKENS && K % 256 == 0 && K >= 1024 && K <= 65536 && tuning().tq2g != 'b';
+  if (p.repack) fmt = BP_TQ2;
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) & ~(size_t)255; return o; };
   p.q = take(act_int8 ? (size_t)T * (size_t)K : 0);
@@ -229,6 +235,7 @@ LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int6
   p.sums = take(out_dtype == BP_F32 ? 0 : 4 * (size_t)T * (size_t)N);
   p.stage_bytes = act_int8 ? bp_grouped_gemm_int8_workspace_bytes(T, N, K, 1, fmt, T) : bp_grouped_gemm_workspace_bytes(x_dtype, T, N, K, 1, fmt, T);
   p.stage = take(p.stage_bytes);
+  p.repacked = take(p.repack ? (size_t)n_terms * repacked_bytes(N, K) : 0);
   p.bytes = at;
   return p;
 }
@@ -271,6 +278,19 @@ extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_
     return rc;
   if (empty) return BP_OK;
   uint16_t* out16 = out_dtype == BP_BF16 ? (uint16_t*)out : nullptr;
+  if (p.repack && g_policy != 1) {
+    GemmArgs b = a;
+    b.fmt = BP_TQ2;
+    b.Kp = K / 4;
+    for (int t = 0; t < n_terms; ++t) b.packed[t] = ws + p.repacked + (size_t)t * repacked_bytes(N, K);
+    GemmArgs probe = b;  // (float32 / fp16 activations run as a bf16 pair)
+    if (!act_int8) probe.x_dtype = BP_BF16;
+    if (mfma_supports(probe)) {
+      for (int t = 0; t < n_terms; ++t)
+        if (const int rc = launch_tq1_to_tq2(const_cast<uint8_t*>(b.packed[t]), a.packed[t], N, K, s)) return rc;
+      a = b;
+    }
+  }
   if (act_int8 && x_dtype == BP_BF16 && a.stage && g_policy != 1) {  // token tiles of 128: the conversion pass quantises the rows
     GemmArgs w = a;
     w.x_dtype = BP_BF16;

@@ -164,6 +164,8 @@ size_t gemm_tq2f_workspace_bytes(int64_t T, int64_t K, int64_t E);
 // ... of the int8 GEMM over token tiles of 128 rows.
 size_t gemm_i8w_workspace_bytes(int64_t T, int64_t K, int64_t E);
 int launch_general(const GemmArgs& a, hipStream_t s);
+// bp_repack.hip: TQ1 rows as TQ2 rows
+int launch_tq1_to_tq2(uint8_t* out, const uint8_t* in, int64_t rows, int64_t K, hipStream_t s);
 // Returns BP_ERR_UNSUPPORTED (without setting an error message) when the shape is outside the
 // tuned kernels' preconditions.
 int launch_mfma(const GemmArgs& a, hipStream_t s);
