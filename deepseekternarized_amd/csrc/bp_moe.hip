@@ -18,6 +18,7 @@ namespace bp {
 int kernel_policy();  // bp_api.hip
 int sort_with_inverse(int64_t* order, int64_t* offsets, int64_t* inv, const int64_t* ids, int64_t n, int64_t E, int32_t* workspace,
                       int32_t* bad, hipStream_t stream);  // bp_route.hip
+int64_t sort_with_inverse_ints(int64_t n, int64_t E);  // its workspace
 int moe_combine(void* out, const void* y, bool y16, const int64_t* inv, const void* w, const int64_t* experts, int64_t T, int64_t k, int64_t H,
                 void* stream);  // bp_route.hip
 int moe_combine_v4(void* out, int out_dtype, const void* y, bool y16, const int64_t* inv, const int64_t* experts, int64_t T, int64_t k, int64_t H,
@@ -215,7 +216,7 @@ Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k
   p.order = (int64_t*)c.take(8 * (size_t)n);
   p.offsets = (int64_t*)c.take(8 * (size_t)(E + 1));
   p.inv = (int64_t*)c.take(8 * (size_t)n);
-  p.sort_ws = (int32_t*)c.take(4 * (size_t)bp_sort_workspace_ints(n, E));
+  p.sort_ws = (int32_t*)c.take(4 * (size_t)sort_with_inverse_ints(n, E));
   p.tile_cap = (n + TILE_ROWS - 1) / TILE_ROWS + E;
   p.tiles = (int32_t*)c.take(8 * (size_t)p.tile_cap);
   p.tile_count = (int32_t*)c.take(4);

@@ -2,6 +2,7 @@
 // row gather (the x[order // k] permute), and the two elementwise stages of an expert MLP
 // (SwiGLU, weighted combine) with the reference engine's bf16 rounding points.
 #include <mutex>
+#include <type_traits>
 
 #include "bp_common.h"
 
@@ -113,6 +114,82 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort(int64_t* __restrict__ ord
   }
 }
 
+// Many ids (a prompt's routing): the same sort over workgroups of 1024 ids, in two launches - one workgroup alone takes
+// 81 us for 65,536 ids and 26 for 12,288. k_sort_count leaves every block's histogram in ws[block][E]; in k_sort_place every
+// block adds up the histograms of all blocks (the experts' first slots) and of the blocks before it, ranks its ids - a
+// wave's 64 by ballots as in k_sort, the waves through their counts in LDS - and writes them.
+constexpr int SORT_BLOCK = 1024;
+constexpr int64_t SORT_BLOCKS_FROM = 4096;  // ids from which the two launches win
+constexpr int64_t SORT_BLOCKS_MAX_E = 512;  // (k_sort_place: 64 bytes of LDS per expert)
+__global__ __launch_bounds__(SORT_BLOCK) void k_sort_count(const int64_t* __restrict__ ids, int64_t n, int E, int32_t* __restrict__ ws, int32_t* __restrict__ bad) {
+  __shared__ int32_t hist[SORT_BLOCKS_MAX_E];
+  if ((int)threadIdx.x < E) hist[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t i = (int64_t)blockIdx.x * SORT_BLOCK + threadIdx.x;
+  if (i < n) {
+    const int64_t id = ids[i];
+    if (id >= 0 && id < E) atomicAdd(&hist[id], 1);
+    else if (bad) *bad = 1;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < E) ws[(int64_t)blockIdx.x * E + threadIdx.x] = hist[threadIdx.x];
+}
+__global__ __launch_bounds__(SORT_BLOCK) void k_sort_place(int64_t* __restrict__ order, int64_t* __restrict__ offsets, const int64_t* __restrict__ ids, int64_t n,
+                                                           int E, const int32_t* __restrict__ ws, int64_t* __restrict__ inv) {
+  extern __shared__ int32_t slots[];  // [SORT_WAVES][E]: a wave's counts, then its first slot of every expert
+  __shared__ int32_t wave_total[SORT_WAVES];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, e = threadIdx.x;
+  const int64_t i = (int64_t)blockIdx.x * SORT_BLOCK + threadIdx.x;
+  const int64_t id = i < n ? ids[i] : -1;
+  const bool todo = id >= 0 && id < E;
+  for (int j = threadIdx.x; j < SORT_WAVES * E; j += SORT_BLOCK) slots[j] = 0;
+  int32_t all = 0, before = 0;  // expert e's ids in all blocks and in those before this one
+  if (e < E) {
+#pragma unroll 8
+    for (int b = 0; b < (int)gridDim.x; ++b) {
+      const int32_t c = ws[(int64_t)b * E + e];
+      all += c;
+      before += b < (int)blockIdx.x ? c : 0;
+    }
+  }
+  int32_t incl = all;  // inclusive prefix sum over the experts
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t up = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += up;
+  }
+  if (lane == 63) wave_total[wave] = incl;
+  int nbits = 1;
+  while ((1 << nbits) < E) ++nbits;
+  unsigned long long same = __ballot(todo);
+  for (int bit = 0; bit < nbits; ++bit) {
+    const unsigned long long set = __ballot(todo && ((id >> bit) & 1));
+    same &= ((id >> bit) & 1) ? set : ~set;
+  }
+  __syncthreads();
+  if (todo && lane == __ffsll((long long)same) - 1) slots[wave * E + id] = (int32_t)__popcll(same);
+  for (int w = 0; w < wave; ++w) incl += wave_total[w];
+  __syncthreads();
+  if (e < E) {
+    if (blockIdx.x == 0) {
+      offsets[e] = incl - all;
+      if (e == E - 1) offsets[E] = incl;
+    }
+    int32_t run = incl - all + before;
+    for (int w = 0; w < SORT_WAVES; ++w) {
+      const int32_t c = slots[w * E + e];
+      slots[w * E + e] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+  if (todo) {
+    const int64_t slot = (int64_t)slots[wave * E + id] + __popcll(same & ((1ull << lane) - 1ull));
+    order[slot] = i;
+    if (inv) inv[i] = slot;
+  }
+}
+
 // Few ids (n <= SORT_SMALL_N = 128): one pass, no histograms. Element i goes to slot #(valid ids below id_i) + #(equal ids
 // before i) - the stable order - and offsets[e] = #(valid ids below e); every thread scans the ids held in LDS
 // (a broadcast read per step). Decode batches sort a few dozen ids: this takes a quarter of the general kernel's time.
@@ -211,6 +288,67 @@ __global__ __launch_bounds__(256) void k_swiglu4(uint16_t* __restrict__ h, const
 // every thread reads its 4 columns of all k rows (independent loads) and accumulates them in that order.
 // Y16: the rows of y are bf16 already (the down projection rounded them itself: the rounding the sum starts with).
 constexpr int COMBINE_COLS = 1024;
+// Rows whose column count is a multiple of 8: eight columns per thread (16-byte loads of bf16 rows), 2048 per workgroup.
+constexpr int COMBINE8_COLS = 2048;
+template <bool V4 /* float32 sums, no routing weights */, bool OUT_BF16, bool Y16>
+__global__ __launch_bounds__(256) void k_combine8(void* __restrict__ out, const void* __restrict__ y, const int64_t* __restrict__ inv,
+                                                  const uint16_t* __restrict__ w, const int64_t* __restrict__ experts, int k, int64_t H) {
+  const int64_t t = blockIdx.x;
+  __shared__ int64_t row_of[64];
+  __shared__ float weight_of[64];
+  if (threadIdx.x < 64) {  // the first wave: slot = lane, its place in ascending expert order (ties: slot order) by rank
+    const int sl = threadIdx.x;
+    const int64_t mine = sl < k ? experts[t * k + sl] : 0;
+    const int64_t row = sl < k ? clamp_i64(inv[t * k + sl], 0, (int64_t)gridDim.x * k - 1) : 0;
+    const float ws = !V4 && sl < k ? bf16_bits_to_f32(w[t * k + sl]) : 1.f;
+    int rank = 0;
+    for (int j = 0; j < k; ++j) {
+      const int64_t other = __shfl(mine, j, 64);
+      rank += (other < mine || (other == mine && j < sl)) ? 1 : 0;
+    }
+    if (sl < k) {
+      row_of[rank] = row;
+      weight_of[rank] = ws;
+    }
+  }
+  __syncthreads();
+  const int64_t c0 = (int64_t)blockIdx.y * COMBINE8_COLS + 8 * threadIdx.x;
+  if (c0 >= H) return;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < k; s0 += 4) {  // four rows on their way at a time
+    uint4 v[4][Y16 ? 1 : 2];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int64_t at = row_of[s0 + s < k ? s0 + s : k - 1] * H + c0;
+      if (Y16) {
+        v[s][0] = *(const uint4*)((const uint16_t*)y + at);
+      } else {
+        v[s][0] = *(const uint4*)((const float*)y + at);
+        v[s][Y16 ? 0 : 1] = *(const uint4*)((const float*)y + at + 4);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      if (s0 + s >= k) break;
+      const float ws = weight_of[s0 + s];
+      const unsigned b[8] = {v[s][0].x, v[s][0].y, v[s][0].z, v[s][0].w, v[s][Y16 ? 0 : 1].x, v[s][Y16 ? 0 : 1].y, v[s][Y16 ? 0 : 1].z, v[s][Y16 ? 0 : 1].w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float e = Y16 ? __uint_as_float((i & 1) ? (b[i >> 1] & 0xffff0000u) : (b[i >> 1] << 16)) : round_bf16(__uint_as_float(b[i]));
+        acc[i] = V4 ? acc[i] + e : round_bf16(acc[i] + round_bf16(e * ws));
+      }
+    }
+  }
+  if (OUT_BF16) {
+    unsigned o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (unsigned)f32_to_bf16_bits(acc[2 * i]) | ((unsigned)f32_to_bf16_bits(acc[2 * i + 1]) << 16);
+    *(uint4*)((uint16_t*)out + t * H + c0) = make_uint4(o[0], o[1], o[2], o[3]);
+  } else {
+    *(float4*)((float*)out + t * H + c0) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    *(float4*)((float*)out + t * H + c0 + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+  }
+}
 template <bool Y16>
 __global__ __launch_bounds__(256) void k_combine(uint16_t* __restrict__ out, const float* __restrict__ y,
                                                  const int64_t* __restrict__ inv, const uint16_t* __restrict__ w,
@@ -353,6 +491,31 @@ __global__ __launch_bounds__(256) void k_check_rows(int32_t* __restrict__ flag, 
 // rounds of a wave arg-max over (score, expert) with ties to the lower expert, the winner's entry taken out after each:
 // the slots come out in descending score like torch.topk's. `renorm`: the k scores are divided by their sum
 // (norm_topk_prob) before they are rounded to the output dtype.
+// A wave's butterflies stay in the vector ALU (a shuffle through the LDS pipeline has several times the latency, and a
+// round of the arg-max is six of them in a row): lane + 32 and lane + 16 by register swaps, then rotations within a row of
+// 16 - after each step the values repeat with half the period, so a rotation by 8, 4, 2, 1 meets the same value as lane ^ 8 ...
+struct LanePair { unsigned a, b; };
+template <int STEP>
+__device__ __forceinline__ LanePair lane_pair(unsigned v) {  // the lane's value and its partner's, in either order
+  if constexpr (STEP == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return {r[0], r[1]};
+  } else if constexpr (STEP == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return {r[0], r[1]};
+  } else {
+    return {v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + STEP /* row_ror */, 0xf, 0xf, false)};
+  }
+}
+template <class F>
+__device__ __forceinline__ void butterfly(F&& f) {
+  f(std::integral_constant<int, 32>{});
+  f(std::integral_constant<int, 16>{});
+  f(std::integral_constant<int, 8>{});
+  f(std::integral_constant<int, 4>{});
+  f(std::integral_constant<int, 2>{});
+  f(std::integral_constant<int, 1>{});
+}
 constexpr int ROUTE_PER_LANE = 16;  // experts per lane at most: up to 1024 experts
 template <int LDT, bool W_BF16, int PER /* experts per lane: E <= 64 PER */>
 __global__ __launch_bounds__(256) void k_route_topk(void* __restrict__ weights, int64_t* __restrict__ experts, const void* __restrict__ logits,
@@ -368,16 +531,20 @@ __global__ __launch_bounds__(256) void k_route_topk(void* __restrict__ weights, 
     sc[j] = e < E ? load_act_f32(logits, LDT, t * E + e) : -INFINITY;
     mx = fmaxf(mx, sc[j]);
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+  butterfly([&](auto step) {
+    const LanePair p = lane_pair<decltype(step)::value>(__float_as_uint(mx));
+    mx = fmaxf(__uint_as_float(p.a), __uint_as_float(p.b));
+  });
   float sum = 0.f;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     sc[j] = lane + 64 * j < E ? expf(sc[j] - mx) : 0.f;
     sum += sc[j];
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  butterfly([&](auto step) {
+    const LanePair p = lane_pair<decltype(step)::value>(__float_as_uint(sum));
+    sum = __uint_as_float(p.a) + __uint_as_float(p.b);
+  });
 #pragma unroll
   for (int j = 0; j < PER; ++j) sc[j] = lane + 64 * j < E ? sc[j] / sum : -1.f;  // (scores are >= 0: -1 marks "no expert")
   float mine = 0.f;  // lane s keeps the score of slot s
@@ -389,12 +556,13 @@ __global__ __launch_bounds__(256) void k_route_topk(void* __restrict__ weights, 
 #pragma unroll
     for (int j = 0; j < PER; ++j)  // (ascending expert: a later equal score does not replace an earlier one)
       if (sc[j] > best) { best = sc[j]; best_e = lane + 64 * j; }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(best, off, 64);
-      const int oe = __shfl_xor(best_e, off, 64);
-      if (ov > best || (ov == best && oe < best_e)) { best = ov; best_e = oe; }
-    }
+    butterfly([&](auto step) {
+      const LanePair v = lane_pair<decltype(step)::value>(__float_as_uint(best)), x = lane_pair<decltype(step)::value>((unsigned)best_e);
+      const float va = __uint_as_float(v.a), vb = __uint_as_float(v.b);
+      const bool b = vb > va || (vb == va && (int)x.b < (int)x.a);
+      best = b ? vb : va;
+      best_e = (int)(b ? x.b : x.a);
+    });
     if ((best_e & 63) == lane) {  // the winner leaves its lane's list
 #pragma unroll
       for (int j = 0; j < PER; ++j)
@@ -435,8 +603,18 @@ static int launch_sort(int64_t* order, int64_t* offsets, const int64_t* ids, int
 
 namespace bp {
 // bp_sort_by_expert that also writes the inverse permutation (the MoE layer's preparation; arguments checked by its caller)
+// Its workspace: bp_sort_workspace_ints, or the blocks' histograms where those sort.
+static bool sort_in_blocks(int64_t n, int64_t E) { return n >= SORT_BLOCKS_FROM && E > 0 && E <= SORT_BLOCKS_MAX_E; }
+int64_t sort_with_inverse_ints(int64_t n, int64_t E) { return sort_in_blocks(n, E) ? (n + SORT_BLOCK - 1) / SORT_BLOCK * E : bp_sort_workspace_ints(n, E); }
 int sort_with_inverse(int64_t* order, int64_t* offsets, int64_t* inv, const int64_t* ids, int64_t n, int64_t E, int32_t* workspace,
                       int32_t* bad, hipStream_t stream) {
+  if (sort_in_blocks(n, E)) {
+    const unsigned blocks = (unsigned)((n + SORT_BLOCK - 1) / SORT_BLOCK);
+    hipLaunchKernelGGL(k_sort_count, dim3(blocks), dim3(SORT_BLOCK), 0, stream, ids, n, (int)E, workspace, bad);
+    if (const int rc = check_launch("sort_count")) return rc;
+    hipLaunchKernelGGL(k_sort_place, dim3(blocks), dim3(SORT_BLOCK), (size_t)(SORT_WAVES * E) * sizeof(int32_t), stream, order, offsets, ids, n, (int)E, workspace, inv);
+    return check_launch("sort_place");
+  }
   return launch_sort(order, offsets, ids, n, E, bp_sort_workspace_ints(n, E) > 0 ? workspace : (int32_t*)nullptr, bad, stream, inv);
 }
 }  // namespace bp
@@ -503,6 +681,8 @@ extern "C" int bp_swiglu_bf16(void* h, const float* gate, const float* up, int64
 }
 
 namespace bp {
+// (whole 16-byte pieces of every row)
+static bool combine8(const void* out, const void* y, int64_t H) { return H % 8 == 0 && (((uintptr_t)out | (uintptr_t)y) & 15) == 0; }
 // the two combines with rows of y that are float32 (the entry points) or bf16 already (y16: bp_moe_layer_* after a down
 // projection that wrote bf16)
 int moe_combine(void* out, const void* y, bool y16, const int64_t* inv, const void* w, const int64_t* experts, int64_t T, int64_t k, int64_t H,
@@ -510,6 +690,12 @@ int moe_combine(void* out, const void* y, bool y16, const int64_t* inv, const vo
   if (T < 0 || k <= 0 || k > 64 || H <= 0 || T > 0x7fffffff) return fail(BP_ERR_ARG, "invalid combine dimensions (top-k up to 64)");
   if (T == 0) return BP_OK;
   if (!out || !y || !inv || !w || !experts) return fail(BP_ERR_ARG, "null pointer");
+  if (combine8(out, y, H)) {
+    const dim3 grid8((unsigned)T, (unsigned)((H + COMBINE8_COLS - 1) / COMBINE8_COLS));
+    if (y16) hipLaunchKernelGGL((k_combine8<false, true, true>), grid8, dim3(256), 0, (hipStream_t)stream, out, y, inv, (const uint16_t*)w, experts, (int)k, H);
+    else hipLaunchKernelGGL((k_combine8<false, true, false>), grid8, dim3(256), 0, (hipStream_t)stream, out, y, inv, (const uint16_t*)w, experts, (int)k, H);
+    return check_launch("moe_combine");
+  }
   const dim3 grid((unsigned)T, (unsigned)((H + COMBINE_COLS - 1) / COMBINE_COLS));
   if (y16) hipLaunchKernelGGL(k_combine<true>, grid, dim3(256), 0, (hipStream_t)stream, (uint16_t*)out, (const float*)y, inv, (const uint16_t*)w, experts, k, H);
   else hipLaunchKernelGGL(k_combine<false>, grid, dim3(256), 0, (hipStream_t)stream, (uint16_t*)out, (const float*)y, inv, (const uint16_t*)w, experts, k, H);
@@ -525,6 +711,19 @@ int moe_combine_v4(void* out, int out_dtype, const void* y, bool y16, const int6
   const dim3 grid((unsigned)T, (unsigned)((H + COMBINE_COLS - 1) / COMBINE_COLS));
   const float* yf = (const float*)y;
   const hipStream_t s = (hipStream_t)stream;
+  if (combine8(out, y, H)) {
+    const dim3 grid8((unsigned)T, (unsigned)((H + COMBINE8_COLS - 1) / COMBINE8_COLS));
+#define BP_C8(OUT, Y) hipLaunchKernelGGL((k_combine8<true, OUT, Y>), grid8, dim3(256), 0, s, out, y, inv, (const uint16_t*)nullptr, experts, (int)k, H)
+    if (out_dtype == BP_BF16) {
+      if (y16) BP_C8(true, true);
+      else BP_C8(true, false);
+    } else {
+      if (y16) BP_C8(false, true);
+      else BP_C8(false, false);
+    }
+#undef BP_C8
+    return check_launch("moe_combine_v4");
+  }
   if (out_dtype == BP_BF16) {
     if (y16) hipLaunchKernelGGL((k_combine_v4<true, true>), grid, dim3(256), 0, s, out, yf, inv, experts, k, H);
     else hipLaunchKernelGGL((k_combine_v4<true, false>), grid, dim3(256), 0, s, out, yf, inv, experts, k, H);
