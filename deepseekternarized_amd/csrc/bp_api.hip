@@ -213,8 +213,8 @@ extern "C" int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype
 
 // ---- one dense linear from its float activations to its output rows, in one call: the quantisation to int8 (act_int8),
 // the product, the rounding to bf16. The kernels write bf16 rows themselves where they can (GemmArgs::out16), so that the
-// usual call is one launch, or two with the quantisation; a zero-fill, a product that adds to float32 rows and a rounding
-// pass are left for the calls in which a kernel takes several passes over an output.
+// usual call is one launch, or two with the quantisation; float32 rows and a rounding pass are left for the calls in which a
+// kernel takes several passes over an output.
 namespace bp {
 namespace {
 struct LinearPlan {  // offsets into the workspace
@@ -240,9 +240,6 @@ LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int6
   return p;
 }
 
-__global__ __launch_bounds__(256) void k_zero4(float* __restrict__ p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0.f;
-}
 __global__ __launch_bounds__(256) void k_round_bf16(uint16_t* __restrict__ out, const float* __restrict__ in, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) out[i] = f32_to_bf16_bits(in[i]);
 }
@@ -309,11 +306,9 @@ extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_
     const int rc = run_gemm(a, s);
     if (rc != ERR_NO_OUT16) return rc;
     a.out16 = nullptr;
-    a.overwrite = 0;
     a.out = (float*)(ws + p.sums);
   }
-  hipLaunchKernelGGL(k_zero4, dim3(fill_grid(T * N)), dim3(256), 0, s, a.out, T * N);
-  if (const int rc = check_launch("zero")) return rc;
+  a.overwrite = 1;
   if (const int rc = run_gemm(a, s)) return rc;
   if (!out16) return BP_OK;
   hipLaunchKernelGGL(k_round_bf16, dim3(fill_grid(T * N)), dim3(256), 0, s, out16, a.out, T * N);
@@ -389,6 +384,7 @@ int run_gemm(const GemmArgs& a, hipStream_t s) {
     b.x = hi;
     if (const int rc = run_gemm(b, s)) return rc;
     b.x = lo;
+    b.overwrite = 0;
     return run_gemm(b, s);
   }
   if (g_policy != 1 && mfma_supports(a)) {

@@ -175,9 +175,12 @@ bool mfma_supports(const GemmArgs& a);
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
 
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {  // round to nearest even, NaN kept quiet
-  const uint32_t u = __float_as_uint(f);
-  const uint32_t rounded = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16, quiet = (u >> 16) | 0x0040u;
-  return (uint16_t)(f != f ? quiet : rounded);  // (a select: epilogues convert dozens of values per lane)
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_bit_cast(uint16_t, (__bf16)f);  // v_cvt_pk_bf16_f32: one instruction, the same bits for every float32 value
+#else
+  const uint32_t u = __builtin_bit_cast(uint32_t, f);
+  return (uint16_t)(f != f ? (u >> 16) | 0x0040u : (u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+#endif
 }
 
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t b) {
@@ -189,6 +192,21 @@ __device__ __forceinline__ float load_scale(const void* p, int dtype, int64_t i)
   if (dtype == BP_F32) return ((const float*)p)[i];
   const uint16_t b = ((const uint16_t*)p)[i];
   return dtype == BP_F16 ? f16_bits_to_f32(b) : bf16_bits_to_f32(b);
+}
+
+// SwiGLU of one pair of gate and up sums with the rounding points of bp_swiglu_bf16 or (V4) of bp_swiglu_v4, as bf16 bits.
+template <bool V4>
+__device__ __forceinline__ uint16_t swiglu_bits(float gate, float up, bool weighted, float weight, float limit) {
+  float g = bf16_bits_to_f32(f32_to_bf16_bits(gate)), u = bf16_bits_to_f32(f32_to_bf16_bits(up));
+  if (V4) {
+    if (limit > 0.f) {  // torch.clamp: a NaN stays a NaN
+      u = u < -limit ? -limit : (u > limit ? limit : u);
+      g = g > limit ? limit : g;
+    }
+    const float v = (g / (1.0f + expf(-g))) * u;
+    return f32_to_bf16_bits(weighted ? weight * v : v);
+  }
+  return f32_to_bf16_bits(bf16_bits_to_f32(f32_to_bf16_bits(g / (1.0f + expf(-g)))) * u);
 }
 
 // One finished output: bf16 in place of the float32 one, or the float32 one replaced or added to.

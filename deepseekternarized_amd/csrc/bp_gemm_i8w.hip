@@ -14,7 +14,8 @@
 // The activations are laid out beforehand (k_stage_i8w): the KiB that a wave reads as operand A of one instruction is
 // contiguous in lane order, every 16 of its bytes are transposed to the decode's code order, and the group sums that take
 // the codes' offset off again are made there, so that the GEMM only copies them to LDS (two windows of 256 k, one barrier
-// per window). The pass also gathers routed rows through an index, and quantises bf16 rows on the way (the arithmetic of
+// per window). 8192 x 2048 x 6144: 441 us on the 32-token tiles; this kernel 252 with the compiler's own schedule, 185 with the
+// interleaving of k_gemm_i8w pinned, 157 (1.31 Pop/s) with two small workgroups per CU and the epilogue through LDS. The pass also gathers routed rows through an index, and quantises bf16 rows on the way (the arithmetic of
 // bp_quant_act_int8), which saves the routed copy of the activations and the int8 rows.
 #include <type_traits>
 
@@ -48,8 +49,9 @@ __device__ __forceinline__ unsigned char* staged_tile(const GemmArgs& a, int64_t
 // ---- the conversion: one workgroup per 16 tokens of a token tile. Wave = every eighth group; lane = (token t of 16,
 // quarter q of the group): the 16-element units 2 q and 2 q + 1, which instructions 0 and 1 take in lane block kb.
 // SRC = BP_I8: rows and their scales are copied. SRC = BP_BF16: a row is quantised, operation for operation as k_quant16.
-constexpr int W_KEEP = 4;  // groups per wave whose bf16 activations stay in registers between the two passes (K <= 4096)
-template <int SRC>
+// KEEP: groups per wave whose bf16 activations stay in registers between the two passes (K up to 1024 KEEP; more are read
+// again), no more than K needs: at K = 1024, 4 of them left room for one workgroup per CU (116 us for 65,536 rows).
+template <int SRC, int KEEP>
 __global__ __launch_bounds__(W_THREADS) void k_stage_i8w(GemmArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const TileRef tr = tile_ref<W_TOK>(a, blockIdx.x, blockIdx.z);
@@ -93,7 +95,7 @@ __global__ __launch_bounds__(W_THREADS) void k_stage_i8w(GemmArgs a) {
     if (g < groups) put(g, xp[8 * g], xp[8 * g + 1]);
   } else {
     const u32x4* xp = (const u32x4*)((const uint16_t*)a.x + src * a.K) + 4 * q;
-    u32x4 kept[W_KEEP][4];
+    u32x4 kept[KEEP][4];
     float amax = 0.f;
     bool nan = false;
     auto look = [&](const u32x4& v) {
@@ -105,16 +107,16 @@ __global__ __launch_bounds__(W_THREADS) void k_stage_i8w(GemmArgs a) {
       }
     };
 #pragma unroll
-    for (int i = 0; i < W_KEEP; ++i) {
+    for (int i = 0; i < KEEP; ++i) {
       const int g = wave + i * W_WAVES;
 #pragma unroll
       for (int d = 0; d < 4; ++d) kept[i][d] = g < groups ? xp[16 * g + d] : u32x4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
-    for (int i = 0; i < W_KEEP; ++i)
+    for (int i = 0; i < KEEP; ++i)
 #pragma unroll
       for (int d = 0; d < 4; ++d) look(kept[i][d]);
-    for (int g = wave + W_KEEP * W_WAVES; g < groups; g += W_WAVES)
+    for (int g = wave + KEEP * W_WAVES; g < groups; g += W_WAVES)
 #pragma unroll
       for (int d = 0; d < 4; ++d) look(xp[16 * g + d]);
     if (nan) amax = __builtin_nanf("");
@@ -152,9 +154,9 @@ __global__ __launch_bounds__(W_THREADS) void k_stage_i8w(GemmArgs a) {
       put(g, u0, u1);
     };
 #pragma unroll
-    for (int i = 0; i < W_KEEP; ++i)
+    for (int i = 0; i < KEEP; ++i)
       if (wave + i * W_WAVES < groups) put16(wave + i * W_WAVES, kept[i]);
-    for (int g = wave + W_KEEP * W_WAVES; g < groups; g += W_WAVES) {
+    for (int g = wave + KEEP * W_WAVES; g < groups; g += W_WAVES) {
       const u32x4 v[4] = {xp[16 * g], xp[16 * g + 1], xp[16 * g + 2], xp[16 * g + 3]};
       put16(g, v);
     }
@@ -538,8 +540,11 @@ int launch_gemm_i8w(const GemmArgs& a, hipStream_t s) {
   const int64_t slots = a.tiles ? a.tile_cap : a.E;
   const unsigned z = a.tiles ? 1u : (unsigned)((a.max_rows + W_TOK - 1) / W_TOK);
   const dim3 sgrid((unsigned)slots, W_TOK / 16, z);
-  if (a.quant) hipLaunchKernelGGL(k_stage_i8w<BP_BF16>, sgrid, dim3(W_THREADS), W_WAVES * 16 * 4, s, a);
-  else hipLaunchKernelGGL(k_stage_i8w<BP_I8>, sgrid, dim3(W_THREADS), 0, s, a);
+  const int red = W_WAVES * 16 * 4;  // bytes of LDS for the row maxima
+  if (!a.quant) hipLaunchKernelGGL((k_stage_i8w<BP_I8, 1>), sgrid, dim3(W_THREADS), 0, s, a);
+  else if (a.K <= 1024) hipLaunchKernelGGL((k_stage_i8w<BP_BF16, 1>), sgrid, dim3(W_THREADS), red, s, a);
+  else if (a.K <= 2048) hipLaunchKernelGGL((k_stage_i8w<BP_BF16, 2>), sgrid, dim3(W_THREADS), red, s, a);
+  else hipLaunchKernelGGL((k_stage_i8w<BP_BF16, 4>), sgrid, dim3(W_THREADS), red, s, a);
   if (const int rc = check_launch("stage_i8w")) return rc;
   return i8w_wr(a) == 2 ? launch_i8w<2>(a, s) : launch_i8w<4>(a, s);
 }

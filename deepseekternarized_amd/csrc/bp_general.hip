@@ -92,7 +92,7 @@ __global__ __launch_bounds__(GEN_WAVES * 64) void k_general(GemmArgs a) {
   if (lane == 0) {
 #pragma unroll
     for (int r = 0; r < GEN_TOK; ++r)
-      if (r < rows) a.out[(row0 + r) * a.N + n] = __fadd_rn(a.out[(row0 + r) * a.N + n], total[r]);
+      if (r < rows) a.out[(row0 + r) * a.N + n] = __fadd_rn(a.overwrite ? 0.f : a.out[(row0 + r) * a.N + n], total[r]);
   }
 }
 
@@ -262,22 +262,25 @@ __global__ __launch_bounds__(256) void k_quant(int8_t* __restrict__ q, float* __
 // The same for 16-bit activations in rows of whole 16-byte pieces (K % 8 == 0, K <= 8192, aligned pointers): a thread keeps
 // its up to four pieces of the row in registers between the two passes, so the row is read once, in 16-byte loads, and
 // written in 8-byte stores. Same arithmetic as k_quant, operation for operation.
-constexpr int QUANT_VPT = 4;
+// `index` (or NULL): row m is quantised from row index[m] / div of x, which has src_rows rows (a routed layer's gather).
+constexpr int QUANT_VPT = 4;  // pieces per thread at most (VPT: as many as K needs)
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-template <int DT>
-__global__ __launch_bounds__(256) void k_quant16(int8_t* __restrict__ q, float* __restrict__ s, const uint16_t* __restrict__ x, int64_t K) {
+template <int DT, int VPT>
+__global__ __launch_bounds__(256) void k_quant16(int8_t* __restrict__ q, float* __restrict__ s, const uint16_t* __restrict__ x, int64_t K,
+                                                 const int64_t* __restrict__ index, int64_t div, int64_t src_rows) {
   __shared__ float part[4];
   const int64_t m = blockIdx.x;
+  const int64_t from = index ? clamp_i64(index[m] / div, 0, src_rows - 1) : m;
   const int pieces = (int)(K / 8);
-  u32x4 raw[QUANT_VPT];
+  u32x4 raw[VPT];
   float amax = 0.f;
   bool nan = false;
 #pragma unroll
-  for (int i = 0; i < QUANT_VPT; ++i) {
+  for (int i = 0; i < VPT; ++i) {
     const int pc = threadIdx.x + 256 * i;
     raw[i] = u32x4{0u, 0u, 0u, 0u};
-    if (pc < pieces) raw[i] = *(const u32x4*)(x + m * K + 8 * (int64_t)pc);
+    if (pc < pieces) raw[i] = *(const u32x4*)(x + from * K + 8 * (int64_t)pc);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const uint16_t h = (uint16_t)(raw[i][j >> 1] >> (16 * (j & 1)));
@@ -301,7 +304,7 @@ __global__ __launch_bounds__(256) void k_quant16(int8_t* __restrict__ q, float* 
   sc = sc != sc ? sc : fmaxf(sc, 1e-8f);  // clamp(min=1e-8) keeps NaN
   if (threadIdx.x == 0) s[m] = sc;
 #pragma unroll
-  for (int i = 0; i < QUANT_VPT; ++i) {
+  for (int i = 0; i < VPT; ++i) {
     const int pc = threadIdx.x + 256 * i;
     unsigned out[2] = {0u, 0u};
 #pragma unroll
@@ -313,6 +316,77 @@ __global__ __launch_bounds__(256) void k_quant16(int8_t* __restrict__ q, float* 
       out[j >> 2] |= ((unsigned)(r != r ? 0 : (int)r) & 0xffu) << (8 * (j & 3));
     }
     if (pc < pieces) *(u32x2*)(q + m * K + 8 * (int64_t)pc) = u32x2{out[0], out[1]};
+  }
+}
+
+template <int DT>
+void launch_quant16(int8_t* q, float* s, const void* x, int64_t M, int64_t K, const int64_t* index, int64_t div, int64_t src_rows, hipStream_t st) {
+  const dim3 grid((unsigned)M), block(256);
+  const uint16_t* xh = (const uint16_t*)x;
+  if (K <= 8 * 256) hipLaunchKernelGGL((k_quant16<DT, 1>), grid, block, 0, st, q, s, xh, K, index, div, src_rows);
+  else if (K <= 2 * 8 * 256) hipLaunchKernelGGL((k_quant16<DT, 2>), grid, block, 0, st, q, s, xh, K, index, div, src_rows);
+  else hipLaunchKernelGGL((k_quant16<DT, QUANT_VPT>), grid, block, 0, st, q, s, xh, K, index, div, src_rows);
+}
+
+// SwiGLU of a row of float32 gate | up sums and the quantisation of its bf16 result, without writing it: a thread keeps its
+// up to VPT x 4 values between the row maximum and the rounding. The same values as k_swiglu4 or k_swiglu_v4 followed by k_quant16.
+template <bool V4, int VPT>
+__global__ __launch_bounds__(256) void k_swiglu_quant(int8_t* __restrict__ q, float* __restrict__ s, const float* __restrict__ gate, const float* __restrict__ up,
+                                                      const float* __restrict__ weights, const int64_t* __restrict__ order, int64_t pairs, float limit, int64_t I,
+                                                      int64_t ld) {
+  __shared__ float part[4];
+  const int64_t m = blockIdx.x;
+  float w = 1.f;
+  if (V4 && weights) w = weights[order ? clamp_i64(order[m], 0, pairs - 1) : m];
+  float h[VPT][4];
+  float amax = 0.f;
+  bool nan = false;
+  float4 g4[VPT], u4[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int64_t c = 4 * (int64_t)(threadIdx.x + 256 * i);
+    g4[i] = u4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (c < I) {
+      g4[i] = *(const float4*)(gate + m * ld + c);
+      u4[i] = *(const float4*)(up + m * ld + c);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const float gs[4] = {g4[i].x, g4[i].y, g4[i].z, g4[i].w}, us[4] = {u4[i].x, u4[i].y, u4[i].z, u4[i].w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float v = bf16_bits_to_f32(swiglu_bits<V4>(gs[j], us[j], weights != nullptr, w, limit));
+      h[i][j] = v;
+      nan |= v != v;
+      amax = fmaxf(amax, fabsf(v));
+    }
+  }
+  if (nan) amax = __builtin_nanf("");
+  float t = amax;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float o = __shfl_xor(t, off, 64);
+    t = (t != t || o != o) ? __builtin_nanf("") : fmaxf(t, o);
+  }
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = t;
+  __syncthreads();
+  float a = part[0];
+  for (int i = 1; i < 4; ++i) a = (a != a || part[i] != part[i]) ? __builtin_nanf("") : fmaxf(a, part[i]);
+  float sc = __fdiv_rn(a, 127.0f);
+  sc = sc != sc ? sc : fmaxf(sc, 1e-8f);
+  if (threadIdx.x == 0) s[m] = sc;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int64_t c = 4 * (int64_t)(threadIdx.x + 256 * i);
+    unsigned out = 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float r = rintf(__fdiv_rn(h[i][j], sc));
+      r = fminf(fmaxf(r, -127.f), 127.f);
+      out |= ((unsigned)(r != r ? 0 : (int)r) & 0xffu) << (8 * j);
+    }
+    if (c < I) *(unsigned*)(q + m * I + c) = out;
   }
 }
 
@@ -467,6 +541,32 @@ __global__ __launch_bounds__(256) void k_absmean_pack_lds(uint8_t* __restrict__ 
 
 }  // namespace
 
+// Rows index[m] / div of bf16 x (src_rows of them) as int8 rows m of q. BP_ERR_UNSUPPORTED: rows that the kernel does not take.
+int quant_gathered(int8_t* q, float* s, const void* x, const int64_t* index, int64_t div, int64_t src_rows, int64_t M, int64_t K, hipStream_t st) {
+  if (K % 8 != 0 || K > 8 * 256 * QUANT_VPT || (((uintptr_t)x & 15) | ((uintptr_t)q & 7)) != 0 || M > 0x7fffffff) return BP_ERR_UNSUPPORTED;
+  launch_quant16<BP_BF16>(q, s, x, M, K, index, div, src_rows, st);
+  return check_launch("quant_gathered");
+}
+
+// SwiGLU of float32 gate | up rows (v4: bp_swiglu_v4's, otherwise bp_swiglu_bf16's) and its int8 rows. BP_ERR_UNSUPPORTED as above.
+int swiglu_quant(bool v4, int8_t* q, float* s, const float* gate, const float* up, const float* weights, const int64_t* order, int64_t pairs, float limit,
+                 int64_t rows, int64_t I, int64_t ld, hipStream_t st) {
+  if (I % 4 != 0 || ld % 4 != 0 || I > 4096 || (((uintptr_t)gate | (uintptr_t)up) & 15) != 0 || ((uintptr_t)q & 3) != 0 || rows > 0x7fffffff) return BP_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)rows), block(256);
+#define BP_SQ(V4, VPT) hipLaunchKernelGGL((k_swiglu_quant<V4, VPT>), grid, block, 0, st, q, s, gate, up, weights, order, pairs, limit, I, ld)
+  if (v4) {
+    if (I <= 1024) BP_SQ(true, 1);
+    else if (I <= 2048) BP_SQ(true, 2);
+    else BP_SQ(true, 4);
+  } else {
+    if (I <= 1024) BP_SQ(false, 1);
+    else if (I <= 2048) BP_SQ(false, 2);
+    else BP_SQ(false, 4);
+  }
+#undef BP_SQ
+  return check_launch("swiglu_quant");
+}
+
 int launch_general(const GemmArgs& a, hipStream_t s) {
   if (a.max_rows <= 0 || a.N == 0 || a.E == 0) return BP_OK;
   const int64_t zt = (a.max_rows + GEN_TOK - 1) / GEN_TOK;
@@ -545,8 +645,10 @@ extern "C" int bp_quant_act_int8(int8_t* q, float* s, const void* x, int x_dtype
   if (M == 0) return BP_OK;
   if (!q || !s || !x) return fail(BP_ERR_ARG, "null pointer");
   const bool pieces = x_dtype != BP_F32 && K % 8 == 0 && K <= 8 * 256 * QUANT_VPT && ((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 7) == 0;
-  if (pieces && x_dtype == BP_BF16) hipLaunchKernelGGL(k_quant16<BP_BF16>, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, q, s, (const uint16_t*)x, K);
-  else if (pieces) hipLaunchKernelGGL(k_quant16<BP_F16>, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, q, s, (const uint16_t*)x, K);
+  if (pieces) {
+    if (x_dtype == BP_BF16) launch_quant16<BP_BF16>(q, s, x, M, K, nullptr, 1, 0, (hipStream_t)stream);
+    else launch_quant16<BP_F16>(q, s, x, M, K, nullptr, 1, 0, (hipStream_t)stream);
+  }
   else hipLaunchKernelGGL(k_quant, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, q, s, x, x_dtype, K);
   return check_launch("quant_act_int8");
 }

@@ -99,22 +99,10 @@ __device__ __forceinline__ float scale_at(const u32x4 (&raw)[2], int i) {  // i-
   return __uint_as_float((i & 1) ? (v & 0xffff0000u) : (v << 16));
 }
 
-// SwiGLU of one pair of gate and up sums with the rounding points of bp_swiglu_bf16 or, with a.glu_v4, of bp_swiglu_v4.
+// SwiGLU in a GEMM's epilogue (GemmArgs::glu_h).
 __device__ __forceinline__ uint16_t swiglu_value(const GemmArgs& a, float gate, float up, float weight) {
-  float g = bf16_bits_to_f32(f32_to_bf16_bits(gate)), u = bf16_bits_to_f32(f32_to_bf16_bits(up));
-  float v;
-  if (a.glu_v4) {
-    if (a.glu_limit > 0.f) {  // torch.clamp: a NaN stays a NaN
-      u = u < -a.glu_limit ? -a.glu_limit : (u > a.glu_limit ? a.glu_limit : u);
-      g = g > a.glu_limit ? a.glu_limit : g;
-    }
-    v = (g / (1.0f + expf(-g))) * u;
-    if (a.glu_weights) v = weight * v;
-  } else {
-    const float sg = bf16_bits_to_f32(f32_to_bf16_bits(g / (1.0f + expf(-g))));
-    v = sg * u;
-  }
-  return f32_to_bf16_bits(v);
+  if (a.glu_v4) return swiglu_bits<true>(gate, up, a.glu_weights != nullptr, weight, a.glu_limit);
+  return swiglu_bits<false>(gate, up, false, 1.f, 0.f);
 }
 
 }  // namespace

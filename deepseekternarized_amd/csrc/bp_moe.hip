@@ -23,6 +23,10 @@ int moe_combine(void* out, const void* y, bool y16, const int64_t* inv, const vo
                 void* stream);  // bp_route.hip
 int moe_combine_v4(void* out, int out_dtype, const void* y, bool y16, const int64_t* inv, const int64_t* experts, int64_t T, int64_t k, int64_t H,
                    void* stream);
+// bp_general.hip
+int quant_gathered(int8_t* q, float* s, const void* x, const int64_t* index, int64_t div, int64_t src_rows, int64_t M, int64_t K, hipStream_t st);
+int swiglu_quant(bool v4, int8_t* q, float* s, const float* gate, const float* up, const float* weights, const int64_t* order, int64_t pairs, float limit,
+                 int64_t rows, int64_t I, int64_t ld, hipStream_t st);
 namespace {
 
 constexpr int TILE_ROWS = 32;  // token tile of k_gemm_tq1 / k_gemm_tq2
@@ -69,36 +73,26 @@ __global__ __launch_bounds__(1024) void k_tile_list(int32_t* __restrict__ tiles,
   if (threadIdx.x == 0) count[0] = carry < cap ? carry : (int)cap;
 }
 
-// The row gather xg[r] = x[order[r] / k] (rows of 16-byte pieces) and, in the same launch, the zero-fill of the two float32
-// outputs that the GEMMs accumulate into (z0_16 = z1_16 = 0 where they write instead).
-__global__ __launch_bounds__(256) void k_gather_zero(u32x4* __restrict__ xg, const u32x4* __restrict__ x, const int64_t* __restrict__ order, int64_t n,
-                                                     int64_t k, int64_t T, int64_t row16, u32x4* __restrict__ z0, int64_t z0_16, u32x4* __restrict__ z1,
-                                                     int64_t z1_16) {
+// The row gather xg[r] = x[order[r] / k] (rows of 16-byte pieces).
+__global__ __launch_bounds__(256) void k_gather16(u32x4* __restrict__ xg, const u32x4* __restrict__ x, const int64_t* __restrict__ order, int64_t n,
+                                                  int64_t k, int64_t T, int64_t row16) {
   const int64_t gtid = (int64_t)blockIdx.x * 256 + threadIdx.x, gsz = (int64_t)gridDim.x * 256;
   for (int64_t w = gtid; w < n * row16; w += gsz) {
     const int64_t r = w / row16, c = w - r * row16;
     const int64_t src = clamp_i64(order[r] / k, 0, T - 1);
     xg[r * row16 + c] = x[src * row16 + c];
   }
-  for (int64_t w = gtid; w < z0_16; w += gsz) z0[w] = u32x4{0u, 0u, 0u, 0u};
-  for (int64_t w = gtid; w < z1_16; w += gsz) z1[w] = u32x4{0u, 0u, 0u, 0u};
-}
-
-__global__ __launch_bounds__(256) void k_zero16(u32x4* __restrict__ p, int64_t n16) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (int64_t)gridDim.x * 256) p[i] = u32x4{0u, 0u, 0u, 0u};
 }
 
 // A few routed rows (n <= ROUTE_SMALL_N): the layer's whole preparation in one launch instead of five - stable sort of
 // the expert ids (every workgroup ranks the ids for itself in LDS: element i goes to slot #(ids below id_i) + #(equal
-// ids before i); workgroup 0 writes order, offsets and the inverse permutation), the row gather xg[r] = x[order[r] / k],
-// and the zero-fill of the two float32 outputs that the small-batch kernels accumulate into - or, where the GEMMs run
-// over the list of token tiles, that list (position r of the order starts a tile when it is a multiple of 32 rows into
-// its expert; the tiles come out in expert order) instead of the zero-fill.
+// ids before i); workgroup 0 writes order, offsets and the inverse permutation), the row gather xg[r] = x[order[r] / k]
+// and, where the GEMMs run over the list of token tiles, that list (position r of the order starts a tile when it is a
+// multiple of 32 rows into its expert; the tiles come out in expert order).
 constexpr int ROUTE_SMALL_N = 256, ROUTE_SMALL_THREADS = 256;
 __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __restrict__ order, int64_t* __restrict__ offsets, int64_t* __restrict__ inv,
                                                                      const int64_t* __restrict__ ids, int n, int64_t E, int32_t* __restrict__ bad,
                                                                      u32x4* __restrict__ xg, const u32x4* __restrict__ x, int k, int64_t T, int64_t row16,
-                                                                     u32x4* __restrict__ z0, int64_t z0_16, u32x4* __restrict__ z1, int64_t z1_16,
                                                                      int32_t* __restrict__ tiles, int32_t* __restrict__ tile_count, int64_t tile_cap) {
   __shared__ __attribute__((aligned(16))) int32_t sid[ROUTE_SMALL_N];  // (entries from n on: 0x7fffffff, "no expert")
   __shared__ int32_t ord[ROUTE_SMALL_N];
@@ -172,12 +166,12 @@ __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __
       xg[r * row16 + c] = x[src * row16 + c];
     }
   }
-  for (int64_t w = gtid; w < z0_16; w += gsz) z0[w] = u32x4{0u, 0u, 0u, 0u};
-  for (int64_t w = gtid; w < z1_16; w += gsz) z1[w] = u32x4{0u, 0u, 0u, 0u};
 }
 
-// Layers whose two GEMMs run on the int8 kernel for token tiles of 128: int8 activations, TQ2, 128 rows per expert on average (the
-// tiles of an expert mostly full; below, the kernel for tiles of 32 computes less padding).
+// Layers whose two GEMMs run on the int8 kernel for token tiles of 128: int8 activations, TQ2, 64 rows per expert on average.
+// Whole layer with skewed routing against the kernel for tiles of 32, us: 2048 / 1024, 64 experts top-8, 512 tokens (64 rows) 137.5 / 164.3,
+// 768 145 / 219, 8192 957 / 2186 at the start; 4096 / 2048, top-6, 768 tokens (72 rows) 370 / 465, 2048 675 / 1027. With fewer rows the tiles are
+// mostly padding (48 rows: 137 on tiles of 32, which 75 tiles of 128 take as well).
 bool moe_wide(int act, int fmt, int64_t n, int64_t T, int64_t E) { return act == BP_I8 && fmt == BP_TQ2 && T > 64 && n >= 128 * E; }
 
 struct Carve {
@@ -240,14 +234,6 @@ Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k
   return p;
 }
 
-int zero(void* p, size_t bytes, hipStream_t s) {  // (a fill kernel, not a memset node: the call may be captured in a graph)
-  const int64_t n16 = (int64_t)(bytes / 16);
-  int64_t g = (n16 + 255) / 256;
-  if (g > 8192) g = 8192;
-  if (g > 0) hipLaunchKernelGGL(k_zero16, dim3((unsigned)g), dim3(256), 0, s, (u32x4*)p, n16);
-  return check_launch("zero");
-}
-
 }  // namespace
 }  // namespace bp
 
@@ -286,8 +272,6 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   const int per = fmt == BP_TQ2 ? 4 : 5;
 
   int rc = BP_OK;
-  // (the outputs' zero-fill rides along only where both GEMMs are going to accumulate: no tile list, and a policy that
-  // lets them run; rows of 16-byte multiples: H % 8 == 0 is checked above)
   // Tokens beyond which the GEMMs run over the tile list. Up to 64 no expert can have more than 64 rows and the small-batch
   // kernels take the launch by that bound; TQ1 with bf16 activations changes over at 24 already: the launches of 8 rows
   // cost what their widest expert costs (an expert with 9 rows means a second pass over few CUs), the tile kernel a flat
@@ -296,7 +280,9 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   const bool tiles = T > tiles_from;
   const bool small = n <= ROUTE_SMALL_N && (((uintptr_t)x | (uintptr_t)p.xg) & 15) == 0;
   const bool aligned16 = (((uintptr_t)x | (uintptr_t)p.xg) & 15) == 0;
-  const bool prezeroed = aligned16 && !tiles;  // the zero-fill rides along with the gather (the GEMMs over the tile list write instead of accumulate)
+  // int8 activations: the rows are quantised where they are gathered, and SwiGLU's result where it is made, when the rows'
+  // lengths suit those kernels - two launches and two copies of the rows less
+  const bool quant_in = act == BP_I8 && aligned16 && H <= 8192;
   // The gate | up projection as the grouped GEMM over converted activations with SwiGLU in its epilogue (bf16 h written,
   // no float32 gate | up rows), where that kernel takes the call: over the tile list, bf16 activations. Its conversion
   // pass then also does the row gather (rows read through `order`): no routed copy of the activations is written.
@@ -346,33 +332,31 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     wide = mfma_supports(a) && mfma_supports(probe) && gemm_i8w_applies(a) == BP_OK && gemm_i8w_applies(d) == BP_OK;
   }
   if (small) {
-    const int64_t z0 = prezeroed ? (int64_t)(4 * (size_t)n * 2 * I / 16) : 0, z1 = prezeroed ? (int64_t)(4 * (size_t)n * H / 16) : 0;
-    const int64_t row16 = fuse && fused.x_index ? 0 : H / 8;  // (no rows to copy where the gate | up launch reads them through `order`)
-    int64_t g = (z0 + z1 + (int64_t)n * row16 + ROUTE_SMALL_THREADS - 1) / ROUTE_SMALL_THREADS;
+    const int64_t row16 = (fuse && fused.x_index) || quant_in ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
+    int64_t g = ((int64_t)n * row16 + ROUTE_SMALL_THREADS - 1) / ROUTE_SMALL_THREADS;
     g = g < 1 ? 1 : (g > 256 ? 256 : g);
     hipLaunchKernelGGL(k_route_small, dim3((unsigned)g), dim3(ROUTE_SMALL_THREADS), 0, s, p.order, p.offsets, p.inv, experts, (int)n, E, bad,
-                       (u32x4*)p.xg, (const u32x4*)x, (int)k, T, row16, (u32x4*)p.gu, z0, (u32x4*)p.y, z1, tiles ? p.tiles : nullptr, p.tile_count,
+                       (u32x4*)p.xg, (const u32x4*)x, (int)k, T, row16, tiles ? p.tiles : nullptr, p.tile_count,
                        p.tile_cap);
     if ((rc = check_launch("route_small")) != BP_OK) return rc;
   } else {
     if ((rc = sort_with_inverse(p.order, p.offsets, p.inv, experts, n, E, p.sort_ws, bad, s)) != BP_OK) return rc;
     if (wide) {
       if ((rc = bp_quant_act_int8(p.q, p.q_scale, x, BP_BF16, T, H, s)) != BP_OK) return rc;
-    } else if (fuse && fused.x_index) {
+    } else if ((fuse && fused.x_index) || quant_in) {
       // (no routed copy of the activations: the gate | up launch's conversion pass reads them through `order`)
     } else if (aligned16) {
-      const int64_t z0 = prezeroed ? (int64_t)(4 * (size_t)n * 2 * I / 16) : 0, z1 = prezeroed ? (int64_t)(4 * (size_t)n * H / 16) : 0;
-      int64_t g = (z0 + z1 + n * (H / 8) + 255) / 256;
+      int64_t g = (n * (H / 8) + 255) / 256;
       g = g < 1 ? 1 : (g > 4096 ? 4096 : g);
-      hipLaunchKernelGGL(k_gather_zero, dim3((unsigned)g), dim3(256), 0, s, (u32x4*)p.xg, (const u32x4*)x, p.order, n, k, T, H / 8, (u32x4*)p.gu, z0,
-                         (u32x4*)p.y, z1);
-      if ((rc = check_launch("gather_zero")) != BP_OK) return rc;
+      hipLaunchKernelGGL(k_gather16, dim3((unsigned)g), dim3(256), 0, s, (u32x4*)p.xg, (const u32x4*)x, p.order, n, k, T, H / 8);
+      if ((rc = check_launch("gather")) != BP_OK) return rc;
     } else if ((rc = bp_gather_rows(p.xg, x, p.order, k, n, T, 2 * H, s)) != BP_OK) return rc;
   }
 
   // `o16`: the caller takes bf16 rows (the combine rounds the down projection's rows to bf16 first); set to whether
-  // the launch wrote them - the grouped GEMM over converted activations does, into the same buffer.
-  auto gemm = [&](float* o, const void* in, const uint8_t* const* packed, const void* const* scale, int64_t N, int64_t K, bool tiles, bool* o16) -> int {
+  // the launch wrote them, into the same buffer. `quantised`: p.q and p.q_scale hold the int8 rows already. Every launch
+  // replaces what its output held.
+  auto gemm = [&](float* o, const void* in, const uint8_t* const* packed, const void* const* scale, int64_t N, int64_t K, bool tiles, bool* o16, bool quantised) -> int {
     const bool want16 = o16 && *o16;
     if (o16) *o16 = false;
     GemmArgs a;
@@ -381,8 +365,10 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     a.x = in;
     a.offsets = p.offsets;
     a.x_dtype = act;
+    a.overwrite = 1;
     if (act == BP_I8) {
-      if (const int q = bp_quant_act_int8(p.q, p.q_scale, in, BP_BF16, n, K, s)) return q;
+      if (quantised) {
+      } else if (const int q = bp_quant_act_int8(p.q, p.q_scale, in, BP_BF16, n, K, s)) return q;
       a.x = p.q;
       a.x_scale = p.q_scale;
     }
@@ -397,7 +383,6 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     if (tiles) {
       a.tiles = p.tiles; a.tile_count = p.tile_count; a.tile_cap = p.tile_cap;
       if (kernel_policy() != 1 && gemm_tiles_supported(a)) {
-        a.overwrite = 1;
         a.max_rows = TILE_ROWS;
         if (want16 && tuning().glu != 'n' && tuning().tq2g != 'b') {
           a.out16 = (uint16_t*)o;
@@ -411,8 +396,15 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
       }
       a.tiles = nullptr;  // no tile kernel for this shape: the launch covers the bound (every expert up to T rows)
     }
-    if (!prezeroed)
-      if (const int z = zero(o, 4 * (size_t)n * N, s)) return z;
+    if (want16) {
+      a.out16 = (uint16_t*)o;
+      const int got = run_gemm(a, s);
+      if (got != ERR_NO_OUT16) {
+        *o16 = true;
+        return got;
+      }
+      a.out16 = nullptr;
+    }
     return run_gemm(a, s);
   };
   if (tiles && !small) {
@@ -425,16 +417,22 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     if (v4) return moe_combine_v4(out, out_dtype, p.y, true, p.inv, experts, T, k, H, s);
     return moe_combine(out, p.y, true, p.inv, weights, experts, T, k, H, s);
   }
+  bool quant_h = false;
   if (fuse) {
     rc = launch_gemm_tq2f(fused, s);
   } else {
-    if ((rc = gemm(p.gu, p.xg, gate_up_packed, gate_up_scale, 2 * I, H, tiles, nullptr)) != BP_OK) return rc;
-    if (v4) rc = bp_swiglu_v4(p.h, p.gu, p.gu + I, (const float*)weights, p.order, n, limit, n, I, 2 * I, s);
+    if (quant_in && (rc = quant_gathered(p.q, p.q_scale, x, p.order, k, T, n, H, s)) != BP_OK) return rc;
+    if ((rc = gemm(p.gu, p.xg, gate_up_packed, gate_up_scale, 2 * I, H, tiles, nullptr, quant_in)) != BP_OK) return rc;
+    rc = BP_ERR_UNSUPPORTED;
+    if (act == BP_I8) rc = swiglu_quant(v4, p.q, p.q_scale, p.gu, p.gu + I, v4 ? (const float*)weights : nullptr, p.order, n, limit, n, I, 2 * I, s);
+    quant_h = rc == BP_OK;
+    if (quant_h) {
+    } else if (v4) rc = bp_swiglu_v4(p.h, p.gu, p.gu + I, (const float*)weights, p.order, n, limit, n, I, 2 * I, s);
     else rc = bp_swiglu_bf16(p.h, p.gu, p.gu + I, n, I, 2 * I, s);
   }
   if (rc != BP_OK) return rc;
   bool y16 = true;
-  if ((rc = gemm(p.y, p.h, down_packed, down_scale, H, I, tiles, &y16)) != BP_OK) return rc;
+  if ((rc = gemm(p.y, p.h, down_packed, down_scale, H, I, tiles, &y16, quant_h)) != BP_OK) return rc;
   if (fuse) note_kernel_suffix(fused.x_index ? "+glu+gather" : "+glu");  // (bp_last_kernel: the down projection's kernel, and that the gate | up one applied SwiGLU)
   if (y16) note_kernel_suffix("+y16");  // (... and that the down projection wrote bf16 rows)
   if (v4) return moe_combine_v4(out, out_dtype, p.y, y16, p.inv, experts, T, k, H, s);

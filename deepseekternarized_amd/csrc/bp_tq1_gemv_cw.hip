@@ -101,7 +101,7 @@ __global__ __launch_bounds__(CW_WAVES * 64) void k_tq1_gemv_cw(GemmArgs a, int n
 #pragma unroll
   for (int u = 0; u < CW_STAGE_PER_THREAD; ++u) {
     const int o = (int)threadIdx.x + u * THREADS;
-    was[u] = !a.out16 && o < n_stage && ((o >> 4) % NTOK) < ntok ? a.out[out_index(o)] : 0.f;
+    was[u] = !a.out16 && !a.overwrite && o < n_stage && ((o >> 4) % NTOK) < ntok ? a.out[out_index(o)] : 0.f;
   }
 
   // ---- loaders: state of the current term (the expert's rows and scales as buffers of their own: a tile past N reads

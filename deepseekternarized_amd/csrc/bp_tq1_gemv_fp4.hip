@@ -190,13 +190,14 @@ __global__ __launch_bounds__(WAVES * 64, KS ? 2 : 4) void k_tq1_gemv_fp4(GemmArg
     // with stacked terms the value may be one this wave stored a term ago.)
     // (up to 4 tokens; beyond, the registers are not there)
     constexpr bool EARLY = NTOK <= 4;
+    const bool fresh = a.out16 || (a.overwrite && term == 0 && first_chunk == 0);  // nothing to add to
     float before[NTOK > 1 ? NTOK : GR];
 #pragma unroll
     for (int s = 0; s < (NTOK > 1 ? NTOK : GR); ++s) {
       total[s] = 0.f;
       const int tile = NTOK > 1 ? 0 : s, tt = NTOK > 1 ? s : 0;
       before[s] = 0.f;
-      if (EARLY && !a.out16 && kb == 0 && wave_live && n0 + 16 * tile < a.N && tt < ntok && (!KS || wave == 0))
+      if (EARLY && !fresh && kb == 0 && wave_live && n0 + 16 * tile < a.N && tt < ntok && (!KS || wave == 0))
         before[s] = __hip_atomic_load(a.out + (tok + tt) * a.N + n0 + 16 * tile + r16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // chunk c of this block, or (c >= nchunks, chained) chunk c - nchunks of the next one: row offset (scalar) and chunk
@@ -503,7 +504,7 @@ __global__ __launch_bounds__(WAVES * 64, KS ? 2 : 4) void k_tq1_gemv_fp4(GemmArg
         continue;
       }
       float* o = a.out + at;
-      const float was = EARLY ? before[s] : __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const float was = EARLY ? before[s] : fresh ? 0.f : __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       *o = was + v;
     }
   }

@@ -149,7 +149,7 @@ __global__ __launch_bounds__(1024) void k_tq2_gemv_ks(GemmArgs a, int nw, int ti
 #pragma unroll
   for (int u = 0; u < KV_OPT; ++u) {
     const int o = (int)threadIdx.x + u * nw * 64;
-    total[u] = !a.out16 && out_live(o) ? a.out[out_at(o)] : 0.f;
+    total[u] = !a.out16 && !a.overwrite && out_live(o) ? a.out[out_at(o)] : 0.f;
   }
   i32x8 A[2 * KV_S];
   float cinit[4], inv2[NTOK], cinitb[4], inv2b[2];  // (b: four tokens, the second step; inv2 / inv2b then hold the lane's two tokens)
