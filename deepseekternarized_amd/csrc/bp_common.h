@@ -33,6 +33,7 @@ struct GemmArgs {
   const int32_t* tiles;
   const int32_t* tile_count;
   int64_t tile_cap;
+  int row_grid;   // decode launches: one blockIdx.y per token row instead of one per expert (expert_of_block; set by launch_mfma)
   int overwrite;  // tile-list mode: the kernel's result replaces `out` instead of being added to it (one launch covers all of K and all terms)
   // Workspace of the caller for kernels that convert the activations in a pass of their own (NULL: those kernels are not used).
   unsigned char* stage;
@@ -58,6 +59,37 @@ struct GemmArgs {
 };
 
 __device__ __forceinline__ int64_t clamp_i64(int64_t v, int64_t lo, int64_t hi) { return v < lo ? lo : (v > hi ? hi : v); }
+
+// The expert of a decode launch's blockIdx.y. With many fewer token rows than experts (one token of a routed layer: 6 of 64)
+// the grid holds one y per row, and y = j is the j-th expert that has rows - every wave looks for it in the offsets - rather than
+// one y per expert, most of whose workgroups would only take a CU's LDS, read two offsets and leave.
+inline bool rows_in_grid(int64_t T, int64_t E) { return 2 * T <= E; }  // (GemmArgs::row_grid)
+inline unsigned grid_experts(const GemmArgs& a) { return (unsigned)(a.row_grid ? a.T : a.E); }
+constexpr unsigned NO_EXPERT = 0xffffffffu;
+__device__ __forceinline__ unsigned expert_of_block(const GemmArgs& a, unsigned j) {
+  if (__builtin_expect(!a.row_grid, 1)) return j;
+  const int lane = threadIdx.x & 63;
+  for (int64_t base = 0; base < a.E; base += 256) {
+    unsigned long long has[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t x = base + 64 * i + lane;
+      bool rows = false;
+      if (x < a.E) rows = clamp_i64(a.offsets[x + 1], 0, a.T) > clamp_i64(a.offsets[x], 0, a.T);
+      has[i] = __ballot(rows);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned n = (unsigned)__popcll(has[i]);
+      if (j < n) {
+        for (; j > 0; --j) has[i] &= has[i] - 1;
+        return (unsigned)base + 64u * (unsigned)i + (unsigned)(__ffsll((long long)has[i]) - 1);
+      }
+      j -= n;
+    }
+  }
+  return NO_EXPERT;  // fewer experts with rows
+}
 
 // Which token tile of ROWS rows a workgroup takes: `slot` is its expert (list entry in tile-list mode), z its token tile.
 struct TileRef {

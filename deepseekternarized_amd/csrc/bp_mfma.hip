@@ -37,7 +37,9 @@ bool gemm_tiles_supported(const GemmArgs& a) {
   return true;
 }
 
-int launch_mfma(const GemmArgs& a, hipStream_t s) {
+int launch_mfma(const GemmArgs& call, hipStream_t s) {
+  GemmArgs a = call;
+  a.row_grid = rows_in_grid(a.T, a.E) ? 1 : 0;
   if (a.tiles) {  // tile-list mode: only the 32-token-tile kernels read the list
     if (!gemm_tiles_supported(a)) return BP_ERR_UNSUPPORTED;
     return a.fmt == BP_TQ1 ? launch_gemm_tq1(a, s) : launch_gemm_tq2(a, s);

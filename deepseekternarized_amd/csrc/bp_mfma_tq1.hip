@@ -79,7 +79,9 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq1(GemmArgs a, int CPT 
   // the wave index through readfirstlane: everything derived from it stays in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int r16 = lane & 15, b = lane >> 4;
-  const int64_t e = blockIdx.y;
+  const unsigned ey = expert_of_block(a, blockIdx.y);
+  if (ey == NO_EXPERT) return;  // (uniform)
+  const int64_t e = ey;
   const int64_t o0 = clamp_i64(a.offsets[e], 0, a.T), o1 = clamp_i64(a.offsets[e + 1], 0, a.T);
   const int64_t tok0 = o0 + (int64_t)blockIdx.z * 16;
   if (tok0 >= o1) return;  // uniform for the workgroup
@@ -345,7 +347,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq1(GemmArgs a, int CPT 
 template <int SDT, int WAVES, int NQ, int SL, int MULTI, int ABL = 0>
 int launch_tq1_k(const GemmArgs& a, hipStream_t s, const char* name, int64_t cpt, int64_t tokens, size_t lds) {
   const int64_t rows_per_wg = (int64_t)WAVES * 16;
-  const dim3 grid((unsigned)((a.N + rows_per_wg - 1) / rows_per_wg), (unsigned)a.E, (unsigned)((a.max_rows + 15) / 16));
+  const dim3 grid((unsigned)((a.N + rows_per_wg - 1) / rows_per_wg), grid_experts(a), (unsigned)((a.max_rows + 15) / 16));
   if (const int rc = raise_lds_limit<k_mfma_tq1<SDT, WAVES, NQ, SL, MULTI, ABL>>(T1_LDS_MAX)) return rc;
   note_kernel(name);
   hipLaunchKernelGGL((k_mfma_tq1<SDT, WAVES, NQ, SL, MULTI, ABL>), grid, dim3(WAVES * 64), lds, s, a, (int)cpt, (int)tokens);

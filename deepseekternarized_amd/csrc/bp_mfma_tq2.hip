@@ -28,7 +28,9 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq2(GemmArgs a, int KC, 
   // the wave index through readfirstlane: everything derived from it stays in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int r16 = lane & 15, b = lane >> 4;
-  const int64_t e = blockIdx.y;
+  const unsigned ey = expert_of_block(a, blockIdx.y);
+  if (ey == NO_EXPERT) return;  // (uniform)
+  const int64_t e = ey;
   const int64_t o0 = clamp_i64(a.offsets[e], 0, a.T), o1 = clamp_i64(a.offsets[e + 1], 0, a.T);
   const int64_t tok0 = o0 + (int64_t)blockIdx.z * (16 * MT);
   if (tok0 >= o1) return;  // uniform for the workgroup: no barrier is skipped by part of it
@@ -322,7 +324,7 @@ template <int ACT, int SDT, int R, int MT, int WAVES, int XKB, int ABL = 0, int 
 int launch_tq2(const GemmArgs& a, hipStream_t s, const char* name) {
   constexpr int XB = ACT == BP_BF16 ? 2 : 1;
   const int64_t rows_per_wg = (int64_t)WAVES * 16 * R;
-  const dim3 grid((unsigned)((a.N + rows_per_wg - 1) / rows_per_wg), (unsigned)a.E,
+  const dim3 grid((unsigned)((a.N + rows_per_wg - 1) / rows_per_wg), grid_experts(a),
                   (unsigned)((a.max_rows + 16 * MT - 1) / (16 * MT)));
   // chunk length: as much of K as the tile budget holds for the widest token tile, in blocks of 4 steps
   const int64_t tokens = a.max_rows < 16 * MT ? a.max_rows : 16 * MT;

@@ -92,7 +92,9 @@ __global__ __launch_bounds__(WAVES * 64, KS ? 2 : 4) void k_tq1_gemv_fp4(GemmArg
 
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int r16 = lane & 15, kb = lane >> 4;
-  const int64_t e = blockIdx.y;
+  const unsigned ey = expert_of_block(a, blockIdx.y);
+  if (ey == NO_EXPERT) return;  // (uniform)
+  const int64_t e = ey;
   const int64_t o0 = clamp_i64(a.offsets[e], 0, a.T), o1 = clamp_i64(a.offsets[e + 1], 0, a.T);
   // A launch takes the expert's token rows first_row .. first_row + NTOK - 1 (one token: its first row); an expert with
   // more rows than that gets further launches, one without any in this range is done at once (uniform).
@@ -532,7 +534,7 @@ int launch_f4_k(const GemmArgs& a, hipStream_t s, const char* name, int nchunks,
   const int64_t experts = a.E < a.T ? a.E : a.T;  // (an expert without a token returns at once)
   int64_t bpw = blocks * experts / resident;
   bpw = bpw < 1 || KS ? 1 : bpw > blocks ? blocks : bpw;
-  const dim3 grid((unsigned)((blocks + bpw - 1) / bpw), (unsigned)a.E, 1u);
+  const dim3 grid((unsigned)((blocks + bpw - 1) / bpw), grid_experts(a), 1u);
   note_kernel(name);
   const int per = seg_chunks > 0 ? seg_chunks : nchunks;
   for (int cb = 0; cb < nchunks; cb += per) {
