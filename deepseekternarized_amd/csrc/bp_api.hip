@@ -185,7 +185,7 @@ extern "C" size_t bp_grouped_gemm_workspace_bytes(int x_dtype, int64_t T, int64_
 
 extern "C" size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows) {
   if (fmt != BP_TQ2 || T <= 0 || E <= 0 || N <= 0 || K <= 0 || max_rows <= 16 || tuning().tq2g == 'b') return 0;
-  return tuning().tq2g == 'f' || i8w_pays(T, N, E) ? gemm_i8w_workspace_bytes(T, K, E) : 0;
+  return tuning().tq2g == 'f' || i8w_pays(T, N, K, E) ? gemm_i8w_workspace_bytes(T, K, E) : 0;
 }
 
 static size_t staged_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows) {
@@ -221,12 +221,16 @@ struct LinearPlan {  // offsets into the workspace
   size_t q, q_scale, sums, stage, stage_bytes, repacked, bytes;
   bool repack;  // TQ1 weights are rewritten as TQ2 ones first
 };
-// TQ1 linears of this many tokens and more rewrite their weights as TQ2 ones, which the token-tile kernels decode faster.
-constexpr int64_t REPACK_TOKENS = 256;
+// TQ1 linears whose weights are rewritten as TQ2 ones first, which the TQ2 kernels decode faster. From five tokens on while
+// the rewriting (0.45 bytes of traffic per weight) stays in the order of its launch; whole call against the TQ1 kernels, us:
+// 2048 x 2048 at 6 tokens 20 / 21.7 (at 4 tokens 20 / 15.6), 4096 x 4096 at 6 / 16 / 128 tokens 20 / 32, 20 / 40, 32 / 56, 2048 x 7168 at 16 tokens
+// 27 / 60. Larger weights, which the TQ1 kernels' few large workgroups fill the device with, from the number of tokens at which those decode
+// every weight for eight token tiles (4096 tokens x 4096 x 4096: 159 / 283).
+bool repack_pays(int64_t T, int64_t N, int64_t K) { return T >= 256 || (T >= 5 && N <= ((int64_t)1 << 26) / K); }
 size_t repacked_bytes(int64_t N, int64_t K) { return ((size_t)N * (size_t)(K / 4) + 255) & ~(size_t)255; }
 LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int fmt, int n_terms) {
   LinearPlan p;
-  p.repack = fmt == BP_TQ1 && T >= REPACK_TOKENS && K % 256 == 0 && K >= 1024 && K <= 65536 && tuning().tq2g != 'b';
+  p.repack = fmt == BP_TQ1 && repack_pays(T, N, K) && K % 256 == 0 && K >= 1024 && K <= 65536 && tuning().tq2g != 'b';
   if (p.repack) fmt = BP_TQ2;
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) & ~(size_t)255; return o; };

@@ -30,9 +30,12 @@ int gemm_tq2f_applies(const GemmArgs& a);  // BP_OK where launch_gemm_tq2f takes
 constexpr int I8W_TOK = 128;
 int launch_gemm_i8w(const GemmArgs& a, hipStream_t s);
 int gemm_i8w_applies(const GemmArgs& a);  // BP_OK where launch_gemm_i8w takes the call (nothing is launched)
-// Calls that run on it when the caller brings a workspace.
-inline bool i8w_pays(int64_t T, int64_t N, int64_t E) {
-  return T >= 64 * E && (T + I8W_TOK - 1) / I8W_TOK * ((N + 255) / 256) >= 192;
+// Calls that run on it when the caller brings a workspace: launches that fill most of the device, with less for rows that
+// run as two small workgroups per CU. Linears on it against the 32-token tiles, us: 1024 tokens x 2048 x 7168 41.6 / 58.7,
+// 768 x 2048 x 6144 (144 blocks) 40.2 / 45.7, 2048 x 2048 x 2048 (128) 33.1 / 36.6, 512 x 2048 x 6144 (96) 31.1 / 32.2, 256 x 2048 x 6144
+// 30.4 / 19.4; eight waves: 2048 x 4096 x 4096 (256) 68.0 / 92.8, 1024 x 4096 x 4096 (128) 62.6 / 50.2, 2048 x 7168 x 2048 (128) 99 / 77.8.
+inline bool i8w_pays(int64_t T, int64_t N, int64_t K, int64_t E) {
+  return T >= 64 * E && (T + I8W_TOK - 1) / I8W_TOK * ((N + 255) / 256) >= (K <= 3328 ? 128 : 192);
 }
 // bp_gemm_tq1.hip: TQ1 with token tiles of 32 on the fp8 x fp4 matrix instruction (experts with more than 8 token rows);
 // BP_ERR_UNSUPPORTED without a message when the call is outside its preconditions

@@ -15,6 +15,13 @@ def _weights(fmt, N, K, group, terms, sdt, seed=3):
                           (0.02 * torch.rand(N, -(-K // group), device="cuda", generator=gen)).to(sdt)) for _ in range(terms)], gen
 
 
+def _as_tq2(weights, K):
+    """What a TQ1 linear of five tokens and more multiplies: the same digits as 2-bit codes."""
+    import deepseekternarized_amd as bp
+
+    return [bp.PackedTerm(bp.pack(bp.unpack(w.packed, "tq1", K), "tq2"), w.scale) for w in weights]
+
+
 def _steps(x, terms, K, group, fmt, act, out_dtype):
     import deepseekternarized_amd as bp
     from deepseekternarized_amd.kernels.ternary_hip import dense_offsets
@@ -36,8 +43,9 @@ def test_linear_call_equals_its_steps(T, fmt, act, xdt, N, K, group, terms):
     weights, gen = _weights(fmt, N, K, group, terms, torch.float16)
     x = torch.randn(T, K, device="cuda", generator=gen).to(xdt)
     lin = bp.TernaryLinear(weights, K, fmt, group, act=act)
+    same, same_fmt = (weights, fmt) if fmt == "tq2" or T < 5 or K % 256 else (_as_tq2(weights, K), "tq2")
     for out_dtype in (torch.bfloat16, torch.float32):
-        assert torch.equal(lin(x, out_dtype), _steps(x, weights, K, group, fmt, act, out_dtype)), out_dtype
+        assert torch.equal(lin(x, out_dtype), _steps(x, same, K, group, same_fmt, act, out_dtype)), out_dtype
 
 
 def test_linear_call_with_leading_dimensions():
@@ -47,3 +55,20 @@ def test_linear_call_with_leading_dimensions():
     lin = bp.TernaryLinear(weights, 1024, "tq2", 128)
     x = torch.randn(2, 3, 1024, device="cuda", generator=gen).bfloat16()
     assert torch.equal(lin(x), lin(x.view(6, 1024)).view(2, 3, 256))
+
+
+# every digit that a row's 64-code pieces can start at inside a byte, rows at every address modulo 4, one row tile and more rows
+# than a workgroup stages, bytes past 242 (which decode to trit 0)
+@pytest.mark.parametrize("K", [1024, 1280, 1536, 1792, 2048, 7168])
+@pytest.mark.parametrize("N,offset", [(16, 0), (48, 1), (2064, 2), (1024, 3)])
+def test_tq1_rows_rewritten_as_tq2(K, N, offset):
+    import deepseekternarized_amd as bp
+
+    gen = torch.Generator(device="cuda").manual_seed(K + N)
+    Kp = bp.packed_cols("tq1", K)
+    bytes_ = torch.randint(0, 256, (N * Kp + offset,), dtype=torch.uint8, device="cuda", generator=gen)
+    packed = bytes_[offset:].view(N, Kp)
+    weights = [bp.PackedTerm(packed, (0.02 * torch.rand(N, K // 128, device="cuda", generator=gen)).half())]
+    x = torch.randn(6, K, device="cuda", generator=gen).bfloat16()
+    got = bp.TernaryLinear(weights, K, "tq1", 128, act="bf16")(x, torch.float32)
+    assert torch.equal(got, _steps(x, _as_tq2(weights, K), K, 128, "tq2", "bf16", torch.float32))
