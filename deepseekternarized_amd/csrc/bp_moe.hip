@@ -170,7 +170,7 @@ __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __
 
 // Layers whose two GEMMs run on the int8 kernel for token tiles of 128: int8 activations, TQ2, 64 rows per expert on average.
 // Whole layer with skewed routing against the kernel for tiles of 32, us: 2048 / 1024, 64 experts top-8, 512 tokens (64 rows) 137.5 / 164.3,
-// 768 145 / 219, 8192 957 / 2186 at the start; 4096 / 2048, top-6, 768 tokens (72 rows) 370 / 465, 2048 675 / 1027. With fewer rows the tiles are
+// 768 145 / 219, 8192 957 / 2175; 4096 / 2048, top-6, 768 tokens (72 rows) 370 / 465, 2048 675 / 1027. With fewer rows the tiles are
 // mostly padding (48 rows: 137 on tiles of 32, which 75 tiles of 128 take as well).
 bool moe_wide(int act, int fmt, int64_t n, int64_t T, int64_t E) { return act == BP_I8 && fmt == BP_TQ2 && T > 64 && n >= 64 * E; }
 
