@@ -106,9 +106,7 @@ __global__ __launch_bounds__(1024) void k_tq2_gemv_ks(GemmArgs a, int nw, int ti
   constexpr int SB = SDT == BP_F32 ? 4 : 2, NSL = SB / 2;  // bytes per scale; a wave's 16-byte loads of a round's scales
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int n = lane & 15, kb = lane >> 4;
-  const unsigned ey = expert_of_block(a, blockIdx.y);
-  if (ey == NO_EXPERT) return;  // (uniform)
-  const int64_t e = ey;
+  const int64_t e = blockIdx.y;
   const int64_t tok = clamp_i64(a.offsets[e], 0, a.T), o1 = clamp_i64(a.offsets[e + 1], 0, a.T);
   if (tok >= o1) return;  // (uniform: an expert without a token row)
   const int ntok = o1 - tok < NTOK ? (int)(o1 - tok) : NTOK;
@@ -442,7 +440,7 @@ int launch_tq2_gemv_fp4(const GemmArgs& a, hipStream_t s) {
   // stays whole rounds of the resident workgroups - 96 tiles per expert at four rows as 4 x 24, not 3 x 32)
   for (int64_t k = 2; per > per_max; ++k) per = ((tiles + k * wpe - 1) / (k * wpe) + KV_R - 1) / KV_R * KV_R;
   const size_t lds = (size_t)(slots + per * nw * 64 * ntok);
-  const dim3 grid((unsigned)((tiles + per - 1) / per), grid_experts(a), 1u);
+  const dim3 grid((unsigned)((tiles + per - 1) / per), (unsigned)a.E, 1u);
   if (a.E > 65535) return BP_ERR_UNSUPPORTED;
   if (a.scale_dtype == BP_F32) return launch_kv<BP_F32>(a, s, (int)nw, per, grid, lds, ntok);
   return a.scale_dtype == BP_F16 ? launch_kv<BP_F16>(a, s, (int)nw, per, grid, lds, ntok) : launch_kv<BP_BF16>(a, s, (int)nw, per, grid, lds, ntok);
