@@ -7,6 +7,7 @@
 #include <mutex>
 
 #include "../../include/bp_ternary.h"
+#include "bp_xcd.h"
 
 namespace bp {
 
@@ -116,30 +117,23 @@ __device__ __forceinline__ TileRef tile_ref(const GemmArgs& a, int64_t slot, uns
   return r;
 }
 
-// Which token tile and which block of output rows a workgroup of a token-tile kernel takes, from its linear index.
-// Workgroups are dealt to the 8 XCDs round-robin by linear index and each XCD has its own L2. The row blocks of a token
-// tile read the same activations and the token tiles of an expert the same weights, so an XCD takes its experts one after
-// the other, an expert's token tiles one after the other and a tile's row blocks one after the other: the workgroups
-// that run on it at one time share what they stream through its L2. In tile-list mode an expert's tiles are neighbours
-// in the list, and an XCD takes the list in runs of TILE_RUN entries. Without a list the launch's (expert, token tile,
-// row block) triples are one sequence, of which each XCD takes a contiguous eighth: with whole experts per XCD instead a
-// dense call (one expert) ran on a single XCD - a linear of 777 tokens x 4096 x 2048, TQ1 in two terms, 389 us against
-// 115, 8192 x 2048 x 6144 int8 on the 32-token tiles 2877 against 441.
+// Which token tile and which block of output rows a workgroup of a token-tile kernel takes, from its linear index. In
+// tile-list mode an expert's tiles are neighbours in the list, and an XCD takes the list in runs of TILE_RUN entries, a tile's
+// row blocks one after the other; without a list see bp_xcd.h.
 constexpr int TILE_RUN = 4;
 template <int ROWS = 32>
 __device__ __forceinline__ TileRef tile_of_workgroup(const GemmArgs& a, unsigned linear, int row_blocks, int& row_block) {
-  const unsigned xcd = linear & 7;
-  unsigned q = linear >> 3;
   if (a.tiles) {
+    const unsigned xcd = linear & 7;
+    unsigned q = linear >> 3;
     row_block = (int)(q % (unsigned)row_blocks);
     q /= (unsigned)row_blocks;
     return tile_ref<ROWS>(a, (int64_t)(q / TILE_RUN) * (8 * TILE_RUN) + xcd * TILE_RUN + q % TILE_RUN, 0);
   }
-  const unsigned tiles_per_expert = (unsigned)((a.max_rows + ROWS - 1) / ROWS);
-  const unsigned item = xcd * (gridDim.x >> 3) + q;  // (the grid is a multiple of 8: tile_workgroups; items past the experts are not live)
-  row_block = (int)(item % (unsigned)row_blocks);
-  const unsigned tile = item / (unsigned)row_blocks;
-  return tile_ref<ROWS>(a, tile / tiles_per_expert, tile % tiles_per_expert);
+  unsigned expert = 0, tile = 0, block = 0;
+  if (!tile_item(tile_split(a.E, a.max_rows, ROWS), linear, gridDim.x, (unsigned)row_blocks, expert, tile, block)) return {0, 0, 0, false};
+  row_block = (int)block;
+  return tile_ref<ROWS>(a, expert, tile);
 }
 // Workgroups of such a launch (-1: more than a grid's x extent holds).
 template <int ROWS = 32>
@@ -148,9 +142,7 @@ inline int64_t tile_workgroups(const GemmArgs& a, int64_t row_blocks) {
     const int64_t rounds = (a.tile_cap + 8 * TILE_RUN - 1) / (8 * TILE_RUN);
     return rounds > 0x7fffffff / (row_blocks * 8 * TILE_RUN) ? -1 : row_blocks * 8 * TILE_RUN * rounds;
   }
-  const int64_t z = (a.max_rows + ROWS - 1) / ROWS;
-  if (z > 0x7ffffff8 / row_blocks || a.E > 0x7ffffff8 / (row_blocks * z)) return -1;
-  return (a.E * z * row_blocks + 7) & ~(int64_t)7;
+  return tile_items(tile_split(a.E, a.max_rows, ROWS), row_blocks);
 }
 
 // Development overrides of the kernel selection (environment variables BP_TUNE_*), read once when the library is first

@@ -1,0 +1,76 @@
+// How a launch over token tiles deals its work out to the 8 XCDs. Plain integer arithmetic, for the host as well.
+#pragma once
+#include <stdint.h>
+
+#ifdef __HIPCC__
+#define BP_HOST_DEVICE __host__ __device__ __forceinline__
+#else
+#define BP_HOST_DEVICE inline
+#endif
+
+namespace bp {
+
+// Workgroups are dealt to the XCDs round-robin by linear index and each XCD has its own L2. A launch without a tile list has
+// (expert, token tile, row block) triples: the row blocks of a tile read the same activations, the tiles of an expert the same
+// weights. They are put in one sequence, of which XCD x takes the x-th contiguous eighth: a tile's row blocks are neighbours,
+// then a run's tiles (128 token rows of an expert), and the runs are ordered so that an eighth is what one XCD should have:
+//  * whole groups of eight experts: class c of the group i holds run 0 of expert 8 i + c, run 1 of expert 8 i + c - 1 (mod 8), ...
+//    Neighbouring experts fall on different XCDs, and an expert with many rows is spread over them by runs, whichever
+//    experts those are (a launch often has few experts with rows, next to each other or at some stride);
+//  * the E % 8 experts that are left over, or a launch of fewer than eight (one: a dense linear): one after the other, in
+//    whole, so that the eighths are equal whatever E is.
+// 64 experts x 2048 x 2048, 4096 rows, us (whole experts dealt by expert % 8 / the triples in plain expert order / this order): TQ1, bf16:
+// 64 rows each 108 / 111 / 105; 512 rows in eight neighbours 121 / 795 / 127, in every eighth expert 772 / 123 / 220; 1 to 127 rows,
+// ascending, 143 / 182 / 140. TQ2, int8, 512 rows in eight neighbours: 92 / 330 / 82.
+struct TileSplit {
+  unsigned experts, tiles_per_expert, tiles_per_run, runs;  // runs of an expert
+};
+BP_HOST_DEVICE TileSplit tile_split(int64_t E, int64_t max_rows, int tile_rows) {
+  TileSplit s;
+  s.experts = (unsigned)E;
+  s.tiles_per_expert = (unsigned)((max_rows + tile_rows - 1) / tile_rows);
+  const unsigned most = 128u / (unsigned)tile_rows;
+  s.runs = E < 8 ? 1u : (s.tiles_per_expert + most - 1) / most;
+  s.tiles_per_run = s.runs ? (s.tiles_per_expert + s.runs - 1) / s.runs : 0u;
+  return s;
+}
+// Items of the whole sequence, a multiple of 8 (-1: more than a grid's x extent holds). Some are empty (tile_item: false).
+inline int64_t tile_items(const TileSplit& s, int64_t row_blocks) {
+  const int64_t per_expert = (int64_t)s.runs * s.tiles_per_run;
+  if (per_expert > 0x7ffffff8 / row_blocks || (int64_t)s.experts > 0x7ffffff8 / (row_blocks * (per_expert > 0 ? per_expert : 1))) return -1;
+  return ((int64_t)s.experts * per_expert * row_blocks + 7) & ~(int64_t)7;
+}
+// The triple of workgroup `linear` of `items`; false: none.
+BP_HOST_DEVICE bool tile_item(const TileSplit& s, unsigned linear, unsigned items, unsigned row_blocks, unsigned& expert, unsigned& tile, unsigned& row_block) {
+  const unsigned item = (linear & 7) * (items >> 3) + (linear >> 3);
+  unsigned at = item / row_blocks;
+  row_block = item - at * row_blocks;
+  unsigned run = at / s.tiles_per_run;
+  tile = at - run * s.tiles_per_run;
+  const unsigned whole = s.experts >> 3, left = s.experts & 7;  // groups of eight, experts past them
+  // the classes in order: the first `left` of them hold one of the experts that are left over as well
+  const unsigned len = whole * s.runs, len1 = len + s.runs;
+  unsigned c;
+  if (run < left * len1) {
+    c = run / len1;
+    run -= c * len1;
+  } else {
+    if (len == 0) return false;
+    run -= left * len1;
+    const unsigned k = run / len;
+    c = left + k;
+    run -= k * len;
+    if (c >= 8) return false;
+  }
+  if (run < len) {
+    const unsigned i = run / s.runs, r = run - i * s.runs;
+    expert = 8 * i + ((c - r) & 7);
+    tile += r * s.tiles_per_run;
+  } else {
+    expert = 8 * whole + c;
+    tile += (run - len) * s.tiles_per_run;
+  }
+  return tile < s.tiles_per_expert;
+}
+
+}  // namespace bp
