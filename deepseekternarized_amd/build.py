@@ -17,6 +17,8 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "libbp_ternary_hip.so"
 SOURCES = ["bp_api.hip", "bp_general.hip", "bp_repack.hip", "bp_route.hip", "bp_gguf.hip", "bp_huffman.hip", "bp_moe.hip", "bp_mfma.hip", "bp_mfma_tq2.hip", "bp_gemm_tq2.hip", "bp_gemm_tq2f.hip", "bp_gemm_i8w.hip", "bp_mfma_tq1.hip", "bp_gemm_tq1.hip", "bp_tq1_gemv.hip", "bp_tq1_gemv_fp4.hip", "bp_tq1_gemv_cw.hip", "bp_tq2_gemv_fp4.hip"]
+# Compiled twice, for launches that add to their outputs and for those that replace them (BP_REPLACES in bp_common.h).
+TWICE = {"bp_mfma_tq2.hip", "bp_gemm_tq2.hip", "bp_mfma_tq1.hip", "bp_gemm_tq1.hip", "bp_tq1_gemv_fp4.hip", "bp_tq1_gemv_cw.hip"}
 # packed FP32 VALU ops are disabled for every device object of this library
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function", "-Wno-int-to-pointer-cast",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
@@ -29,10 +31,21 @@ NO_STATIC_LDS = {"bp_mfma_tq2.hip", "bp_gemm_tq2.hip", "bp_gemm_tq2f.hip", "bp_g
 _REMARK = "[-Rpass-analysis=kernel-resource-usage]"
 
 
-def _compile(src: str) -> Path:
-    obj = CSRC / (src + ".o")
+def _units() -> list[tuple[str, str]]:
+    """(source, case) of every object, the ones that take longest first; the case is "" or, of a source in TWICE, "add" or "set"."""
+    units = [(s, c) for s in SOURCES for c in (("add", "set") if s in TWICE else ("",))]
+    return sorted(units, key=lambda u: u[0] not in ("bp_tq1_gemv_cw.hip", "bp_tq1_gemv_fp4.hip"))
+
+
+def _object(unit: tuple[str, str]) -> Path:
+    return CSRC / (unit[0] + ("." + unit[1] if unit[1] else "") + ".o")
+
+
+def _compile(unit: tuple[str, str]) -> Path:
+    src, case = unit
+    obj = _object(unit)
     check = src in NO_STATIC_LDS
-    cmd = ["hipcc", *FLAGS, *(["-Rpass-analysis=kernel-resource-usage"] if check else []), "-c", str(CSRC / src), "-o", str(obj)]
+    cmd = ["hipcc", *FLAGS, *([f"-DBP_REPLACES={int(case == 'set')}"] if case else []), *(["-Rpass-analysis=kernel-resource-usage"] if check else []), "-c", str(CSRC / src), "-o", str(obj)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     noise = "is not a recognized feature for this target"
     lines = [l for l in res.stderr.splitlines() if noise not in l]
@@ -58,21 +71,21 @@ def _compile(src: str) -> Path:
     return obj
 
 
-def _fresh(src: str) -> bool:
-    """The object of `src` is newer than the source and every header (used by --incremental only)."""
-    obj = CSRC / (src + ".o")
+def _fresh(unit: tuple[str, str]) -> bool:
+    """The unit's object is newer than its source and every header (used by --incremental only)."""
+    obj = _object(unit)
     if not obj.exists():
         return False
-    deps = [CSRC / src, *CSRC.glob("*.h"), HERE.parent / "include" / "bp_ternary.h", Path(__file__)]
+    deps = [CSRC / unit[0], *CSRC.glob("*.h"), HERE.parent / "include" / "bp_ternary.h", Path(__file__)]
     return all(obj.stat().st_mtime > d.stat().st_mtime for d in deps)
 
 
 def build(verbose: bool = True, incremental: bool = False) -> Path:
     """Compiles every source (``incremental``: only those older than their inputs) and links the library."""
-    todo = [s for s in SOURCES if not (incremental and _fresh(s))]
+    todo = [u for u in _units() if not (incremental and _fresh(u))]
     with ThreadPoolExecutor(max_workers=7) as pool:
         list(pool.map(_compile, todo))
-    objs = [CSRC / (s + ".o") for s in SOURCES]
+    objs = [_object(u) for u in _units()]
     cmd = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,--no-undefined", *map(str, objs), "-o", str(LIB)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

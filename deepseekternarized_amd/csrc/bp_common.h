@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/bp_ternary.h"
 #include "bp_xcd.h"
@@ -35,7 +36,7 @@ struct GemmArgs {
   const int32_t* tile_count;
   int64_t tile_cap;
   int row_grid;   // decode launches: one blockIdx.y per token row instead of one per expert (expert_of_block; set by launch_mfma)
-  int overwrite;  // tile-list mode: the kernel's result replaces `out` instead of being added to it (one launch covers all of K and all terms)
+  int overwrite;  // the results replace `out` instead of being added to it
   // Workspace of the caller for kernels that convert the activations in a pass of their own (NULL: those kernels are not used).
   unsigned char* stage;
   int64_t stage_bytes;
@@ -235,11 +236,32 @@ __device__ __forceinline__ uint16_t swiglu_bits(float gate, float up, bool weigh
   return f32_to_bf16_bits(bf16_bits_to_f32(f32_to_bf16_bits(g / (1.0f + expf(-g)))) * u);
 }
 
-// One finished output: bf16 in place of the float32 one, or the float32 one replaced or added to.
-__device__ __forceinline__ void store_out(const GemmArgs& a, int64_t i, float v) {
-  if (a.out16) a.out16[i] = f32_to_bf16_bits(v);
-  else a.out[i] = (a.overwrite ? 0.f : a.out[i]) + v;
+// What happens to the outputs. A source is compiled for both cases where its kernels feel the difference (build.py,
+// BP_REPLACES): launches that add to float32 `out`, the grouped entry point's contract, and launches of a linear or a layer
+// that replace it or write bf16 `out16` instead. Elsewhere GemmArgs::overwrite decides. Tested at run time in every kernel, the
+// second case cost the first: spilled scalar registers in the streaming TQ1 kernels (192 against 185 with six loads per loader, two
+// tokens 34 against 24), and 2 - 10 % of a grouped launch's time (int8, 64 experts x 32 rows x 2048 x 2048: TQ1 61.0 -> 70.2 us).
+namespace {
+#ifdef BP_REPLACES
+constexpr int OUTPUTS = BP_REPLACES;  // 0: added to, 1: replaced
+#else
+constexpr int OUTPUTS = -1;  // by GemmArgs::overwrite
+#endif
+__device__ __forceinline__ bool replaces(const GemmArgs& a) { return OUTPUTS < 0 ? a.overwrite != 0 : OUTPUTS == 1; }
+// A kernel's epilogue f(OUT16): once for bf16 outputs and once for float32 ones, so that the branch is outside its loops (inside,
+// it kept the compiler from grouping an epilogue's loads).
+template <class F>
+__device__ __forceinline__ void with_output(const GemmArgs& a, F&& f) {
+  if (OUTPUTS != 0 && a.out16) f(std::true_type{});
+  else f(std::false_type{});
 }
+// One finished output.
+template <bool OUT16>
+__device__ __forceinline__ void store_out(const GemmArgs& a, int64_t i, float v) {
+  if (OUT16) a.out16[i] = f32_to_bf16_bits(v);
+  else a.out[i] = (replaces(a) ? 0.f : a.out[i]) + v;
+}
+}  // namespace
 
 __device__ __forceinline__ float load_act_f32(const void* p, int dtype, int64_t i) {
   if (dtype == BP_F32) return ((const float*)p)[i];

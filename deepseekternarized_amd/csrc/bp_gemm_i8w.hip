@@ -482,7 +482,7 @@ __global__ __launch_bounds__(WR * W_WT * 64, 2) void k_gemm_i8w(GemmArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int tk = 64 * wt + 16 * m + 4 * b + i;
-          if (tk < ntok) store_out(a, (tok0 + tk) * a.N + row + r16, total[r][m][i] * xs[m][i]);
+          if (tk < ntok) store_out<false>(a, (tok0 + tk) * a.N + row + r16, total[r][m][i] * xs[m][i]);
         }
     }
   }

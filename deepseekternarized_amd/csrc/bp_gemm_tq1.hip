@@ -431,24 +431,26 @@ __global__ __launch_bounds__(Q_THREADS, 2) void k_gemm_tq1(GemmArgs a) {
     }
 
     // ---- epilogue: lane holds tokens 4 kb + i of each token tile, output row n_wave + 16 r + r16
+    with_output(a, [&](auto out16) {
 #pragma unroll
-    for (int t = 0; t < TT; ++t) {
+      for (int t = 0; t < TT; ++t) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int tk = 16 * t + 4 * kb + i;
-        if (tk < ntok) {
-          const int64_t tok = tok0 + tk;
-          const float xs = ACT == BP_I8 ? a.x_scale[tok] : 1.0f;
+        for (int i = 0; i < 4; ++i) {
+          const int tk = 16 * t + 4 * kb + i;
+          if (tk < ntok) {
+            const int64_t tok = tok0 + tk;
+            const float xs = ACT == BP_I8 ? a.x_scale[tok] : 1.0f;
 #pragma unroll
-          for (int r = 0; r < Q_RT; ++r) {
-            const int64_t row = n_wave + 16 * r;
-            if (row < a.N) {
-              store_out(a, tok * a.N + row + r16, total[r][t][i] * xs);
+            for (int r = 0; r < Q_RT; ++r) {
+              const int64_t row = n_wave + 16 * r;
+              if (row < a.N) {
+                store_out<decltype(out16)::value>(a, tok * a.N + row + r16, total[r][t][i] * xs);
+              }
             }
           }
         }
       }
-    }
+    });
   };
   if (two) all_terms(QC<2>{});
   else all_terms(QC<1>{});
@@ -471,7 +473,7 @@ int launch_gemm_tq1_k(const GemmArgs& a, hipStream_t s, const char* name) {
 // Preconditions (beyond mfma_supports: groups of 128 or 256, K % 256 == 0, K >= 1024, N % 16 == 0, 16-byte aligned x):
 // bf16 or int8 activations; 4-byte aligned scale rows; K small enough for 32-bit offsets into a 32-token activation tile.
 // BP_ERR_UNSUPPORTED (no message): the caller falls back to its other kernels.
-int launch_gemm_tq1(const GemmArgs& a, hipStream_t s) {
+int BP_OUTPUTS(launch_gemm_tq1)(const GemmArgs& a, hipStream_t s) {
   if (a.stage && tuning().tq2g != 'b') {  // with a workspace: one matrix instruction per scale group over converted activations (bp_gemm_tq2f.hip; development: BP_TUNE_TQ2G=bf16 keeps this file's kernel)
     const int rc = launch_gemm_tq2f(a, s);
     if (rc != BP_ERR_UNSUPPORTED) return rc;

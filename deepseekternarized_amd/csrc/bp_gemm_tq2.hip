@@ -385,23 +385,25 @@ __global__ __launch_bounds__(GTHREADS, 2) void k_gemm_tq2(GemmArgs a) {
   else all_terms(std::integral_constant<int, 1>{});
 
   // ---- epilogue: lane holds tokens 4b + q of each token sub-tile, output row n0 + 16r + r16
+  with_output(a, [&](auto out16) {
 #pragma unroll
-  for (int mt = 0; mt < GT; ++mt) {
+    for (int mt = 0; mt < GT; ++mt) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int t = 16 * mt + 4 * b + q;
-      if (t < ntok) {
-        const int64_t tok = tok0 + t;
-        const float xs = ACT == BP_I8 ? a.x_scale[tok] : 1.0f;
+      for (int q = 0; q < 4; ++q) {
+        const int t = 16 * mt + 4 * b + q;
+        if (t < ntok) {
+          const int64_t tok = tok0 + t;
+          const float xs = ACT == BP_I8 ? a.x_scale[tok] : 1.0f;
 #pragma unroll
-        for (int r = 0; r < GR; ++r) {
-          if (rows_valid[r]) {
-            store_out(a, tok * a.N + n0 + 16 * r + r16, total[r][mt][q] * xs);
+          for (int r = 0; r < GR; ++r) {
+            if (rows_valid[r]) {
+              store_out<decltype(out16)::value>(a, tok * a.N + n0 + 16 * r + r16, total[r][mt][q] * xs);
+            }
           }
         }
       }
     }
-  }
+  });
 }
 
 template <int ACT, int SDT, int SL, int ABL = 0>
@@ -429,7 +431,7 @@ int launch_gemm_sd(const GemmArgs& a, hipStream_t s, const char* name, const cha
 }  // namespace
 
 // Preconditions (checked by mfma_supports): group 128, K % 256 == 0, K >= 1024, N % 16 == 0, 16-byte aligned x / packed / scales.
-int launch_gemm_tq2(const GemmArgs& a, hipStream_t s) {
+int BP_OUTPUTS(launch_gemm_tq2)(const GemmArgs& a, hipStream_t s) {
   if (a.stage && a.x_dtype == BP_I8 && !a.tiles && tuning().tq2g != 'b' && (tuning().tq2g == 'f' || i8w_pays(a.T, a.N, a.K, a.E))) {
     const int rc = launch_gemm_i8w(a, s);
     if (rc != BP_ERR_UNSUPPORTED) return rc;

@@ -650,23 +650,25 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a) {
       }
       return;
     }
+    with_output(a, [&](auto out16) {
 #pragma unroll
-    for (int t = 0; t < TT; ++t) {
+      for (int t = 0; t < TT; ++t) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int tk = 16 * t + 4 * kb + i;
-        if (tk < ntok) {
-          const int64_t tok = tok0 + tk;
+        for (int i = 0; i < 4; ++i) {
+          const int tk = 16 * t + 4 * kb + i;
+          if (tk < ntok) {
+            const int64_t tok = tok0 + tk;
 #pragma unroll
-          for (int r = 0; r < F_RT; ++r) {
-            const int64_t row = tile_row(wave, r);
-            if (row >= 0) {
-              store_out(a, tok * a.N + row + r16, total[r][t][i]);
+            for (int r = 0; r < F_RT; ++r) {
+              const int64_t row = tile_row(wave, r);
+              if (row >= 0) {
+                store_out<decltype(out16)::value>(a, tok * a.N + row + r16, total[r][t][i]);
+              }
             }
           }
         }
       }
-    }
+    });
   };
   if (two) all_windows(FC<2>{});
   else all_windows(FC<1>{});

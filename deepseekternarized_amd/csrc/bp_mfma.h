@@ -19,11 +19,23 @@
 
 namespace bp {
 
+// A launcher whose source is compiled twice (BP_REPLACES in bp_common.h): NAME_add for launches that add to their outputs,
+// NAME_set for those that replace them.
+#define BP_LAUNCHER(NAME, PARAMS, ARGS) \
+  int NAME##_add PARAMS;                \
+  int NAME##_set PARAMS;                \
+  inline int NAME PARAMS { return a.overwrite ? NAME##_set ARGS : NAME##_add ARGS; }
+#if defined(BP_REPLACES) && BP_REPLACES
+#define BP_OUTPUTS(NAME) NAME##_set
+#else
+#define BP_OUTPUTS(NAME) NAME##_add
+#endif
+
 // implemented in bp_mfma_tq2.hip / bp_mfma_tq1.hip; R, MT, waves: the tiling chosen by launch_mfma
-int launch_mfma_tq2(const GemmArgs& a, hipStream_t s, int R, int MT, int waves);
-int launch_mfma_tq1(const GemmArgs& a, hipStream_t s, int waves);
+BP_LAUNCHER(launch_mfma_tq2, (const GemmArgs& a, hipStream_t s, int R, int MT, int waves), (a, s, R, MT, waves))
+BP_LAUNCHER(launch_mfma_tq1, (const GemmArgs& a, hipStream_t s, int waves), (a, s, waves))
 // bp_gemm_tq2.hip: TQ2 with token tiles of 32 (experts with more than 16 token rows)
-int launch_gemm_tq2(const GemmArgs& a, hipStream_t s);
+BP_LAUNCHER(launch_gemm_tq2, (const GemmArgs& a, hipStream_t s), (a, s))
 int launch_gemm_tq2f(const GemmArgs& a, hipStream_t s);
 int gemm_tq2f_applies(const GemmArgs& a);  // BP_OK where launch_gemm_tq2f takes the call (nothing is launched)
 // bp_gemm_i8w.hip: TQ2 with int8 activations (or bf16 ones that it quantises: GemmArgs::quant) and token tiles of 128
@@ -39,7 +51,7 @@ inline bool i8w_pays(int64_t T, int64_t N, int64_t K, int64_t E) {
 }
 // bp_gemm_tq1.hip: TQ1 with token tiles of 32 on the fp8 x fp4 matrix instruction (experts with more than 8 token rows);
 // BP_ERR_UNSUPPORTED without a message when the call is outside its preconditions
-int launch_gemm_tq1(const GemmArgs& a, hipStream_t s);
+BP_LAUNCHER(launch_gemm_tq1, (const GemmArgs& a, hipStream_t s), (a, s))
 // TQ1 calls of seven or eight token rows per expert that run on the tile kernel over converted activations when the
 // caller brings a workspace, rather than as two launches of the four-row decode kernel: dense batches (four rows per
 // expert on average) of at least 512 blocks of 512 output rows. Measured with 8 rows per expert: 128 experts x 2048 x
@@ -53,7 +65,7 @@ int launch_tq1_gemv(const GemmArgs& a, hipStream_t s, int waves);
 // bp_tq1_gemv_fp4.hip: the same through the fp8 x fp4 matrix instruction (16-bit and int8 activations), and small
 // batches: up to 8 token rows per expert, or up to 64 in launches of 8 when the experts average at most 4 rows;
 // BP_ERR_UNSUPPORTED without a message when the call is outside its preconditions
-int launch_tq1_gemv_fp4(const GemmArgs& a, hipStream_t s);
+BP_LAUNCHER(launch_tq1_gemv_fp4, (const GemmArgs& a, hipStream_t s), (a, s))
 // bp_tq2_gemv_fp4.hip: TQ2, one to four token rows per expert, on the fp8 x fp4 matrix instruction with K split over the waves;
 // BP_ERR_UNSUPPORTED without a message when the call is outside its preconditions
 int launch_tq2_gemv_fp4(const GemmArgs& a, hipStream_t s);

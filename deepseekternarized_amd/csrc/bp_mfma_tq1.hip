@@ -335,13 +335,15 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq1(GemmArgs a, int CPT 
     }
   }
   // ---- epilogue: lane holds tokens 4b + q of output row n0 + r16 (NQ = 1: only token 0 is kept)
+  with_output(a, [&](auto out16) {
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int t = 4 * b + q;
-    if (t < ntok && wave_live) {
-      store_out(a, (tok0 + t) * a.N + n0 + r16, x_i8 ? total[q] * a.x_scale[tok0 + t] : total[q]);
+    for (int q = 0; q < NQ; ++q) {
+      const int t = 4 * b + q;
+      if (t < ntok && wave_live) {
+        store_out<decltype(out16)::value>(a, (tok0 + t) * a.N + n0 + r16, x_i8 ? total[q] * a.x_scale[tok0 + t] : total[q]);
+      }
     }
-  }
+  });
 }
 
 template <int SDT, int WAVES, int NQ, int SL, int MULTI, int ABL = 0>
@@ -387,7 +389,7 @@ int launch_tq1_v(const GemmArgs& a, hipStream_t s, const char* name_sl, const ch
 
 }  // namespace
 
-int launch_mfma_tq1(const GemmArgs& a, hipStream_t s, int waves) {
+int BP_OUTPUTS(launch_mfma_tq1)(const GemmArgs& a, hipStream_t s, int waves) {
 #ifdef BP_DEV_ABLATIONS  // timing ablations (results are wrong): development builds only
   if (const char* t = getenv("BP_TUNE_ABL")) {
     if (atoi(t) == 1) return launch_tq1<BP_F16, 16, 1, 1, 1>(a, s, "abl1_tq1");

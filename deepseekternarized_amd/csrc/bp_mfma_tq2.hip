@@ -301,23 +301,25 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq2(GemmArgs a, int KC, 
     }
   }
   // ---- epilogue: lane holds tokens 4b + q (q = 0..3) of each token tile, output row n0 + 16r + r16
+  with_output(a, [&](auto out16) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
+    for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {  // NQ = 1: single-token launches keep only the sums of token 0
-      const int t = 16 * mt + 4 * b + q;
-      if (t < ntok) {
-        const int64_t tok = tok0 + t;
-        const float xs = ACT == BP_I8 ? a.x_scale[tok] : 1.0f;
+      for (int q = 0; q < NQ; ++q) {  // NQ = 1: single-token launches keep only the sums of token 0
+        const int t = 16 * mt + 4 * b + q;
+        if (t < ntok) {
+          const int64_t tok = tok0 + t;
+          const float xs = ACT == BP_I8 ? a.x_scale[tok] : 1.0f;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          if (rows_valid[r]) {
-            store_out(a, tok * a.N + n0 + 16 * r + r16, total[r][mt][q] * xs);
+          for (int r = 0; r < R; ++r) {
+            if (rows_valid[r]) {
+              store_out<decltype(out16)::value>(a, tok * a.N + n0 + 16 * r + r16, total[r][mt][q] * xs);
+            }
           }
         }
       }
     }
-  }
+  });
 }
 
 template <int ACT, int SDT, int R, int MT, int WAVES, int XKB, int ABL = 0, int NQ = 4, int SL = 1>
@@ -362,7 +364,7 @@ int launch_tq2_sd(const GemmArgs& a, hipStream_t s, const char* name) {
 
 }  // namespace
 
-int launch_mfma_tq2(const GemmArgs& a, hipStream_t s, int R, int MT, int waves) {
+int BP_OUTPUTS(launch_mfma_tq2)(const GemmArgs& a, hipStream_t s, int R, int MT, int waves) {
   const bool bf = a.x_dtype == BP_BF16;
 #ifdef BP_DEV_ABLATIONS  // timing ablations (results are wrong): development builds only
   if (const char* t = getenv("BP_TUNE_ABL")) {

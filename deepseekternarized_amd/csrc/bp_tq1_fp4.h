@@ -10,7 +10,7 @@ namespace bp {
 
 // bp_tq1_gemv_cw.hip: the kernel that streams the rows through LDS tile by tile (one token row per expert or a pair,
 // rows first_row .. of every expert); BP_ERR_UNSUPPORTED without a message where it does not apply
-int launch_tq1_gemv_cw(const GemmArgs& a, hipStream_t s, int ntok, int64_t nchunks, int cus, int first_row);
+BP_LAUNCHER(launch_tq1_gemv_cw, (const GemmArgs& a, hipStream_t s, int ntok, int64_t nchunks, int cus, int first_row), (a, s, ntok, nchunks, cus, first_row))
 
 namespace {
 

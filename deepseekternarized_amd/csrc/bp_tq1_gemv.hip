@@ -275,7 +275,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_tq1_gemv(GemmArgs a, int CPT 
   total += __shfl_xor(total, 16);
   total += __shfl_xor(total, 32);
   if (b == 0 && wave_live) {
-    store_out(a, tok * a.N + n0 + r16, a.x_dtype == BP_I8 ? total * a.x_scale[tok] : total);
+    with_output(a, [&](auto out16) { store_out<decltype(out16)::value>(a, tok * a.N + n0 + r16, a.x_dtype == BP_I8 ? total * a.x_scale[tok] : total); });
   }
 }
 

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(CW_WAVES * 64) void k_tq1_gemv_cw(GemmArgs a, int n
 #pragma unroll
   for (int u = 0; u < CW_STAGE_PER_THREAD; ++u) {
     const int o = (int)threadIdx.x + u * THREADS;
-    was[u] = !a.out16 && !a.overwrite && o < n_stage && ((o >> 4) % NTOK) < ntok ? a.out[out_index(o)] : 0.f;
+    was[u] = !replaces(a) && o < n_stage && ((o >> 4) % NTOK) < ntok ? a.out[out_index(o)] : 0.f;
   }
 
   // ---- loaders: state of the current term (the expert's rows and scales as buffers of their own: a tile past N reads
@@ -439,7 +439,7 @@ __global__ __launch_bounds__(CW_WAVES * 64) void k_tq1_gemv_cw(GemmArgs a, int n
         if (tt % lpg == lidx && tile < tile_end && tt < ntok) {
           const int64_t at = (tok + tt) * a.N + tile * 16 + r16;
           const float v = __uint_as_float(*(const lds_u32*)(stage + (unsigned)((((int)(tile - tile0) * NTOK + tt) * 16 + r16) * 4)));
-          if (a.out16) a.out16[at] = f32_to_bf16_bits(v);
+          if (OUTPUTS == 1 && a.out16) a.out16[at] = f32_to_bf16_bits(v);
           else a.out[at] = v;
         }
       }
@@ -515,7 +515,7 @@ int launch_cw(const GemmArgs& a, hipStream_t s, int64_t nchunks, int cus, int fi
 
 }  // namespace
 
-int launch_tq1_gemv_cw(const GemmArgs& a, hipStream_t s, int ntok, int64_t nchunks, int cus, int first_row) {
+int BP_OUTPUTS(launch_tq1_gemv_cw)(const GemmArgs& a, hipStream_t s, int ntok, int64_t nchunks, int cus, int first_row) {
   if (ntok == 4) {  // (2-byte scales)
     if (a.scale_dtype == BP_F16) return launch_cw<BP_F16, 4>(a, s, nchunks, cus, first_row);
     if (a.scale_dtype == BP_BF16) return launch_cw<BP_BF16, 4>(a, s, nchunks, cus, first_row);

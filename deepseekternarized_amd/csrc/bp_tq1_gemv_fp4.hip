@@ -192,7 +192,7 @@ __global__ __launch_bounds__(WAVES * 64, KS ? 2 : 4) void k_tq1_gemv_fp4(GemmArg
     // with stacked terms the value may be one this wave stored a term ago.)
     // (up to 4 tokens; beyond, the registers are not there)
     constexpr bool EARLY = NTOK <= 4;
-    const bool fresh = a.out16 || (a.overwrite && term == 0 && first_chunk == 0);  // nothing to add to
+    const bool fresh = replaces(a) && (a.out16 || (term == 0 && first_chunk == 0));  // nothing to add to
     float before[NTOK > 1 ? NTOK : GR];
 #pragma unroll
     for (int s = 0; s < (NTOK > 1 ? NTOK : GR); ++s) {
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(WAVES * 64, KS ? 2 : 4) void k_tq1_gemv_fp4(GemmArg
     if (kb == 0 && wave_live && n0 + 16 * tile < a.N && tt < ntok) {
       const int64_t at = (tok + tt) * a.N + n0 + 16 * tile + r16;
       const float v = a.x_dtype == BP_I8 ? t * xsc[tt] : t;
-      if (a.out16) {  // (one term, all of K in this launch)
+      if (OUTPUTS == 1 && a.out16) {  // (one term, all of K in this launch)
         a.out16[at] = f32_to_bf16_bits(v);
         continue;
       }
@@ -660,7 +660,7 @@ int launch_f4_any(const GemmArgs& a, hipStream_t s) {
 }
 }  // namespace
 
-int launch_tq1_gemv_fp4(const GemmArgs& a, hipStream_t s) {
+int BP_OUTPUTS(launch_tq1_gemv_fp4)(const GemmArgs& a, hipStream_t s) {
   if (a.x_dtype != BP_BF16 && a.x_dtype != BP_F16 && a.x_dtype != BP_I8) return BP_ERR_UNSUPPORTED;
   if (a.max_rows > 1 && a.x_dtype == BP_F16) return BP_ERR_UNSUPPORTED;  // (11 significant bits need the third piece)
   int64_t few = 4;  // "most experts have few rows": at most this many routed rows per expert on average
