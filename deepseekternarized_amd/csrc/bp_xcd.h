@@ -45,6 +45,11 @@ BP_HOST_DEVICE bool tile_item(const TileSplit& s, unsigned linear, unsigned item
   const unsigned item = (linear & 7) * (items >> 3) + (linear >> 3);
   unsigned at = item / row_blocks;
   row_block = item - at * row_blocks;
+  if (s.experts == 1) {  // (a dense call: no more divisions)
+    expert = 0;
+    tile = at;
+    return tile < s.tiles_per_expert;
+  }
   unsigned run = at / s.tiles_per_run;
   tile = at - run * s.tiles_per_run;
   const unsigned whole = s.experts >> 3, left = s.experts & 7;  // groups of eight, experts past them
