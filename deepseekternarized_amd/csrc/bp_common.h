@@ -118,20 +118,15 @@ __device__ __forceinline__ TileRef tile_ref(const GemmArgs& a, int64_t slot, uns
   return r;
 }
 
-// Which token tile and which block of output rows a workgroup of a token-tile kernel takes, from its linear index. In
-// tile-list mode an expert's tiles are neighbours in the list, and an XCD takes the list in runs of TILE_RUN entries, a tile's
-// row blocks one after the other; without a list see bp_xcd.h.
-constexpr int TILE_RUN = 4;
+// Which token tile and which block of output rows a workgroup of a token-tile kernel takes, from its linear index: bp_xcd.h.
 template <int ROWS = 32>
 __device__ __forceinline__ TileRef tile_of_workgroup(const GemmArgs& a, unsigned linear, int row_blocks, int& row_block) {
-  if (a.tiles) {
-    const unsigned xcd = linear & 7;
-    unsigned q = linear >> 3;
-    row_block = (int)(q % (unsigned)row_blocks);
-    q /= (unsigned)row_blocks;
-    return tile_ref<ROWS>(a, (int64_t)(q / TILE_RUN) * (8 * TILE_RUN) + xcd * TILE_RUN + q % TILE_RUN, 0);
-  }
   unsigned expert = 0, tile = 0, block = 0;
+  if (a.tiles) {
+    const unsigned slot = list_item(ROWS, linear, (unsigned)row_blocks, block);
+    row_block = (int)block;
+    return tile_ref<ROWS>(a, slot, 0);
+  }
   if (!tile_item(tile_split(a.E, a.max_rows, ROWS), linear, gridDim.x, (unsigned)row_blocks, expert, tile, block)) return {0, 0, 0, false};
   row_block = (int)block;
   return tile_ref<ROWS>(a, expert, tile);
@@ -139,11 +134,7 @@ __device__ __forceinline__ TileRef tile_of_workgroup(const GemmArgs& a, unsigned
 // Workgroups of such a launch (-1: more than a grid's x extent holds).
 template <int ROWS = 32>
 inline int64_t tile_workgroups(const GemmArgs& a, int64_t row_blocks) {
-  if (a.tiles) {
-    const int64_t rounds = (a.tile_cap + 8 * TILE_RUN - 1) / (8 * TILE_RUN);
-    return rounds > 0x7fffffff / (row_blocks * 8 * TILE_RUN) ? -1 : row_blocks * 8 * TILE_RUN * rounds;
-  }
-  return tile_items(tile_split(a.E, a.max_rows, ROWS), row_blocks);
+  return a.tiles ? list_items(ROWS, a.tile_cap, row_blocks) : tile_items(tile_split(a.E, a.max_rows, ROWS), row_blocks);
 }
 
 // Development overrides of the kernel selection (environment variables BP_TUNE_*), read once when the library is first

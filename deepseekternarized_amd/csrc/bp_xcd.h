@@ -78,4 +78,18 @@ BP_HOST_DEVICE bool tile_item(const TileSplit& s, unsigned linear, unsigned item
   return tile < s.tiles_per_expert;
 }
 
+// With a list of the token tiles that exist, in expert order: an XCD takes the list in runs of 128 token rows, a tile's row
+// blocks one after the other. (Runs of four tiles whatever their rows left a layer with 16 tiles of 128 to four XCDs: 8 experts
+// top-2, 1024 rows, hidden 7168 / intermediate 2048, int8, 287 us against 177.)
+BP_HOST_DEVICE unsigned list_item(int tile_rows, unsigned linear, unsigned row_blocks, unsigned& row_block) {
+  const unsigned run = 128u / (unsigned)tile_rows, xcd = linear & 7, q = linear >> 3, at = q / row_blocks;
+  row_block = q - at * row_blocks;
+  return at / run * (8 * run) + xcd * run + at % run;
+}
+// Workgroups for a list of up to `cap` tiles (-1: as above); positions past the list's end hold no tile.
+inline int64_t list_items(int tile_rows, int64_t cap, int64_t row_blocks) {
+  const int64_t per = 8 * (128 / tile_rows), rounds = (cap + per - 1) / per;
+  return rounds > 0x7fffffff / (row_blocks * per) ? -1 : row_blocks * per * rounds;
+}
+
 }  // namespace bp

@@ -21,6 +21,15 @@ extern "C" void deal(long E, long max_rows, int rows, long blocks, int* out) {  
     out[3 * i] = any ? (int)e : -1, out[3 * i + 1] = any ? (int)t : -1, out[3 * i + 2] = any ? (int)b : -1;
   }
 }
+extern "C" long listed(long cap, int rows, long blocks) { return bp::list_items(rows, cap, blocks); }
+extern "C" void deal_list(long cap, int rows, long blocks, int* out) {  // per workgroup: position in the list, row block
+  const unsigned n = (unsigned)bp::list_items(rows, cap, blocks);
+  for (unsigned i = 0; i < n; ++i) {
+    unsigned b = 0;
+    out[2 * i] = (int)bp::list_item(rows, i, (unsigned)blocks, b);
+    out[2 * i + 1] = (int)b;
+  }
+}
 """
 
 
@@ -39,7 +48,15 @@ def deal(tmp_path_factory):
         lib.deal(E, max_rows, rows, blocks, out)
         return [(i & 7, out[3 * i], out[3 * i + 1], out[3 * i + 2]) for i in range(n) if out[3 * i] >= 0], n
 
-    run.items = lib.items
+    def run_list(cap, rows, blocks):
+        n = lib.listed(cap, rows, blocks)
+        out = (C.c_int * (2 * n))()
+        lib.deal_list(cap, rows, blocks, out)
+        return [(i & 7, out[2 * i], out[2 * i + 1]) for i in range(n)]
+
+    lib.listed.restype, lib.listed.argtypes = C.c_long, [C.c_long, C.c_int, C.c_long]
+    lib.deal_list.argtypes = [C.c_long, C.c_int, C.c_long, C.POINTER(C.c_int)]
+    run.items, run.list = lib.items, run_list
     return run
 
 
@@ -72,3 +89,12 @@ def test_hot_experts_are_spread(deal, E, hot, rows_each, worst):
 def test_more_workgroups_than_a_grid_holds(deal):
     assert deal.items(65535, 1 << 20, 32, 64) == -1 and deal.items(1, 1 << 31, 32, 1 << 10) == -1
     assert 0 < deal.items(1, 1 << 20, 32, 32) <= 0x7FFFFFF8
+
+
+@pytest.mark.parametrize("rows", [32, 128])
+def test_lists_of_tiles(deal, rows):
+    """Every position of a list once with every row block; 128 token rows in a row on one XCD, the next 128 on the next."""
+    for cap in (1, 7, 16, 100):
+        got = deal.list(cap, rows, 3)
+        assert sorted(g[1:] for g in got) == [(p, b) for p in range(len(got) // 3) for b in range(3)] and len(got) // 3 >= cap
+        assert all(xcd == p * rows // 128 % 8 for xcd, p, _ in got)
