@@ -168,11 +168,17 @@ __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __
   }
 }
 
-// Layers whose two GEMMs run on the int8 kernel for token tiles of 128: int8 activations, TQ2, 64 rows per expert on average.
-// Whole layer with skewed routing against the kernel for tiles of 32, us: 2048 / 1024, 64 experts top-8, 512 tokens (64 rows) 137.5 / 164.3,
-// 768 145 / 219, 8192 957 / 2175; 4096 / 2048, top-6, 768 tokens (72 rows) 370 / 465, 2048 675 / 1027. With fewer rows the tiles are
-// mostly padding (48 rows: 137 on tiles of 32, which 75 tiles of 128 take as well).
-bool moe_wide(int act, int fmt, int64_t n, int64_t T, int64_t E) { return act == BP_I8 && fmt == BP_TQ2 && T > 64 && n >= 64 * E; }
+// Layers whose two GEMMs run on the int8 kernel for token tiles of 128: int8 activations, TQ2, 64 rows per expert on average, 1024
+// rows and 80 blocks of 128 rows x 256 gate | up rows (128 with stacked terms). Whole layer against the kernel for tiles of 32, us
+// (hidden / intermediate, experts, rows): 2048 / 1024, 64 experts, 4096 rows (64 per expert) 137.5 / 164.3 (48 per expert: 137 on tiles of
+// 32, which 75 tiles of 128, mostly padding, take as well); 4096 / 2048, 8 experts, 768 rows 108 / 103, 1024 rows 119 / 171; 2048 / 4096, 8
+// experts, 768 rows 121 / 114, 1024 rows 148 / 189; 2048 / 1024, 4 experts, 512 rows 66 / 53, 1024 rows (64 blocks) 70 / 77, in two terms
+// 103 / 99; 1024 / 1024, 16 experts, 1024 rows 60.5 / 59.2, 1536 rows (96 blocks) 64.1 / 63.4 and in two terms 78.4 / 73.2, 2048 rows
+// 69.9 / 85.0 and 88.1 / 100.5.
+bool moe_wide(int act, int fmt, int64_t n, int64_t T, int64_t E, int64_t I, int n_terms) {
+  return act == BP_I8 && fmt == BP_TQ2 && T > 64 && n >= 64 * E && n >= 1024 &&
+         n / I8W_TOK * ((2 * I + 255) / 256) >= (n_terms == 1 ? 80 : 128);
+}
 
 struct Carve {
   unsigned char* base;
@@ -221,7 +227,7 @@ Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k
   p.h = c.take(2 * (size_t)n * I);
   p.y = (float*)c.take(4 * (size_t)n * H);
   p.stage_bytes = 0;
-  if (moe_wide(act, fmt, n, T, E)) {
+  if (moe_wide(act, fmt, n, T, E, I, 1)) {  // (the size covers any number of terms)
     const size_t a = gemm_i8w_workspace_bytes(n, H, E), b = gemm_i8w_workspace_bytes(n, I, E);
     p.stage_bytes = a > b ? a : b;
   }
@@ -309,7 +315,7 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   // pass of either GEMM gathers or quantises its rows; gate | up applies SwiGLU and the down projection writes bf16 rows.
   GemmArgs wide_gu, wide_down;
   bool wide = false;
-  if (moe_wide(act, fmt, n, T, E) && tiles && !small && aligned16 && kernel_policy() != 1 && tuning().glu != 'n' && tuning().tq2g != 'b') {
+  if (moe_wide(act, fmt, n, T, E, I, n_terms) && tiles && !small && aligned16 && kernel_policy() != 1 && tuning().glu != 'n' && tuning().tq2g != 'b') {
     memset(&wide_gu, 0, sizeof(wide_gu));
     GemmArgs& a = wide_gu;
     a.offsets = p.offsets; a.x_dtype = BP_I8; a.scale_dtype = scale_dtype; a.n_terms = n_terms; a.fmt = fmt; a.group = group;

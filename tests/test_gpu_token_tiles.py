@@ -127,3 +127,26 @@ def test_int8_layer_on_tiles_of_128(tune, pattern, T, E, k, terms):
         ref = moe.composed(x, logits)
     assert torch.isfinite(got).all()
     assert float((got.double() - ref.double()).norm() / ref.double().norm()) <= 4e-3
+
+
+# either side of the line: 896 and 1024 rows, 72 and 80 blocks of 128 rows x 256 gate | up rows (two terms: 120 and 128)
+@pytest.mark.parametrize("T,E,k,I,terms,wide", [(448, 8, 2, 4096, 1, False), (512, 8, 2, 4096, 1, True), (1152, 4, 1, 1024, 1, False), (1280, 4, 1, 1024, 1, True),
+                                                (960, 8, 2, 1024, 2, False), (1024, 8, 2, 1024, 2, True)])
+def test_int8_layers_with_few_blocks_stay_on_tiles_of_32(T, E, k, I, terms, wide):
+    import deepseekternarized_amd as bp
+    from deepseekternarized_amd.moe import TernaryMoE
+
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    H = 1024
+
+    def terms_of(N, K):
+        return [(bp.pack(torch.randint(-1, 2, (E * N, K), dtype=torch.int8, device="cuda", generator=gen), "tq2").view(E, N, -1),
+                 (0.02 * torch.rand(E, N, K // 128, device="cuda", generator=gen)).half()) for _ in range(terms)]
+
+    moe = TernaryMoE(terms_of(I, H), terms_of(I, H), terms_of(H, I), H, I, k, "tq2", 128, act="int8")
+    x = torch.randn(T, H, device="cuda", generator=gen).bfloat16()
+    logits = torch.randn(T, E, device="cuda", generator=gen)
+    got = moe(x, logits)
+    assert ("i8w" in bp.ext().last_kernel()) == wide
+    ref = moe.composed(x, logits)
+    assert float((got.double() - ref.double()).norm() / ref.double().norm()) <= 4e-3  # (bf16 roundings and int8 steps that fall otherwise)
