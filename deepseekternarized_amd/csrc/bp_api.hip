@@ -183,9 +183,10 @@ extern "C" size_t bp_grouped_gemm_workspace_bytes(int x_dtype, int64_t T, int64_
   return staged_workspace_bytes(T, N, K, E, fmt, max_rows);
 }
 
-extern "C" size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows) {
-  if (fmt != BP_TQ2 || T <= 0 || E <= 0 || N <= 0 || K <= 0 || max_rows <= 16 || tuning().tq2g == 'b') return 0;
-  return tuning().tq2g == 'f' || i8w_pays(T, N, K, E) ? gemm_i8w_workspace_bytes(T, K, E) : 0;
+extern "C" size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t group, int64_t E, int fmt, int n_terms, int64_t max_rows) {
+  if (fmt != BP_TQ2 || T <= 0 || E <= 0 || N <= 0 || K <= 0 || n_terms < 1 || n_terms > BP_MAX_TERMS || max_rows <= 16 || tuning().tq2g == 'b') return 0;
+  if (!i8w_takes(N, K, group, n_terms, max_rows < T ? max_rows : T)) return 0;
+  return tuning().tq2g == 'f' || i8w_pays(T, N, K, E, n_terms) ? gemm_i8w_workspace_bytes(T, K, E) : 0;
 }
 
 static size_t staged_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows) {
@@ -228,7 +229,7 @@ struct LinearPlan {  // offsets into the workspace
 // every weight for eight token tiles (4096 tokens x 4096 x 4096: 159 / 283).
 bool repack_pays(int64_t T, int64_t N, int64_t K) { return T >= 256 || (T >= 5 && N <= ((int64_t)1 << 26) / K); }
 size_t repacked_bytes(int64_t N, int64_t K) { return ((size_t)N * (size_t)(K / 4) + 255) & ~(size_t)255; }
-LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int fmt, int n_terms) {
+LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int64_t group, int fmt, int n_terms) {
   LinearPlan p;
   p.repack = fmt == BP_TQ1 && repack_pays(T, N, K) && K % 256 == 0 && K >= 1024 && K <= 65536 && tuning().tq2g != 'b';
   if (p.repack) fmt = BP_TQ2;
@@ -237,7 +238,7 @@ LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int6
   p.q = take(act_int8 ? (size_t)T * (size_t)K : 0);
   p.q_scale = take(act_int8 ? 4 * (size_t)T : 0);
   p.sums = take(out_dtype == BP_F32 ? 0 : 4 * (size_t)T * (size_t)N);
-  p.stage_bytes = act_int8 ? bp_grouped_gemm_int8_workspace_bytes(T, N, K, 1, fmt, T) : bp_grouped_gemm_workspace_bytes(x_dtype, T, N, K, 1, fmt, T);
+  p.stage_bytes = act_int8 ? bp_grouped_gemm_int8_workspace_bytes(T, N, K, group, 1, fmt, n_terms, T) : bp_grouped_gemm_workspace_bytes(x_dtype, T, N, K, 1, fmt, T);
   p.stage = take(p.stage_bytes);
   p.repacked = take(p.repack ? (size_t)n_terms * repacked_bytes(N, K) : 0);
   p.bytes = at;
@@ -251,9 +252,9 @@ unsigned fill_grid(int64_t n) { return (unsigned)((n + 255) / 256 > 16384 ? 1638
 }  // namespace
 }  // namespace bp
 
-extern "C" size_t bp_ternary_linear_workspace_bytes(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int fmt, int n_terms) {
+extern "C" size_t bp_ternary_linear_workspace_bytes(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int64_t group, int fmt, int n_terms) {
   if (T <= 0 || N <= 0 || K <= 0 || n_terms < 1 || n_terms > BP_MAX_TERMS) return 0;
-  return linear_plan(x_dtype, act_int8, out_dtype, T, N, K, fmt, n_terms).bytes;
+  return linear_plan(x_dtype, act_int8, out_dtype, T, N, K, group, fmt, n_terms).bytes;
 }
 
 extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_dtype, int act_int8, const int64_t* offsets,
@@ -268,7 +269,7 @@ extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_
   const hipStream_t s = (hipStream_t)stream;
   unsigned char* ws = (unsigned char*)workspace;
   LinearPlan p = {};
-  if (T > 0 && N > 0 && K > 0 && n_terms >= 1 && n_terms <= BP_MAX_TERMS) p = linear_plan(x_dtype, act_int8, out_dtype, T, N, K, fmt, n_terms);
+  if (T > 0 && N > 0 && K > 0 && n_terms >= 1 && n_terms <= BP_MAX_TERMS) p = linear_plan(x_dtype, act_int8, out_dtype, T, N, K, group, fmt, n_terms);
   if (p.bytes && (!ws || workspace_bytes < p.bytes)) return fail(BP_ERR_ARG, "the workspace must hold bp_ternary_linear_workspace_bytes() = %zu bytes", p.bytes);
   GemmArgs a;
   bool empty;

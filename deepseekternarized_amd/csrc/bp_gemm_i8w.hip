@@ -496,18 +496,16 @@ __global__ __launch_bounds__(WR * W_WT * 64, 2) void k_gemm_i8w(GemmArgs a) {
   }
 }
 
-int64_t i8w_lds_bytes(const GemmArgs& a, int WR) { return W_SC + a.n_terms * i8w_rows(WR) * (a.K / 128 + 2) * 4; }
 int64_t i8w_row_blocks(const GemmArgs& a, int WR) {
   const int64_t rows = a.glu_h ? a.N / 2 : a.N, per = a.glu_h ? i8w_rows(WR) / 2 : i8w_rows(WR);
   return (rows + per - 1) / per;
 }
-// Two workgroups to a CU where their LDS allows it.
-int i8w_wr(const GemmArgs& a) { return i8w_lds_bytes(a, 2) <= 80 * 1024 ? 2 : 4; }
+static_assert(W_SC == I8W_STAGED && i8w_rows(2) == 64 * 2, "i8w_lds_bytes");
 template <int WR>
 int launch_i8w(const GemmArgs& a, hipStream_t s) {
   if (const int rc = raise_lds_limit<k_gemm_i8w<WR>>(160 * 1024)) return rc;
   note_kernel("gemm_tq2_i8w");
-  hipLaunchKernelGGL(k_gemm_i8w<WR>, dim3((unsigned)tile_workgroups<W_TOK>(a, i8w_row_blocks(a, WR))), dim3(WR * W_WT * 64), (size_t)i8w_lds_bytes(a, WR), s, a);
+  hipLaunchKernelGGL(k_gemm_i8w<WR>, dim3((unsigned)tile_workgroups<W_TOK>(a, i8w_row_blocks(a, WR))), dim3(WR * W_WT * 64), (size_t)i8w_lds_bytes(a.K, a.n_terms, WR), s, a);
   return check_launch("gemm_tq2_i8w");
 }
 
@@ -526,12 +524,10 @@ int gemm_i8w_applies(const GemmArgs& a) {
   if (!a.stage || ((uintptr_t)a.stage & 255) != 0) return BP_ERR_UNSUPPORTED;
   const size_t need = gemm_i8w_workspace_bytes(a.T, a.K, a.E);
   if (need == 0 || (size_t)a.stage_bytes < need) return BP_ERR_UNSUPPORTED;
-  if (a.K > ((int64_t)1 << 20) || a.N * a.Kp > ((int64_t)1 << 31) - 4096) return BP_ERR_UNSUPPORTED;
-  const int WR = i8w_wr(a);
-  if (i8w_lds_bytes(a, WR) > 160 * 1024) return BP_ERR_UNSUPPORTED;
+  if (!i8w_takes(a.N, a.K, a.group, a.n_terms, a.max_rows)) return BP_ERR_UNSUPPORTED;
+  const int WR = i8w_wr(a.K, a.n_terms);
   if (a.glu_h && a.N % 32 != 0) return BP_ERR_UNSUPPORTED;
   if ((((uintptr_t)a.glu_h | (uintptr_t)a.out16) & 15) != 0) return BP_ERR_UNSUPPORTED;  // (16-byte pieces of bf16 rows)
-  if ((a.max_rows + W_TOK - 1) / W_TOK > 65535) return BP_ERR_UNSUPPORTED;
   return tile_workgroups<W_TOK>(a, i8w_row_blocks(a, WR)) < 0 ? BP_ERR_UNSUPPORTED : BP_OK;
 }
 
@@ -546,7 +542,7 @@ int launch_gemm_i8w(const GemmArgs& a, hipStream_t s) {
   else if (a.K <= 2048) hipLaunchKernelGGL((k_stage_i8w<BP_BF16, 2>), sgrid, dim3(W_THREADS), red, s, a);
   else hipLaunchKernelGGL((k_stage_i8w<BP_BF16, 4>), sgrid, dim3(W_THREADS), red, s, a);
   if (const int rc = check_launch("stage_i8w")) return rc;
-  return i8w_wr(a) == 2 ? launch_i8w<2>(a, s) : launch_i8w<4>(a, s);
+  return i8w_wr(a.K, a.n_terms) == 2 ? launch_i8w<2>(a, s) : launch_i8w<4>(a, s);
 }
 
 }  // namespace bp

@@ -432,7 +432,7 @@ int launch_gemm_sd(const GemmArgs& a, hipStream_t s, const char* name, const cha
 
 // Preconditions (checked by mfma_supports): group 128, K % 256 == 0, K >= 1024, N % 16 == 0, 16-byte aligned x / packed / scales.
 int BP_OUTPUTS(launch_gemm_tq2)(const GemmArgs& a, hipStream_t s) {
-  if (a.stage && a.x_dtype == BP_I8 && !a.tiles && tuning().tq2g != 'b' && (tuning().tq2g == 'f' || i8w_pays(a.T, a.N, a.K, a.E))) {
+  if (a.stage && a.x_dtype == BP_I8 && !a.tiles && tuning().tq2g != 'b' && (tuning().tq2g == 'f' || i8w_pays(a.T, a.N, a.K, a.E, a.n_terms))) {
     const int rc = launch_gemm_i8w(a, s);
     if (rc != BP_ERR_UNSUPPORTED) return rc;
   }

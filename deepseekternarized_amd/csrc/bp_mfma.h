@@ -40,14 +40,29 @@ int launch_gemm_tq2f(const GemmArgs& a, hipStream_t s);
 int gemm_tq2f_applies(const GemmArgs& a);  // BP_OK where launch_gemm_tq2f takes the call (nothing is launched)
 // bp_gemm_i8w.hip: TQ2 with int8 activations (or bf16 ones that it quantises: GemmArgs::quant) and token tiles of 128
 constexpr int I8W_TOK = 128;
+constexpr int I8W_STAGED = 2 * (2 * 2 * (I8W_TOK / 16) * 1024 + 2 * I8W_TOK * 4);  // LDS: two staged windows of the activations
 int launch_gemm_i8w(const GemmArgs& a, hipStream_t s);
 int gemm_i8w_applies(const GemmArgs& a);  // BP_OK where launch_gemm_i8w takes the call (nothing is launched)
-// Calls that run on it when the caller brings a workspace: launches that fill most of the device, with less for rows that
-// run as two small workgroups per CU. Linears on it against the 32-token tiles, us: 1024 tokens x 2048 x 7168 41.6 / 58.7,
-// 768 x 2048 x 6144 (144 blocks) 40.2 / 45.7, 2048 x 2048 x 2048 (128) 33.1 / 36.6, 512 x 2048 x 6144 (96) 31.1 / 32.2, 256 x 2048 x 6144
-// 30.4 / 19.4; eight waves: 2048 x 4096 x 4096 (256) 68.0 / 92.8, 1024 x 4096 x 4096 (128) 62.6 / 50.2, 2048 x 7168 x 2048 (128) 99 / 77.8.
-inline bool i8w_pays(int64_t T, int64_t N, int64_t K, int64_t E) {
-  return T >= 64 * E && (T + I8W_TOK - 1) / I8W_TOK * ((N + 255) / 256) >= (K <= 3328 ? 128 : 192);
+// LDS of a workgroup of 64 WR rows: the staged windows and the rows' scales of all terms, float32. WR = 2 where two workgroups
+// fit a CU, else 4, or 0 where that does not fit either.
+inline int64_t i8w_lds_bytes(int64_t K, int n_terms, int WR) { return I8W_STAGED + (int64_t)n_terms * 64 * WR * (K / 128 + 2) * 4; }
+inline int i8w_wr(int64_t K, int n_terms) { return i8w_lds_bytes(K, n_terms, 2) <= 80 * 1024 ? 2 : i8w_lds_bytes(K, n_terms, 4) <= 160 * 1024 ? 4 : 0; }
+// Sizes that the kernel takes (beside them: alignments and workspace, gemm_i8w_applies and mfma_supports).
+inline bool i8w_takes(int64_t N, int64_t K, int64_t group, int n_terms, int64_t max_rows) {
+  return (group == 128 || (group == 256 && K >= 2048)) && K % 256 == 0 && K >= 1024 && K <= ((int64_t)1 << 20) && N % 16 == 0 && i8w_wr(K, n_terms) != 0 &&
+         N * (K / 4) <= ((int64_t)1 << 31) - 4096 && (max_rows + I8W_TOK - 1) / I8W_TOK <= 65535;
+}
+// Calls that run on it when the caller brings a workspace, by the blocks of 128 tokens x 256 rows that hold work if every tile is full.
+// One expert: from 128 blocks on as two small workgroups per CU (WR = 2), from 192 as one of eight waves, which takes as long for 64
+// blocks as for 256. us on it / on the 32-token tiles: 2048 x 2048 x 2048 (128 blocks) 32.8 / 35.5, 512 x 2048 x 6144 (96) 31.1 / 31.9,
+// 1024 x 2048 x 2048 (64) 30.9 / 20.4; eight waves: 3072 x 4096 x 2048 (192) 65.7 / 73.5, 2048 x 4096 x 2048 (128) 63.7 / 51.8, in two
+// terms 2048 x 2048 x 2048 (128) 56.8 / 51.2, 3072 x 2048 x 2048 (192) 60.0 / 73.3, 1024 x 7168 x 6144 (192) 100.6 / 103.9.
+// Several experts, whose last tiles are partly empty: from 112 rows per expert and 384 blocks on. 64 experts x 2048 x 2048, 64 / 80 / 96 /
+// 112 / 128 rows each: 1.26 / 1.03 / 1.02 / 0.86 / 0.80 of the time on the 32-token tiles (with 0 to twice as many rows: 1.04 / 1.01 / 0.99 /
+// 0.91 / 0.88); 16 experts x 2048 x 4096 at 256 rows (256 blocks) 0.91 and 1.09, 16 x 4096 x 1024 at 192 (384) 1.05 and 0.94.
+inline bool i8w_pays(int64_t T, int64_t N, int64_t K, int64_t E, int n_terms) {
+  const int64_t blocks = (T + I8W_TOK - 1) / I8W_TOK * ((N + 255) / 256);
+  return E == 1 ? blocks >= (i8w_wr(K, n_terms) == 2 ? 128 : 192) : T >= 112 * E && blocks >= 384;
 }
 // bp_gemm_tq1.hip: TQ1 with token tiles of 32 on the fp8 x fp4 matrix instruction (experts with more than 8 token rows);
 // BP_ERR_UNSUPPORTED without a message when the call is outside its preconditions

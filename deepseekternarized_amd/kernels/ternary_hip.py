@@ -97,7 +97,7 @@ class _HipTernary:
             # one (small calls, a loose max_rows); decode-sized bf16 / int8 calls never do and skip the query.
             need = 0
             if max_rows > 16 and xdt == _lib.BP_I8:
-                need = self.lib.bp_grouped_gemm_int8_workspace_bytes(T, N, int(K), E, int(fmt), int(max_rows))
+                need = self.lib.bp_grouped_gemm_int8_workspace_bytes(T, N, int(K), int(group), E, int(fmt), len(packed_l), int(max_rows))
             elif xdt != _lib.BP_I8 and (max_rows > _DECODE_ROWS or xdt != _lib.BP_BF16):
                 need = self.lib.bp_grouped_gemm_workspace_bytes(xdt, T, N, int(K), E, int(fmt), int(max_rows))
             if need > _WORKSPACE_CAP:  # (up to 2.1 bytes per activation: a call this large keeps its memory and runs the kernels without one)
@@ -138,7 +138,7 @@ class _HipTernary:
         xdt, odt, sdc = _lib.dtype_code(x.dtype), _lib.dtype_code(out_dtype), _lib.dtype_code(sdt)
         offsets = dense_offsets(dev, T)
         out = torch.empty(T, N, dtype=out_dtype, device=dev)
-        need = self.lib.bp_ternary_linear_workspace_bytes(xdt, act_int8, odt, T, N, K, fmt, n)
+        need = self.lib.bp_ternary_linear_workspace_bytes(xdt, act_int8, odt, T, N, K, group, fmt, n)
         ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
         prev = torch.cuda.current_device()
         index = dev.index if dev.index is not None else prev

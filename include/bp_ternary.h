@@ -95,9 +95,10 @@ int bp_ternary_grouped_gemm(float* out, const void* x, int x_dtype, const float*
  * runs on them as well: the activations are split into a bf16 pair x = hi + lo (exact for fp16, to 2^-17 |x| for float32)
  * and both products are added into out. Without one they run on the general kernel. */
 size_t bp_grouped_gemm_workspace_bytes(int x_dtype, int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows);
-/* The same for int8 activations and TQ2: the workspace of the kernel for token tiles of 128 rows (large calls with at least
- * 64 rows per expert on average), 0 where bp_ternary_grouped_gemm_ws would not use one. */
-size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows);
+/* The same for int8 activations and TQ2: the workspace of the kernel for token tiles of 128 rows (large dense calls, and
+ * grouped ones with at least 112 rows per expert on average), 0 where the call's sizes and number of terms mean that
+ * bp_ternary_grouped_gemm_ws would not use one (beside them it needs the alignments that the tuned kernels need). */
+size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t group, int64_t E, int fmt, int n_terms, int64_t max_rows);
 int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype, const float* x_scale,
                                const int64_t* offsets, const int64_t* offsets_host,
                                const uint8_t* const* packed, const void* const* w_scale, int scale_dtype,
@@ -114,7 +115,7 @@ int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype, const flo
  *   offsets  device i64 {0, T}
  *   packed[t] device u8 [N, Kp], w_scale[t] device [N, G]; n_terms stacked terms
  *   workspace device memory, 256-byte aligned, at least bp_ternary_linear_workspace_bytes(...) bytes (NULL if that is 0) */
-size_t bp_ternary_linear_workspace_bytes(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int fmt, int n_terms);
+size_t bp_ternary_linear_workspace_bytes(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int64_t group, int fmt, int n_terms);
 int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_dtype, int act_int8, const int64_t* offsets,
                       const uint8_t* const* packed, const void* const* w_scale, int scale_dtype, int n_terms,
                       int64_t T, int64_t N, int64_t K, int64_t Kp, int64_t G, int64_t group, int fmt, void* workspace,

@@ -150,3 +150,18 @@ def test_int8_layers_with_few_blocks_stay_on_tiles_of_32(T, E, k, I, terms, wide
     assert ("i8w" in bp.ext().last_kernel()) == wide
     ref = moe.composed(x, logits)
     assert float((got.double() - ref.double()).norm() / ref.double().norm()) <= 4e-3  # (bf16 roundings and int8 steps that fall otherwise)
+
+
+# the rows of tests/test_workspace_sizes.py that lie at a line, as the launch sees them
+@pytest.mark.parametrize("T,N,K,terms,wide", [(2048, 2048, 1536, 2, True), (2048, 2048, 2048, 2, False), (2048, 2048, 2048, 1, True), (3072, 2048, 1792, 2, True), (1536, 4096, 7168, 2, False)])
+def test_int8_linears_take_the_variant_their_terms_fit(T, N, K, terms, wide):
+    import deepseekternarized_amd as bp
+
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    weights = [bp.PackedTerm(bp.pack(torch.randint(-1, 2, (N, K), dtype=torch.int8, device="cuda", generator=gen), "tq2"),
+                             (0.02 * torch.rand(N, K // 128, device="cuda", generator=gen)).half()) for _ in range(terms)]
+    x = torch.randn(T, K, device="cuda", generator=gen).bfloat16()
+    got = bp.TernaryLinear(weights, K, "tq2", 128)(x, torch.float32)
+    assert ("i8w" in bp.ext().last_kernel()) == wide
+    ref = bp.TernaryLinear(weights, K, "tq2", 128, backend="torch")(x, torch.float32)
+    _close(got, ref, "int8")
