@@ -239,18 +239,25 @@ constexpr int OUTPUTS = BP_REPLACES;  // 0: added to, 1: replaced
 constexpr int OUTPUTS = -1;  // by GemmArgs::overwrite
 #endif
 __device__ __forceinline__ bool replaces(const GemmArgs& a) { return OUTPUTS < 0 ? a.overwrite != 0 : OUTPUTS == 1; }
-// A kernel's epilogue f(OUT16): once for bf16 outputs and once for float32 ones, so that the branch is outside its loops (inside,
-// it kept the compiler from grouping an epilogue's loads).
+// Where a kernel's epilogue writes: copies of the arguments, not a reference, through which every output would load them again.
+struct Output {
+  float* out;
+  uint16_t* out16;
+  bool replace;
+};
+__device__ __forceinline__ Output output_of(const GemmArgs& a) { return {a.out, OUTPUTS == 0 ? nullptr : a.out16, replaces(a)}; }
+// An epilogue f(OUT16): once for bf16 outputs and once for float32 ones, so that the branch is outside its loops (inside, it kept the
+// compiler from grouping an epilogue's loads).
 template <class F>
-__device__ __forceinline__ void with_output(const GemmArgs& a, F&& f) {
-  if (OUTPUTS != 0 && a.out16) f(std::true_type{});
+__device__ __forceinline__ void with_output(const Output& o, F&& f) {
+  if (OUTPUTS != 0 && o.out16) f(std::true_type{});
   else f(std::false_type{});
 }
 // One finished output.
 template <bool OUT16>
-__device__ __forceinline__ void store_out(const GemmArgs& a, int64_t i, float v) {
-  if (OUT16) a.out16[i] = f32_to_bf16_bits(v);
-  else a.out[i] = (replaces(a) ? 0.f : a.out[i]) + v;
+__device__ __forceinline__ void store_out(const Output& o, int64_t i, float v) {
+  if (OUT16) o.out16[i] = f32_to_bf16_bits(v);
+  else o.out[i] = (o.replace ? 0.f : o.out[i]) + v;
 }
 }  // namespace
 

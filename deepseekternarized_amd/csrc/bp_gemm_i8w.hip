@@ -473,6 +473,7 @@ __global__ __launch_bounds__(WR * W_WT * 64, 2) void k_gemm_i8w(GemmArgs a) {
 #pragma unroll
         for (int r = 0; r < W_RT; ++r) park(16 * m + 4 * b + i, 16 * r + r16, f32_to_bf16_bits(total[r][m][i] * xs[m][i]));
   } else {
+    const Output o = output_of(a);
 #pragma unroll
     for (int r = 0; r < W_RT; ++r) {
       const int64_t row = tile_row(wr, r);
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(WR * W_WT * 64, 2) void k_gemm_i8w(GemmArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int tk = 64 * wt + 16 * m + 4 * b + i;
-          if (tk < ntok) store_out<false>(a, (tok0 + tk) * a.N + row + r16, total[r][m][i] * xs[m][i]);
+          if (tk < ntok) store_out<false>(o, (tok0 + tk) * NH + row + r16, total[r][m][i] * xs[m][i]);
         }
     }
   }

@@ -431,7 +431,10 @@ __global__ __launch_bounds__(Q_THREADS, 2) void k_gemm_tq1(GemmArgs a) {
     }
 
     // ---- epilogue: lane holds tokens 4 kb + i of each token tile, output row n_wave + 16 r + r16
-    with_output(a, [&](auto out16) {
+    const Output o = output_of(a);
+    const int64_t N = a.N;
+    const float* const x_scale = a.x_scale;
+    with_output(o, [&](auto out16) {
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
 #pragma unroll
@@ -439,12 +442,13 @@ __global__ __launch_bounds__(Q_THREADS, 2) void k_gemm_tq1(GemmArgs a) {
           const int tk = 16 * t + 4 * kb + i;
           if (tk < ntok) {
             const int64_t tok = tok0 + tk;
-            const float xs = ACT == BP_I8 ? a.x_scale[tok] : 1.0f;
+            const int64_t at = tok * N + n_wave + r16;
+            const float xs = ACT == BP_I8 ? x_scale[tok] : 1.0f;
 #pragma unroll
             for (int r = 0; r < Q_RT; ++r) {
               const int64_t row = n_wave + 16 * r;
-              if (row < a.N) {
-                store_out<decltype(out16)::value>(a, tok * a.N + row + r16, total[r][t][i] * xs);
+              if (row < N) {
+                store_out<decltype(out16)::value>(o, at + 16 * r, total[r][t][i] * xs);
               }
             }
           }

@@ -650,7 +650,9 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a) {
       }
       return;
     }
-    with_output(a, [&](auto out16) {
+    const Output o = output_of(a);
+    const int64_t N = a.N;
+    with_output(o, [&](auto out16) {
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
 #pragma unroll
@@ -662,7 +664,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a) {
             for (int r = 0; r < F_RT; ++r) {
               const int64_t row = tile_row(wave, r);
               if (row >= 0) {
-                store_out<decltype(out16)::value>(a, tok * a.N + row + r16, total[r][t][i]);
+                store_out<decltype(out16)::value>(o, tok * N + row + r16, total[r][t][i]);
               }
             }
           }

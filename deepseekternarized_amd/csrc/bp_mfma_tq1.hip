@@ -335,12 +335,15 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq1(GemmArgs a, int CPT 
     }
   }
   // ---- epilogue: lane holds tokens 4b + q of output row n0 + r16 (NQ = 1: only token 0 is kept)
-  with_output(a, [&](auto out16) {
+  const Output o = output_of(a);
+  const int64_t N = a.N;
+  const float* const x_scale = a.x_scale;
+  with_output(o, [&](auto out16) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       const int t = 4 * b + q;
       if (t < ntok && wave_live) {
-        store_out<decltype(out16)::value>(a, (tok0 + t) * a.N + n0 + r16, x_i8 ? total[q] * a.x_scale[tok0 + t] : total[q]);
+        store_out<decltype(out16)::value>(o, (tok0 + t) * N + n0 + r16, x_i8 ? total[q] * x_scale[tok0 + t] : total[q]);
       }
     }
   });

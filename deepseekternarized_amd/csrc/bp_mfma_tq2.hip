@@ -301,7 +301,10 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq2(GemmArgs a, int KC, 
     }
   }
   // ---- epilogue: lane holds tokens 4b + q (q = 0..3) of each token tile, output row n0 + 16r + r16
-  with_output(a, [&](auto out16) {
+  const Output o = output_of(a);
+  const int64_t N = a.N;
+  const float* const x_scale = a.x_scale;
+  with_output(o, [&](auto out16) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
@@ -309,11 +312,12 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_mfma_tq2(GemmArgs a, int KC, 
         const int t = 16 * mt + 4 * b + q;
         if (t < ntok) {
           const int64_t tok = tok0 + t;
-          const float xs = ACT == BP_I8 ? a.x_scale[tok] : 1.0f;
+          const int64_t at = tok * N + n0 + r16;
+          const float xs = ACT == BP_I8 ? x_scale[tok] : 1.0f;
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             if (rows_valid[r]) {
-              store_out<decltype(out16)::value>(a, tok * a.N + n0 + 16 * r + r16, total[r][mt][q] * xs);
+              store_out<decltype(out16)::value>(o, at + 16 * r, total[r][mt][q] * xs);
             }
           }
         }

@@ -275,7 +275,8 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_tq1_gemv(GemmArgs a, int CPT 
   total += __shfl_xor(total, 16);
   total += __shfl_xor(total, 32);
   if (b == 0 && wave_live) {
-    with_output(a, [&](auto out16) { store_out<decltype(out16)::value>(a, tok * a.N + n0 + r16, a.x_dtype == BP_I8 ? total * a.x_scale[tok] : total); });
+    const Output o = output_of(a);
+    with_output(o, [&](auto out16) { store_out<decltype(out16)::value>(o, tok * a.N + n0 + r16, a.x_dtype == BP_I8 ? total * a.x_scale[tok] : total); });
   }
 }
 
