@@ -120,21 +120,24 @@ __device__ __forceinline__ TileRef tile_ref(const GemmArgs& a, int64_t slot, uns
 
 // Which token tile and which block of output rows a workgroup of a token-tile kernel takes, from its linear index: bp_xcd.h.
 template <int ROWS = 32>
-__device__ __forceinline__ TileRef tile_of_workgroup(const GemmArgs& a, unsigned linear, int row_blocks, int& row_block) {
+__device__ __forceinline__ TileRef tile_of_workgroup(const GemmArgs& a, const TileSplit& split, unsigned linear, int& row_block) {
   unsigned expert = 0, tile = 0, block = 0;
   if (a.tiles) {
-    const unsigned slot = list_item(ROWS, linear, (unsigned)row_blocks, block);
+    const unsigned slot = list_item(split, ROWS, linear, block);
     row_block = (int)block;
     return tile_ref<ROWS>(a, slot, 0);
   }
-  if (!tile_item(tile_split(a.E, a.max_rows, ROWS), linear, gridDim.x, (unsigned)row_blocks, expert, tile, block)) return {0, 0, 0, false};
+  if (!tile_item(split, linear, expert, tile, block)) return {0, 0, 0, false};
   row_block = (int)block;
   return tile_ref<ROWS>(a, expert, tile);
 }
-// Workgroups of such a launch (-1: more than a grid's x extent holds).
+// Workgroups of such a launch and its split (-1: more than a grid's x extent holds).
 template <int ROWS = 32>
-inline int64_t tile_workgroups(const GemmArgs& a, int64_t row_blocks) {
-  return a.tiles ? list_items(ROWS, a.tile_cap, row_blocks) : tile_items(tile_split(a.E, a.max_rows, ROWS), row_blocks);
+inline int64_t split_tiles(TileSplit& split, const GemmArgs& a, int64_t row_blocks) {
+  split = tile_split(a.E, a.max_rows, ROWS, row_blocks);
+  const int64_t wgs = a.tiles ? list_items(ROWS, a.tile_cap, row_blocks) : tile_items(split);
+  split.eighth = (unsigned)(wgs / 8);
+  return wgs;
 }
 
 // Development overrides of the kernel selection (environment variables BP_TUNE_*), read once when the library is first

@@ -167,7 +167,7 @@ __global__ __launch_bounds__(W_THREADS) void k_stage_i8w(GemmArgs a) {
 // of it (K up to 3328 with one term): one loads its first windows and writes its results while the other multiplies, which
 // is a third of a workgroup's time at K = 2048. WR = 4: eight waves, 256 x 128, for longer rows.
 template <int WR>
-__global__ __launch_bounds__(WR * W_WT * 64, 2) void k_gemm_i8w(GemmArgs a) {
+__global__ __launch_bounds__(WR * W_WT * 64, 2) void k_gemm_i8w(GemmArgs a, TileSplit split) {
   constexpr int W_WR = WR, W_ROWS = i8w_rows(WR), W_THREADS = WR * W_WT * 64;
   constexpr int NB = W_OPS / (4 * 16 * W_THREADS);  // batches of four pieces per thread in a staged window
   static_assert(NB == 1 || NB == 2, "");
@@ -177,9 +177,8 @@ __global__ __launch_bounds__(WR * W_WT * 64, 2) void k_gemm_i8w(GemmArgs a) {
   // SwiGLU in the epilogue: a wave's four row tiles are two of the gate and the same two of the up projection
   const bool glu = a.glu_h != nullptr;
   const int64_t NH = glu ? a.N / 2 : a.N;
-  const int row_blocks = (int)(glu ? (NH + W_ROWS / 2 - 1) / (W_ROWS / 2) : (a.N + W_ROWS - 1) / W_ROWS);
   int wg_block;
-  const TileRef tr = tile_of_workgroup<W_TOK>(a, blockIdx.x, row_blocks, wg_block);
+  const TileRef tr = tile_of_workgroup<W_TOK>(a, split, blockIdx.x, wg_block);
   if (!tr.live) return;  // uniform for the workgroup
   const int64_t e = tr.e, tok0 = tr.tok0;
   const int ntok = (int)(tr.o1 - tok0 < W_TOK ? tr.o1 - tok0 : W_TOK);
@@ -505,8 +504,11 @@ static_assert(W_SC == I8W_STAGED && i8w_rows(2) == 64 * 2, "i8w_lds_bytes");
 template <int WR>
 int launch_i8w(const GemmArgs& a, hipStream_t s) {
   if (const int rc = raise_lds_limit<k_gemm_i8w<WR>>(160 * 1024)) return rc;
+  TileSplit split;
+  const int64_t wgs = split_tiles<W_TOK>(split, a, i8w_row_blocks(a, WR));
+  if (wgs < 0) return BP_ERR_UNSUPPORTED;  // (gemm_i8w_applies)
   note_kernel("gemm_tq2_i8w");
-  hipLaunchKernelGGL(k_gemm_i8w<WR>, dim3((unsigned)tile_workgroups<W_TOK>(a, i8w_row_blocks(a, WR))), dim3(WR * W_WT * 64), (size_t)i8w_lds_bytes(a.K, a.n_terms, WR), s, a);
+  hipLaunchKernelGGL(k_gemm_i8w<WR>, dim3((unsigned)wgs), dim3(WR * W_WT * 64), (size_t)i8w_lds_bytes(a.K, a.n_terms, WR), s, a, split);
   return check_launch("gemm_tq2_i8w");
 }
 
@@ -529,7 +531,8 @@ int gemm_i8w_applies(const GemmArgs& a) {
   const int WR = i8w_wr(a.K, a.n_terms);
   if (a.glu_h && a.N % 32 != 0) return BP_ERR_UNSUPPORTED;
   if ((((uintptr_t)a.glu_h | (uintptr_t)a.out16) & 15) != 0) return BP_ERR_UNSUPPORTED;  // (16-byte pieces of bf16 rows)
-  return tile_workgroups<W_TOK>(a, i8w_row_blocks(a, WR)) < 0 ? BP_ERR_UNSUPPORTED : BP_OK;
+  TileSplit split;
+  return split_tiles<W_TOK>(split, a, i8w_row_blocks(a, WR)) < 0 ? BP_ERR_UNSUPPORTED : BP_OK;
 }
 
 int launch_gemm_i8w(const GemmArgs& a, hipStream_t s) {

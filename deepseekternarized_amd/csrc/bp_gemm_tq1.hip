@@ -62,15 +62,14 @@ __device__ __forceinline__ constexpr int q_split_byte(int J) { return J == 1 ? 9
 __device__ __forceinline__ constexpr int q_split_digits(int J) { return J == 1 ? 3 : J == 3 ? 1 : J == 4 ? 4 : J == 6 ? 2 : 0; }
 
 template <int ACT, int SDT>
-__global__ __launch_bounds__(Q_THREADS, 2) void k_gemm_tq1(GemmArgs a) {
+__global__ __launch_bounds__(Q_THREADS, 2) void k_gemm_tq1(GemmArgs a, TileSplit split) {
   constexpr int XB = ACT == BP_BF16 ? 2 : 1;   // bytes per activation
   constexpr int SB = SDT == BP_F32 ? 4 : 2;
 
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int r16 = lane & 15, kb = lane >> 4;
-  const int row_blocks = (int)((a.N + Q_ROWS - 1) / Q_ROWS);
   int wg_block;
-  const TileRef tr = tile_of_workgroup(a, blockIdx.x, row_blocks, wg_block);
+  const TileRef tr = tile_of_workgroup(a, split, blockIdx.x, wg_block);
   if (!tr.live) return;  // uniform for the workgroup
   const int64_t e = tr.e, tok0 = tr.tok0, o1 = tr.o1;
   const int ntok = (int)(o1 - tok0 < 32 ? o1 - tok0 : 32);
@@ -464,11 +463,12 @@ template <int ACT, int SDT>
 int launch_gemm_tq1_k(const GemmArgs& a, hipStream_t s, const char* name) {
   if (const int rc = raise_lds_limit<k_gemm_tq1<ACT, SDT>>(q_lds_bytes(SDT == BP_F32 ? 4 : 2))) return rc;
   const int64_t row_blocks = (a.N + Q_ROWS - 1) / Q_ROWS;
-  const int64_t wgs = tile_workgroups(a, row_blocks);
+  TileSplit split;
+  const int64_t wgs = split_tiles(split, a, row_blocks);
   if (wgs < 0) return BP_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)wgs, 1, 1);
   note_kernel(name);
-  hipLaunchKernelGGL((k_gemm_tq1<ACT, SDT>), grid, dim3(Q_THREADS), q_lds_bytes(SDT == BP_F32 ? 4 : 2), s, a);
+  hipLaunchKernelGGL((k_gemm_tq1<ACT, SDT>), grid, dim3(Q_THREADS), q_lds_bytes(SDT == BP_F32 ? 4 : 2), s, a, split);
   return check_launch(name);
 }
 

@@ -36,7 +36,7 @@ constexpr int gemm_tile_bytes() { return 16 * GT * GKC * (ACT == BP_BF16 ? 2 : 1
 // KiB at ((g * NJ + j) * GT + mt) * 1024; lane l = 16 b + t of it holds, for token 16 mt + t, the KM
 // elements the lane multiplies in that MFMA (k-block b of the decode's slot order).
 template <int ACT, int SDT, int SL, int ABL = 0>
-__global__ __launch_bounds__(GTHREADS, 2) void k_gemm_tq2(GemmArgs a) {
+__global__ __launch_bounds__(GTHREADS, 2) void k_gemm_tq2(GemmArgs a, TileSplit split) {
   constexpr int XB = ACT == BP_BF16 ? 2 : 1;
   constexpr int KM = ACT == BP_BF16 ? 8 : 16;
   constexpr int NJ = 32 / KM;
@@ -50,9 +50,8 @@ __global__ __launch_bounds__(GTHREADS, 2) void k_gemm_tq2(GemmArgs a) {
 
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int r16 = lane & 15, b = lane >> 4;
-  const int row_tiles = (int)((a.N + GROWS - 1) / GROWS);
   int wg_tile;
-  const TileRef tr = tile_of_workgroup(a, blockIdx.x, row_tiles, wg_tile);
+  const TileRef tr = tile_of_workgroup(a, split, blockIdx.x, wg_tile);
   if (!tr.live) return;  // uniform for the workgroup
   const int64_t e = tr.e, tok0 = tr.tok0, o1 = tr.o1;
   const int ntok = (int)(o1 - tok0 < 16 * GT ? o1 - tok0 : 16 * GT);
@@ -414,11 +413,12 @@ template <int ACT, int SDT, int SL, int ABL = 0>
 int launch_gemm_k(const GemmArgs& a, hipStream_t s, size_t lds, const char* name) {
   if (const int rc = raise_lds_limit<k_gemm_tq2<ACT, SDT, SL, ABL>>(160 * 1024)) return rc;
   static_assert(16 * GT == 32, "tile_of_workgroup counts token tiles of 32");
-  const int64_t wgs = tile_workgroups(a, (a.N + GROWS - 1) / GROWS);
+  TileSplit split;
+  const int64_t wgs = split_tiles(split, a, (a.N + GROWS - 1) / GROWS);
   if (wgs < 0) return BP_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)wgs, 1, 1);
   note_kernel(name);
-  hipLaunchKernelGGL((k_gemm_tq2<ACT, SDT, SL, ABL>), grid, dim3(GTHREADS), lds, s, a);
+  hipLaunchKernelGGL((k_gemm_tq2<ACT, SDT, SL, ABL>), grid, dim3(GTHREADS), lds, s, a, split);
   return check_launch(name);
 }
 

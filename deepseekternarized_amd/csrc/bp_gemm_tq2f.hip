@@ -177,7 +177,7 @@ __global__ __launch_bounds__(F_THREADS) void k_stage_tq2f(GemmArgs a) {
 
 // GS = 1: scale groups of 256 (the two groups of a window share a scale); 0: of 128.
 template <int SDT, int FMT, int GS>
-__global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a) {
+__global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSplit split) {
   constexpr int SB = SDT == BP_F32 ? 4 : 2;
   constexpr bool Q1 = FMT == BP_TQ1;
   constexpr unsigned LB = Q1 ? F_LUT : 0;  // LDS address of the staged windows
@@ -188,9 +188,8 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a) {
   // of the gate (r = 0, 1) and the same two of the up projection (r = 2, 3): a row block covers F_ROWS / 2 of either
   const bool glu = a.glu_h != nullptr;
   const int64_t NH = glu ? a.N / 2 : a.N;
-  const int row_blocks = glu ? (int)((NH + F_ROWS / 2 - 1) / (F_ROWS / 2)) : (int)((a.N + F_ROWS - 1) / F_ROWS);
   int wg_block;
-  const TileRef tr = tile_of_workgroup(a, blockIdx.x, row_blocks, wg_block);
+  const TileRef tr = tile_of_workgroup(a, split, blockIdx.x, wg_block);
   if (!tr.live) return;  // uniform for the workgroup
   const int64_t e = tr.e, tok0 = tr.tok0, o1 = tr.o1;
   const int ntok = (int)(o1 - tok0 < 32 ? o1 - tok0 : 32);
@@ -683,7 +682,8 @@ int launch_gemm_tq2f_g(const GemmArgs& a, hipStream_t s) {
   const char* name = FMT == BP_TQ1 ? "gemm_tq1f_bf16" : "gemm_tq2f_bf16";
   if (const int rc = raise_lds_limit<k_gemm_tq2f<SDT, FMT, GS>>(LDS)) return rc;
   const int64_t row_blocks = a.glu_h ? (a.N / 2 + F_ROWS / 2 - 1) / (F_ROWS / 2) : (a.N + F_ROWS - 1) / F_ROWS;
-  const int64_t wgs = tile_workgroups(a, row_blocks);
+  TileSplit split;
+  const int64_t wgs = split_tiles(split, a, row_blocks);
   if (wgs < 0) return BP_ERR_UNSUPPORTED;
   const int64_t slots = a.tiles ? a.tile_cap : a.E;
   const unsigned z = a.tiles ? 1u : (unsigned)((a.max_rows + 31) / 32);
@@ -691,7 +691,7 @@ int launch_gemm_tq2f_g(const GemmArgs& a, hipStream_t s) {
   if (const int rc = check_launch("stage_tq2f")) return rc;
   const dim3 grid((unsigned)wgs, 1, 1);
   note_kernel(name);
-  hipLaunchKernelGGL((k_gemm_tq2f<SDT, FMT, GS>), grid, dim3(F_THREADS), LDS, s, a);
+  hipLaunchKernelGGL((k_gemm_tq2f<SDT, FMT, GS>), grid, dim3(F_THREADS), LDS, s, a, split);
   return check_launch(name);
 }
 
@@ -735,8 +735,8 @@ int gemm_tq2f_applies(const GemmArgs& a) {
       if ((((uintptr_t)a.packed[t] ^ (uintptr_t)a.packed[0]) & 3) != 0) return BP_ERR_UNSUPPORTED;
   }
   const int64_t row_blocks = a.glu_h ? (a.N / 2 + F_ROWS / 2 - 1) / (F_ROWS / 2) : (a.N + F_ROWS - 1) / F_ROWS;
-  if (tile_workgroups(a, row_blocks) < 0) return BP_ERR_UNSUPPORTED;
-  return BP_OK;
+  TileSplit split;
+  return split_tiles(split, a, row_blocks) < 0 ? BP_ERR_UNSUPPORTED : BP_OK;
 }
 
 int launch_gemm_tq2f(const GemmArgs& a, hipStream_t s) {
