@@ -215,11 +215,12 @@ extern "C" int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype
 // ---- one dense linear from its float activations to its output rows, in one call: the quantisation to int8 (act_int8),
 // the product, the rounding to bf16. The kernels write bf16 rows themselves where they can (GemmArgs::out16), so that the
 // usual call is one launch, or two with the quantisation; float32 rows and a rounding pass are left for the calls in which a
-// kernel takes several passes over an output.
+// kernel takes several passes over an output (fp16 and float32 activations as a bf16 pair, TQ1 with few rows).
 namespace bp {
 namespace {
+size_t split_bytes(int64_t T, int64_t K);  // of one of a pair
 struct LinearPlan {  // offsets into the workspace
-  size_t q, q_scale, sums, stage, stage_bytes, repacked, bytes;
+  size_t q, q_scale, sums, sums_bytes, stage, stage_bytes, repacked, bytes;
   bool repack;  // TQ1 weights are rewritten as TQ2 ones first
 };
 // TQ1 linears whose weights are rewritten as TQ2 ones first, which the TQ2 kernels decode faster. From five tokens on while
@@ -228,18 +229,27 @@ struct LinearPlan {  // offsets into the workspace
 // 27 / 60. Larger weights, which the TQ1 kernels' few large workgroups fill the device with, from the number of tokens at which those decode
 // every weight for eight token tiles (4096 tokens x 4096 x 4096: 159 / 283).
 bool repack_pays(int64_t T, int64_t N, int64_t K) { return T >= 256 || (T >= 5 && N <= ((int64_t)1 << 26) / K); }
+// Memory that a call only runs faster with - converted activations, rewritten weights - is asked for up to this size of either; a
+// larger call runs without it.
+constexpr size_t OPTIONAL_BYTES = (size_t)8 << 30;
 size_t repacked_bytes(int64_t N, int64_t K) { return ((size_t)N * (size_t)(K / 4) + 255) & ~(size_t)255; }
 LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int64_t group, int fmt, int n_terms) {
   LinearPlan p;
-  p.repack = fmt == BP_TQ1 && repack_pays(T, N, K) && K % 256 == 0 && K >= 1024 && K <= 65536 && tuning().tq2g != 'b';
+  const bool few_tq1 = fmt == BP_TQ1 && T <= 64;
+  p.repack = fmt == BP_TQ1 && repack_pays(T, N, K) && K % 256 == 0 && K >= 1024 && K <= 65536 && tuning().tq2g != 'b' &&
+             N <= (int64_t)(OPTIONAL_BYTES / (size_t)n_terms) / (K / 4);
   if (p.repack) fmt = BP_TQ2;
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) & ~(size_t)255; return o; };
   p.q = take(act_int8 ? (size_t)T * (size_t)K : 0);
   p.q_scale = take(act_int8 ? 4 * (size_t)T : 0);
-  p.sums = take(out_dtype == BP_F32 ? 0 : 4 * (size_t)T * (size_t)N);
   p.stage_bytes = act_int8 ? bp_grouped_gemm_int8_workspace_bytes(T, N, K, group, 1, fmt, n_terms, T) : bp_grouped_gemm_workspace_bytes(x_dtype, T, N, K, 1, fmt, T);
+  const bool floats = !act_int8 && x_dtype != BP_BF16;  // (a bf16 pair, and its conversion as far as there is room)
+  if (p.stage_bytes > OPTIONAL_BYTES) p.stage_bytes = floats && 2 * split_bytes(T, K) <= OPTIONAL_BYTES ? 2 * split_bytes(T, K) : 0;
   p.stage = take(p.stage_bytes);
+  const bool pair = floats && p.stage_bytes;
+  p.sums_bytes = out_dtype == BP_BF16 && (pair || few_tq1) ? 4 * (size_t)T * (size_t)N : 0;
+  p.sums = take(p.sums_bytes);
   p.repacked = take(p.repack ? (size_t)n_terms * repacked_bytes(N, K) : 0);
   p.bytes = at;
   return p;
@@ -310,6 +320,7 @@ extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_
     a.overwrite = 1;
     const int rc = run_gemm(a, s);
     if (rc != ERR_NO_OUT16) return rc;
+    if (!p.sums_bytes) return fail(BP_ERR_UNSUPPORTED, "no workspace for this linear's float32 rows");  // (linear_plan knows the kernels that need them)
     a.out16 = nullptr;
     a.out = (float*)(ws + p.sums);
   }
@@ -398,7 +409,6 @@ int run_gemm(const GemmArgs& a, hipStream_t s) {
   }
   if (a.tiles) return fail(BP_ERR_UNSUPPORTED, "tile-list mode needs one of the 32-token-tile kernels");
   if (g_policy == 2) return fail(BP_ERR_UNSUPPORTED, "shape is outside the tuned kernels (policy 2 forbids the general kernel)");
-  if (a.out16) return ERR_NO_OUT16;
   return launch_general(a, s);
 }
 }  // namespace bp

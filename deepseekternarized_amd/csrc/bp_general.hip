@@ -91,8 +91,12 @@ __global__ __launch_bounds__(GEN_WAVES * 64) void k_general(GemmArgs a) {
   }
   if (lane == 0) {
 #pragma unroll
-    for (int r = 0; r < GEN_TOK; ++r)
-      if (r < rows) a.out[(row0 + r) * a.N + n] = __fadd_rn(a.overwrite ? 0.f : a.out[(row0 + r) * a.N + n], total[r]);
+    for (int r = 0; r < GEN_TOK; ++r) {
+      if (r >= rows) break;
+      const int64_t at = (row0 + r) * a.N + n;
+      if (a.out16) a.out16[at] = f32_to_bf16_bits(__fadd_rn(0.f, total[r]));
+      else a.out[at] = __fadd_rn(a.overwrite ? 0.f : a.out[at], total[r]);
+    }
   }
 }
 

@@ -114,7 +114,8 @@ int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype, const flo
  *   x        device [T, K] of x_dtype BP_BF16, BP_F16 or BP_F32
  *   offsets  device i64 {0, T}
  *   packed[t] device u8 [N, Kp], w_scale[t] device [N, G]; n_terms stacked terms
- *   workspace device memory, 256-byte aligned, at least bp_ternary_linear_workspace_bytes(...) bytes (NULL if that is 0) */
+ *   workspace device memory, 256-byte aligned, at least bp_ternary_linear_workspace_bytes(...) bytes (NULL if that is 0).
+ *             Converted activations and rewritten weights, which only make a call faster, are part of it up to 8 GiB each. */
 size_t bp_ternary_linear_workspace_bytes(int x_dtype, int act_int8, int out_dtype, int64_t T, int64_t N, int64_t K, int64_t group, int fmt, int n_terms);
 int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_dtype, int act_int8, const int64_t* offsets,
                       const uint8_t* const* packed, const void* const* w_scale, int scale_dtype, int n_terms,

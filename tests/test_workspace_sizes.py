@@ -25,3 +25,33 @@ def lib():
     (8192, 2048, 2048, 128, 1, TQ1, 1, False), (64 * 96, 2048, 2048, 128, 64, TQ2, 1, False), (64 * 112, 2048, 2048, 128, 64, TQ2, 1, True), (16 * 256, 2048, 2048, 128, 16, TQ2, 1, False)])
 def test_int8_calls_ask_for_what_they_use(lib, T, N, K, group, E, fmt, terms, asks):
     assert (lib.bp_grouped_gemm_int8_workspace_bytes(T, N, K, group, E, fmt, terms, T) > 0) == asks
+
+
+I8, BF16, F16, F32 = 0, 1, 2, 3
+
+
+def _linear(lib, T, N, K, x=BF16, int8=0, out=BF16, fmt=TQ2, terms=1):
+    return lib.bp_ternary_linear_workspace_bytes(x, int8, out, T, N, K, 128, fmt, terms)
+
+
+def test_linears_ask_for_float32_rows_only_where_a_kernel_needs_them(lib):
+    from deepseekternarized_amd.kernels import _lib
+
+    assert (BF16, F16, F32, I8) == (_lib.BP_BF16, _lib.BP_F16, _lib.BP_F32, _lib.BP_I8)
+    # bf16 rows from the kernel: as much as float32 rows from it
+    for T, N, K, int8, fmt in [(8192, 6144, 2048, 1, TQ2), (8192, 6144, 2048, 0, TQ2), (200, 4096, 4096, 0, TQ2), (4096, 4096, 4096, 1, TQ1), (8192, 4096, 200, 0, TQ2)]:
+        assert _linear(lib, T, N, K, int8=int8, fmt=fmt) == _linear(lib, T, N, K, int8=int8, fmt=fmt, out=F32)
+    # TQ1 with few rows (a launch per term or segment), activations as a bf16 pair
+    assert _linear(lib, 4, 2048, 7168, fmt=TQ1) == 4 * 4 * 2048
+    assert _linear(lib, 512, 2048, 2048, x=F32) == _linear(lib, 512, 2048, 2048, x=F32, out=F32) + 4 * 512 * 2048
+
+
+@pytest.mark.parametrize("int8,x,fmt", [(0, BF16, TQ2), (1, BF16, TQ2), (0, F32, TQ2), (0, BF16, TQ1), (1, F16, TQ1)])
+def test_large_linears_ask_for_no_more_than_they_must(lib, int8, x, fmt):
+    """Conversions of more than 8 GiB are left out, as in the grouped call: 4 Mi rows ask for their int8 rows at most."""
+    T, K, N = 1 << 22, 7168, 8192
+    assert _linear(lib, T, N, K, x=x, int8=int8, fmt=fmt) <= int8 * (T * K + 4 * T) + (N * K // 4 if fmt == TQ1 else 0) + 1024
+    assert _linear(lib, T // 64, N, K, x=x, int8=int8, fmt=fmt) > int8 * (T * K + 4 * T) // 64 + (1 << 27)
+    if x == F32:  # the bf16 pair still fits, its conversion does not
+        assert _linear(lib, T // 16, N, K, x=x, int8=int8, fmt=fmt, out=F32) == 2 * 2 * T // 16 * K
+    assert _linear(lib, 1 << 16, 1 << 21, 1 << 15, int8=1, fmt=TQ1, terms=2) < 6 << 30  # (17 GiB of weights a term)
