@@ -119,7 +119,10 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort(int64_t* __restrict__ ord
 // block adds up the histograms of all blocks (the experts' first slots) and of the blocks before it, ranks its ids - a
 // wave's 64 by ballots as in k_sort, the waves through their counts in LDS - and writes them.
 constexpr int SORT_BLOCK = 1024;
-constexpr int64_t SORT_BLOCKS_FROM = 4096;  // ids from which the two launches win
+// Ids for which the two launches win. The placement reads all blocks' histograms in every block, so its time grows with the square of
+// the ids: 64 / 512 experts, us against one workgroup, 1 Mi ids 74 / 111 against 1332 / 1601, 4 Mi 862 / 1697 against 5260 / 6314; at 16 Mi it
+// would be behind.
+constexpr int64_t SORT_BLOCKS_FROM = 4096, SORT_BLOCKS_TO = (int64_t)8 << 20;
 constexpr int64_t SORT_BLOCKS_MAX_E = 512;  // (k_sort_place: 64 bytes of LDS per expert)
 __global__ __launch_bounds__(SORT_BLOCK) void k_sort_count(const int64_t* __restrict__ ids, int64_t n, int E, int32_t* __restrict__ ws, int32_t* __restrict__ bad) {
   __shared__ int32_t hist[SORT_BLOCKS_MAX_E];
@@ -604,7 +607,7 @@ static int launch_sort(int64_t* order, int64_t* offsets, const int64_t* ids, int
 namespace bp {
 // bp_sort_by_expert that also writes the inverse permutation (the MoE layer's preparation; arguments checked by its caller)
 // Its workspace: bp_sort_workspace_ints, or the blocks' histograms where those sort.
-static bool sort_in_blocks(int64_t n, int64_t E) { return n >= SORT_BLOCKS_FROM && E > 0 && E <= SORT_BLOCKS_MAX_E; }
+static bool sort_in_blocks(int64_t n, int64_t E) { return n >= SORT_BLOCKS_FROM && n <= SORT_BLOCKS_TO && E > 0 && E <= SORT_BLOCKS_MAX_E; }
 int64_t sort_with_inverse_ints(int64_t n, int64_t E) { return sort_in_blocks(n, E) ? (n + SORT_BLOCK - 1) / SORT_BLOCK * E : bp_sort_workspace_ints(n, E); }
 int sort_with_inverse(int64_t* order, int64_t* offsets, int64_t* inv, const int64_t* ids, int64_t n, int64_t E, int32_t* workspace,
                       int32_t* bad, hipStream_t stream) {

@@ -55,3 +55,10 @@ def test_large_linears_ask_for_no_more_than_they_must(lib, int8, x, fmt):
     if x == F32:  # the bf16 pair still fits, its conversion does not
         assert _linear(lib, T // 16, N, K, x=x, int8=int8, fmt=fmt, out=F32) == 2 * 2 * T // 16 * K
     assert _linear(lib, 1 << 16, 1 << 21, 1 << 15, int8=1, fmt=TQ1, terms=2) < 6 << 30  # (17 GiB of weights a term)
+
+
+def test_very_many_ids_sort_without_block_histograms(lib):
+    """Beyond 8 Mi routed rows, where placing them block by block would read more than one workgroup sorting them takes: the
+    layer's workspace loses the 8192 x 512 counters."""
+    size = lambda T: lib.bp_moe_layer_workspace_bytes(T, 8, 8, 512, 8, BF16, TQ2)  # noqa: E731
+    assert size((1 << 20) + 1) < size(1 << 20) - 4 * 8192 * 512 + (1 << 16)
