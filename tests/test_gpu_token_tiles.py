@@ -70,6 +70,21 @@ def test_int8_tiles_of_128(tune, counts, N, K, group, terms, sdt):
     assert bp.ext().last_kernel() == "gemm_tq2_i8w"
 
 
+# the same with eight waves of 256 rows per workgroup: rows whose scales leave room for one workgroup per CU - one term from K = 3584
+# on, two from 1792, three always -, an odd number of windows, one scale per 256, remainders of 1, 63, 65 and 127 rows
+@pytest.mark.parametrize("counts", [(129, 0, 63), (193, 65, 255)])
+@pytest.mark.parametrize("N,K,group,terms,sdt", [(272, 3584, 128, 1, torch.float16), (528, 4352, 128, 1, torch.float32), (256, 2048, 128, 2, torch.bfloat16),
+                                                 (272, 2304, 128, 2, torch.float16), (528, 4096, 256, 1, torch.float16), (272, 1280, 128, 3, torch.float32)])
+def test_int8_tiles_of_128_with_eight_waves(tune, counts, N, K, group, terms, sdt):
+    import deepseekternarized_amd as bp
+
+    tune("BP_TUNE_TQ2G", "f")
+    got, _ = _call("tq2", "int8", counts, N, K, 13, terms, group, sdt, max_rows=300, ref=False)
+    assert bp.ext().last_kernel() == "gemm_tq2_i8w"
+    _, ref = _call("tq2", "int8", counts, N, K, 13, terms, group, sdt, max_rows=300)  # (the reference-order kernel's)
+    _close(got, ref, "int8")
+
+
 @pytest.mark.parametrize("T,K,scale", [(129, 1024, 1.0), (200, 1280, 1e-6), (130, 4352, 100.0)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_linear_quantises_in_the_conversion_pass(tune, T, K, scale, out_dtype):
@@ -93,17 +108,24 @@ def test_linear_quantises_in_the_conversion_pass(tune, T, K, scale, out_dtype):
     ref = bp.grouped_ternary_gemm(q, qs, dense_offsets(x.device, T), [packed[None]], [s[None]], K, 128, "tq2", max_rows=T).to(out_dtype)
     assert torch.equal(got.isnan(), ref.isnan()) and bool(ref[5].isnan().all())
     assert torch.equal(got.nan_to_num(), ref.nan_to_num())
+    # ... and the product itself against the reference-order kernel (both references above run on this kernel)
+    ref = bp.grouped_ternary_gemm(q, qs, dense_offsets(x.device, T), [packed[None]], [s[None]], K, 128, "tq2", max_rows=T, backend="torch")
+    keep = torch.arange(T, device="cuda") != 5
+    bound = 4e-6 if out_dtype == torch.float32 else 2**-9  # (bf16: half a step)
+    assert float((got[keep].double() - ref[keep].double()).norm() / ref[keep].double().norm()) <= bound
 
 
-@pytest.mark.parametrize("pattern,T,E,k,terms", [("standard", 1100, 8, 1, 1), ("standard", 700, 16, 4, 2), ("v4", 520, 4, 2, 1)])
-def test_int8_layer_on_tiles_of_128(tune, pattern, T, E, k, terms):
+@pytest.mark.parametrize("pattern,T,E,k,terms,H", [("standard", 1100, 8, 1, 1, 1024), ("standard", 700, 16, 4, 2, 1024), ("v4", 520, 4, 2, 1, 1024),
+                                                   ("standard", 1100, 8, 1, 1, 4096), ("standard", 700, 4, 3, 2, 2048), ("v4", 520, 4, 2, 1, 4096)])
+def test_int8_layer_on_tiles_of_128(tune, pattern, T, E, k, terms, H):
     """The layer on the 128-token kernel against the same layer as separate launches (standard), or on the 32-token kernel (v4):
-    the same rounding points over float32 sums that differ in order, so a few bf16 roundings and int8 steps fall otherwise."""
+    the same rounding points over float32 sums that differ in order, so a few bf16 roundings and int8 steps fall otherwise.
+    H = 4096, and 2048 in two terms: the gate | up launch, with SwiGLU and the gather, on eight waves."""
     import deepseekternarized_amd as bp
     from deepseekternarized_amd.moe import TernaryMoE
 
     gen = torch.Generator(device="cuda").manual_seed(10)
-    H, I = 1024, 1280
+    I = 1280
 
     def terms_of(N, K):
         return [(torch.stack([bp.pack(torch.randint(-1, 2, (N, K), dtype=torch.int8, device="cuda", generator=gen), "tq2") for _ in range(E)]),
