@@ -28,8 +28,8 @@ struct GemmArgs {
   const void* w_scale[BP_MAX_TERMS];
   int x_dtype, scale_dtype, n_terms, fmt;
   int64_t T, N, K, Kp, G, group, E, max_rows;
-  // Tile-list mode of the 32-token-tile kernels (set by callers that keep the routing on the device, where the widest
-  // expert's row count is unknown to the host): tiles = (expert, first row) pairs of the token tiles that exist, in
+  // Tile-list mode of the token-tile kernels, with tiles of 32 or 128 rows (set by callers that keep the routing on the device, where
+  // the widest expert's row count is unknown to the host): tiles = (expert, first row) pairs of the token tiles that exist, in
   // expert order, tile_count[0] of them (device memory, written by a kernel earlier on the stream); the launch covers
   // tile_cap entries and workgroups past the count leave at once. NULL: token tiles are counted by blockIdx.z up to max_rows.
   const int32_t* tiles;
@@ -40,18 +40,18 @@ struct GemmArgs {
   // Workspace of the caller for kernels that convert the activations in a pass of their own (NULL: those kernels are not used).
   unsigned char* stage;
   int64_t stage_bytes;
-  // SwiGLU in the epilogue of the grouped GEMM over converted activations (glu_h != NULL; tile-list mode with overwrite):
-  // the N output rows are N / 2 gate rows followed by N / 2 up rows, and the kernel writes bf16 glu_h[T, N / 2] instead
-  // of `out`, with the rounding points of bp_swiglu_bf16 (glu_v4 = 0) or of bp_swiglu_v4 (glu_v4 = 1: clamp by glu_limit
-  // when positive, float32 product times glu_weights[glu_order[row]] when glu_weights is set, one rounding to bf16).
-  // Row gather in the conversion pass of that kernel (x_index != NULL): row r of the launch is row
-  // x_index[r] / x_div of x, which has x_rows rows (the routed copy of the activations is never materialised).
+  // Row gather in the conversion pass of the grouped GEMMs over converted activations (x_index != NULL): row r of the launch is
+  // row x_index[r] / x_div of x, which has x_rows rows (the routed copy of the activations is never materialised).
   const int64_t* x_index;
   int64_t x_div, x_rows;
   int quant;  // x is bf16 and the conversion pass of the int8 kernel for 128-token tiles quantises its rows (x_scale unused)
   // bf16 out16[T, N] is written instead of float32 `out` (one launch that covers all of K and all terms; a kernel that
   // takes several passes over an output returns ERR_NO_OUT16 instead).
   uint16_t* out16;
+  // SwiGLU in the epilogue of the same GEMMs (glu_h != NULL; tile-list mode with overwrite): the N output rows are N / 2 gate
+  // rows followed by N / 2 up rows, and the kernel writes bf16 glu_h[T, N / 2] instead of `out`, with the rounding points of
+  // bp_swiglu_bf16 (glu_v4 = 0) or of bp_swiglu_v4 (glu_v4 = 1: clamp by glu_limit when positive, float32 product times
+  // glu_weights[glu_order[row]] when glu_weights is set, one rounding to bf16).
   uint16_t* glu_h;
   int glu_v4;
   float glu_limit;

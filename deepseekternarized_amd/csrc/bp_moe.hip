@@ -5,7 +5,7 @@
 //
 // Nothing is read back to the host. The reference sizes its grouped launch from `int(offsets.diff().max())`
 // (boilerplate/kernels/ternary_cuda.py:97), a device-to-host copy in the middle of the layer; here a kernel writes
-// the list of 32-row token tiles that exist (k_tile_list), and the grouped GEMMs run over that list. Up to 64 tokens
+// the list of token tiles that exist (k_tile_list; 32 rows each, 128 in large int8 layers), and the grouped GEMMs run over it. Up to 64 tokens
 // no expert can have more than 64 rows, and the launch is sized by that bound instead (the small-batch kernels).
 //
 // All intermediate tensors live in a workspace the caller provides (bp_moe_layer_workspace_bytes): the library

@@ -149,6 +149,8 @@ __global__ __launch_bounds__(1024) void k_tq2_gemv_ks(GemmArgs a, int nw, int ti
 #pragma unroll
   for (int u = 0; u < KV_OPT; ++u) {
     const int o = (int)threadIdx.x + u * nw * 64;
+    // (tested at run time, not a second object as elsewhere: without the test four tokens spill 11 vector registers instead of 3,
+    // 128 x 2048 x 7168 111.6 us against 108.8)
     total[u] = !a.out16 && !a.overwrite && out_live(o) ? a.out[out_at(o)] : 0.f;
   }
   i32x8 A[2 * KV_S];
