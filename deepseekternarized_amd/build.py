@@ -18,7 +18,7 @@ CSRC = HERE / "csrc"
 LIB = HERE / "libbp_ternary_hip.so"
 SOURCES = ["bp_api.hip", "bp_general.hip", "bp_repack.hip", "bp_route.hip", "bp_gguf.hip", "bp_huffman.hip", "bp_moe.hip", "bp_mfma.hip", "bp_mfma_tq2.hip", "bp_gemm_tq2.hip", "bp_gemm_tq2f.hip", "bp_gemm_i8w.hip", "bp_mfma_tq1.hip", "bp_gemm_tq1.hip", "bp_tq1_gemv.hip", "bp_tq1_gemv_fp4.hip", "bp_tq1_gemv_cw.hip", "bp_tq2_gemv_fp4.hip"]
 # Compiled twice, for launches that add to their outputs and for those that replace them (BP_REPLACES in bp_common.h).
-TWICE = {"bp_mfma_tq2.hip", "bp_gemm_tq2.hip", "bp_mfma_tq1.hip", "bp_gemm_tq1.hip", "bp_tq1_gemv_fp4.hip", "bp_tq1_gemv_cw.hip"}
+TWICE = {"bp_mfma_tq2.hip", "bp_gemm_tq2.hip", "bp_mfma_tq1.hip", "bp_gemm_tq1.hip", "bp_tq1_gemv_fp4.hip", "bp_tq1_gemv_cw.hip", "bp_tq2_gemv_fp4.hip"}
 # packed FP32 VALU ops are disabled for every device object of this library
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function", "-Wno-int-to-pointer-cast",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

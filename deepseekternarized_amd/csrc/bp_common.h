@@ -234,7 +234,7 @@ __device__ __forceinline__ uint16_t swiglu_bits(float gate, float up, bool weigh
 // BP_REPLACES): launches that add to float32 `out`, the grouped entry point's contract, and launches of a linear or a layer
 // that replace it or write bf16 `out16` instead. Elsewhere GemmArgs::overwrite decides. Tested at run time in every kernel, the
 // second case cost the first: spilled scalar registers in the streaming TQ1 kernels (192 against 185 with six loads per loader, two
-// tokens 34 against 24), and 2 - 10 % of a grouped launch's time (int8, 64 experts x 32 rows x 2048 x 2048: TQ1 61.0 -> 70.2 us).
+// tokens 43 against 24), and 2 - 15 % of a grouped launch's time (int8, 64 experts x 32 rows x 2048 x 2048: TQ1 61.0 -> 70.2 us).
 namespace {
 #ifdef BP_REPLACES
 constexpr int OUTPUTS = BP_REPLACES;  // 0: added to, 1: replaced

@@ -83,7 +83,7 @@ int launch_tq1_gemv(const GemmArgs& a, hipStream_t s, int waves);
 BP_LAUNCHER(launch_tq1_gemv_fp4, (const GemmArgs& a, hipStream_t s), (a, s))
 // bp_tq2_gemv_fp4.hip: TQ2, one to four token rows per expert, on the fp8 x fp4 matrix instruction with K split over the waves;
 // BP_ERR_UNSUPPORTED without a message when the call is outside its preconditions
-int launch_tq2_gemv_fp4(const GemmArgs& a, hipStream_t s);
+BP_LAUNCHER(launch_tq2_gemv_fp4, (const GemmArgs& a, hipStream_t s), (a, s))
 
 namespace {
 

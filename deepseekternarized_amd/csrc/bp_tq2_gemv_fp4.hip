@@ -149,9 +149,9 @@ __global__ __launch_bounds__(1024) void k_tq2_gemv_ks(GemmArgs a, int nw, int ti
 #pragma unroll
   for (int u = 0; u < KV_OPT; ++u) {
     const int o = (int)threadIdx.x + u * nw * 64;
-    // (tested at run time, not a second object as elsewhere: without the test four tokens spill 11 vector registers instead of 3,
+    // (four tokens: tested at run time in either object - without the test they spill 11 vector registers instead of 3,
     // 128 x 2048 x 7168 111.6 us against 108.8)
-    total[u] = !a.out16 && !a.overwrite && out_live(o) ? a.out[out_at(o)] : 0.f;
+    total[u] = !(NTOK == 4 ? a.out16 || a.overwrite : replaces(a)) && out_live(o) ? a.out[out_at(o)] : 0.f;
   }
   i32x8 A[2 * KV_S];
   float cinit[4], inv2[NTOK], cinitb[4], inv2b[2];  // (b: four tokens, the second step; inv2 / inv2b then hold the lane's two tokens)
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(1024) void k_tq2_gemv_ks(GemmArgs a, int nw, int ti
   for (int u = 0; u < KV_OPT; ++u) {
     const int o = (int)threadIdx.x + u * nw * 64;
     if (!out_live(o)) continue;
-    if (a.out16) a.out16[out_at(o)] = f32_to_bf16_bits(total[u]);
+    if ((NTOK == 4 || OUTPUTS != 0) && a.out16) a.out16[out_at(o)] = f32_to_bf16_bits(total[u]);
     else a.out[out_at(o)] = total[u];
   }
 }
@@ -399,7 +399,7 @@ int launch_kv(const GemmArgs& a, hipStream_t s, int nw, int64_t per, const dim3&
 }  // namespace
 
 // BP_ERR_UNSUPPORTED (no message) where the kernel does not apply: the caller goes on to its other kernels.
-int launch_tq2_gemv_fp4(const GemmArgs& a, hipStream_t s) {
+int BP_OUTPUTS(launch_tq2_gemv_fp4)(const GemmArgs& a, hipStream_t s) {
   const char force = tuning().tq2v;
   if (force == 'n') return BP_ERR_UNSUPPORTED;
   if (a.fmt != BP_TQ2 || a.max_rows < 1 || a.max_rows > 4 || a.tiles) return BP_ERR_UNSUPPORTED;
