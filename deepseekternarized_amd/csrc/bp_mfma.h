@@ -52,8 +52,9 @@ inline bool i8w_takes(int64_t N, int64_t K, int64_t group, int n_terms, int64_t 
   return (group == 128 || (group == 256 && K >= 2048)) && K % 256 == 0 && K >= 1024 && K <= ((int64_t)1 << 20) && N % 16 == 0 && i8w_wr(K, n_terms) != 0 &&
          N * (K / 4) <= ((int64_t)1 << 31) - 4096 && (max_rows + I8W_TOK - 1) / I8W_TOK <= 65535;
 }
-// Calls that run on it when the caller brings a workspace, by the blocks of 128 tokens x 256 rows that hold work if every tile is full.
-// One expert: from 128 blocks on as two small workgroups per CU (WR = 2), from 192 as one of eight waves, which takes as long for 64
+// Calls that run on it when the caller brings a workspace, by their blocks of 128 tokens x 256 rows.
+// One expert: from 96 tokens (64 / 96 tokens x 2048 x 32768, 128 blocks each, 1.50 / 0.94 of the time on the 32-token tiles, x 65536 1.12 /
+// 0.87; a second tile may be nearly empty: 140 tokens x 2048 x 16384 0.94) and 128 blocks on as two small workgroups per CU (WR = 2), from 192 as one of eight waves, which takes as long for 64
 // blocks as for 256. us on it / on the 32-token tiles: 2048 x 2048 x 2048 (128 blocks) 32.8 / 35.5, 512 x 2048 x 6144 (96) 31.1 / 31.9,
 // 1024 x 2048 x 2048 (64) 30.9 / 20.4; eight waves: 3072 x 4096 x 2048 (192) 65.7 / 73.5, 2048 x 4096 x 2048 (128) 63.7 / 51.8, in two
 // terms 2048 x 2048 x 2048 (128) 56.8 / 51.2, 3072 x 2048 x 2048 (192) 60.0 / 73.3, 1024 x 7168 x 6144 (192) 100.6 / 103.9.
@@ -62,7 +63,7 @@ inline bool i8w_takes(int64_t N, int64_t K, int64_t group, int n_terms, int64_t 
 // 0.91 / 0.88); 16 experts x 2048 x 4096 at 256 rows (256 blocks) 0.91 and 1.09, 16 x 4096 x 1024 at 192 (384) 1.05 and 0.94.
 inline bool i8w_pays(int64_t T, int64_t N, int64_t K, int64_t E, int n_terms) {
   const int64_t blocks = (T + I8W_TOK - 1) / I8W_TOK * ((N + 255) / 256);
-  return E == 1 ? blocks >= (i8w_wr(K, n_terms) == 2 ? 128 : 192) : T >= 112 * E && blocks >= 384;
+  return E == 1 ? T >= 96 && blocks >= (i8w_wr(K, n_terms) == 2 ? 128 : 192) : T >= 112 * E && blocks >= 384;
 }
 // bp_gemm_tq1.hip: TQ1 with token tiles of 32 on the fp8 x fp4 matrix instruction (experts with more than 8 token rows);
 // BP_ERR_UNSUPPORTED without a message when the call is outside its preconditions
