@@ -42,7 +42,7 @@ namespace {
 std::atomic<const Tuning*> g_tuning{nullptr};
 std::once_flag g_tuning_once;
 void read_tuning() {
-  Tuning* t = new Tuning{0, 0, 0, 0, 0, 0, -1, 0, -1, 0};
+  Tuning* t = new Tuning{0, 0, 0, 0, 0, 0, -1, 0, -1, -1, 0};
   if (const char* v = getenv("BP_TUNE_R")) t->r = atoi(v);
   if (const char* v = getenv("BP_TUNE_WAVES")) t->waves = atoi(v);
   if (const char* v = getenv("BP_TUNE_TQ1")) t->tq1 = v[0];
@@ -52,6 +52,7 @@ void read_tuning() {
   if (const char* v = getenv("BP_TUNE_F4T")) t->f4t = atoi(v);
   if (const char* v = getenv("BP_TUNE_CPT")) t->cpt = atoi(v);
   if (const char* v = getenv("BP_TUNE_TILES")) t->tiles = atoi(v);
+  if (const char* v = getenv("BP_TUNE_F4")) t->f4 = atoi(v);
   if (const char* v = getenv("BP_TUNE_GLU")) t->glu = v[0];
   g_tuning.store(t, std::memory_order_release);
 }
@@ -186,16 +187,16 @@ extern "C" size_t bp_grouped_gemm_workspace_bytes(int x_dtype, int64_t T, int64_
 extern "C" size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t group, int64_t E, int fmt, int n_terms, int64_t max_rows) {
   if (fmt != BP_TQ2 || T <= 0 || E <= 0 || N <= 0 || K <= 0 || n_terms < 1 || n_terms > BP_MAX_TERMS || max_rows <= 16 || tuning().tq2g == 'b') return 0;
   if (!i8w_takes(N, K, group, n_terms, max_rows < T ? max_rows : T)) return 0;
-  return tuning().tq2g == 'f' || i8w_pays(T, N, K, E, n_terms) ? gemm_i8w_workspace_bytes(T, K, E) : 0;
+  return tuning().tq2g == 'f' || i8w_pays(T, N, K, E, n_terms) ? gemm_f4_workspace_bytes(BP_I8, T, K, E) : 0;
 }
 
 static size_t staged_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows) {
   if (tuning().tq2g == 'b') return 0;
   // (the launcher's own thresholds, so that a call it would turn down does not make its caller allocate)
-  if (fmt == BP_TQ2 && tuning().tq2g != 'f' && (N < 1024 || (T + 31) / 32 * ((N + 511) / 512) < 768)) return 0;  // at least two blocks of 512 output rows, three rounds of one workgroup per CU
+  if (fmt == BP_TQ2 && !f4_pays_bf16(T, N)) return 0;
   if (fmt == BP_TQ1 && max_rows <= 8 && tuning().tq2g != 'f' && !tq1_rows_on_tiles(max_rows, E, T, N)) return 0;  // (the small-batch kernels take these)
   if (max_rows <= 0 || (max_rows + 31) / 32 * 32 * E > 4 * T + 32 * E) return 0;  // a loose bound on the rows per expert: mostly token tiles that do not exist
-  return gemm_tq2f_workspace_bytes(T, K, E);
+  return fmt == BP_TQ2 ? gemm_f4_workspace_bytes(BP_BF16, T, K, E) : gemm_tq2f_workspace_bytes(T, K, E);
 }
 
 extern "C" int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype, const float* x_scale,
@@ -221,6 +222,7 @@ namespace {
 size_t split_bytes(int64_t T, int64_t K);  // of one of a pair
 struct LinearPlan {  // offsets into the workspace
   size_t q, q_scale, sums, sums_bytes, stage, stage_bytes, repacked, bytes;
+  bool f4;      // the conversion pass of the kernel for token tiles of 64 quantises the rows
   bool repack;  // TQ1 weights are rewritten as TQ2 ones first
 };
 // TQ1 linears whose weights are rewritten as TQ2 ones first, which the TQ2 kernels decode faster. From five tokens on while
@@ -229,6 +231,10 @@ struct LinearPlan {  // offsets into the workspace
 // 27 / 60. Larger weights, which the TQ1 kernels' few large workgroups fill the device with, from the number of tokens at which those decode
 // every weight for eight token tiles (4096 tokens x 4096 x 4096: 159 / 283).
 bool repack_pays(int64_t T, int64_t N, int64_t K) { return T >= 256 || (T >= 5 && N <= ((int64_t)1 << 26) / K); }
+// int8 linears on the kernel for token tiles of 64, from 256 workgroups of 64 tokens x 256 rows on: us on it / on the 32-token tiles
+// 8 x 32 of them (2048 x 7168 x 2048) 74 / 77, 13 x 24 (777 x 2048 x 6144) 34.5 / 42, in two terms 51 / 72; 13 x 8 (777 x 7168 x
+// 2048, two terms) 110 / 66, 5 x 24 (300 x 2048 x 6144) 28 / 20.
+bool f4_linear(int64_t T, int64_t N) { return (T + F4_TOK - 1) / F4_TOK * ((N + 255) / 256) >= (tuning().f4 >= 0 ? tuning().f4 : 256); }
 // Memory that a call only runs faster with - converted activations, rewritten weights - is asked for up to this size of either; a
 // larger call runs without it.
 constexpr size_t OPTIONAL_BYTES = (size_t)8 << 30;
@@ -244,6 +250,8 @@ LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int6
   p.q = take(act_int8 ? (size_t)T * (size_t)K : 0);
   p.q_scale = take(act_int8 ? 4 * (size_t)T : 0);
   p.stage_bytes = act_int8 ? bp_grouped_gemm_int8_workspace_bytes(T, N, K, group, 1, fmt, n_terms, T) : bp_grouped_gemm_workspace_bytes(x_dtype, T, N, K, 1, fmt, T);
+  p.f4 = act_int8 && x_dtype == BP_BF16 && fmt == BP_TQ2 && tuning().tq2g != 'b' && (p.stage_bytes || f4_linear(T, N)) && (group == 128 || (group == 256 && K >= 2048)) && N % 16 == 0;
+  if (p.f4) p.stage_bytes = gemm_f4_workspace_bytes(BP_I8, T, K, 1);
   const bool floats = !act_int8 && x_dtype != BP_BF16;  // (a bf16 pair, and its conversion as far as there is room)
   if (p.stage_bytes > OPTIONAL_BYTES) p.stage_bytes = floats && 2 * split_bytes(T, K) <= OPTIONAL_BYTES ? 2 * split_bytes(T, K) : 0;
   p.stage = take(p.stage_bytes);
@@ -303,13 +311,14 @@ extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_
       a = b;
     }
   }
-  if (act_int8 && x_dtype == BP_BF16 && a.stage && g_policy != 1) {  // token tiles of 128: the conversion pass quantises the rows
+  if (p.f4 && a.stage && g_policy != 1) {
     GemmArgs w = a;
     w.x_dtype = BP_BF16;
     w.quant = 1;
     w.overwrite = 1;
     w.out16 = out16;
-    if (mfma_supports(a) && gemm_i8w_applies(w) == BP_OK) return launch_gemm_i8w(w, s);
+    const bool wide = i8w_takes(N, K, group, n_terms, T) && (tuning().tq2g == 'f' || i8w_pays(T, N, K, 1, n_terms));  // (a grouped call's lines)
+    if (mfma_supports(a) && gemm_f4_applies(w) == BP_OK) return launch_gemm_f4(w, s, wide ? "gemm_tq2_i8w" : "gemm_tq2_i8f");
   }
   if (act_int8) {
     if (const int rc = bp_quant_act_int8((int8_t*)(ws + p.q), (float*)(ws + p.q_scale), x, x_dtype, T, K, stream)) return rc;

@@ -28,7 +28,7 @@ struct GemmArgs {
   const void* w_scale[BP_MAX_TERMS];
   int x_dtype, scale_dtype, n_terms, fmt;
   int64_t T, N, K, Kp, G, group, E, max_rows;
-  // Tile-list mode of the token-tile kernels, with tiles of 32 or 128 rows (set by callers that keep the routing on the device, where
+  // Tile-list mode of the token-tile kernels, with tiles of 32 or 64 rows (set by callers that keep the routing on the device, where
   // the widest expert's row count is unknown to the host): tiles = (expert, first row) pairs of the token tiles that exist, in
   // expert order, tile_count[0] of them (device memory, written by a kernel earlier on the stream); the launch covers
   // tile_cap entries and workgroups past the count leave at once. NULL: token tiles are counted by blockIdx.z up to max_rows.
@@ -44,7 +44,7 @@ struct GemmArgs {
   // row x_index[r] / x_div of x, which has x_rows rows (the routed copy of the activations is never materialised).
   const int64_t* x_index;
   int64_t x_div, x_rows;
-  int quant;  // x is bf16 and the conversion pass of the int8 kernel for 128-token tiles quantises its rows (x_scale unused)
+  int quant;  // x is bf16 and the conversion pass of the kernel for 64-token tiles quantises its rows (x_scale unused)
   // bf16 out16[T, N] is written instead of float32 `out` (one launch that covers all of K and all terms; a kernel that
   // takes several passes over an output returns ERR_NO_OUT16 instead).
   uint16_t* out16;
@@ -152,6 +152,7 @@ struct Tuning {
   int f4t;     // BP_TUNE_F4T: routed rows per expert up to which launches of 8 rows are used (-1 = default)
   int cpt;     // BP_TUNE_CPT: chunks per table pass of the table-lookup GEMV
   int tiles;   // BP_TUNE_TILES: tokens from which bp_moe_layer_* runs its GEMMs over the device-side list of token tiles (-1 = default)
+  int f4;      // BP_TUNE_F4: token rows (per expert on average) from which TQ2 layers and linears run on the GEMM over tiles of 64 (-1 = default)
   char glu;    // BP_TUNE_GLU: 'n' bp_moe_layer_* never lets the gate | up GEMM apply SwiGLU itself (a launch of its own instead), 'g' it does but the row gather stays a launch of its own
 };
 const Tuning& tuning();
@@ -180,10 +181,10 @@ constexpr int ERR_NO_OUT16 = -100;
 int run_gemm(const GemmArgs& a, hipStream_t s);
 // True when a launch in tile-list mode would run on one of the 32-token-tile kernels (which honour tiles / overwrite).
 bool gemm_tiles_supported(const GemmArgs& a);
-// Workspace bytes of the TQ2 grouped GEMM over converted activations (GemmArgs::stage) for T rows in all; 0: not available.
+// Workspace bytes of the TQ1 grouped GEMM over converted activations (GemmArgs::stage) for T rows in all; 0: not available.
 size_t gemm_tq2f_workspace_bytes(int64_t T, int64_t K, int64_t E);
-// ... of the int8 GEMM over token tiles of 128 rows.
-size_t gemm_i8w_workspace_bytes(int64_t T, int64_t K, int64_t E);
+// ... of the GEMM over token tiles of 64 rows (act: BP_BF16 or BP_I8).
+size_t gemm_f4_workspace_bytes(int act, int64_t T, int64_t K, int64_t E);
 int launch_general(const GemmArgs& a, hipStream_t s);
 // bp_repack.hip: TQ1 rows as TQ2 rows
 int launch_tq1_to_tq2(uint8_t* out, const uint8_t* in, int64_t rows, int64_t K, hipStream_t s);

@@ -436,12 +436,10 @@ int launch_gemm_sd(const GemmArgs& a, hipStream_t s, const char* name, const cha
 
 // Preconditions (checked by mfma_supports): group 128, K % 256 == 0, K >= 1024, N % 16 == 0, 16-byte aligned x / packed / scales.
 int BP_OUTPUTS(launch_gemm_tq2)(const GemmArgs& a, hipStream_t s) {
-  if (a.stage && a.x_dtype == BP_I8 && !a.tiles && tuning().tq2g != 'b' && (tuning().tq2g == 'f' || i8w_pays(a.T, a.N, a.K, a.E, a.n_terms))) {
-    const int rc = launch_gemm_i8w(a, s);
-    if (rc != BP_ERR_UNSUPPORTED) return rc;
-  }
-  if (a.stage && tuning().tq2g != 'b') {  // with a workspace: the fp8 x fp4 kernel over converted activations (development: BP_TUNE_TQ2G=bf16 keeps this file's kernel)
-    const int rc = launch_gemm_tq2f(a, s);
+  // with a workspace: over converted activations (development: BP_TUNE_TQ2G=bf16 keeps this file's kernel)
+  if (a.stage && tuning().tq2g != 'b' &&
+      (a.x_dtype == BP_I8 ? !a.tiles && (tuning().tq2g == 'f' || i8w_pays(a.T, a.N, a.K, a.E, a.n_terms)) : f4_pays_bf16(a.T, a.N))) {
+    const int rc = launch_gemm_f4(a, s, a.x_dtype == BP_I8 ? "gemm_tq2_i8w" : "gemm_tq2f_bf16");
     if (rc != BP_ERR_UNSUPPORTED) return rc;
   }
 #ifdef BP_DEV_ABLATIONS  // timing ablations (results are wrong): development builds only

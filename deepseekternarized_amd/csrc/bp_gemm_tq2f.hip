@@ -1,42 +1,30 @@
-// TQ2 grouped GEMM for bf16 activations and token tiles of 16 or 32 rows on the scaled fp8 x fp4 matrix instruction
-// (v_mfma_scale_f32_16x16x128_f8f6f4), over activations converted beforehand: 2-bit codes become fp4 operands with four
-// vector instructions per 16 weights, and one matrix instruction covers exactly one 128-wide scale group.
+// TQ1 grouped GEMM for bf16 activations and token tiles of 16 or 32 rows on the scaled fp8 x fp4 matrix instruction
+// (v_mfma_scale_f32_16x16x128_f8f6f4), over activations converted beforehand; one matrix instruction covers exactly one 128-wide scale group.
 //
 // Contract as everywhere (boilerplate/kernels/ternary_cuda.py:58-63, boilerplate/kernels/csrc/ternary_cuda_kernel.cu:44-99):
 // out[t, n] += sum_g scale[n, g] * sum_{k in g} x[t, k] * trit[n, k], float32 accumulation.
 //
-//  * Weights as fp4. A code u = trit + 1 placed at bits [2:1] of a nibble is the E2M1 number u (0000 = 0, 0010 = 1,
-//    0100 = 2), so a packed dword (16 codes) becomes two operand dwords by (w << 1) & 0x66666666 (even codes) and
-//    (w >> 1) & 0x66666666 (odd codes): no table, no LDS. The products then carry sum x * u; every group's accumulator
-//    starts from -sum x, which leaves sum x * (u - 1). The unused code 3 reads 4 - 1 = +3 (pack never writes it).
-//  * A lane loads 16 bytes of its row per 64-byte window (rows are 16-byte aligned: K % 256 == 0); two
-//    v_permlane32_swap leave every lane with 8 bytes of each of the window's two groups, so the four lanes of a row
-//    supply the 128 weights of ONE group to a matrix instruction: lane quarter kb holds the group's weights
-//    64 (kb % 2) + 32 (kb / 2) .. + 31.
 //  * Activations as two fp8 (E4M3) pieces under a power-of-two block scale that the instruction applies itself: the
 //    32 activations that meet one lane of operand B (32 consecutive k) share one E8M0 scale 2^(e - 7), e the exponent
 //    of the block's largest magnitude; y = x / scale = p0 + p1, p0 = y rounded to E4M3, p1 the rounded remainder.
-//    bf16 activations are exactly p0 + p1 down to 2^-9 of their block's largest magnitude; less than 2^-17 of it is
-//    dropped below. Products fp8 x fp4 are exact. A block that holds a NaN or an infinity makes the token's outputs NaN.
+//    Less than 2^-17 of a block's largest magnitude is dropped below. p0 is a multiple of 2^-5, because the instruction drops what lies
+//    13 bits below the largest of the 8 products that it aligns (bp_gemm_f4.hip; error of a layer against 64 bits 5.1e-4 -> 2.7e-4).
+//    Products fp8 x fp4 are exact. A block that holds a NaN or an infinity makes the token's outputs NaN.
 //  * The conversion is vector-ALU work, about as many cycles per token as a workgroup's matrix instructions, and every
 //    row block of an expert would repeat it. So it runs once, in a kernel of its own (k_stage_tq2f), into a workspace of
-//    the caller: per token tile of 32 and 64-byte window, 17 KiB in exactly the layout the GEMM's LDS buffer has
-//    (operands in operand-A register order, block scales, offset sums). The GEMM copies a window's 17 KiB from there.
+//    the caller: per token tile of 32 and window of 256 k, 16.5 KiB in exactly the layout the GEMM's LDS buffer has
+//    (operands in operand-A register order, block scales). The GEMM copies them from there.
 //  * A GEMM workgroup (8 waves) owns 512 output rows x 32 tokens; a wave 64 rows (4 row tiles) x 32 tokens (2 token
 //    tiles): an operand A read from LDS feeds 4 matrix instructions, a decoded weight meets 32 tokens. Weights, scales
 //    and staged activations are requested two windows ahead, one load after each row tile's matrix instructions (all at
 //    once they fill the CU's vector-memory queue and the waves that come last wait thousands of cycles to issue theirs);
 //    every wave issues the same loads in the same order in every window and the stacked terms run as one sequence of
 //    windows, so every wait is for loads at least a window old and counts the younger ones exactly. One barrier per window.
-//
-// TQ1 (FMT = BP_TQ1) runs on the same kernel; only how a lane gets its 32 weights of a group differs. Base-3 bytes have no
-// bit fields and groups of 128 digits end inside bytes (128 / 5 = 25.6), so the lane takes the 8 bytes that hold its 32
-// digits - bytes floor(t / 5) .. + 7 of its row, t = 128 g + 64 (kb % 2) + 32 (kb / 2) the slice's first digit - looks each
-// up in a table byte -> 5 fp4 codes (-1, 0, +1 as E2M1; 20 bits; one copy per lane in LDS, so the address is one
-// v_perm_b32 and no two lanes share a bank), strings the 8 entries together to 160 bits and shifts them right by the
-// 0..4 digits the slice starts inside its first byte (4 v_alignbit_b32): 128 bits = the lane's operand B in k order, one
-// matrix instruction per scale group. The codes are signed: no offset sums. The staged activations are the same, with
-// the 16 activations of a thread in consecutive bytes instead of TQ2's even / odd order.
+//  * Base-3 bytes have no bit fields and groups of 128 digits end inside bytes (128 / 5 = 25.6), so a lane takes the 8 bytes that hold its
+//    32 digits of a group - bytes floor(t / 5) .. + 7 of its row, t = 128 g + 64 (kb % 2) + 32 (kb / 2) the slice's first digit - looks each
+//    up in a table byte -> 5 fp4 codes (-1, 0, +1 as E2M1; 20 bits; one copy per lane in LDS, so the address is one
+//    v_perm_b32 and no two lanes share a bank), strings the 8 entries together to 160 bits and shifts them right by the
+//    0..4 digits the slice starts inside its first byte (4 v_alignbit_b32): 128 bits = the lane's operand B in k order.
 // A window's bytes come from memory the way the cache likes them, not the way the matrix instruction wants them: four
 // neighbouring lanes load the 64 bytes (at a dword-aligned address) that hold a row's 51.2 bytes of the window - 16
 // cache requests per wave load, where a load in the instruction's own lane order (neighbouring lanes = different rows)
@@ -65,12 +53,11 @@ constexpr int F_THREADS = F_WAVES * 64;
 constexpr int F_ROWS = F_WAVES * 16 * F_RT;        // output rows per workgroup
 constexpr int F_OPS = 2 * 2 * 2 * 2048;            // operands of a window: 2 groups x 2 token tiles x 2 pieces x 2 KiB
 constexpr int F_SCL = 2 * 64 * 4;                  // ... the block scales: per token tile one dword per lane (byte g = group g)
-constexpr int F_SUM = 2 * 32 * 4;                  // ... and the offset sums: [group][token] float
-constexpr int F_TAIL = F_SCL + F_SUM;              // (48 x 16 bytes)
-constexpr int F_FB = 32 * 544;                     // a staged window of a token tile: operands, scales, sums, padding (544 bytes per token: a multiple of 16)
+constexpr int F_TAIL = F_SCL;                      // (32 x 16 bytes)
+constexpr int F_FB = 32 * 528;                     // a staged window of a token tile: operands, scales (528 bytes per token: a multiple of 16)
 static_assert(F_OPS + F_TAIL <= F_FB && F_OPS == F_THREADS * 32 && F_TAIL % 16 == 0, "a staged window: two 16-byte pieces per thread and a tail");
 constexpr int F_SC = 2 * F_FB;                     // LDS: two staged windows, then the rows' scales: 2 slots of [512 rows][8 scales] as stored
-constexpr int f_lds_bytes(int scale_bytes) { return F_SC + 2 * F_ROWS * 8 * scale_bytes; }  // 51,200 (16-bit scales) / 67,584 (float32)
+constexpr int f_lds_bytes(int scale_bytes) { return F_SC + 2 * F_ROWS * 8 * scale_bytes; }  // (16-bit scales)
 constexpr int F_LUT = 256 * 256;                   // TQ1: the byte table at LDS address 0 (entry v, copy c at 256 v + 4 c), everything else behind it
 constexpr int F_TP = 72;                           // TQ1: pitch of a row's 64 bytes in the transit area (18 dwords: 16 rows start in 16 different banks), and the area of a wave's row tile
 constexpr int F_TR = 16 * F_TP;
@@ -93,9 +80,7 @@ __device__ __forceinline__ unsigned char* staged_tile(const GemmArgs& a, int64_t
 // mh); lane = (token m3 of 8, quarter kbA of operand A's lanes, half hi of its registers): the thread converts the 16
 // activations that fill registers 4 hi .. 4 hi + 3 of A lane (m, kbA) for the group's instruction: k = 64 (kbA / 2) +
 // 32 hi + 16 (kbA % 2) .. + 15 of the group. A token's group is the 8 lanes (kbA, hi) of one wave: 256 consecutive bytes.
-// NAT: activation j of the thread's 16 goes to register j / 4, byte j % 4 (operand B in k order: TQ1); otherwise to
-// register 2 (j % 2) + j / 8, byte (j % 8) / 2 (operand B as the even and the odd codes of a packed TQ2 dword).
-template <bool NAT>
+// Activation j of the thread's 16 goes to register j / 4, byte j % 4 (operand B in k order).
 __global__ __launch_bounds__(F_THREADS) void k_stage_tq2f(GemmArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const TileRef tr = tile_ref(a, blockIdx.x, blockIdx.z);
@@ -107,9 +92,8 @@ __global__ __launch_bounds__(F_THREADS) void k_stage_tq2f(GemmArgs a) {
   const int m3 = lane & 7, kbA = (lane >> 3) & 3, hi = lane >> 5;
   const int sm = 8 * mh + m3;
   unsigned char* dst = staged_tile(a, tr.e, tok0) + (int64_t)s * F_FB;
-  if (stt == 1 && ntok <= 16) {  // no second token tile: its scales and sums are read all the same (and multiply nothing that is stored)
+  if (stt == 1 && ntok <= 16) {  // no second token tile: its scales are read all the same (and multiply nothing that is stored)
     if ((kbA & 1) == 0) dst[F_OPS + (stt * 64 + ((kbA >> 1) + 2 * hi) * 16 + sm) * 4 + sg] = 127;
-    if (kbA == 0 && hi == 0) *(float*)(dst + F_OPS + F_SCL + (sg * 32 + 16 * stt + sm) * 4) = 0.f;
     return;
   }
   int srow = 16 * stt + sm;
@@ -141,22 +125,18 @@ __global__ __launch_bounds__(F_THREADS) void k_stage_tq2f(GemmArgs a) {
   float mult = __uint_as_float((unsigned)(127 + sh) << 23);
   if (ex == 255) mult = __uint_as_float(0x7fc00000u);  // a NaN or an infinity in the block: every slot becomes NaN
   u32x4 p0, p1;
-  float used = 0.f;  // sum of what the two pieces represent, in the block's scaled domain
+  const float R = 393216.f;  // (1.5 x 2^18: a float near it is a multiple of 2^-5)
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
-    const int v1 = d >> 1, v0 = d & 1;
     int c0 = 0, c1 = 0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const float f0 = y[NAT ? 4 * d + 2 * h : 8 * v0 + 4 * h + v1] * mult, f1 = y[NAT ? 4 * d + 2 * h + 1 : 8 * v0 + 4 * h + 2 + v1] * mult;
-      c0 = h == 0 ? __builtin_amdgcn_cvt_pk_fp8_f32(f0, f1, c0, false) : __builtin_amdgcn_cvt_pk_fp8_f32(f0, f1, c0, true);
+      const float f0 = y[4 * d + 2 * h] * mult, f1 = y[4 * d + 2 * h + 1] * mult;
+      const float g0 = (f0 + R) - R, g1 = (f1 + R) - R;
+      c0 = h == 0 ? __builtin_amdgcn_cvt_pk_fp8_f32(g0, g1, c0, false) : __builtin_amdgcn_cvt_pk_fp8_f32(g0, g1, c0, true);
       const float b0 = h == 0 ? __builtin_amdgcn_cvt_f32_fp8(c0, 0) : __builtin_amdgcn_cvt_f32_fp8(c0, 2);
       const float b1 = h == 0 ? __builtin_amdgcn_cvt_f32_fp8(c0, 1) : __builtin_amdgcn_cvt_f32_fp8(c0, 3);
-      const float r0 = f0 - b0, r1 = f1 - b1;
-      c1 = h == 0 ? __builtin_amdgcn_cvt_pk_fp8_f32(r0, r1, c1, false) : __builtin_amdgcn_cvt_pk_fp8_f32(r0, r1, c1, true);
-      const float e0 = h == 0 ? __builtin_amdgcn_cvt_f32_fp8(c1, 0) : __builtin_amdgcn_cvt_f32_fp8(c1, 2);
-      const float e1 = h == 0 ? __builtin_amdgcn_cvt_f32_fp8(c1, 1) : __builtin_amdgcn_cvt_f32_fp8(c1, 3);
-      used += (b0 + e0) + (b1 + e1);
+      c1 = h == 0 ? __builtin_amdgcn_cvt_pk_fp8_f32(f0 - b0, f1 - b1, c1, false) : __builtin_amdgcn_cvt_pk_fp8_f32(f0 - b0, f1 - b1, c1, true);
     }
     p0[d] = (unsigned)c0;
     p1[d] = (unsigned)c1;
@@ -166,21 +146,13 @@ __global__ __launch_bounds__(F_THREADS) void k_stage_tq2f(GemmArgs a) {
   *(u32x4*)(ob + 2048) = p1;
   // the block's scale: byte sg of the scale operand's dword in lane (m, kb) with kb % 2 = kbA / 2, kb / 2 = hi
   if ((kbA & 1) == 0) dst[F_OPS + (stt * 64 + ((kbA >> 1) + 2 * hi) * 16 + sm) * 4 + sg] = (unsigned char)(127 - sh);
-  // the group's offset sum: what the pieces represent, back in the activations' units, over the token's 8 lanes
-  float part = used * __uint_as_float((unsigned)(127 - sh) << 23);
-  if (ex == 255) part = __uint_as_float(0x7fc00000u);
-  part += __shfl_xor(part, 8, 64);
-  part += __shfl_xor(part, 16, 64);
-  part += __shfl_xor(part, 32, 64);
-  if (kbA == 0 && hi == 0) *(float*)(dst + F_OPS + F_SCL + (sg * 32 + 16 * stt + sm) * 4) = -part;
 }
 
 // GS = 1: scale groups of 256 (the two groups of a window share a scale); 0: of 128.
-template <int SDT, int FMT, int GS>
+template <int SDT, int GS>
 __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSplit split) {
-  constexpr int SB = SDT == BP_F32 ? 4 : 2;
-  constexpr bool Q1 = FMT == BP_TQ1;
-  constexpr unsigned LB = Q1 ? F_LUT : 0;  // LDS address of the staged windows
+  constexpr int SB = 2;  // (16-bit scales)
+  constexpr unsigned LB = F_LUT;  // LDS address of the staged windows
 
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int r16 = lane & 15, kb = lane >> 4;
@@ -209,7 +181,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
   constexpr int gs = GS;
 
   const unsigned alane = LB + (unsigned)(kb * 512 + r16 * 16);
-  if constexpr (Q1) {  // the byte table: two threads per byte value, 32 copies each
+  {  // the byte table: two threads per byte value, 32 copies each
     unsigned v = threadIdx.x >> 1, ent = 0;
     if (v < 243) {
 #pragma unroll
@@ -231,7 +203,6 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
   // ---- the load stream. Window w of the sequence is window w % nwin of term w / nwin; (lterm, ls) names the next window
   // to request. Per window every wave issues, in this order: the thread's three pieces of the staged window, the thread's
   // row's two scales, the wave's four weight loads. Requests past the last window repeat it (never used).
-  const unsigned voff = (unsigned)r16 * (unsigned)a.Kp + 16u * kb;
   // TQ1: first digit of the lane's slice of a window's first group (the second group's: + 128)
   const unsigned cg0 = 64u * (kb & 1) + 32u * (kb >> 1);
   auto slice_of = [&](unsigned s, unsigned g, unsigned& first_byte, unsigned& digit) {  // of window s of a term: byte offset past floor(256 s / 5), digit 0..4 inside it
@@ -251,7 +222,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
   // for every term: a precondition). Loading lane L takes piece L % 4 of row L / 4 of a tile: lpre[r] = byte offset of
   // that piece for window 0, before alignment. Reading lane (r16, kb): upre[r] = byte offset of its row (the low two
   // bits of it and the window's first byte say where the row's bytes start in its 64-byte image).
-  const unsigned mis = Q1 ? (unsigned)((uintptr_t)(a.packed[0] + e * a.N * a.Kp) & 3) : 0u;
+  const unsigned mis = (unsigned)((uintptr_t)(a.packed[0] + e * a.N * a.Kp) & 3);
   unsigned lpre[F_RT], upre[F_RT];
 #pragma unroll
   for (int r = 0; r < F_RT; ++r) {
@@ -271,7 +242,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
     // (TQ1: the range ends with the dword that holds the tensor's last byte - a dword that straddled the end of the range
     // would read as zero, valid bytes included; up to 3 bytes behind the tensor are read with it, inside a dword of which
     // the tensor owns a byte, and never used; whole dwords past that read as zero)
-    wrs = make_rsrc(wbeg + e * a.N * a.Kp - mis, Q1 ? (((a.E - e) * a.N * a.Kp + mis + 3) & ~(int64_t)3) : (a.E - e) * a.N * a.Kp);
+    wrs = make_rsrc(wbeg + e * a.N * a.Kp - mis, ((a.E - e) * a.N * a.Kp + mis + 3) & ~(int64_t)3);
     const unsigned char* sbeg = (const unsigned char*)a.w_scale[term];
     const unsigned char* expert_scales = sbeg + e * a.N * a.G * SB;
     srs = make_rsrc(expert_scales, (sbeg + a.E * a.N * a.G * SB) - expert_scales);
@@ -294,8 +265,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
   auto request = [&](auto p_c, auto part_c) {
     constexpr int P = decltype(p_c)::value, PART = decltype(part_c)::value;
     const unsigned s = (unsigned)ls;
-    if constexpr (PART < F_RT && !Q1) W[P][PART] = buf_load16(wrs, voff, wrow[PART] + 64u * s);
-    if constexpr (PART < F_RT && Q1) W[P][PART] = buf_load16(wrs, (lpre[PART] + lq) & ~3u, 0u);
+    if constexpr (PART < F_RT) W[P][PART] = buf_load16(wrs, (lpre[PART] + lq) & ~3u, 0u);
     if (PART == 4) {
       if (starts_block((int)s)) {  // uniform
         unsigned first;
@@ -314,7 +284,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
         ls = 0;
         set_term(lterm);
       }
-      if constexpr (Q1) lq = (256u * (unsigned)ls) / 5u;
+      lq = (256u * (unsigned)ls) / 5u;
     }
   };
   auto request_all = [&](auto p_c) {
@@ -365,7 +335,6 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
     // it a wave writes the next window's staged activations and scales to LDS, after it it reads them.
     constexpr int DT = TT - 1;       // the token tile whose sums wait for the next group's batch 0
     i32x8 A[TT][2];
-    f32x4 base[TT];
     int sa[2][TT];                   // [window parity][token tile]
     unsigned sraw[2][F_RT][SB / 2];  // [window parity]: the window's two scales of the lane's row of each row tile, as stored
     float scp[F_RT];                 // the scales of the group whose token tile DT is still to be summed
@@ -383,13 +352,6 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
       const u32x4 lo = *(const lds_u32x4*)at, hi4 = *(const lds_u32x4*)(at + 256);
       A[t][pp] = i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi4.x, (int)hi4.y, (int)hi4.z, (int)hi4.w};
     };
-    auto read_base = [&](unsigned ab, int g) {
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if constexpr (Q1) base[t] = f32x4{0.f, 0.f, 0.f, 0.f};  // (signed codes: nothing to take off)
-        else base[t] = __builtin_bit_cast(f32x4, *(const lds_u32x4*)(ab + F_OPS + F_SCL + (unsigned)((g * 32 + 16 * t + 4 * kb) * 4)));
-      }
-    };
     auto read_window_scales = [&](auto h_c, int sw) {  // block scales and row scales of the window of parity H, window sw of its term
       constexpr int H = decltype(h_c)::value;
       const unsigned ab = LB + (unsigned)(H * F_FB);
@@ -402,16 +364,8 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
 #pragma unroll
       for (int r = 0; r < F_RT; ++r) {
         const unsigned at = sb + (unsigned)(16 * r * 8 * SB);
-        if (SB == 2) {
-          if (gs) sraw[H][r][0] = (unsigned)*(const lds_u16*)at * 0x10001u;  // (one scale for both groups)
-          else sraw[H][r][0] = *(const lds_u32*)at;
-        } else if (gs) {
-          sraw[H][r][0] = sraw[H][r][SB / 2 - 1] = *(const lds_u32*)at;
-        } else {
-          const u32x2 v = *(const lds_u32x2*)at;
-          sraw[H][r][0] = v.x;
-          sraw[H][r][SB / 2 - 1] = v.y;
-        }
+        if (gs) sraw[H][r][0] = (unsigned)*(const lds_u16*)at * 0x10001u;  // (one scale for both groups)
+        else sraw[H][r][0] = *(const lds_u32*)at;
       }
     };
     read_a(0u, 0, FC<0>{}, FC<0>{});
@@ -420,10 +374,8 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
       read_a(0u, 0, FC<1>{}, FC<0>{});
       read_a(0u, 0, FC<1>{}, FC<1>{});
     }
-    read_base(0u, 0);
     read_window_scales(FC<0>{}, 0);
 
-    unsigned D[F_RT][2][2];  // TQ2: the window's bytes regrouped: D[r][g] = the lane's 8 bytes (32 weights) of group g
     // TQ1: operand B of a group is made while the group before it is multiplied, in three steps per row tile, each
     // behind the matrix instructions of another batch so that no wave waits for the LDS between a read and its use:
     // the three dwords around the lane's slice are read from the transit area (T), shifted into place and looked up in
@@ -483,7 +435,7 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
         unxt[r] = (upre[r] + qn) & 3u;
       }
     };
-    if constexpr (Q1) {  // the first group's operands (window 0 of term 0 has arrived with the prologue's barrier)
+    {  // the first group's operands (window 0 of term 0 has arrived with the prologue's barrier)
       window_slices(0, 0);
       transit_write(W[0]);
 #pragma unroll
@@ -502,7 +454,6 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
         return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, cv, 0 /* A: E4M3 */, 4 /* B: E2M1 */, g, sav, 0, ones);
       };
       auto row_scale = [&](int r) {
-        if (SDT == BP_F32) return __uint_as_float(sraw[H][r][g == 0 ? 0 : SB / 2 - 1]);
         const unsigned rawsc = g == 0 ? sraw[H][r][0] & 0xffffu : sraw[H][r][0] >> 16;
         return SDT == BP_F16 ? f16_bits_to_f32((uint16_t)rawsc) : __uint_as_float(rawsc << 16);
       };
@@ -513,21 +464,16 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
       const unsigned sh_next = shq[g == 0 ? 1 : 2], fb_next = fbq[g == 0 ? 1 : 2];
       auto step_t = [&](int slot, int r) { transit_read(tb[slot], r, (g == 0 ? ucur[r] : unxt[r]) + fb_next); };
       auto step_l = [&](int slot, int r) { lookups(en[slot], tb[slot], (g == 0 ? ucur[r] : unxt[r]) + fb_next); };
-      if constexpr (Q1 && g == 1) transit_write(W[H ^ 1]);
+      if constexpr (g == 1) transit_write(W[H ^ 1]);
       static_for<F_RT>([&](auto r_c) {
         constexpr int r = decltype(r_c)::value;
-        if constexpr (Q1) {
-          B[r] = i32x8{(int)Bq[g][r].x, (int)Bq[g][r].y, (int)Bq[g][r].z, (int)Bq[g][r].w, 0, 0, 0, 0};
-        } else {
-          const unsigned d0 = D[r][g][0], d1 = D[r][g][1];
-          B[r] = i32x8{(int)((d0 << 1) & m66), (int)((d0 >> 1) & m66), (int)((d1 << 1) & m66), (int)((d1 >> 1) & m66), 0, 0, 0, 0};
-        }
+        B[r] = i32x8{(int)Bq[g][r].x, (int)Bq[g][r].y, (int)Bq[g][r].z, (int)Bq[g][r].w, 0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < 4; ++i) total[r][DT][i] += scp[r] * C[r][DT][i];
         asm volatile("" : "+v"(total[r][DT]));
-        C[r][0] = mfma(A[0][0], B[r], base[0], sa[H][0]);
+        C[r][0] = mfma(A[0][0], B[r], f32x4{0.f, 0.f, 0.f, 0.f}, sa[H][0]);
         asm volatile("" : "+v"(C[r][0]) : : "memory");
-        if constexpr (Q1 && r >= 2) step_t(r - 2, r - 2);
+        if constexpr (r >= 2) step_t(r - 2, r - 2);
         __builtin_amdgcn_sched_barrier(0);
       });
       read_a(nb, ng, FC<0>{}, FC<0>{});
@@ -538,14 +484,14 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
       if constexpr (TT == 2) {
         static_for<F_RT>([&](auto r_c) {
           constexpr int r = decltype(r_c)::value;
-          C[r][1] = mfma(A[1][0], B[r], base[1], sa[H][1]);
+          C[r][1] = mfma(A[1][0], B[r], f32x4{0.f, 0.f, 0.f, 0.f}, sa[H][1]);
           asm volatile("" : "+v"(C[r][1]) : : "memory");
-          if constexpr (Q1 && r < 2) step_l(r, r);
-          if constexpr (Q1 && r >= 2) step_t(r - 2, r);
+          if constexpr (r < 2) step_l(r, r);
+          if constexpr (r >= 2) step_t(r - 2, r);
           __builtin_amdgcn_sched_barrier(0);
         });
         read_a(nb, ng, FC<1>{}, FC<0>{});
-      } else if constexpr (Q1) {
+      } else {
         step_l(0, 0);
         step_l(1, 1);
         step_t(0, 2);
@@ -559,12 +505,11 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
         constexpr int r = decltype(r_c)::value;
         C[r][0] = mfma(A[0][1], B[r], C[r][0], sa[H][0]);
         asm volatile("" : "+v"(C[r][0]) : : "memory");
-        if constexpr (Q1 && r < 2) Bq[ng][r] = strung(en[r], sh_next);
-        if constexpr (Q1 && r >= 2) step_l(r - 2, r);
+        if constexpr (r < 2) Bq[ng][r] = strung(en[r], sh_next);
+        if constexpr (r >= 2) step_l(r - 2, r);
         __builtin_amdgcn_sched_barrier(0);
       });
       read_a(nb, ng, FC<0>{}, FC<1>{});
-      read_base(nb, ng);  // (the accumulators' starting values were last read by batch 1)
       if (g == 1) read_window_scales(FC<H ^ 1>{}, ns);
       request(h_c, FC<g == 0 ? 7 : 2>{});
       __builtin_amdgcn_sched_barrier(0);
@@ -579,38 +524,24 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
           for (int i = 0; i < 4; ++i) total[r][0][i] += sc * C[r][0][i];
           asm volatile("" : "+v"(total[r][0]));
           scp[r] = sc;
-          if constexpr (Q1 && r >= 2) Bq[ng][r] = strung(en[r - 2], sh_next);
+          if constexpr (r >= 2) Bq[ng][r] = strung(en[r - 2], sh_next);
           __builtin_amdgcn_sched_barrier(0);
         });
         read_a(nb, ng, FC<1>{}, FC<1>{});
       } else {
 #pragma unroll
         for (int r = 0; r < F_RT; ++r) scp[r] = row_scale(r);
-        if constexpr (Q1) {
-          Bq[ng][2] = strung(en[0], sh_next);
-          Bq[ng][3] = strung(en[1], sh_next);
-        }
+        Bq[ng][2] = strung(en[0], sh_next);
+        Bq[ng][3] = strung(en[1], sh_next);
       }
       request(h_c, FC<g == 0 ? 4 : 3>{});
       if (g == 1) request(h_c, FC<8>{});
       __builtin_amdgcn_sched_barrier(0);
     };
     auto pwindow = [&](auto h_c) {
-      constexpr int H = decltype(h_c)::value;
-#pragma unroll
-      for (int r = 0; r < F_RT; ++r) {  // (in place: the registers of W[H] are requested again only in this window's second group, after D's last use)
-        if constexpr (!Q1) {
-          const auto s0 = __builtin_amdgcn_permlane32_swap(W[H][r].x, W[H][r].z, false, false);
-          const auto s1 = __builtin_amdgcn_permlane32_swap(W[H][r].y, W[H][r].w, false, false);
-          D[r][0][0] = s0[0];
-          D[r][0][1] = s1[0];
-          D[r][1][0] = s0[1];
-          D[r][1][1] = s1[1];
-        }
-      }
       __builtin_amdgcn_sched_barrier(0);
       ns = cs + 1 < nwin ? cs + 1 : 0;  // the next window's index in its term
-      if constexpr (Q1) window_slices(cs, ns);
+      window_slices(cs, ns);
       pgroup(h_c, FC<0>{});
       __syncthreads();
       pgroup(h_c, FC<1>{});
@@ -675,29 +606,29 @@ __global__ __launch_bounds__(F_THREADS, 2) void k_gemm_tq2f(GemmArgs a, TileSpli
   else all_windows(FC<1>{});
 }
 
-template <int SDT, int FMT, int GS>
+template <int SDT, int GS>
 int launch_gemm_tq2f_g(const GemmArgs& a, hipStream_t s) {
-  constexpr int LDS = f_lds_bytes(SDT == BP_F32 ? 4 : 2) + (FMT == BP_TQ1 ? F_LUT + F_WAVES * F_RT * F_TR : 0);
+  constexpr int LDS = f_lds_bytes(2) + F_LUT + F_WAVES * F_RT * F_TR;
   static_assert(LDS <= 160 * 1024, "LDS of a workgroup");
-  const char* name = FMT == BP_TQ1 ? "gemm_tq1f_bf16" : "gemm_tq2f_bf16";
-  if (const int rc = raise_lds_limit<k_gemm_tq2f<SDT, FMT, GS>>(LDS)) return rc;
+  const char* name = "gemm_tq1f_bf16";
+  if (const int rc = raise_lds_limit<k_gemm_tq2f<SDT, GS>>(LDS)) return rc;
   const int64_t row_blocks = a.glu_h ? (a.N / 2 + F_ROWS / 2 - 1) / (F_ROWS / 2) : (a.N + F_ROWS - 1) / F_ROWS;
   TileSplit split;
   const int64_t wgs = split_tiles(split, a, row_blocks);
   if (wgs < 0) return BP_ERR_UNSUPPORTED;
   const int64_t slots = a.tiles ? a.tile_cap : a.E;
   const unsigned z = a.tiles ? 1u : (unsigned)((a.max_rows + 31) / 32);
-  hipLaunchKernelGGL((k_stage_tq2f<FMT == BP_TQ1>), dim3((unsigned)slots, (unsigned)(a.K / 256), z), dim3(F_THREADS), 0, s, a);
+  hipLaunchKernelGGL(k_stage_tq2f, dim3((unsigned)slots, (unsigned)(a.K / 256), z), dim3(F_THREADS), 0, s, a);
   if (const int rc = check_launch("stage_tq2f")) return rc;
   const dim3 grid((unsigned)wgs, 1, 1);
   note_kernel(name);
-  hipLaunchKernelGGL((k_gemm_tq2f<SDT, FMT, GS>), grid, dim3(F_THREADS), LDS, s, a, split);
+  hipLaunchKernelGGL((k_gemm_tq2f<SDT, GS>), grid, dim3(F_THREADS), LDS, s, a, split);
   return check_launch(name);
 }
 
-template <int SDT, int FMT>
+template <int SDT>
 int launch_gemm_tq2f_k(const GemmArgs& a, hipStream_t s) {
-  return a.group == 256 ? launch_gemm_tq2f_g<SDT, FMT, 1>(a, s) : launch_gemm_tq2f_g<SDT, FMT, 0>(a, s);
+  return a.group == 256 ? launch_gemm_tq2f_g<SDT, 1>(a, s) : launch_gemm_tq2f_g<SDT, 0>(a, s);
 }
 
 }  // namespace
@@ -716,24 +647,16 @@ size_t gemm_tq2f_workspace_bytes(int64_t T, int64_t K, int64_t E) {
 // (the conversion runs one workgroup per tile and window: a loose bound on the rows per expert would launch mostly
 // empty ones). BP_ERR_UNSUPPORTED (no message): the caller falls back to its other kernels.
 int gemm_tq2f_applies(const GemmArgs& a) {
-  if (a.x_dtype != BP_BF16 || !a.stage || ((uintptr_t)a.stage & 15) != 0) return BP_ERR_UNSUPPORTED;
+  if (a.fmt != BP_TQ1 || a.x_dtype != BP_BF16 || !a.stage || ((uintptr_t)a.stage & 15) != 0) return BP_ERR_UNSUPPORTED;
   if (a.glu_h && (!a.tiles || !a.overwrite || a.N % 32 != 0)) return BP_ERR_UNSUPPORTED;  // (whole row tiles of either half, one launch for all of K)
   if ((size_t)a.stage_bytes < gemm_tq2f_workspace_bytes(a.T, a.K, a.E) || gemm_tq2f_workspace_bytes(a.T, a.K, a.E) == 0) return BP_ERR_UNSUPPORTED;
   if (a.K > ((int64_t)1 << 24) || a.N * a.Kp > ((int64_t)1 << 31) - 4096) return BP_ERR_UNSUPPORTED;
-  if (a.fmt == BP_TQ2 && tuning().tq2g != 'f') {  // (development: BP_TUNE_TQ2G=fp4 runs this kernel wherever it can)
-    if (a.N < 2 * F_ROWS) return BP_ERR_UNSUPPORTED;  // (one or two row blocks: converting first saves nothing)
-    // One workgroup of 8 waves takes a CU: below three rounds of them (a round = 256 workgroups) the last, partly filled
-    // round costs more than the kernel gains over the one that runs two smaller workgroups per CU.
-    if ((a.T + 31) / 32 * ((a.N + F_ROWS - 1) / F_ROWS) < 768) return BP_ERR_UNSUPPORTED;
-  }
   if (!a.tiles && ((a.max_rows + 31) / 32 > 65535 || (a.max_rows + 31) / 32 * 32 * a.E > 4 * a.T + 32 * a.E)) return BP_ERR_UNSUPPORTED;
   if (a.K / 256 > 65535) return BP_ERR_UNSUPPORTED;
   if (a.group == 256 && a.scale_dtype != BP_F32 && a.G % 2 != 0) return BP_ERR_UNSUPPORTED;  // (rows of scales not dword-aligned)
-  if (a.fmt == BP_TQ1) {
-    if (a.Kp != (a.K + 4) / 5 || a.scale_dtype == BP_F32) return BP_ERR_UNSUPPORTED;
-    for (int t = 1; t < a.n_terms; ++t)  // (one byte alignment of the rows for all terms)
-      if ((((uintptr_t)a.packed[t] ^ (uintptr_t)a.packed[0]) & 3) != 0) return BP_ERR_UNSUPPORTED;
-  }
+  if (a.Kp != (a.K + 4) / 5 || a.scale_dtype == BP_F32) return BP_ERR_UNSUPPORTED;  // (float32 scales: the table, the transit area and their ring do not fit in LDS together)
+  for (int t = 1; t < a.n_terms; ++t)  // (one byte alignment of the rows for all terms)
+    if ((((uintptr_t)a.packed[t] ^ (uintptr_t)a.packed[0]) & 3) != 0) return BP_ERR_UNSUPPORTED;
   const int64_t row_blocks = a.glu_h ? (a.N / 2 + F_ROWS / 2 - 1) / (F_ROWS / 2) : (a.N + F_ROWS - 1) / F_ROWS;
   TileSplit split;
   return split_tiles(split, a, row_blocks) < 0 ? BP_ERR_UNSUPPORTED : BP_OK;
@@ -741,13 +664,7 @@ int gemm_tq2f_applies(const GemmArgs& a) {
 
 int launch_gemm_tq2f(const GemmArgs& a, hipStream_t s) {
   if (const int rc = gemm_tq2f_applies(a)) return rc;
-  if (a.fmt == BP_TQ1) {
-    if (a.scale_dtype == BP_F16) return launch_gemm_tq2f_k<BP_F16, BP_TQ1>(a, s);
-    return launch_gemm_tq2f_k<BP_BF16, BP_TQ1>(a, s);  // (float32 scales: the table, the transit area and their ring do not fit in LDS together)
-  }
-  if (a.scale_dtype == BP_F16) return launch_gemm_tq2f_k<BP_F16, BP_TQ2>(a, s);
-  if (a.scale_dtype == BP_BF16) return launch_gemm_tq2f_k<BP_BF16, BP_TQ2>(a, s);
-  return launch_gemm_tq2f_k<BP_F32, BP_TQ2>(a, s);
+  return a.scale_dtype == BP_F16 ? launch_gemm_tq2f_k<BP_F16>(a, s) : launch_gemm_tq2f_k<BP_BF16>(a, s);
 }
 
 }  // namespace bp

@@ -37,32 +37,28 @@ BP_LAUNCHER(launch_mfma_tq1, (const GemmArgs& a, hipStream_t s, int waves), (a, 
 // bp_gemm_tq2.hip: TQ2 with token tiles of 32 (experts with more than 16 token rows)
 BP_LAUNCHER(launch_gemm_tq2, (const GemmArgs& a, hipStream_t s), (a, s))
 int launch_gemm_tq2f(const GemmArgs& a, hipStream_t s);
-int gemm_tq2f_applies(const GemmArgs& a);  // BP_OK where launch_gemm_tq2f takes the call (nothing is launched)
-// bp_gemm_i8w.hip: TQ2 with int8 activations (or bf16 ones that it quantises: GemmArgs::quant) and token tiles of 128
-constexpr int I8W_TOK = 128;
-constexpr int I8W_STAGED = 2 * (2 * 2 * (I8W_TOK / 16) * 1024 + 2 * I8W_TOK * 4);  // LDS: two staged windows of the activations
-int launch_gemm_i8w(const GemmArgs& a, hipStream_t s);
-int gemm_i8w_applies(const GemmArgs& a);  // BP_OK where launch_gemm_i8w takes the call (nothing is launched)
-// LDS of a workgroup of 64 WR rows: the staged windows and the rows' scales of all terms, float32. WR = 2 where two workgroups
-// fit a CU, else 4, or 0 where that does not fit either.
-inline int64_t i8w_lds_bytes(int64_t K, int n_terms, int WR) { return I8W_STAGED + (int64_t)n_terms * 64 * WR * (K / 128 + 2) * 4; }
+int gemm_tq2f_applies(const GemmArgs& a);  // TQ1: BP_OK where launch_gemm_tq2f takes the call (nothing is launched)
+// bp_gemm_f4.hip: TQ2 over token tiles of 64, weights as fp4, bf16 activations (or int8 ones, or bf16 ones to be quantised:
+// GemmArgs::quant) as two exact pieces. With a tile list (GemmArgs::tiles, entries of 64 rows): max_rows = F4_TOK.
+constexpr int F4_TOK = 64;
+int launch_gemm_f4(const GemmArgs& a, hipStream_t s, const char* name);
+int gemm_f4_applies(const GemmArgs& a);  // BP_OK where launch_gemm_f4 takes the call (nothing is launched)
+// bf16 calls that run on it: at least two blocks of 512 output rows, and as many tokens as make 768 tiles of 32 x 512. Below, the kernels
+// on bf16 matrix instructions (k_gemm_tq2) sum more exactly (1.4e-7 of a float32 output's size where the fp8 pieces leave 5e-7).
+inline bool f4_pays_bf16(int64_t T, int64_t N) {
+  return tuning().tq2g == 'f' || (N >= 1024 && (T + 31) / 32 * ((N + 511) / 512) >= 768);
+}
+// Int8 grouped calls that ask for its workspace (bp_grouped_gemm_int8_workspace_bytes). The sizes and lines are those that callers
+// know, of the kernel over tiles of 128 that it replaced: that one kept all scales of its 128 or 256 rows in LDS, as float32 beside
+// 67,584 bytes of activations.
+inline int64_t i8w_lds_bytes(int64_t K, int n_terms, int WR) { return 67584 + (int64_t)n_terms * 64 * WR * (K / 128 + 2) * 4; }
 inline int i8w_wr(int64_t K, int n_terms) { return i8w_lds_bytes(K, n_terms, 2) <= 80 * 1024 ? 2 : i8w_lds_bytes(K, n_terms, 4) <= 160 * 1024 ? 4 : 0; }
-// Sizes that the kernel takes (beside them: alignments and workspace, gemm_i8w_applies and mfma_supports).
 inline bool i8w_takes(int64_t N, int64_t K, int64_t group, int n_terms, int64_t max_rows) {
   return (group == 128 || (group == 256 && K >= 2048)) && K % 256 == 0 && K >= 1024 && K <= ((int64_t)1 << 20) && N % 16 == 0 && i8w_wr(K, n_terms) != 0 &&
-         N * (K / 4) <= ((int64_t)1 << 31) - 4096 && (max_rows + I8W_TOK - 1) / I8W_TOK <= 65535;
+         N * (K / 4) <= ((int64_t)1 << 31) - 4096 && (max_rows + 127) / 128 <= 65535;
 }
-// Calls that run on it when the caller brings a workspace, by their blocks of 128 tokens x 256 rows.
-// One expert: from 96 tokens (64 / 96 tokens x 2048 x 32768, 128 blocks each, 1.50 / 0.94 of the time on the 32-token tiles, x 65536 1.12 /
-// 0.87; a second tile may be nearly empty: 140 tokens x 2048 x 16384 0.94) and 128 blocks on as two small workgroups per CU (WR = 2), from 192 as one of eight waves, which takes as long for 64
-// blocks as for 256. us on it / on the 32-token tiles: 2048 x 2048 x 2048 (128 blocks) 32.8 / 35.5, 512 x 2048 x 6144 (96) 31.1 / 31.9,
-// 1024 x 2048 x 2048 (64) 30.9 / 20.4; eight waves: 3072 x 4096 x 2048 (192) 65.7 / 73.5, 2048 x 4096 x 2048 (128) 63.7 / 51.8, in two
-// terms 2048 x 2048 x 2048 (128) 56.8 / 51.2, 3072 x 2048 x 2048 (192) 60.0 / 73.3, 1024 x 7168 x 6144 (192) 100.6 / 103.9.
-// Several experts, whose last tiles are partly empty: from 112 rows per expert and 384 blocks on. 64 experts x 2048 x 2048, 64 / 80 / 96 /
-// 112 / 128 rows each: 1.26 / 1.03 / 1.02 / 0.86 / 0.80 of the time on the 32-token tiles (with 0 to twice as many rows: 1.04 / 1.01 / 0.99 /
-// 0.91 / 0.88); 16 experts x 2048 x 4096 at 256 rows (256 blocks) 0.91 and 1.09, 16 x 4096 x 1024 at 192 (384) 1.05 and 0.94.
 inline bool i8w_pays(int64_t T, int64_t N, int64_t K, int64_t E, int n_terms) {
-  const int64_t blocks = (T + I8W_TOK - 1) / I8W_TOK * ((N + 255) / 256);
+  const int64_t blocks = (T + 127) / 128 * ((N + 255) / 256);
   return E == 1 ? T >= 96 && blocks >= (i8w_wr(K, n_terms) == 2 ? 128 : 192) : T >= 112 * E && blocks >= 384;
 }
 // bp_gemm_tq1.hip: TQ1 with token tiles of 32 on the fp8 x fp4 matrix instruction (experts with more than 8 token rows);

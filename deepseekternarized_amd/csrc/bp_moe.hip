@@ -88,12 +88,12 @@ __global__ __launch_bounds__(256) void k_gather16(u32x4* __restrict__ xg, const 
 // the expert ids (every workgroup ranks the ids for itself in LDS: element i goes to slot #(ids below id_i) + #(equal
 // ids before i); workgroup 0 writes order, offsets and the inverse permutation), the row gather xg[r] = x[order[r] / k]
 // and, where the GEMMs run over the list of token tiles, that list (position r of the order starts a tile when it is a
-// multiple of 32 rows into its expert; the tiles come out in expert order).
+// multiple of tile_rows, 32 or 64, into its expert; the tiles come out in expert order).
 constexpr int ROUTE_SMALL_N = 256, ROUTE_SMALL_THREADS = 256;
 __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __restrict__ order, int64_t* __restrict__ offsets, int64_t* __restrict__ inv,
                                                                      const int64_t* __restrict__ ids, int n, int64_t E, int32_t* __restrict__ bad,
                                                                      u32x4* __restrict__ xg, const u32x4* __restrict__ x, int k, int64_t T, int64_t row16,
-                                                                     int32_t* __restrict__ tiles, int32_t* __restrict__ tile_count, int64_t tile_cap) {
+                                                                     int32_t* __restrict__ tiles, int32_t* __restrict__ tile_count, int64_t tile_cap, int tile_rows) {
   __shared__ __attribute__((aligned(16))) int32_t sid[ROUTE_SMALL_N];  // (entries from n on: 0x7fffffff, "no expert")
   __shared__ int32_t ord[ROUTE_SMALL_N];
   __shared__ __attribute__((aligned(16))) int32_t tstart[ROUTE_SMALL_N];  // position r of the order starts a token tile
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __
     }
     rank += lower;
     ord[rank] = i;
-    if (((rank - lower) & (TILE_ROWS - 1)) == 0) tstart[rank] = 1;
+    if (((rank - lower) & (tile_rows - 1)) == 0) tstart[rank] = 1;
     if (blockIdx.x == 0) {
       order[rank] = i;
       inv[i] = rank;
@@ -168,16 +168,19 @@ __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __
   }
 }
 
-// Layers whose two GEMMs run on the int8 kernel for token tiles of 128: int8 activations, TQ2, 64 rows per expert on average, 1024
-// rows and 80 blocks of 128 rows x 256 gate | up rows (128 with stacked terms). Whole layer against the kernel for tiles of 32, us
-// (hidden / intermediate, experts, rows): 2048 / 1024, 64 experts, 4096 rows (64 per expert) 137.5 / 164.3 (48 per expert: 137 on tiles of
-// 32, which 75 tiles of 128, mostly padding, take as well); 4096 / 2048, 8 experts, 768 rows 108 / 103, 1024 rows 119 / 171; 2048 / 4096, 8
-// experts, 768 rows 121 / 114, 1024 rows 148 / 189; 2048 / 1024, 4 experts, 512 rows 66 / 53, 1024 rows (64 blocks) 70 / 77, in two terms
-// 103 / 99; 1024 / 1024, 16 experts, 1024 rows 60.5 / 59.2, 1536 rows (96 blocks) 64.1 / 63.4 and in two terms 78.4 / 73.2, 2048 rows
-// 69.9 / 85.0 and 88.1 / 100.5.
-bool moe_wide(int act, int fmt, int64_t n, int64_t T, int64_t E, int64_t I, int n_terms) {
-  return act == BP_I8 && fmt == BP_TQ2 && T > 64 && n >= 64 * E && n >= 1024 &&
-         n / I8W_TOK * ((2 * I + 255) / 256) >= (n_terms == 1 ? 80 : 128);
+// Layers whose two GEMMs run on the kernel for token tiles of 64 (TQ2). int8: from 16 rows per expert on average. Whole layer on it / on
+// the 32-token tiles, us: 2048 / 1024 (hidden / intermediate), 64 experts, 16 rows each 71 / 83, 50 rows 112 / 146; 4096 / 2048, 64
+// experts, 12 rows 166 / 163, 37 rows 203 / 305; 384 experts, 6 rows 760 / 740, 19 rows 785 / 930, 62 rows 1350 / 2194.
+// bf16: where one of the two products alone would (f4_pays_bf16).
+bool moe_f4(int act, int fmt, int64_t n, int64_t H, int64_t I, int64_t E) {
+  if (fmt != BP_TQ2 || tuning().tq2g == 'b') return false;
+  if (act == BP_I8) return n >= (tuning().f4 >= 0 ? tuning().f4 : 16) * E;
+  return f4_pays_bf16(n, 2 * I) || f4_pays_bf16(n, H);
+}
+// ... of them, the int8 layers that are named as grouped calls of many rows are: 64 rows per expert, 1024 rows and 80 blocks of 128 rows
+// x 256 gate | up rows (128 with stacked terms).
+bool moe_wide(int64_t n, int64_t T, int64_t E, int64_t I, int n_terms) {
+  return T > 64 && n >= 64 * E && n >= 1024 && n / 128 * ((2 * I + 255) / 256) >= (n_terms == 1 ? 80 : 128);
 }
 
 struct Carve {
@@ -227,13 +230,13 @@ Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k
   p.h = c.take(2 * (size_t)n * I);
   p.y = (float*)c.take(4 * (size_t)n * H);
   p.stage_bytes = 0;
-  if (moe_wide(act, fmt, n, T, E, I, 1)) {  // (the size covers any number of terms)
-    const size_t a = gemm_i8w_workspace_bytes(n, H, E), b = gemm_i8w_workspace_bytes(n, I, E);
-    p.stage_bytes = a > b ? a : b;
-  }
   if (act == BP_BF16) {
     const size_t a = gemm_tq2f_workspace_bytes(n, H, E), b = gemm_tq2f_workspace_bytes(n, I, E);
     p.stage_bytes = a > b ? a : b;
+  }
+  if (moe_f4(act, fmt, n, H, I, E)) {
+    const size_t a = gemm_f4_workspace_bytes(act, n, H, E), b = gemm_f4_workspace_bytes(act, n, I, E), more = a > b ? a : b;
+    p.stage_bytes = more > p.stage_bytes ? more : p.stage_bytes;
   }
   p.stage = (unsigned char*)c.take(p.stage_bytes);
   p.bytes = c.used;
@@ -295,7 +298,7 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   GemmArgs fused;
   memset(&fused, 0, sizeof(fused));
   bool fuse = false;
-  if (tiles && act == BP_BF16 && p.stage_bytes && kernel_policy() != 1 && tuning().glu != 'n' && tuning().tq2g != 'b') {
+  if (tiles && fmt == BP_TQ1 && act == BP_BF16 && p.stage_bytes && kernel_policy() != 1 && tuning().glu != 'n' && tuning().tq2g != 'b') {
     GemmArgs& a = fused;
     a.out = p.gu; a.x = p.xg; a.offsets = p.offsets; a.x_dtype = act;
     for (int t = 0; t < n_terms; ++t) { a.packed[t] = gate_up_packed[t]; a.w_scale[t] = gate_up_scale[t]; }
@@ -311,45 +314,52 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     }
     fuse = gemm_tiles_supported(a) && gemm_tq2f_applies(a) == BP_OK;
   }
-  // The same for int8 activations where experts have many rows each: the token rows are quantised once and the conversion
-  // pass of either GEMM gathers or quantises its rows; gate | up applies SwiGLU and the down projection writes bf16 rows.
-  GemmArgs wide_gu, wide_down;
-  bool wide = false;
-  if (moe_wide(act, fmt, n, T, E, I, n_terms) && tiles && !small && aligned16 && kernel_policy() != 1 && tuning().glu != 'n' && tuning().tq2g != 'b') {
-    memset(&wide_gu, 0, sizeof(wide_gu));
-    GemmArgs& a = wide_gu;
-    a.offsets = p.offsets; a.x_dtype = BP_I8; a.scale_dtype = scale_dtype; a.n_terms = n_terms; a.fmt = fmt; a.group = group;
-    a.T = n; a.E = E; a.max_rows = I8W_TOK; a.overwrite = 1;
+  // TQ2 over token tiles of 64, either activation type: the conversion passes gather (int8: the token rows are quantised once) and
+  // quantise h; gate | up applies SwiGLU and the down projection writes bf16 rows. A down projection that the kernel does not take runs
+  // elsewhere, unless it would need the list of 32-row tiles.
+  GemmArgs f4_gu, f4_down;
+  bool f4 = false, f4_both = false;
+  const bool f4_glu = tuning().glu != 'n', f4_gather = f4_glu && tuning().glu != 'g';
+  if (moe_f4(act, fmt, n, H, I, E) && aligned16 && kernel_policy() != 1 && (f4_gather || act == BP_BF16)) {
+    memset(&f4_gu, 0, sizeof(f4_gu));
+    GemmArgs& a = f4_gu;
+    a.offsets = p.offsets; a.x_dtype = act; a.scale_dtype = scale_dtype; a.n_terms = n_terms; a.fmt = fmt; a.group = group;
+    a.T = n; a.E = E; a.max_rows = F4_TOK; a.overwrite = 1;
     a.stage = p.stage; a.stage_bytes = (int64_t)p.stage_bytes;
-    a.tiles = p.tiles; a.tile_count = p.tile_count; a.tile_cap = (n + I8W_TOK - 1) / I8W_TOK + E;
-    wide_down = a;
+    a.tiles = p.tiles; a.tile_count = p.tile_count; a.tile_cap = (n + F4_TOK - 1) / F4_TOK + E;
+    f4_down = a;
     for (int t = 0; t < n_terms; ++t) { a.packed[t] = gate_up_packed[t]; a.w_scale[t] = gate_up_scale[t]; }
-    a.x = p.q; a.x_scale = p.q_scale; a.x_index = p.order; a.x_div = k; a.x_rows = T;
+    a.x = p.xg;
+    if (f4_gather) { a.x = act == BP_I8 ? (const void*)p.q : x; a.x_scale = p.q_scale; a.x_index = p.order; a.x_div = k; a.x_rows = T; }
     a.N = 2 * I; a.K = H; a.Kp = (H + per - 1) / per; a.G = (H + group - 1) / group;
-    a.glu_h = (uint16_t*)p.h; a.glu_v4 = v4 ? 1 : 0; a.glu_limit = limit;
-    a.glu_weights = v4 ? (const float*)weights : nullptr; a.glu_order = p.order; a.glu_pairs = n;
-    GemmArgs& d = wide_down;
+    a.out = p.gu;
+    if (f4_glu) {
+      a.glu_h = (uint16_t*)p.h; a.glu_v4 = v4 ? 1 : 0; a.glu_limit = limit;
+      a.glu_weights = v4 ? (const float*)weights : nullptr; a.glu_order = p.order; a.glu_pairs = n;
+    }
+    GemmArgs& d = f4_down;
     for (int t = 0; t < n_terms; ++t) { d.packed[t] = down_packed[t]; d.w_scale[t] = down_scale[t]; }
-    d.x = p.h; d.x_dtype = BP_BF16; d.quant = 1;
+    d.x = p.h; d.x_dtype = BP_BF16; d.quant = act == BP_I8 ? 1 : 0;
     d.N = H; d.K = I; d.Kp = (I + per - 1) / per; d.G = (I + group - 1) / group;
-    d.out16 = (uint16_t*)p.y;
+    d.out = p.y;
+    d.out16 = f4_glu ? (uint16_t*)p.y : nullptr;
     GemmArgs probe = d;  // (mfma_supports knows the product's own activation type)
-    probe.x_dtype = BP_I8;
-    wide = mfma_supports(a) && mfma_supports(probe) && gemm_i8w_applies(a) == BP_OK && gemm_i8w_applies(d) == BP_OK;
+    probe.x_dtype = act;
+    f4_both = mfma_supports(probe) && gemm_f4_applies(d) == BP_OK;
+    f4 = mfma_supports(a) && gemm_f4_applies(a) == BP_OK && (f4_both || !gemm_tiles_supported(probe));
   }
+  const char* f4_name = act == BP_BF16 ? "gemm_tq2f_bf16" : moe_wide(n, T, E, I, n_terms) ? "gemm_tq2_i8w" : "gemm_tq2_i8f";
   if (small) {
-    const int64_t row16 = (fuse && fused.x_index) || quant_in ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
+    const int64_t row16 = (f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4) ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
     int64_t g = ((int64_t)n * row16 + ROUTE_SMALL_THREADS - 1) / ROUTE_SMALL_THREADS;
     g = g < 1 ? 1 : (g > 256 ? 256 : g);
     hipLaunchKernelGGL(k_route_small, dim3((unsigned)g), dim3(ROUTE_SMALL_THREADS), 0, s, p.order, p.offsets, p.inv, experts, (int)n, E, bad,
-                       (u32x4*)p.xg, (const u32x4*)x, (int)k, T, row16, tiles ? p.tiles : nullptr, p.tile_count,
-                       p.tile_cap);
+                       (u32x4*)p.xg, (const u32x4*)x, (int)k, T, row16, tiles || f4 ? p.tiles : nullptr, p.tile_count,
+                       p.tile_cap, f4 ? F4_TOK : TILE_ROWS);
     if ((rc = check_launch("route_small")) != BP_OK) return rc;
   } else {
     if ((rc = sort_with_inverse(p.order, p.offsets, p.inv, experts, n, E, p.sort_ws, bad, s)) != BP_OK) return rc;
-    if (wide) {
-      if ((rc = bp_quant_act_int8(p.q, p.q_scale, x, BP_BF16, T, H, s)) != BP_OK) return rc;
-    } else if ((fuse && fused.x_index) || quant_in) {
+    if ((f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4)) {
       // (no routed copy of the activations: the gate | up launch's conversion pass reads them through `order`)
     } else if (aligned16) {
       int64_t g = (n * (H / 8) + 255) / 256;
@@ -413,15 +423,22 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     }
     return run_gemm(a, s);
   };
-  if (tiles && !small) {
-    hipLaunchKernelGGL(k_tile_list, dim3(1), dim3(1024), 0, s, p.tiles, p.tile_count, p.offsets, E, n, p.tile_cap, wide ? I8W_TOK : TILE_ROWS);
+  if ((tiles || f4) && !small) {
+    hipLaunchKernelGGL(k_tile_list, dim3(1), dim3(1024), 0, s, p.tiles, p.tile_count, p.offsets, E, n, p.tile_cap, f4 ? F4_TOK : TILE_ROWS);
     if ((rc = check_launch("tile_list")) != BP_OK) return rc;
   }
-  if (wide) {
-    if ((rc = launch_gemm_i8w(wide_gu, s)) != BP_OK || (rc = launch_gemm_i8w(wide_down, s)) != BP_OK) return rc;
-    note_kernel_suffix("+glu+gather+y16");
-    if (v4) return moe_combine_v4(out, out_dtype, p.y, true, p.inv, experts, T, k, H, s);
-    return moe_combine(out, p.y, true, p.inv, weights, experts, T, k, H, s);
+  if (f4) {
+    if (act == BP_I8 && (rc = bp_quant_act_int8(p.q, p.q_scale, x, BP_BF16, T, H, s)) != BP_OK) return rc;
+    if ((rc = launch_gemm_f4(f4_gu, s, f4_name)) != BP_OK) return rc;
+    if (!f4_glu) rc = v4 ? bp_swiglu_v4(p.h, p.gu, p.gu + I, (const float*)weights, p.order, n, limit, n, I, 2 * I, s) : bp_swiglu_bf16(p.h, p.gu, p.gu + I, n, I, 2 * I, s);
+    if (rc != BP_OK) return rc;
+    bool y16 = f4_glu;
+    rc = f4_both ? launch_gemm_f4(f4_down, s, f4_name) : gemm(p.y, p.h, down_packed, down_scale, H, I, false, &y16, false);
+    if (rc != BP_OK) return rc;
+    if (f4_glu) note_kernel_suffix(f4_gather ? "+glu+gather" : "+glu");
+    if (y16) note_kernel_suffix("+y16");
+    if (v4) return moe_combine_v4(out, out_dtype, p.y, y16, p.inv, experts, T, k, H, s);
+    return moe_combine(out, p.y, y16, p.inv, weights, experts, T, k, H, s);
   }
   bool quant_h = false;
   if (fuse) {

@@ -1,0 +1,80 @@
+"""The GEMM over token tiles of 64: its lines, tiles of at most 32 rows, odd sizes, and what its two pieces of an activation keep."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _terms(E, N, K, terms, gen, sdt=torch.float16, group=128):
+    import deepseekternarized_amd as bp
+
+    return [(bp.pack(torch.randint(-1, 2, (E * N, K), dtype=torch.int8, device="cuda", generator=gen), "tq2").view(E, N, -1),
+             (0.02 * torch.rand(E, N, K // group, device="cuda", generator=gen)).to(sdt)) for _ in range(terms)]
+
+
+# int8 layers either side of the line of 16 rows per expert on average; up to 256 routed rows (preparation and tile list in one launch)
+# and more; against the kernels over tiles of 32, whose exact group sums are scaled and added in the same order
+@pytest.mark.parametrize("pattern,T,E,k,terms,I,wide", [("standard", 127, 16, 2, 1, 1040, False), ("standard", 128, 16, 2, 1, 1040, True), ("v4", 70, 8, 2, 2, 1024, True),
+                                                        ("standard", 333, 16, 3, 2, 1280, True)])
+def test_int8_layers_from_sixteen_rows_per_expert(tune, pattern, T, E, k, terms, I, wide):
+    import deepseekternarized_amd as bp
+    from deepseekternarized_amd.moe import TernaryMoE
+
+    gen = torch.Generator(device="cuda").manual_seed(21)
+    H, v4 = 1280, pattern == "v4"
+    moe = TernaryMoE(_terms(E, I, H, terms, gen), _terms(E, I, H, terms, gen), _terms(E, H, I, terms, gen), H, I, k, "tq2", 128, act="int8", pattern=pattern,
+                     swiglu_limit=10.0 if v4 else 0.0)
+    x = torch.randn(T, H, device="cuda", generator=gen).bfloat16()
+    logits = 1.5 * torch.randn(T, E, device="cuda", generator=gen)
+    logits[:, 3] = -40.0  # an expert without rows
+    w, idx = torch.topk(torch.softmax(logits, -1), k)
+    run = (lambda: moe.routed(x, w, idx)) if v4 else (lambda: moe(x, logits))  # noqa: E731
+    got = run()
+    supported = I % 256 == 0  # (otherwise the down projection runs on the general kernel)
+    name = bp.ext().last_kernel()
+    assert ("+glu+gather" in name) == wide and (not wide or not supported or name == "gemm_tq2_i8f+glu+gather+y16"), name
+    tune("BP_TUNE_TQ2G", "b")
+    ref = run()
+    assert torch.isfinite(got).all()
+    assert float((got.double() - ref.double()).norm() / ref.double().norm()) <= 4e-3  # (bf16 roundings and int8 steps that fall otherwise)
+
+
+# 252 and 256 workgroups of 64 tokens x 256 rows, at a row length whose grouped calls keep to tiles of 32 there; the last tile of 1, 32 and 33 rows
+@pytest.mark.parametrize("T,N,K,name", [(63 * 64 + 1, 1024, 3584, "gemm_tq2_i8f"), (51 * 64 + 32, 1280, 3584, "gemm_tq2_i8f"), (42 * 64 + 33, 1536, 1024, "gemm_tq2_i8w"),
+                                        (63 * 64, 1024, 3584, "gemm_tq2_i8_gs")])
+def test_int8_linears_from_256_workgroups(T, N, K, name):
+    import deepseekternarized_amd as bp
+
+    gen = torch.Generator(device="cuda").manual_seed(22)
+    (packed, scale), = _terms(1, N, K, 1, gen)
+    x = torch.randn(T, K, device="cuda", generator=gen).bfloat16()
+    lin = bp.TernaryLinear([bp.PackedTerm(packed[0], scale[0])], K, "tq2", 128)
+    got = lin(x, torch.float32)
+    assert bp.ext().last_kernel() == name, bp.ext().last_kernel()
+    q, qs = bp.quant_act_int8(x)
+    trits = bp.unpack(packed[0], "tq2", K).double()
+    want = (q.double() @ (trits * scale[0].double().repeat_interleave(128, -1)).T) * qs.double().view(-1, 1)
+    # exact sums of a group; K / 128 scaled additions in float32, each of which rounds by at most 2^-24 of a partial sum
+    assert float((got.double() - want).norm() / want.norm()) <= K / 128 * 2.0**-24
+
+
+@pytest.mark.parametrize("spread", [0, 12])
+def test_bf16_pieces_keep_what_the_matrix_instruction_sums(tune, spread):
+    """bf16 activations of one magnitude and over 2^12 of it: what a value loses below 2^-17 of its block's largest (the instruction
+    aligns the products of 8 k to 13 bits below the largest; the first piece stays above that)."""
+    import deepseekternarized_amd as bp
+
+    T, N, K = 130, 1024, 2048
+    gen = torch.Generator(device="cuda").manual_seed(23)
+    (packed, scale), = _terms(1, N, K, 1, gen)
+    x = torch.randn(T, K, device="cuda", generator=gen) * 2.0 ** -(spread * torch.rand(T, K, device="cuda", generator=gen))
+    x = x.bfloat16()
+    tune("BP_TUNE_TQ2G", "f")
+    got = bp.TernaryLinear([bp.PackedTerm(packed[0], scale[0])], K, "tq2", 128, act="bf16")(x, torch.float32)
+    assert bp.ext().last_kernel() == "gemm_tq2f_bf16"
+    want = x.double() @ (bp.unpack(packed[0], "tq2", K).double() * scale[0].double().repeat_interleave(128, -1)).T
+    # an element's error is at most 2^-17.4 of its block's largest, uniform: 2^-19.2 of it in the mean square; that largest is
+    # about 2.5 (spread 0: 0.3 % of the elements lose anything) to 4.5 (spread 12) times the root mean square
+    bound = 2.5 * 2**-19.2 * 0.003**0.5 + 2**-22 if spread == 0 else 4.5 * 2**-19.2 + 2**-22
+    assert float((got.double() - want).norm() / want.norm()) <= 2 * bound
