@@ -183,6 +183,21 @@ bool moe_wide(int64_t n, int64_t T, int64_t E, int64_t I, int n_terms) {
   return T > 64 && n >= 64 * E && n >= 1024 && n / 128 * ((2 * I + 255) / 256) >= (n_terms == 1 ? 80 : 128);
 }
 
+// TQ1 layers whose weights are rewritten as TQ2 ones first (k_tq1_to_tq2, 0.45 bytes of traffic per weight), in memory that the caller
+// brings beyond bp_moe_layer_workspace_bytes: the products of such a layer run on the kernel for token tiles of 64 then. int8 from 24 rows
+// per expert on average, bf16 from 44 (and from f4_pays_bf16 on). Whole layer with / without, us, int8: 4096 / 2048 (hidden / intermediate),
+// 64 experts, 19 rows each 316 / 284, 28 rows 333 / 406, 375 rows 1133 / 3123; 2048 / 1024, 16 rows 102 / 110 (two terms 177 / 167), 25
+// rows 116 / 182, 1024 rows 899 / 2728; 4096 / 2048, 384 experts, 19 rows 1580 / 1466, 31 rows 1690 / 2038. bf16: 64 experts, 56 rows
+// 420 / 482, 375 rows 1330 / 2259; 384 experts, 31 rows 1779 / 1547, 47 rows 2040 / 2158; 2048 / 1024, 1024 rows 1040 / 2032.
+bool moe_repacks(int act, int fmt, int64_t n, int64_t H, int64_t I, int64_t E, int64_t group) {
+  if (fmt != BP_TQ1 || kernel_policy() == 1 || H % 256 != 0 || I % 256 != 0 || H < 1024 || I < 1024 || H > 65536 || I > 65536) return false;
+  if (group != 128 && !(group == 256 && H % 512 == 0 && I % 512 == 0 && H >= 2048 && I >= 2048)) return false;
+  return moe_f4(act, BP_TQ2, n, H, I, E) && n >= (tuning().f4 >= 0 ? tuning().f4 : act == BP_I8 ? 24 : 44) * E;
+}
+size_t rewritten_bytes(int64_t rows, int64_t K) { return ((size_t)rows * (size_t)(K / 4) + 255) & ~(size_t)255; }
+size_t repack_bytes(int64_t H, int64_t I, int64_t E, int n_terms) { return (size_t)n_terms * (rewritten_bytes(E * 2 * I, H) + rewritten_bytes(E * H, I)); }
+constexpr size_t REPACK_LIMIT = (size_t)8 << 30;
+
 struct Carve {
   unsigned char* base;
   size_t used;
@@ -253,6 +268,14 @@ extern "C" size_t bp_moe_layer_workspace_bytes(int64_t T, int64_t H, int64_t I, 
   return plan(nullptr, T, H, I, E, k, act, fmt).bytes;
 }
 
+extern "C" size_t bp_moe_layer_workspace_bytes_terms(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int64_t group, int n_terms, int act, int fmt) {
+  if (T <= 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0 || n_terms < 1 || n_terms > BP_MAX_TERMS) return 0;
+  const size_t base = plan(nullptr, T, H, I, E, k, act, fmt).bytes;
+  if (!moe_repacks(act, fmt, T * k, H, I, E, group) || repack_bytes(H, I, E, n_terms) > REPACK_LIMIT) return base;
+  const size_t more = plan(nullptr, T, H, I, E, k, act, BP_TQ2).bytes + repack_bytes(H, I, E, n_terms);
+  return more > base ? more : base;
+}
+
 // `v4`: the rounding points of the V4 engine (boilerplate/engine/model.py:376-387, 407-422) instead of the standard
 // decoder's: float32 routing weights applied to the float32 SwiGLU product before the down projection, `limit` clamps,
 // float32 accumulation over a token's experts, output float32 or cast once to bf16 (out_dtype).
@@ -260,7 +283,7 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
                      const uint8_t* const* gate_up_packed, const void* const* gate_up_scale,
                      const uint8_t* const* down_packed, const void* const* down_scale, int scale_dtype,
                      int n_terms, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int64_t group, int fmt,
-                     int act, void* workspace, size_t workspace_bytes, int32_t* bad, void* stream) {
+                     int act, void* workspace, size_t workspace_bytes, int32_t* bad, void* stream, bool rewritten = false) {
   if (T < 0 || H <= 0 || I <= 0 || E <= 0 || E > 65535 || k <= 0 || k > 64 || k > E) return fail(BP_ERR_ARG, "invalid MoE layer dimensions (experts up to 65535, top-k up to 64)");
   if (T * k > ((int64_t)1 << 31) - 1 - 32 * E) return fail(BP_ERR_ARG, "too many routed rows for one call");
   if (fmt != BP_TQ1 && fmt != BP_TQ2) return fail(BP_ERR_ARG, "fmt must be 1 (TQ1) or 2 (TQ2)");
@@ -278,6 +301,24 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   if (((uintptr_t)workspace & 255) != 0) return fail(BP_ERR_ARG, "the workspace must be 256-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   const int64_t n = T * k;
+  if (moe_repacks(act, fmt, n, H, I, E, group) && (((uintptr_t)x | (uintptr_t)out) & 15) == 0) {
+    const size_t own = plan(nullptr, T, H, I, E, k, act, BP_TQ2).bytes, weights2 = repack_bytes(H, I, E, n_terms);
+    bool fits = weights2 <= REPACK_LIMIT && workspace_bytes >= own + weights2;
+    for (int t = 0; t < n_terms; ++t) fits = fits && (((uintptr_t)gate_up_scale[t] | (uintptr_t)down_scale[t]) & 15) == 0;
+    if (fits) {
+      const uint8_t *gu[BP_MAX_TERMS], *dn[BP_MAX_TERMS];
+      unsigned char* at = (unsigned char*)workspace + own;
+      for (int t = 0; t < n_terms; ++t) {
+        gu[t] = at;
+        dn[t] = at + rewritten_bytes(E * 2 * I, H);
+        if (const int rc = launch_tq1_to_tq2(at, gate_up_packed[t], E * 2 * I, H, s)) return rc;
+        if (const int rc = launch_tq1_to_tq2(at + rewritten_bytes(E * 2 * I, H), down_packed[t], E * H, I, s)) return rc;
+        at += rewritten_bytes(E * 2 * I, H) + rewritten_bytes(E * H, I);
+      }
+      return moe_layer(v4, out, out_dtype, limit, x, experts, weights, gu, gate_up_scale, dn, down_scale, scale_dtype, n_terms, T, H, I, E, k, group, BP_TQ2, act,
+                       workspace, own, bad, stream, true);
+    }
+  }
   const int per = fmt == BP_TQ2 ? 4 : 5;
 
   int rc = BP_OK;
@@ -348,7 +389,8 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     f4_both = mfma_supports(probe) && gemm_f4_applies(d) == BP_OK;
     f4 = mfma_supports(a) && gemm_f4_applies(a) == BP_OK && (f4_both || !gemm_tiles_supported(probe));
   }
-  const char* f4_name = act == BP_BF16 ? "gemm_tq2f_bf16" : moe_wide(n, T, E, I, n_terms) ? "gemm_tq2_i8w" : "gemm_tq2_i8f";
+  const char* f4_name = rewritten ? (act == BP_BF16 ? "gemm_tq1_as_tq2f_bf16" : "gemm_tq1_as_tq2_i8f")
+                        : act == BP_BF16 ? "gemm_tq2f_bf16" : moe_wide(n, T, E, I, n_terms) ? "gemm_tq2_i8w" : "gemm_tq2_i8f";
   if (small) {
     const int64_t row16 = (f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4) ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
     int64_t g = ((int64_t)n * row16 + ROUTE_SMALL_THREADS - 1) / ROUTE_SMALL_THREADS;

@@ -262,6 +262,9 @@ int bp_moe_combine_v4(void* out, int out_dtype, const float* y, const int64_t* i
  *   workspace device memory, 256-byte aligned, at least bp_moe_layer_workspace_bytes(T, H, I, E, k, act, fmt) bytes
  *   bad      device i32 flag set to 1 if an expert id is out of range (may be NULL) */
 size_t bp_moe_layer_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int act, int fmt);
+/* ... with the memory in which the weights of a TQ1 layer are rewritten as TQ2 ones where that pays (many token rows per expert; at most
+ * 8 GiB, bp_moe_layer_workspace_bytes otherwise). A layer that gets less runs on the TQ1 kernels. */
+size_t bp_moe_layer_workspace_bytes_terms(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int64_t group, int n_terms, int act, int fmt);
 int bp_moe_layer_bf16(void* out, const void* x, const int64_t* experts, const void* weights,
                       const uint8_t* const* gate_up_packed, const void* const* gate_up_scale,
                       const uint8_t* const* down_packed, const void* const* down_scale, int scale_dtype,

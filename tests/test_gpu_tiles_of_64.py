@@ -78,3 +78,35 @@ def test_bf16_pieces_keep_what_the_matrix_instruction_sums(tune, spread):
     # about 2.5 (spread 0: 0.3 % of the elements lose anything) to 4.5 (spread 12) times the root mean square
     bound = 2.5 * 2**-19.2 * 0.003**0.5 + 2**-22 if spread == 0 else 4.5 * 2**-19.2 + 2**-22
     assert float((got.double() - want).norm() / want.norm()) <= 2 * bound
+
+
+# TQ1 layers either side of the lines from which their weights are rewritten as TQ2 ones: the same trits in either format are the same
+# layer to the bit (int8: exact group sums; bf16: the same kernel). Rows that start at any byte; two terms; groups of 256.
+@pytest.mark.parametrize("act,T,E,k,terms,group,H,I", [("int8", 191, 16, 2, 1, 128, 1280, 1024), ("int8", 192, 16, 2, 1, 128, 1280, 1024), ("int8", 300, 8, 3, 2, 128, 1024, 1792),
+                                                       ("int8", 400, 8, 2, 1, 256, 2048, 2560), ("bf16", 3100, 8, 2, 2, 128, 1024, 1280)])
+def test_tq1_layers_rewritten_as_tq2(act, T, E, k, terms, group, H, I):
+    import deepseekternarized_amd as bp
+    from deepseekternarized_amd.moe import TernaryMoE
+
+    gen = torch.Generator(device="cuda").manual_seed(24)
+
+    def both(N, K):
+        out = {"tq1": [], "tq2": []}
+        for _ in range(terms):
+            trits = torch.randint(-1, 2, (E * N, K), dtype=torch.int8, device="cuda", generator=gen)
+            scale = (0.02 * torch.rand(E, N, K // group, device="cuda", generator=gen)).half()
+            for fmt in out:
+                out[fmt].append((bp.pack(trits, fmt).view(E, N, -1), scale))
+        return out
+
+    gate, up, down = both(I, H), both(I, H), both(H, I)
+    x = torch.randn(T, H, device="cuda", generator=gen).bfloat16()
+    logits = 1.5 * torch.randn(T, E, device="cuda", generator=gen)
+    got = {}
+    for fmt in gate:
+        moe = TernaryMoE(gate[fmt], up[fmt], down[fmt], H, I, k, fmt, group, act=act)
+        got[fmt] = moe(x, logits)
+        rewritten = bp.ext().last_kernel().startswith("gemm_tq1_as_tq2")
+        assert rewritten == (fmt == "tq1" and T * k >= (24 if act == "int8" else 44) * E), bp.ext().last_kernel()
+        assert torch.equal(moe(x, logits), got[fmt])
+    assert torch.isfinite(got["tq1"].float()).all() and torch.equal(got["tq1"], got["tq2"])
