@@ -6,20 +6,34 @@
 // rewritten once, in the workspace, and the call continues as a TQ2 one: the same digits, the same scales.
 // Bound by the memory: 1/5 + 1/4 byte per weight. What kept an earlier version from it was LDS: bytes and a table of one copy, 28
 // conflicting reads for 64 codes. Now a lane loads its 13 or 14 bytes as dwords and has its own copy of the table (64 experts x 3 x
-// 4096 x 2048 weights: 0.73 GB in 280 -> 140 us).
+// 4096 x 2048 weights: 0.73 GB in 280 -> 140 us). The loads are on their way before the table is made.
 #include "bp_mfma.h"
 
 namespace bp {
 namespace {
 
-constexpr int RP_THREADS = 256, RP_EACH = 8;  // pieces of 64 codes that a thread makes
+constexpr int RP_THREADS = 256;
 
 // Pieces of 64 codes, `P` to a row (K = 64 P digits, Kp bytes each, at any byte address). The 13 or 14 bytes that hold a piece's digits
-// through a table byte -> 10 bits, strung together and shifted by the digits that the first byte holds of the codes before.
+// through a table byte -> 10 bits, strung together and shifted by the digits that the first byte holds of the codes before. EACH: pieces
+// that a thread makes.
+template <int EACH>
 __global__ __launch_bounds__(RP_THREADS) void k_tq1_to_tq2(uint4* __restrict__ out, const uint8_t* __restrict__ in, unsigned pieces, unsigned P, Divisor by_P,
                                                            unsigned Kp, int64_t bytes) {
   __shared__ __attribute__((aligned(16))) uint16_t table[256 * 64];  // entry v, copy of lane L at 64 v + L
-  const unsigned lane = threadIdx.x & 63;
+  const unsigned mis = (unsigned)((uintptr_t)in & 3);
+  // (whole dwords: the first and the last one hold a byte of the rows; zeros past them)
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(in - mis, whole_dwords(bytes + mis));
+  const unsigned first_piece = blockIdx.x * (RP_THREADS * EACH) + threadIdx.x;
+  u32x4 w[EACH];
+  unsigned w4[EACH], off[EACH];
+#pragma unroll
+  for (int j = 0; j < EACH; ++j) {
+    const unsigned i = first_piece + RP_THREADS * j, r = quotient(i < pieces ? i : 0u, by_P), p = (i < pieces ? i : 0u) - r * P;
+    off[j] = mis + r * Kp + ((64 * p * 52429u) >> 18);  // (x / 5 for x < 81920)
+    w[j] = buf_load16(rs, off[j] & ~3u, 0u);
+    w4[j] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)((off[j] & ~3u) + 16u), 0, 0);
+  }
   {
     const unsigned v = threadIdx.x;  // (RP_THREADS = 256 entries)
     unsigned c = 0;
@@ -31,22 +45,9 @@ __global__ __launch_bounds__(RP_THREADS) void k_tq1_to_tq2(uint4* __restrict__ o
     for (unsigned i = 0; i < 8; ++i) row[(i + v) & 7] = make_uint4(c, c, c, c);  // (neighbouring threads on different banks)
   }
   __syncthreads();
-  const unsigned mis = (unsigned)((uintptr_t)in & 3);
-  // (whole dwords: the first and the last one hold a byte of the rows; zeros past them)
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(in - mis, whole_dwords(bytes + mis));
-  const uint16_t* mine = table + lane;
-  const unsigned first_piece = blockIdx.x * (RP_THREADS * RP_EACH) + threadIdx.x;
-  u32x4 w[RP_EACH];
-  unsigned w4[RP_EACH], off[RP_EACH];
+  const uint16_t* mine = table + (threadIdx.x & 63);
 #pragma unroll
-  for (int j = 0; j < RP_EACH; ++j) {
-    const unsigned i = first_piece + RP_THREADS * j, r = quotient(i < pieces ? i : 0u, by_P), p = (i < pieces ? i : 0u) - r * P;
-    off[j] = mis + r * Kp + ((64 * p * 52429u) >> 18);  // (x / 5 for x < 81920)
-    w[j] = buf_load16(rs, off[j] & ~3u, 0u);
-    w4[j] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)((off[j] & ~3u) + 16u), 0, 0);
-  }
-#pragma unroll
-  for (int j = 0; j < RP_EACH; ++j) {
+  for (int j = 0; j < EACH; ++j) {
     const unsigned i = first_piece + RP_THREADS * j;
     if (i >= pieces) break;
     const unsigned p = i - quotient(i, by_P) * P, sh = 2 * (64 * p - 5 * ((64 * p * 52429u) >> 18));
@@ -74,8 +75,15 @@ int launch_tq1_to_tq2(uint8_t* out, const uint8_t* in, int64_t rows, int64_t K, 
   const int64_t most = ((int64_t)1 << 30) / Kp;  // rows of a launch (32-bit offsets)
   for (int64_t r = 0; r < rows; r += most) {
     const int64_t n = rows - r < most ? rows - r : most;
-    hipLaunchKernelGGL(k_tq1_to_tq2, dim3((unsigned)((n * P + RP_THREADS * RP_EACH - 1) / (RP_THREADS * RP_EACH))), dim3(RP_THREADS), 0, s, (uint4*)(out + r * (K / 4)),
-                       in + r * Kp, (unsigned)(n * P), (unsigned)P, divisor((unsigned)P), (unsigned)Kp, n * Kp);
+    // Eight pieces per thread, whose workgroups have more loads on their way and a table for more of them, where that leaves a CU
+    // four workgroups; two where the rows are few (a two-term int8 linear of 37 x 4096 x 4096, which rewrites 2 x 128 workgroups of eight:
+    // 37.6 -> 32.3 us).
+    const int64_t pieces = n * P;
+    const bool many = pieces >= (int64_t)1024 * RP_THREADS * 8;
+    const auto kernel = many ? k_tq1_to_tq2<8> : k_tq1_to_tq2<2>;
+    const int64_t per = RP_THREADS * (many ? 8 : 2);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((pieces + per - 1) / per)), dim3(RP_THREADS), 0, s, (uint4*)(out + r * (K / 4)), in + r * Kp, (unsigned)pieces, (unsigned)P,
+                       divisor((unsigned)P), (unsigned)Kp, n * Kp);
     if (const int rc = check_launch("tq1_to_tq2")) return rc;
   }
   return BP_OK;
