@@ -106,17 +106,20 @@ class TernaryMoE:
             values = values / values.sum(-1, keepdim=True)
         return values.to(torch.bfloat16).contiguous(), indices.contiguous()
 
-    def _workspace_bytes(self, tokens: int) -> int:
+    def _workspace(self, tokens: int, device, full: int = 0) -> torch.Tensor:
+        """The layer's workspace. ``full``: the bytes with which the library would also rewrite a TQ1 layer's weights; room for these
+        is taken for the one call, since a layer doesn't hold on to it between calls."""
         e = _need_ext(self.down[0][0])
-        return int(e.lib.bp_moe_layer_workspace_bytes(tokens, self.hidden, self.inter, self.n_experts, self.top_k,
+        ws = getattr(self, "_ws", None)
+        if 0 < full and ws is not None and ws.numel() >= full and ws.device == device:
+            return ws
+        need = int(e.lib.bp_moe_layer_workspace_bytes(tokens, self.hidden, self.inter, self.n_experts, self.top_k,
                                                       _lib.BP_I8 if self.act == "int8" else _lib.BP_BF16, _fmt_code(self.fmt)))
-
-    def _workspace(self, tokens: int, device) -> torch.Tensor:
-        need = self._workspace_bytes(tokens)
+        if full > need:
+            return torch.empty(full, dtype=torch.uint8, device=device)
         device = torch.device(device)
         if device.index is None:  # torch.device("cuda") != torch.device("cuda:0"): compare devices with their index
             device = torch.device(device.type, torch.cuda.current_device())
-        ws = getattr(self, "_ws", None)
         if ws is None or ws.numel() < need or ws.device != device:
             # A HIP graph captured by graphed() holds the address of the workspace it ran in: a workspace that is
             # replaced stays referenced (self._ws_captured) instead of going back to the allocator under that graph.
@@ -146,18 +149,13 @@ class TernaryMoE:
         import ctypes as C
 
         n = len(self.down)
-        # (TQ1 layers with many rows per expert: room for the weights as TQ2 ones, which a layer doesn't hold on to between its calls)
-        more = 0
+        full = 0
         if self.fmt == "tq1":
-            more = int(e.lib.bp_moe_layer_workspace_bytes_terms(T, self.hidden, self.inter, self.n_experts, self.top_k, self.group, n,
-                                                                _lib.BP_I8 if self.act == "int8" else _lib.BP_BF16, _fmt_code(self.fmt)))
-        need = self._workspace_bytes(T)
-        if more > need:
-            ws = torch.empty(more, dtype=torch.uint8, device=flat.device)
-        else:
-            ws = self._workspace(T, flat.device)
-            if torch.cuda.is_current_stream_capturing():
-                self._ws_in_graph = True
+            full = int(e.lib.bp_moe_layer_workspace_bytes_terms(T, self.hidden, self.inter, self.n_experts, self.top_k, self.group, n,
+                                                                _lib.BP_I8 if self.act == "int8" else _lib.BP_BF16, 1))
+        ws = self._workspace(T, flat.device, full)
+        if torch.cuda.is_current_stream_capturing() and ws is getattr(self, "_ws", None):
+            self._ws_in_graph = True
         arr = lambda ts: (C.c_void_p * n)(*[t.data_ptr() for t in ts])
         gp, gs = arr([p for p, _ in self.gate_up]), arr([s for _, s in self.gate_up])
         dp, ds = arr([p for p, _ in self.down]), arr([s for _, s in self.down])
