@@ -42,7 +42,7 @@ namespace {
 std::atomic<const Tuning*> g_tuning{nullptr};
 std::once_flag g_tuning_once;
 void read_tuning() {
-  Tuning* t = new Tuning{0, 0, 0, 0, 0, 0, -1, 0, -1, -1, 0};
+  Tuning* t = new Tuning{0, 0, 0, 0, 0, 0, -1, 0, -1, -1, -1, 0};
   if (const char* v = getenv("BP_TUNE_R")) t->r = atoi(v);
   if (const char* v = getenv("BP_TUNE_WAVES")) t->waves = atoi(v);
   if (const char* v = getenv("BP_TUNE_TQ1")) t->tq1 = v[0];
@@ -53,6 +53,7 @@ void read_tuning() {
   if (const char* v = getenv("BP_TUNE_CPT")) t->cpt = atoi(v);
   if (const char* v = getenv("BP_TUNE_TILES")) t->tiles = atoi(v);
   if (const char* v = getenv("BP_TUNE_F4")) t->f4 = atoi(v);
+  if (const char* v = getenv("BP_TUNE_F4Q")) t->f4q = atoi(v);
   if (const char* v = getenv("BP_TUNE_GLU")) t->glu = v[0];
   g_tuning.store(t, std::memory_order_release);
 }
@@ -187,7 +188,7 @@ extern "C" size_t bp_grouped_gemm_workspace_bytes(int x_dtype, int64_t T, int64_
 extern "C" size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t group, int64_t E, int fmt, int n_terms, int64_t max_rows) {
   if (fmt != BP_TQ2 || T <= 0 || E <= 0 || N <= 0 || K <= 0 || n_terms < 1 || n_terms > BP_MAX_TERMS || max_rows <= 16 || tuning().tq2g == 'b') return 0;
   if (!i8w_takes(N, K, group, n_terms, max_rows < T ? max_rows : T)) return 0;
-  return tuning().tq2g == 'f' || i8w_pays(T, N, K, E, n_terms) ? gemm_f4_workspace_bytes(BP_I8, T, K, E) : 0;
+  return tuning().tq2g == 'f' || i8w_pays(T, N, K, E, n_terms) ? gemm_f4_workspace_bytes(BP_I8, T, K, E, BP_TQ2) : 0;
 }
 
 static size_t staged_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows) {
@@ -196,7 +197,7 @@ static size_t staged_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t E,
   if (fmt == BP_TQ2 && !f4_pays_bf16(T, N)) return 0;
   if (fmt == BP_TQ1 && max_rows <= 8 && tuning().tq2g != 'f' && !tq1_rows_on_tiles(max_rows, E, T, N)) return 0;  // (the small-batch kernels take these)
   if (max_rows <= 0 || (max_rows + 31) / 32 * 32 * E > 4 * T + 32 * E) return 0;  // a loose bound on the rows per expert: mostly token tiles that do not exist
-  return fmt == BP_TQ2 ? gemm_f4_workspace_bytes(BP_BF16, T, K, E) : gemm_tq2f_workspace_bytes(T, K, E);
+  return fmt == BP_TQ2 ? gemm_f4_workspace_bytes(BP_BF16, T, K, E, BP_TQ2) : gemm_tq2f_workspace_bytes(T, K, E);
 }
 
 extern "C" int bp_ternary_grouped_gemm_ws(float* out, const void* x, int x_dtype, const float* x_scale,
@@ -251,7 +252,7 @@ LinearPlan linear_plan(int x_dtype, int act_int8, int out_dtype, int64_t T, int6
   p.q_scale = take(act_int8 ? 4 * (size_t)T : 0);
   p.stage_bytes = act_int8 ? bp_grouped_gemm_int8_workspace_bytes(T, N, K, group, 1, fmt, n_terms, T) : bp_grouped_gemm_workspace_bytes(x_dtype, T, N, K, 1, fmt, T);
   p.f4 = act_int8 && x_dtype == BP_BF16 && fmt == BP_TQ2 && tuning().tq2g != 'b' && (p.stage_bytes || f4_linear(T, N)) && (group == 128 || (group == 256 && K >= 2048)) && N % 16 == 0;
-  if (p.f4) p.stage_bytes = gemm_f4_workspace_bytes(BP_I8, T, K, 1);
+  if (p.f4) p.stage_bytes = gemm_f4_workspace_bytes(BP_I8, T, K, 1, BP_TQ2);
   const bool floats = !act_int8 && x_dtype != BP_BF16;  // (a bf16 pair, and its conversion as far as there is room)
   if (p.stage_bytes > OPTIONAL_BYTES) p.stage_bytes = floats && 2 * split_bytes(T, K) <= OPTIONAL_BYTES ? 2 * split_bytes(T, K) : 0;
   p.stage = take(p.stage_bytes);

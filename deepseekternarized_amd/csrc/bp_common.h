@@ -153,6 +153,7 @@ struct Tuning {
   int cpt;     // BP_TUNE_CPT: chunks per table pass of the table-lookup GEMV
   int tiles;   // BP_TUNE_TILES: tokens from which bp_moe_layer_* runs its GEMMs over the device-side list of token tiles (-1 = default)
   int f4;      // BP_TUNE_F4: token rows (per expert on average) from which TQ2 layers and linears run on the GEMM over tiles of 64 (-1 = default)
+  int f4q;     // BP_TUNE_F4Q: routed rows from which TQ1 layers run on that kernel (-1 = default)
   char glu;    // BP_TUNE_GLU: 'n' bp_moe_layer_* never lets the gate | up GEMM apply SwiGLU itself (a launch of its own instead), 'g' it does but the row gather stays a launch of its own
 };
 const Tuning& tuning();
@@ -183,8 +184,8 @@ int run_gemm(const GemmArgs& a, hipStream_t s);
 bool gemm_tiles_supported(const GemmArgs& a);
 // Workspace bytes of the TQ1 grouped GEMM over converted activations (GemmArgs::stage) for T rows in all; 0: not available.
 size_t gemm_tq2f_workspace_bytes(int64_t T, int64_t K, int64_t E);
-// ... of the GEMM over token tiles of 64 rows (act: BP_BF16 or BP_I8).
-size_t gemm_f4_workspace_bytes(int act, int64_t T, int64_t K, int64_t E);
+// ... of the GEMM on the 32 x 32 x 64 instruction (act: BP_BF16 or BP_I8).
+size_t gemm_f4_workspace_bytes(int act, int64_t T, int64_t K, int64_t E, int fmt);
 int launch_general(const GemmArgs& a, hipStream_t s);
 // bp_repack.hip: TQ1 rows as TQ2 rows
 int launch_tq1_to_tq2(uint8_t* out, const uint8_t* in, int64_t rows, int64_t K, hipStream_t s);

@@ -38,9 +38,9 @@ BP_LAUNCHER(launch_mfma_tq1, (const GemmArgs& a, hipStream_t s, int waves), (a, 
 BP_LAUNCHER(launch_gemm_tq2, (const GemmArgs& a, hipStream_t s), (a, s))
 int launch_gemm_tq2f(const GemmArgs& a, hipStream_t s);
 int gemm_tq2f_applies(const GemmArgs& a);  // TQ1: BP_OK where launch_gemm_tq2f takes the call (nothing is launched)
-// bp_gemm_f4.hip: TQ2 over token tiles of 64, weights as fp4, bf16 activations (or int8 ones, or bf16 ones to be quantised:
-// GemmArgs::quant) as two exact pieces. With a tile list (GemmArgs::tiles, entries of 64 rows): max_rows = F4_TOK.
-constexpr int F4_TOK = 64;
+// bp_gemm_f4.hip: TQ2 over token tiles of 64, TQ1 over tiles of 32, weights as fp4, bf16 activations (or int8 ones, or bf16 ones to be quantised:
+// GemmArgs::quant) as two exact pieces. With a tile list (GemmArgs::tiles, entries of that many rows): max_rows is that.
+constexpr int F4_TOK = 64, F4_TOK1 = 32;  // (TQ2, TQ1)
 int launch_gemm_f4(const GemmArgs& a, hipStream_t s, const char* name);
 int gemm_f4_applies(const GemmArgs& a);  // BP_OK where launch_gemm_f4 takes the call (nothing is launched)
 // bf16 calls that run on it: at least two blocks of 512 output rows, and as many tokens as make 768 tiles of 32 x 512. Below, the kernels

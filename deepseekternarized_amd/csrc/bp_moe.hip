@@ -168,14 +168,24 @@ __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __
   }
 }
 
-// Layers whose two GEMMs run on the kernel for token tiles of 64 (TQ2). int8: from 16 rows per expert on average. Whole layer on it / on
-// the 32-token tiles, us: 2048 / 1024 (hidden / intermediate), 64 experts, 16 rows each 71 / 83, 50 rows 112 / 146; 4096 / 2048, 64
-// experts, 12 rows 166 / 163, 37 rows 203 / 305; 384 experts, 6 rows 760 / 740, 19 rows 785 / 930, 62 rows 1350 / 2194.
-// bf16: where one of the two products alone would (f4_pays_bf16).
-bool moe_f4(int act, int fmt, int64_t n, int64_t H, int64_t I, int64_t E) {
-  if (fmt != BP_TQ2 || tuning().tq2g == 'b') return false;
+// Layers whose two GEMMs run on the kernel for token tiles of 64 (32 for TQ1).
+// TQ2, int8: from 16 rows per expert on average. Whole layer on it / on the 32-token tiles, us: 2048 / 1024 (hidden / intermediate), 64
+// experts, 16 rows each 73 / 82, 50 rows 112 / 146; 4096 / 2048, 64 experts, 12 rows 164 / 163, 37 rows 203 / 305; 384 experts, 6 rows
+// 733 / 739, 19 rows 750 / 920, 62 rows 1350 / 2194. bf16: where one of the two products alone would (f4_pays_bf16).
+// TQ1, int8: from 129 routed rows, where all experts together have 512 workgroups (two to a CU) or there are more than 64 tokens (the old
+// kernels' grids are bounded by the tokens up to there). Whole layer, us: 4096 / 2048, 64 experts of 6, 16 tokens 194 / 181, 32 205 / 316, 64
+// 204 / 221, 251 241 / 372, 1500 765 / 1274; 384 experts, 400 tokens 1038 / 1188, 2000 1357 / 2033; 2048 / 1024, 64 experts of 8, 16 tokens
+// 86 / 86, 64 86 / 89, 200 112 / 182. With fewer workgroups: 7168 / 2048, 16 experts of 8, 17 tokens 188 / 163, 100 179 / 252; 2816 / 1536, 32
+// experts of 4, 34 tokens 99 / 91, 192 130 / 203.
+// TQ1, bf16: from 16 rows per expert, with stacked terms from 44. 4096 / 2048, 64 experts, 6 rows 207 / 199, 12 rows 212 / 209, 23 rows
+// 248 / 295, 37 rows 359 / 402; 384 experts, 6 rows 1080 / 1023, 19 rows 1098 / 1129; 2048 / 1024, 8 rows 84 / 85, 25 rows 111 / 149; in two
+// terms, 64 experts, 37 rows 658 / 622, 47 rows 711 / 730.
+bool moe_f4(int act, int fmt, int64_t T, int64_t n, int64_t H, int64_t I, int64_t E, int n_terms, bool rewritten) {
+  if (tuning().tq2g == 'b') return false;
+  if (fmt == BP_TQ1 && tuning().f4q >= 0) return n >= tuning().f4q;
+  if (fmt == BP_TQ1) return act == BP_I8 ? n > 128 && (T > 64 || E * I >= 512 * 128) : n >= (n_terms == 1 ? 16 : 44) * E;
   if (act == BP_I8) return n >= (tuning().f4 >= 0 ? tuning().f4 : 16) * E;
-  return f4_pays_bf16(n, 2 * I) || f4_pays_bf16(n, H);
+  return rewritten || f4_pays_bf16(n, 2 * I) || f4_pays_bf16(n, H);  // (a TQ1 layer that isn't rewritten runs on fp8 pieces as well)
 }
 // ... of them, the int8 layers that are named as grouped calls of many rows are: 64 rows per expert, 1024 rows and 80 blocks of 128 rows
 // x 256 gate | up rows (128 with stacked terms).
@@ -184,15 +194,16 @@ bool moe_wide(int64_t n, int64_t T, int64_t E, int64_t I, int n_terms) {
 }
 
 // TQ1 layers whose weights are rewritten as TQ2 ones first (k_tq1_to_tq2, 0.45 bytes of traffic per weight), in memory that the caller
-// brings beyond bp_moe_layer_workspace_bytes: the products of such a layer run on the kernel for token tiles of 64 then. int8 from 24 rows
-// per expert on average, bf16 from 44 (and from f4_pays_bf16 on). Whole layer with / without, us, int8: 4096 / 2048 (hidden / intermediate),
-// 64 experts, 19 rows each 316 / 284, 28 rows 333 / 406, 375 rows 1133 / 3123; 2048 / 1024, 16 rows 102 / 110 (two terms 177 / 167), 25
-// rows 116 / 182, 1024 rows 899 / 2728; 4096 / 2048, 384 experts, 19 rows 1580 / 1466, 31 rows 1690 / 2038. bf16: 64 experts, 56 rows
-// 420 / 482, 375 rows 1330 / 2259; 384 experts, 31 rows 1779 / 1547, 47 rows 2040 / 2158; 2048 / 1024, 1024 rows 1040 / 2032.
-bool moe_repacks(int act, int fmt, int64_t n, int64_t H, int64_t I, int64_t E, int64_t group) {
+// brings beyond bp_moe_layer_workspace_bytes: tiles of 64 tokens and no byte table in the products of such a layer then. int8 from 48 rows
+// per expert on average, with stacked terms from 56, bf16 from 64 and 84. Whole layer with / without, us, int8: 4096 / 2048 (hidden /
+// intermediate), 64 experts, 37 rows each 352 / 341, 56 rows 391 / 430, 94 rows 463 / 560, 375 rows 1133 / 1820; 384 experts, 37 rows
+// 1734 / 1690, 56 rows 1904 / 2000; 2048 / 1024, 37 rows 126 / 129, 75 rows 165 / 173. bf16: 64 experts, 47 rows 380 / 362, 66 rows
+// 481 / 480, 94 rows 525 / 580; 384 experts, 56 rows 2197 / 2120, 78 rows 2713 / 2840; 2048 / 1024, 56 rows 162 / 156, 100 rows 186 / 212;
+// in two terms, 64 experts, 75 rows 896 / 890, 94 rows 921 / 1020.
+bool moe_repacks(int act, int fmt, int64_t n, int64_t H, int64_t I, int64_t E, int64_t group, int n_terms) {
   if (fmt != BP_TQ1 || kernel_policy() == 1 || H % 256 != 0 || I % 256 != 0 || H < 1024 || I < 1024 || H > 65536 || I > 65536) return false;
   if (group != 128 && !(group == 256 && H % 512 == 0 && I % 512 == 0 && H >= 2048 && I >= 2048)) return false;
-  return moe_f4(act, BP_TQ2, n, H, I, E) && n >= (tuning().f4 >= 0 ? tuning().f4 : act == BP_I8 ? 24 : 44) * E;
+  return tuning().tq2g != 'b' && n >= (tuning().f4 >= 0 ? tuning().f4 : act == BP_I8 ? (n_terms == 1 ? 48 : 56) : n_terms == 1 ? 64 : 84) * E;
 }
 size_t rewritten_bytes(int64_t rows, int64_t K) { return ((size_t)rows * (size_t)(K / 4) + 255) & ~(size_t)255; }
 size_t repack_bytes(int64_t H, int64_t I, int64_t E, int n_terms) { return (size_t)n_terms * (rewritten_bytes(E * 2 * I, H) + rewritten_bytes(E * H, I)); }
@@ -227,7 +238,7 @@ struct Plan {
   size_t bytes;
 };
 
-Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int act, int fmt) {
+Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int act, int fmt, int n_terms, bool rewritten = false) {
   Carve c = {(unsigned char*)workspace, 0};
   Plan p;
   const int64_t n = T * k;
@@ -249,8 +260,8 @@ Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k
     const size_t a = gemm_tq2f_workspace_bytes(n, H, E), b = gemm_tq2f_workspace_bytes(n, I, E);
     p.stage_bytes = a > b ? a : b;
   }
-  if (moe_f4(act, fmt, n, H, I, E)) {
-    const size_t a = gemm_f4_workspace_bytes(act, n, H, E), b = gemm_f4_workspace_bytes(act, n, I, E), more = a > b ? a : b;
+  if (moe_f4(act, fmt, T, n, H, I, E, n_terms, rewritten)) {
+    const size_t a = gemm_f4_workspace_bytes(act, n, H, E, fmt), b = gemm_f4_workspace_bytes(act, n, I, E, fmt), more = a > b ? a : b;
     p.stage_bytes = more > p.stage_bytes ? more : p.stage_bytes;
   }
   p.stage = (unsigned char*)c.take(p.stage_bytes);
@@ -265,14 +276,14 @@ using namespace bp;
 
 extern "C" size_t bp_moe_layer_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int act, int fmt) {
   if (T < 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0) return 0;
-  return plan(nullptr, T, H, I, E, k, act, fmt).bytes;
+  return plan(nullptr, T, H, I, E, k, act, fmt, 1).bytes;  // (of any count of terms: one has the lowest lines)
 }
 
 extern "C" size_t bp_moe_layer_workspace_bytes_terms(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int64_t group, int n_terms, int act, int fmt) {
   if (T <= 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0 || n_terms < 1 || n_terms > BP_MAX_TERMS) return 0;
-  const size_t base = plan(nullptr, T, H, I, E, k, act, fmt).bytes;
-  if (!moe_repacks(act, fmt, T * k, H, I, E, group) || repack_bytes(H, I, E, n_terms) > REPACK_LIMIT) return base;
-  const size_t more = plan(nullptr, T, H, I, E, k, act, BP_TQ2).bytes + repack_bytes(H, I, E, n_terms);
+  const size_t base = plan(nullptr, T, H, I, E, k, act, fmt, 1).bytes;
+  if (!moe_repacks(act, fmt, T * k, H, I, E, group, n_terms) || repack_bytes(H, I, E, n_terms) > REPACK_LIMIT) return base;
+  const size_t more = plan(nullptr, T, H, I, E, k, act, BP_TQ2, n_terms, true).bytes + repack_bytes(H, I, E, n_terms);
   return more > base ? more : base;
 }
 
@@ -296,13 +307,18 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   if (!out || !x || !experts || !weights || !gate_up_packed || !gate_up_scale || !down_packed || !down_scale) return fail(BP_ERR_ARG, "null pointer");
   for (int t = 0; t < n_terms; ++t)
     if (!gate_up_packed[t] || !gate_up_scale[t] || !down_packed[t] || !down_scale[t]) return fail(BP_ERR_ARG, "null packed or scale pointer in term %d", t);
-  const Plan p = plan(workspace, T, H, I, E, k, act, fmt);
+  const Plan p = plan(workspace, T, H, I, E, k, act, fmt, n_terms, rewritten);
   if (!workspace || workspace_bytes < p.bytes) return fail(BP_ERR_ARG, "the workspace must hold bp_moe_layer_workspace_bytes() = %zu bytes", p.bytes);
   if (((uintptr_t)workspace & 255) != 0) return fail(BP_ERR_ARG, "the workspace must be 256-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   const int64_t n = T * k;
-  if (moe_repacks(act, fmt, n, H, I, E, group) && (((uintptr_t)x | (uintptr_t)out) & 15) == 0) {
-    const size_t own = plan(nullptr, T, H, I, E, k, act, BP_TQ2).bytes, weights2 = repack_bytes(H, I, E, n_terms);
+  // bf16 TQ1 layers on fp8 pieces, rewritten or not: those that k_gemm_tq2f has on pieces too. The others keep the kernel that multiplies bf16.
+  bool pieces = act != BP_BF16 || fmt != BP_TQ1 || (T > 24 && scale_dtype != BP_F32 && (group != 256 || (((H + 255) / 256) % 2 == 0 && ((I + 255) / 256) % 2 == 0)));
+  if (act == BP_BF16 && fmt == BP_TQ1)
+    for (int t = 1; t < n_terms; ++t)
+      pieces = pieces && ((((uintptr_t)gate_up_packed[t] ^ (uintptr_t)gate_up_packed[0]) | ((uintptr_t)down_packed[t] ^ (uintptr_t)down_packed[0])) & 3) == 0;
+  if (pieces && moe_repacks(act, fmt, n, H, I, E, group, n_terms) && (((uintptr_t)x | (uintptr_t)out) & 15) == 0) {
+    const size_t own = plan(nullptr, T, H, I, E, k, act, BP_TQ2, n_terms, true).bytes, weights2 = repack_bytes(H, I, E, n_terms);
     bool fits = weights2 <= REPACK_LIMIT && workspace_bytes >= own + weights2;
     for (int t = 0; t < n_terms; ++t) fits = fits && (((uintptr_t)gate_up_scale[t] | (uintptr_t)down_scale[t]) & 15) == 0;
     if (fits) {
@@ -359,15 +375,16 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   // quantise h; gate | up applies SwiGLU and the down projection writes bf16 rows. A down projection that the kernel does not take runs
   // elsewhere, unless it would need the list of 32-row tiles.
   GemmArgs f4_gu, f4_down;
+  const int f4_tok = fmt == BP_TQ1 ? F4_TOK1 : F4_TOK;
   bool f4 = false, f4_both = false;
   const bool f4_glu = tuning().glu != 'n', f4_gather = f4_glu && tuning().glu != 'g';
-  if (moe_f4(act, fmt, n, H, I, E) && aligned16 && kernel_policy() != 1 && (f4_gather || act == BP_BF16)) {
+  if (moe_f4(act, fmt, T, n, H, I, E, n_terms, rewritten) && pieces && aligned16 && kernel_policy() != 1 && (f4_gather || act == BP_BF16)) {
     memset(&f4_gu, 0, sizeof(f4_gu));
     GemmArgs& a = f4_gu;
     a.offsets = p.offsets; a.x_dtype = act; a.scale_dtype = scale_dtype; a.n_terms = n_terms; a.fmt = fmt; a.group = group;
-    a.T = n; a.E = E; a.max_rows = F4_TOK; a.overwrite = 1;
+    a.T = n; a.E = E; a.max_rows = f4_tok; a.overwrite = 1;
     a.stage = p.stage; a.stage_bytes = (int64_t)p.stage_bytes;
-    a.tiles = p.tiles; a.tile_count = p.tile_count; a.tile_cap = (n + F4_TOK - 1) / F4_TOK + E;
+    a.tiles = p.tiles; a.tile_count = p.tile_count; a.tile_cap = (n + f4_tok - 1) / f4_tok + E;
     f4_down = a;
     for (int t = 0; t < n_terms; ++t) { a.packed[t] = gate_up_packed[t]; a.w_scale[t] = gate_up_scale[t]; }
     a.x = p.xg;
@@ -390,6 +407,7 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     f4 = mfma_supports(a) && gemm_f4_applies(a) == BP_OK && (f4_both || !gemm_tiles_supported(probe));
   }
   const char* f4_name = rewritten ? (act == BP_BF16 ? "gemm_tq1_as_tq2f_bf16" : "gemm_tq1_as_tq2_i8f")
+                        : fmt == BP_TQ1 ? (act == BP_BF16 ? "gemm_tq1f_bf16" : "gemm_tq1_i8f")
                         : act == BP_BF16 ? "gemm_tq2f_bf16" : moe_wide(n, T, E, I, n_terms) ? "gemm_tq2_i8w" : "gemm_tq2_i8f";
   if (small) {
     const int64_t row16 = (f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4) ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
@@ -397,7 +415,7 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     g = g < 1 ? 1 : (g > 256 ? 256 : g);
     hipLaunchKernelGGL(k_route_small, dim3((unsigned)g), dim3(ROUTE_SMALL_THREADS), 0, s, p.order, p.offsets, p.inv, experts, (int)n, E, bad,
                        (u32x4*)p.xg, (const u32x4*)x, (int)k, T, row16, tiles || f4 ? p.tiles : nullptr, p.tile_count,
-                       p.tile_cap, f4 ? F4_TOK : TILE_ROWS);
+                       p.tile_cap, f4 ? f4_tok : TILE_ROWS);
     if ((rc = check_launch("route_small")) != BP_OK) return rc;
   } else {
     if ((rc = sort_with_inverse(p.order, p.offsets, p.inv, experts, n, E, p.sort_ws, bad, s)) != BP_OK) return rc;
@@ -466,7 +484,7 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     return run_gemm(a, s);
   };
   if ((tiles || f4) && !small) {
-    hipLaunchKernelGGL(k_tile_list, dim3(1), dim3(1024), 0, s, p.tiles, p.tile_count, p.offsets, E, n, p.tile_cap, f4 ? F4_TOK : TILE_ROWS);
+    hipLaunchKernelGGL(k_tile_list, dim3(1), dim3(1024), 0, s, p.tiles, p.tile_count, p.offsets, E, n, p.tile_cap, f4 ? f4_tok : TILE_ROWS);
     if ((rc = check_launch("tile_list")) != BP_OK) return rc;
   }
   if (f4) {

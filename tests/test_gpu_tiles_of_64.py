@@ -82,7 +82,7 @@ def test_bf16_pieces_keep_what_the_matrix_instruction_sums(tune, spread):
 
 # TQ1 layers either side of the lines from which their weights are rewritten as TQ2 ones: the same trits in either format are the same
 # layer to the bit (int8: exact group sums; bf16: the same kernel). Rows that start at any byte; two terms; groups of 256.
-@pytest.mark.parametrize("act,T,E,k,terms,group,H,I", [("int8", 191, 16, 2, 1, 128, 1280, 1024), ("int8", 192, 16, 2, 1, 128, 1280, 1024), ("int8", 300, 8, 3, 2, 128, 1024, 1792),
+@pytest.mark.parametrize("act,T,E,k,terms,group,H,I", [("int8", 383, 16, 2, 1, 128, 1280, 1024), ("int8", 384, 16, 2, 1, 128, 1280, 1024), ("int8", 300, 8, 3, 2, 128, 1024, 1792),
                                                        ("int8", 400, 8, 2, 1, 256, 2048, 2560), ("bf16", 3100, 8, 2, 2, 128, 1024, 1280)])
 def test_tq1_layers_rewritten_as_tq2(act, T, E, k, terms, group, H, I):
     import deepseekternarized_amd as bp
@@ -107,6 +107,38 @@ def test_tq1_layers_rewritten_as_tq2(act, T, E, k, terms, group, H, I):
         moe = TernaryMoE(gate[fmt], up[fmt], down[fmt], H, I, k, fmt, group, act=act)
         got[fmt] = moe(x, logits)
         rewritten = bp.ext().last_kernel().startswith("gemm_tq1_as_tq2")
-        assert rewritten == (fmt == "tq1" and T * k >= (24 if act == "int8" else 44) * E), bp.ext().last_kernel()
+        assert rewritten == (fmt == "tq1" and T * k >= (48 if act == "int8" and terms == 1 else 56 if act == "int8" else 84) * E), bp.ext().last_kernel()
         assert torch.equal(moe(x, logits), got[fmt])
     assert torch.isfinite(got["tq1"].float()).all() and torch.equal(got["tq1"], got["tq2"])
+
+
+# TQ1 layers on that kernel as they are, by the byte table: tiles of 32 tokens, rows that start at any byte, windows of an odd count, two
+# terms, groups of 256, scales of 32 bits (bf16 layers of these keep the kernel without pieces); either side of its lines. int8 (exact group sums): the bits of the same trits' TQ2 layer on the
+# kernels over tiles of 32; bf16: of the kernel for 16 x 16 x 128 pieces, whose pieces and order of additions are the same.
+@pytest.mark.parametrize("act,T,E,k,terms,group,H,I,sdt,name", [
+    ("int8", 64, 64, 3, 1, 128, 1280, 1024, torch.float16, "gemm_tq1_i8f"), ("int8", 65, 8, 2, 2, 128, 1792, 1280, torch.float16, "gemm_tq1_i8f"),
+    ("int8", 80, 4, 2, 1, 256, 2048, 2560, torch.float32, "gemm_tq1_i8f"), ("int8", 64, 64, 2, 1, 128, 1280, 1024, torch.float16, None),
+    ("bf16", 64, 8, 2, 1, 128, 1280, 1792, torch.bfloat16, "gemm_tq1f_bf16"), ("bf16", 100, 4, 2, 1, 256, 2048, 2560, torch.float16, "gemm_tq1f_bf16"),
+    ("bf16", 180, 8, 2, 2, 128, 1024, 1280, torch.float16, "gemm_tq1f_bf16"),
+    ("bf16", 180, 8, 2, 2, 128, 1024, 1280, torch.float32, "gemm_tq1_bf16")])
+def test_tq1_layers_by_the_byte_table(tune, act, T, E, k, terms, group, H, I, sdt, name):
+    import deepseekternarized_amd as bp
+    from deepseekternarized_amd.moe import TernaryMoE
+
+    gen = torch.Generator(device="cuda").manual_seed(25)
+    raw = [[(torch.randint(-1, 2, (E * N, K), dtype=torch.int8, device="cuda", generator=gen), (0.02 * torch.rand(E, N, K // group, device="cuda", generator=gen)).to(sdt))
+            for _ in range(terms)] for N, K in ((I, H), (I, H), (H, I))]
+    packed = lambda fmt: [[(bp.pack(t, fmt).view(E, s.shape[1], -1), s) for t, s in part] for part in raw]  # noqa: E731
+    x = torch.randn(T, H, device="cuda", generator=gen).bfloat16()
+    logits = 1.5 * torch.randn(T, E, device="cuda", generator=gen)
+    logits[:, 1] = -40.0  # an expert without rows
+    got = TernaryMoE(*packed("tq1"), H, I, k, "tq1", group, act=act)(x, logits)
+    ran = bp.ext().last_kernel().split("+")[0]
+    assert ran == name if name else not ran.endswith("i8f"), ran
+    if act == "int8":
+        tune("BP_TUNE_F4", "1000000")
+        ref = TernaryMoE(*packed("tq2"), H, I, k, "tq2", group, act=act)(x, logits)
+    else:
+        tune("BP_TUNE_F4Q", "1000000000")
+        ref = TernaryMoE(*packed("tq1"), H, I, k, "tq1", group, act=act)(x, logits)
+    assert torch.isfinite(got.float()).all() and torch.equal(got, ref), bp.ext().last_kernel()
