@@ -187,6 +187,14 @@ size_t gemm_tq2f_workspace_bytes(int64_t T, int64_t K, int64_t E);
 // ... of the GEMM on the 32 x 32 x 64 instruction (act: BP_BF16 or BP_I8).
 size_t gemm_f4_workspace_bytes(int act, int64_t T, int64_t K, int64_t E, int fmt);
 int launch_general(const GemmArgs& a, hipStream_t s);
+// bp_route.hip: where a sort by expert also lists the token tiles of `rows` rows: (expert, first row) of each in expert order, count[0]
+// their number, at most `cap`. tiles NULL: no list.
+struct SortTiles {
+  int32_t* tiles;
+  int32_t* count;
+  int64_t cap;
+  int rows;
+};
 // bp_repack.hip: TQ1 rows as TQ2 rows
 int launch_tq1_to_tq2(uint8_t* out, const uint8_t* in, int64_t rows, int64_t K, hipStream_t s);
 // Returns BP_ERR_UNSUPPORTED (without setting an error message) when the shape is outside the

@@ -5,7 +5,7 @@
 //
 // Nothing is read back to the host. The reference sizes its grouped launch from `int(offsets.diff().max())`
 // (boilerplate/kernels/ternary_cuda.py:97), a device-to-host copy in the middle of the layer; here a kernel writes
-// the list of token tiles that exist (k_tile_list; 32 rows each, 128 in large int8 layers), and the grouped GEMMs run over it. Up to 64 tokens
+// the list of token tiles that exist (made by the sort; 32 or 64 rows each), and the grouped GEMMs run over it. Up to 64 tokens
 // no expert can have more than 64 rows, and the launch is sized by that bound instead (the small-batch kernels).
 //
 // All intermediate tensors live in a workspace the caller provides (bp_moe_layer_workspace_bytes): the library
@@ -17,7 +17,7 @@
 namespace bp {
 int kernel_policy();  // bp_api.hip
 int sort_with_inverse(int64_t* order, int64_t* offsets, int64_t* inv, const int64_t* ids, int64_t n, int64_t E, int32_t* workspace,
-                      int32_t* bad, hipStream_t stream);  // bp_route.hip
+                      int32_t* bad, hipStream_t stream, const SortTiles& t);  // bp_route.hip
 int64_t sort_with_inverse_ints(int64_t n, int64_t E);  // its workspace
 int moe_combine(void* out, const void* y, bool y16, const int64_t* inv, const void* w, const int64_t* experts, int64_t T, int64_t k, int64_t H,
                 void* stream);  // bp_route.hip
@@ -30,48 +30,6 @@ int swiglu_quant(bool v4, int8_t* q, float* s, const float* gate, const float* u
 namespace {
 
 constexpr int TILE_ROWS = 32;  // token tile of k_gemm_tq1 / k_gemm_tq2
-
-// (expert, first row) of every token tile of `tile_rows` rows, in expert order; count[0] = their number. One workgroup; experts in
-// chunks of 1024 with a running total.
-__global__ __launch_bounds__(1024) void k_tile_list(int32_t* __restrict__ tiles, int32_t* __restrict__ count, const int64_t* __restrict__ offsets,
-                                                    int64_t E, int64_t T, int64_t cap, int tile_rows) {
-  __shared__ int part[16];
-  __shared__ int carry;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int64_t base = 0; base < E; base += 1024) {
-    const int64_t e = base + threadIdx.x;
-    int64_t o0 = 0, rows = 0;
-    if (e < E) {
-      o0 = clamp_i64(offsets[e], 0, T);
-      const int64_t o1 = clamp_i64(offsets[e + 1], 0, T);
-      rows = o1 > o0 ? o1 - o0 : 0;
-    }
-    const int mine = (int)((rows + tile_rows - 1) / tile_rows);
-    int incl = mine;  // inclusive prefix sum within the wave
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += up;
-    }
-    if (lane == 63) part[wave] = incl;
-    __syncthreads();
-    int before = carry;
-    for (int w = 0; w < wave; ++w) before += part[w];
-    int64_t at = before + incl - mine;
-    for (int j = 0; j < mine; ++j, ++at) {
-      if (at < cap) {
-        tiles[2 * at] = (int32_t)e;
-        tiles[2 * at + 1] = (int32_t)(o0 + (int64_t)j * tile_rows);
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x == 1023) carry = before + incl;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) count[0] = carry < cap ? carry : (int)cap;
-}
 
 // The row gather xg[r] = x[order[r] / k] (rows of 16-byte pieces).
 __global__ __launch_bounds__(256) void k_gather16(u32x4* __restrict__ xg, const u32x4* __restrict__ x, const int64_t* __restrict__ order, int64_t n,
@@ -418,7 +376,8 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
                        p.tile_cap, f4 ? f4_tok : TILE_ROWS);
     if ((rc = check_launch("route_small")) != BP_OK) return rc;
   } else {
-    if ((rc = sort_with_inverse(p.order, p.offsets, p.inv, experts, n, E, p.sort_ws, bad, s)) != BP_OK) return rc;
+    const SortTiles list = {tiles || f4 ? p.tiles : nullptr, p.tile_count, p.tile_cap, f4 ? f4_tok : TILE_ROWS};
+    if ((rc = sort_with_inverse(p.order, p.offsets, p.inv, experts, n, E, p.sort_ws, bad, s, list)) != BP_OK) return rc;
     if ((f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4)) {
       // (no routed copy of the activations: the gate | up launch's conversion pass reads them through `order`)
     } else if (aligned16) {
@@ -483,10 +442,6 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     }
     return run_gemm(a, s);
   };
-  if ((tiles || f4) && !small) {
-    hipLaunchKernelGGL(k_tile_list, dim3(1), dim3(1024), 0, s, p.tiles, p.tile_count, p.offsets, E, n, p.tile_cap, f4 ? f4_tok : TILE_ROWS);
-    if ((rc = check_launch("tile_list")) != BP_OK) return rc;
-  }
   if (f4) {
     if (act == BP_I8 && (rc = bp_quant_act_int8(p.q, p.q_scale, x, BP_BF16, T, H, s)) != BP_OK) return rc;
     if ((rc = launch_gemm_f4(f4_gu, s, f4_name)) != BP_OK) return rc;

@@ -142,3 +142,24 @@ def test_tq1_layers_by_the_byte_table(tune, act, T, E, k, terms, group, H, I, sd
         tune("BP_TUNE_F4Q", "1000000000")
         ref = TernaryMoE(*packed("tq1"), H, I, k, "tq1", group, act=act)(x, logits)
     assert torch.isfinite(got.float()).all() and torch.equal(got, ref), bp.ext().last_kernel()
+
+
+# The tile list that the sort makes: one workgroup over more experts than it has threads, one over the whole list at 257 and 4095 rows, the
+# two launches from 4096 on; experts without rows. Against the small-batch kernels, which take no list.
+@pytest.mark.parametrize("T,E,k", [(300, 1030, 2), (129, 16, 2), (1365, 16, 3), (1366, 16, 3)])
+def test_tile_lists_from_the_sort(tune, T, E, k):
+    import deepseekternarized_amd as bp
+    from deepseekternarized_amd.moe import TernaryMoE
+
+    gen = torch.Generator(device="cuda").manual_seed(26)
+    H = I = 1024  # noqa: E741
+    moe = TernaryMoE(_terms(E, I, H, 1, gen), _terms(E, I, H, 1, gen), _terms(E, H, I, 1, gen), H, I, k, "tq2", 128)
+    x = torch.randn(T, H, device="cuda", generator=gen).bfloat16()
+    logits = 1.5 * torch.randn(T, E, device="cuda", generator=gen)
+    logits[:, 5] = -40.0
+    got = moe(x, logits)
+    assert bp.ext().last_kernel().startswith("gemm_"), bp.ext().last_kernel()
+    tune("BP_TUNE_TILES", "1000000")
+    ref = moe(x, logits)
+    assert torch.isfinite(got).all() and not bp.ext().last_kernel().startswith("gemm_tq2f")
+    assert float((got.double() - ref.double()).norm() / ref.double().norm()) <= 4e-3  # (sums in another order, each rounded to bf16 three times: 2^-9 once)
