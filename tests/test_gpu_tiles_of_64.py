@@ -10,7 +10,7 @@ def _terms(E, N, K, terms, gen, sdt=torch.float16, group=128):
     import deepseekternarized_amd as bp
 
     return [(bp.pack(torch.randint(-1, 2, (E * N, K), dtype=torch.int8, device="cuda", generator=gen), "tq2").view(E, N, -1),
-             (0.02 * torch.rand(E, N, K // group, device="cuda", generator=gen)).to(sdt)) for _ in range(terms)]
+             (0.02 * torch.rand(E, N, -(-K // group), device="cuda", generator=gen)).to(sdt)) for _ in range(terms)]
 
 
 # int8 layers either side of the line of 16 rows per expert on average; up to 256 routed rows (preparation and tile list in one launch)
