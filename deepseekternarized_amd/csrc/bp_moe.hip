@@ -302,7 +302,6 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   // 0.23 ms from 24 to 64 tokens on config 2's layer, where the small-batch kernels take 0.25 - 0.26 (and 0.18 - 0.21 below).
   const int64_t tiles_from = tuning().tiles >= 0 ? tuning().tiles : (fmt == BP_TQ1 && act == BP_BF16 ? 24 : 64);
   const bool tiles = T > tiles_from;
-  const bool small = n <= ROUTE_SMALL_N && (((uintptr_t)x | (uintptr_t)p.xg) & 15) == 0;
   const bool aligned16 = (((uintptr_t)x | (uintptr_t)p.xg) & 15) == 0;
   // int8 activations: the rows are quantised where they are gathered, and SwiGLU's result where it is made, when the rows'
   // lengths suit those kernels - two launches and two copies of the rows less
@@ -367,8 +366,11 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   const char* f4_name = rewritten ? (act == BP_BF16 ? "gemm_tq1_as_tq2f_bf16" : "gemm_tq1_as_tq2_i8f")
                         : fmt == BP_TQ1 ? (act == BP_BF16 ? "gemm_tq1f_bf16" : "gemm_tq1_i8f")
                         : act == BP_BF16 ? "gemm_tq2f_bf16" : moe_wide(n, T, E, I, n_terms) ? "gemm_tq2_i8w" : "gemm_tq2_i8f";
+  const int64_t row16 = (f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4) ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
+  // A few routed rows in one launch: up to 256 where it gathers, which the sort doesn't, and up to 64 else (every thread reads all ids: 4 us for
+  // 6 rows, 12 for 192, where k_sort takes 5.4 for 384; its histograms grow with the experts. 64 experts of 4096 / 2048, TQ1 bf16, 32 tokens x 6: 198.8 -> 193.5 us).
+  const bool small = n <= (row16 || E > 512 ? ROUTE_SMALL_N : 64) && (((uintptr_t)x | (uintptr_t)p.xg) & 15) == 0;
   if (small) {
-    const int64_t row16 = (f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4) ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
     int64_t g = ((int64_t)n * row16 + ROUTE_SMALL_THREADS - 1) / ROUTE_SMALL_THREADS;
     g = g < 1 ? 1 : (g > 256 ? 256 : g);
     hipLaunchKernelGGL(k_route_small, dim3((unsigned)g), dim3(ROUTE_SMALL_THREADS), 0, s, p.order, p.offsets, p.inv, experts, (int)n, E, bad,
