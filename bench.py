@@ -63,12 +63,13 @@ def arithmetic_of(kernel):
         return "activations as 3 E4M3 pieces under a per-group power-of-two prescale (int8 activations: exact) x 2-bit codes read as E2M1 halves with the offset in the accumulator (v_mfma_f32_16x16x128_f8f6f4), fp32 accumulate, fp16 scale per 128-group applied in fp32"
     if kernel.startswith("fp4_tq1_m"):
         return "activations as 2 E4M3 pieces under a per-group power-of-two prescale x E2M1 weights (v_mfma_f32_16x16x128_f8f6f4), fp32 accumulate"
+    if "f4_" in kernel.split("+")[0] and kernel.startswith("gemm_"):
+        pieces = "int8 activations as 2 E2M3 pieces (exact)" if "_i8" in kernel else "activations as 2 E4M3 pieces under E8M0 block scales (blocks of 32)"
+        return pieces + ", converted once into a workspace, x E2M1 weights (v_mfma_scale_f32_32x32x64_f8f6f4), fp32 accumulate, scale per 128-group applied in fp32"
     if kernel.startswith("gemm_tq1f"):
         return "activations as 2 E4M3 pieces under E8M0 block scales (blocks of 32), converted once into a workspace, x E2M1 weights strung together from a byte table, one v_mfma_scale_f32_16x16x128_f8f6f4 per 128-group, fp32 accumulate, scale per group applied in fp32"
     if kernel.startswith("gemm_tq1"):
         return "activations as 2 E4M3 pieces under E8M0 block scales (blocks of 20) x E2M1 weights (v_mfma_scale_f32_16x16x128_f8f6f4), fp32 accumulate, scale per 128-group applied in fp32"
-    if kernel.startswith("gemm_tq2f"):
-        return "activations as 2 E4M3 pieces under E8M0 block scales (blocks of 32), converted once into a workspace, x E2M1 weights (v_mfma_scale_f32_16x16x128_f8f6f4), fp32 accumulate, scale per 128-group applied in fp32"
     if kernel.startswith(("mfma_tq2_bf16", "gemm_tq2_bf16", "mfma_tq1")):
         return "bf16 activations x bf16-decoded trits (v_mfma_f32_16x16x32_bf16), fp32 accumulate, scale per 128-group applied in fp32"
     if kernel.startswith(("mfma_tq2_i8", "gemm_tq2_i8")):

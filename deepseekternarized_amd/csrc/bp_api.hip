@@ -318,8 +318,7 @@ extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_
     w.quant = 1;
     w.overwrite = 1;
     w.out16 = out16;
-    const bool wide = i8w_takes(N, K, group, n_terms, T) && (tuning().tq2g == 'f' || i8w_pays(T, N, K, 1, n_terms));  // (a grouped call's lines)
-    if (mfma_supports(a) && gemm_f4_applies(w) == BP_OK) return launch_gemm_f4(w, s, wide ? "gemm_tq2_i8w" : "gemm_tq2_i8f");
+    if (mfma_supports(a) && gemm_f4_applies(w) == BP_OK) return launch_gemm_f4(w, s);
   }
   if (act_int8) {
     if (const int rc = bp_quant_act_int8((int8_t*)(ws + p.q), (float*)(ws + p.q_scale), x, x_dtype, T, K, stream)) return rc;

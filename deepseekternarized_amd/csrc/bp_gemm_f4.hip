@@ -781,9 +781,11 @@ int gemm_f4_applies(const GemmArgs& a) {
   return wgs < 0 ? BP_ERR_UNSUPPORTED : BP_OK;
 }
 
-int launch_gemm_f4(const GemmArgs& a, hipStream_t s, const char* name) {
+int launch_gemm_f4(const GemmArgs& a, hipStream_t s, bool rewritten) {
   if (const int rc = gemm_f4_applies(a)) return rc;
-  return a.fmt == BP_TQ1 ? launch_f4_all<BP_TQ1>(a, s, name) : launch_f4_all<BP_TQ2>(a, s, name);
+  const bool i8 = a.quant || a.x_dtype == BP_I8;
+  if (a.fmt == BP_TQ1) return launch_f4_all<BP_TQ1>(a, s, i8 ? "gemm_tq1f4_i8" : "gemm_tq1f4_bf16");
+  return launch_f4_all<BP_TQ2>(a, s, rewritten ? (i8 ? "gemm_tq1_as_tq2f4_i8" : "gemm_tq1_as_tq2f4_bf16") : i8 ? "gemm_tq2f4_i8" : "gemm_tq2f4_bf16");
 }
 
 }  // namespace bp

@@ -439,7 +439,7 @@ int BP_OUTPUTS(launch_gemm_tq2)(const GemmArgs& a, hipStream_t s) {
   // with a workspace: over converted activations (development: BP_TUNE_TQ2G=bf16 keeps this file's kernel)
   if (a.stage && tuning().tq2g != 'b' &&
       (a.x_dtype == BP_I8 ? !a.tiles && (tuning().tq2g == 'f' || i8w_pays(a.T, a.N, a.K, a.E, a.n_terms)) : f4_pays_bf16(a.T, a.N))) {
-    const int rc = launch_gemm_f4(a, s, a.x_dtype == BP_I8 ? "gemm_tq2_i8w" : "gemm_tq2f_bf16");
+    const int rc = launch_gemm_f4(a, s);
     if (rc != BP_ERR_UNSUPPORTED) return rc;
   }
 #ifdef BP_DEV_ABLATIONS  // timing ablations (results are wrong): development builds only

@@ -41,7 +41,7 @@ int gemm_tq2f_applies(const GemmArgs& a);  // TQ1: BP_OK where launch_gemm_tq2f 
 // bp_gemm_f4.hip: TQ2 over token tiles of 64, TQ1 over tiles of 32, weights as fp4, bf16 activations (or int8 ones, or bf16 ones to be quantised:
 // GemmArgs::quant) as two exact pieces. With a tile list (GemmArgs::tiles, entries of that many rows): max_rows is that.
 constexpr int F4_TOK = 64, F4_TOK1 = 32;  // (TQ2, TQ1)
-int launch_gemm_f4(const GemmArgs& a, hipStream_t s, const char* name);
+int launch_gemm_f4(const GemmArgs& a, hipStream_t s, bool rewritten = false);  // rewritten: of TQ1 weights (named so)
 int gemm_f4_applies(const GemmArgs& a);  // BP_OK where launch_gemm_f4 takes the call (nothing is launched)
 // bf16 calls that run on it: at least two blocks of 512 output rows, and as many tokens as make 768 tiles of 32 x 512. Below, the kernels
 // on bf16 matrix instructions (k_gemm_tq2) sum more exactly (1.4e-7 of a float32 output's size where the fp8 pieces leave 5e-7).

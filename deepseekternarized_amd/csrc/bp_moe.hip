@@ -145,11 +145,6 @@ bool moe_f4(int act, int fmt, int64_t T, int64_t n, int64_t H, int64_t I, int64_
   if (act == BP_I8) return n >= (tuning().f4 >= 0 ? tuning().f4 : 16) * E;
   return rewritten || f4_pays_bf16(n, 2 * I) || f4_pays_bf16(n, H);  // (a TQ1 layer that isn't rewritten runs on fp8 pieces as well)
 }
-// ... of them, the int8 layers that are named as grouped calls of many rows are: 64 rows per expert, 1024 rows and 80 blocks of 128 rows
-// x 256 gate | up rows (128 with stacked terms).
-bool moe_wide(int64_t n, int64_t T, int64_t E, int64_t I, int n_terms) {
-  return T > 64 && n >= 64 * E && n >= 1024 && n / 128 * ((2 * I + 255) / 256) >= (n_terms == 1 ? 80 : 128);
-}
 
 // TQ1 layers whose weights are rewritten as TQ2 ones first (k_tq1_to_tq2, 0.45 bytes of traffic per weight), in memory that the caller
 // brings beyond bp_moe_layer_workspace_bytes: tiles of 64 tokens and no byte table in the products of such a layer then. int8 from 48 rows
@@ -363,9 +358,6 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     f4_both = mfma_supports(probe) && gemm_f4_applies(d) == BP_OK;
     f4 = mfma_supports(a) && gemm_f4_applies(a) == BP_OK && (f4_both || !gemm_tiles_supported(probe));
   }
-  const char* f4_name = rewritten ? (act == BP_BF16 ? "gemm_tq1_as_tq2f_bf16" : "gemm_tq1_as_tq2_i8f")
-                        : fmt == BP_TQ1 ? (act == BP_BF16 ? "gemm_tq1f_bf16" : "gemm_tq1_i8f")
-                        : act == BP_BF16 ? "gemm_tq2f_bf16" : moe_wide(n, T, E, I, n_terms) ? "gemm_tq2_i8w" : "gemm_tq2_i8f";
   const int64_t row16 = (f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4) ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
   // A few routed rows in one launch: up to 256 where it gathers, which the sort doesn't, and up to 64 else (every thread reads all ids: 4 us for
   // 6 rows, 12 for 192, where k_sort takes 5.4 for 384; its histograms grow with the experts. 64 experts of 4096 / 2048, TQ1 bf16, 32 tokens x 6: 198.8 -> 193.5 us).
@@ -446,11 +438,11 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   };
   if (f4) {
     if (act == BP_I8 && (rc = bp_quant_act_int8(p.q, p.q_scale, x, BP_BF16, T, H, s)) != BP_OK) return rc;
-    if ((rc = launch_gemm_f4(f4_gu, s, f4_name)) != BP_OK) return rc;
+    if ((rc = launch_gemm_f4(f4_gu, s, rewritten)) != BP_OK) return rc;
     if (!f4_glu) rc = v4 ? bp_swiglu_v4(p.h, p.gu, p.gu + I, (const float*)weights, p.order, n, limit, n, I, 2 * I, s) : bp_swiglu_bf16(p.h, p.gu, p.gu + I, n, I, 2 * I, s);
     if (rc != BP_OK) return rc;
     bool y16 = f4_glu;
-    rc = f4_both ? launch_gemm_f4(f4_down, s, f4_name) : gemm(p.y, p.h, down_packed, down_scale, H, I, false, &y16, false);
+    rc = f4_both ? launch_gemm_f4(f4_down, s, rewritten) : gemm(p.y, p.h, down_packed, down_scale, H, I, false, &y16, false);
     if (rc != BP_OK) return rc;
     if (f4_glu) note_kernel_suffix(f4_gather ? "+glu+gather" : "+glu");
     if (y16) note_kernel_suffix("+y16");

@@ -92,7 +92,7 @@ def test_layer_call_over_the_tile_list_with_converted_activations(tune):
     logits[:, 11] -= 2.5
     tune("BP_TUNE_TQ2G", "fp4")
     got = moe(x, logits).clone()
-    assert ext().last_kernel() == "gemm_tq2f_bf16+glu+gather+y16", ext().last_kernel()  # (the gate | up launch gathered its rows and applied SwiGLU itself)
+    assert ext().last_kernel() == "gemm_tq2f4_bf16+glu+gather+y16", ext().last_kernel()  # (the gate | up launch gathered its rows and applied SwiGLU itself)
     assert torch.equal(moe(x, logits), got)
     tune("BP_TUNE_TQ2G", "bf16")
     want = moe(x, logits)
@@ -243,13 +243,14 @@ def test_swiglu_in_the_gate_up_epilogue_equals_the_separate_launch(tune, fmt, te
     if fmt == "tq2":
         tune("BP_TUNE_TQ2G", "fp4")  # (the shape is below the thresholds of the kernel over converted activations)
     fused = run()
-    assert ext().last_kernel() == "gemm_%sf_bf16+glu+gather+y16" % fmt, ext().last_kernel()
+    kernel = "gemm_%s%s_bf16" % (fmt, "f" if fmt == "tq1" and terms == 2 else "f4")  # (TQ1 in two terms: from 44 rows per expert on k_gemm_f4, here 25)
+    assert ext().last_kernel() == kernel + "+glu+gather+y16", ext().last_kernel()
     tune("BP_TUNE_GLU", "g")  # the routed copy of the activations written by a launch of its own
     assert torch.equal(run(), fused)
-    assert ext().last_kernel() == "gemm_%sf_bf16+glu+y16" % fmt, ext().last_kernel()
+    assert ext().last_kernel() == kernel + "+glu+y16", ext().last_kernel()
     tune("BP_TUNE_GLU", "n")
     apart = run()
-    assert ext().last_kernel() == "gemm_%sf_bf16" % fmt, ext().last_kernel()
+    assert ext().last_kernel() == kernel, ext().last_kernel()
     assert torch.isfinite(fused.float()).all() and torch.equal(fused, apart)
 
 
@@ -408,7 +409,8 @@ def test_router_kernel_ties_go_to_the_lower_expert_and_bad_arguments_are_rejecte
 def test_small_batch_preparation_kernel_writes_the_tile_list(T, E, k):
     """Between 24 tokens (TQ1, bf16: the tile list takes over) and 256 routed rows the preparation kernel also writes the
     list of token tiles - experts without rows, experts with more than one tile of 32 rows - and the layer equals the
-    composed calls bit for bit (the same GEMM kernel, sized by the bound instead of the list)."""
+    composed calls bit for bit (the same GEMM kernel, sized by the bound instead of the list; from 16 rows per expert on the
+    one over the same pieces with the same order of additions)."""
     from deepseekternarized_amd import ext
 
     moe, _ = _layer("tq1", "bf16", 1024, 1024, E, k, seed=T)
@@ -419,6 +421,6 @@ def test_small_batch_preparation_kernel_writes_the_tile_list(T, E, k):
     if E == 4:
         logits[:, 1] += 6.0  # expert 1 is in every token's top-2: more than one tile
     got = moe(x, logits)
-    assert ext().last_kernel() == "gemm_tq1f_bf16+glu+gather+y16", ext().last_kernel()
+    assert ext().last_kernel() == ("gemm_tq1f4_bf16" if T * k >= 16 * E else "gemm_tq1f_bf16") + "+glu+gather+y16", ext().last_kernel()
     want = moe.composed(x, logits)
     assert torch.isfinite(got.float()).all() and torch.equal(got, want)

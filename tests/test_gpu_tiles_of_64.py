@@ -33,7 +33,7 @@ def test_int8_layers_from_sixteen_rows_per_expert(tune, pattern, T, E, k, terms,
     got = run()
     supported = I % 256 == 0  # (otherwise the down projection runs on the general kernel)
     name = bp.ext().last_kernel()
-    assert ("+glu+gather" in name) == wide and (not wide or not supported or name == "gemm_tq2_i8f+glu+gather+y16"), name
+    assert ("+glu+gather" in name) == wide and (not wide or not supported or name == "gemm_tq2f4_i8+glu+gather+y16"), name
     tune("BP_TUNE_TQ2G", "b")
     ref = run()
     assert torch.isfinite(got).all()
@@ -41,7 +41,7 @@ def test_int8_layers_from_sixteen_rows_per_expert(tune, pattern, T, E, k, terms,
 
 
 # 252 and 256 workgroups of 64 tokens x 256 rows, at a row length whose grouped calls keep to tiles of 32 there; the last tile of 1, 32 and 33 rows
-@pytest.mark.parametrize("T,N,K,name", [(63 * 64 + 1, 1024, 3584, "gemm_tq2_i8f"), (51 * 64 + 32, 1280, 3584, "gemm_tq2_i8f"), (42 * 64 + 33, 1536, 1024, "gemm_tq2_i8w"),
+@pytest.mark.parametrize("T,N,K,name", [(63 * 64 + 1, 1024, 3584, "gemm_tq2f4_i8"), (51 * 64 + 32, 1280, 3584, "gemm_tq2f4_i8"), (42 * 64 + 33, 1536, 1024, "gemm_tq2f4_i8"),
                                         (63 * 64, 1024, 3584, "gemm_tq2_i8_gs")])
 def test_int8_linears_from_256_workgroups(T, N, K, name):
     import deepseekternarized_amd as bp
@@ -72,7 +72,7 @@ def test_bf16_pieces_keep_what_the_matrix_instruction_sums(tune, spread):
     x = x.bfloat16()
     tune("BP_TUNE_TQ2G", "f")
     got = bp.TernaryLinear([bp.PackedTerm(packed[0], scale[0])], K, "tq2", 128, act="bf16")(x, torch.float32)
-    assert bp.ext().last_kernel() == "gemm_tq2f_bf16"
+    assert bp.ext().last_kernel() == "gemm_tq2f4_bf16"
     want = x.double() @ (bp.unpack(packed[0], "tq2", K).double() * scale[0].double().repeat_interleave(128, -1)).T
     # an element's error is at most 2^-17.4 of its block's largest, uniform: 2^-19.2 of it in the mean square; that largest is
     # about 2.5 (spread 0: 0.3 % of the elements lose anything) to 4.5 (spread 12) times the root mean square
@@ -106,7 +106,7 @@ def test_tq1_layers_rewritten_as_tq2(act, T, E, k, terms, group, H, I):
     for fmt in gate:
         moe = TernaryMoE(gate[fmt], up[fmt], down[fmt], H, I, k, fmt, group, act=act)
         got[fmt] = moe(x, logits)
-        rewritten = bp.ext().last_kernel().startswith("gemm_tq1_as_tq2")
+        rewritten = bp.ext().last_kernel().startswith("gemm_tq1_as_tq2f4")
         assert rewritten == (fmt == "tq1" and T * k >= (48 if act == "int8" and terms == 1 else 56 if act == "int8" else 84) * E), bp.ext().last_kernel()
         assert torch.equal(moe(x, logits), got[fmt])
     assert torch.isfinite(got["tq1"].float()).all() and torch.equal(got["tq1"], got["tq2"])
@@ -116,10 +116,10 @@ def test_tq1_layers_rewritten_as_tq2(act, T, E, k, terms, group, H, I):
 # terms, groups of 256, scales of 32 bits (bf16 layers of these keep the kernel without pieces); either side of its lines. int8 (exact group sums): the bits of the same trits' TQ2 layer on the
 # kernels over tiles of 32; bf16: of the kernel for 16 x 16 x 128 pieces, whose pieces and order of additions are the same.
 @pytest.mark.parametrize("act,T,E,k,terms,group,H,I,sdt,name", [
-    ("int8", 64, 64, 3, 1, 128, 1280, 1024, torch.float16, "gemm_tq1_i8f"), ("int8", 65, 8, 2, 2, 128, 1792, 1280, torch.float16, "gemm_tq1_i8f"),
-    ("int8", 80, 4, 2, 1, 256, 2048, 2560, torch.float32, "gemm_tq1_i8f"), ("int8", 64, 64, 2, 1, 128, 1280, 1024, torch.float16, None),
-    ("bf16", 64, 8, 2, 1, 128, 1280, 1792, torch.bfloat16, "gemm_tq1f_bf16"), ("bf16", 100, 4, 2, 1, 256, 2048, 2560, torch.float16, "gemm_tq1f_bf16"),
-    ("bf16", 180, 8, 2, 2, 128, 1024, 1280, torch.float16, "gemm_tq1f_bf16"),
+    ("int8", 64, 64, 3, 1, 128, 1280, 1024, torch.float16, "gemm_tq1f4_i8"), ("int8", 65, 8, 2, 2, 128, 1792, 1280, torch.float16, "gemm_tq1f4_i8"),
+    ("int8", 80, 4, 2, 1, 256, 2048, 2560, torch.float32, "gemm_tq1f4_i8"), ("int8", 64, 64, 2, 1, 128, 1280, 1024, torch.float16, None),
+    ("bf16", 64, 8, 2, 1, 128, 1280, 1792, torch.bfloat16, "gemm_tq1f4_bf16"), ("bf16", 100, 4, 2, 1, 256, 2048, 2560, torch.float16, "gemm_tq1f4_bf16"),
+    ("bf16", 180, 8, 2, 2, 128, 1024, 1280, torch.float16, "gemm_tq1f4_bf16"),
     ("bf16", 180, 8, 2, 2, 128, 1024, 1280, torch.float32, "gemm_tq1_bf16")])
 def test_tq1_layers_by_the_byte_table(tune, act, T, E, k, terms, group, H, I, sdt, name):
     import deepseekternarized_amd as bp
@@ -134,7 +134,7 @@ def test_tq1_layers_by_the_byte_table(tune, act, T, E, k, terms, group, H, I, sd
     logits[:, 1] = -40.0  # an expert without rows
     got = TernaryMoE(*packed("tq1"), H, I, k, "tq1", group, act=act)(x, logits)
     ran = bp.ext().last_kernel().split("+")[0]
-    assert ran == name if name else not ran.endswith("i8f"), ran
+    assert ran == name if name else "f4_" not in ran, ran
     if act == "int8":
         tune("BP_TUNE_F4", "1000000")
         ref = TernaryMoE(*packed("tq2"), H, I, k, "tq2", group, act=act)(x, logits)
@@ -161,5 +161,5 @@ def test_tile_lists_from_the_sort(tune, T, E, k):
     assert bp.ext().last_kernel().startswith("gemm_"), bp.ext().last_kernel()
     tune("BP_TUNE_TILES", "1000000")
     ref = moe(x, logits)
-    assert torch.isfinite(got).all() and not bp.ext().last_kernel().startswith("gemm_tq2f")
+    assert torch.isfinite(got).all() and not bp.ext().last_kernel().startswith("gemm_tq2f4")
     assert float((got.double() - ref.double()).norm() / ref.double().norm()) <= 4e-3  # (sums in another order, each rounded to bf16 three times: 2^-9 once)

@@ -67,7 +67,7 @@ def test_int8_tiles_of_128(tune, counts, N, K, group, terms, sdt):
     got, ref = _call("tq2", "int8", counts, N, K, 6, terms, group, sdt, max_rows=300)
     _close(got, ref, "int8")
     _call("tq2", "int8", counts, N, K, 6, terms, group, sdt, max_rows=300, ref=False)
-    assert bp.ext().last_kernel() == "gemm_tq2_i8w"
+    assert bp.ext().last_kernel() == "gemm_tq2f4_i8"
 
 
 # the same with eight waves of 256 rows per workgroup: rows whose scales leave room for one workgroup per CU - one term from K = 3584
@@ -80,7 +80,7 @@ def test_int8_tiles_of_128_with_eight_waves(tune, counts, N, K, group, terms, sd
 
     tune("BP_TUNE_TQ2G", "f")
     got, _ = _call("tq2", "int8", counts, N, K, 13, terms, group, sdt, max_rows=300, ref=False)
-    assert bp.ext().last_kernel() == "gemm_tq2_i8w"
+    assert bp.ext().last_kernel() == "gemm_tq2f4_i8"
     _, ref = _call("tq2", "int8", counts, N, K, 13, terms, group, sdt, max_rows=300)  # (the reference-order kernel's)
     _close(got, ref, "int8")
 
@@ -103,7 +103,7 @@ def test_linear_quantises_in_the_conversion_pass(tune, T, K, scale, out_dtype):
     x = x.bfloat16()
     tune("BP_TUNE_TQ2G", "f")
     got = bp.TernaryLinear([bp.PackedTerm(packed, s)], K, "tq2", 128)(x, out_dtype)
-    assert bp.ext().last_kernel() == "gemm_tq2_i8w"
+    assert bp.ext().last_kernel() == "gemm_tq2f4_i8"
     q, qs = bp.quant_act_int8(x)
     ref = bp.grouped_ternary_gemm(q, qs, dense_offsets(x.device, T), [packed[None]], [s[None]], K, 128, "tq2", max_rows=T).to(out_dtype)
     assert torch.equal(got.isnan(), ref.isnan()) and bool(ref[5].isnan().all())
@@ -141,7 +141,7 @@ def test_int8_layer_on_tiles_of_128(tune, pattern, T, E, k, terms, H):
     else:
         run = lambda: moe(x, logits)  # noqa: E731
     got = run()
-    assert bp.ext().last_kernel() == "gemm_tq2_i8w+glu+gather+y16"
+    assert bp.ext().last_kernel() == "gemm_tq2f4_i8+glu+gather+y16"
     if v4:
         tune("BP_TUNE_TQ2G", "b")
         ref = run()
@@ -151,10 +151,9 @@ def test_int8_layer_on_tiles_of_128(tune, pattern, T, E, k, terms, H):
     assert float((got.double() - ref.double()).norm() / ref.double().norm()) <= 4e-3
 
 
-# either side of the line: 896 and 1024 rows, 72 and 80 blocks of 128 rows x 256 gate | up rows (two terms: 120 and 128)
-@pytest.mark.parametrize("T,E,k,I,terms,wide", [(448, 8, 2, 4096, 1, False), (512, 8, 2, 4096, 1, True), (1152, 4, 1, 1024, 1, False), (1280, 4, 1, 1024, 1, True),
-                                                (960, 8, 2, 1024, 2, False), (1024, 8, 2, 1024, 2, True)])
-def test_int8_layers_with_few_blocks_stay_on_tiles_of_32(T, E, k, I, terms, wide):
+# few experts with many rows each: 896 to 2048 rows, one and two terms
+@pytest.mark.parametrize("T,E,k,I,terms", [(448, 8, 2, 4096, 1), (512, 8, 2, 4096, 1), (1152, 4, 1, 1024, 1), (1280, 4, 1, 1024, 1), (960, 8, 2, 1024, 2), (1024, 8, 2, 1024, 2)])
+def test_int8_layers_of_few_experts(T, E, k, I, terms):
     import deepseekternarized_amd as bp
     from deepseekternarized_amd.moe import TernaryMoE
 
@@ -169,14 +168,14 @@ def test_int8_layers_with_few_blocks_stay_on_tiles_of_32(T, E, k, I, terms, wide
     x = torch.randn(T, H, device="cuda", generator=gen).bfloat16()
     logits = torch.randn(T, E, device="cuda", generator=gen)
     got = moe(x, logits)
-    assert ("i8w" in bp.ext().last_kernel()) == wide
+    assert bp.ext().last_kernel() == "gemm_tq2f4_i8+glu+gather+y16"
     ref = moe.composed(x, logits)
     assert float((got.double() - ref.double()).norm() / ref.double().norm()) <= 4e-3  # (bf16 roundings and int8 steps that fall otherwise)
 
 
-# the rows of tests/test_workspace_sizes.py that lie at a line, as the launch sees them
-@pytest.mark.parametrize("T,N,K,terms,wide", [(2048, 2048, 1536, 2, True), (2048, 2048, 2048, 2, False), (2048, 2048, 2048, 1, True), (3072, 2048, 1792, 2, True), (1536, 4096, 7168, 2, False)])
-def test_int8_linears_take_the_variant_their_terms_fit(T, N, K, terms, wide):
+# the rows of tests/test_workspace_sizes.py that lie at a line of the grouped calls', which linears don't have
+@pytest.mark.parametrize("T,N,K,terms", [(2048, 2048, 1536, 2), (2048, 2048, 2048, 2), (2048, 2048, 2048, 1), (3072, 2048, 1792, 2), (1536, 4096, 7168, 2)])
+def test_int8_linears_on_either_side_of_the_grouped_calls_lines(T, N, K, terms):
     import deepseekternarized_amd as bp
 
     gen = torch.Generator(device="cuda").manual_seed(12)
@@ -184,6 +183,6 @@ def test_int8_linears_take_the_variant_their_terms_fit(T, N, K, terms, wide):
                              (0.02 * torch.rand(N, K // 128, device="cuda", generator=gen)).half()) for _ in range(terms)]
     x = torch.randn(T, K, device="cuda", generator=gen).bfloat16()
     got = bp.TernaryLinear(weights, K, "tq2", 128)(x, torch.float32)
-    assert ("i8w" in bp.ext().last_kernel()) == wide
+    assert bp.ext().last_kernel() == "gemm_tq2f4_i8"
     ref = bp.TernaryLinear(weights, K, "tq2", 128, backend="torch")(x, torch.float32)
     _close(got, ref, "int8")

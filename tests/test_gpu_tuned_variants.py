@@ -769,10 +769,10 @@ def test_tq2_bf16_scales_and_f32_scales(bp):
 @pytest.fixture(params=["fp4", "bf16"])
 def tq2_gemm_kernel(request, tune):
     """More than 16 rows per expert, bf16 activations: the fp8 x fp4 grouped GEMM over activations converted into a
-    workspace (kernel name gemm_tq2f_bf16; BP_TUNE_TQ2G=fp4 runs it on shapes below its thresholds too) and the bf16
-    MFMA kernel (gemm_tq2_bf16*; BP_TUNE_TQ2G=bf16). int8 activations run gemm_tq2_i8* either way."""
+    workspace (kernel name gemm_tq2f4_bf16; BP_TUNE_TQ2G=fp4 runs it on shapes below its thresholds too) and the bf16
+    MFMA kernel (gemm_tq2_bf16*; BP_TUNE_TQ2G=bf16); int8 activations likewise (gemm_tq2f4_i8, gemm_tq2_i8*)."""
     tune("BP_TUNE_TQ2G", request.param)
-    return "gemm_tq2f_" if request.param == "fp4" else "gemm_tq2_"
+    return "gemm_tq2f4_" if request.param == "fp4" else "gemm_tq2_"
 
 
 @pytest.mark.parametrize("act", ["bf16", "int8"])
@@ -788,7 +788,7 @@ def tq2_gemm_kernel(request, tune):
 )
 def test_tq2_gemm_tiles(bp, act, E, N, K, counts, terms, tq2_gemm_kernel):
     got, want, kern = _run(bp, "tq2", E, N, K, counts, act, terms=terms, seed=K + N)
-    assert kern.startswith(tq2_gemm_kernel if act == "bf16" else "gemm_tq2_i8"), kern
+    assert kern.startswith(tq2_gemm_kernel + ("bf16" if act == "bf16" else "i8")), kern
     _check(got, want)
 
 
@@ -803,7 +803,7 @@ def test_tq2_gemm_fp8_pieces_keep_small_activations(bp, tune):
     x = orc.bf16_round(x)
     offsets = np.concatenate([[0], np.cumsum(counts)])
     got = bp.grouped_ternary_gemm(dev(x).to(torch.bfloat16), None, dev(offsets), dev(packed[0]), dev(scales[0]), K, GROUP, "tq2", max_rows=max(counts))
-    assert bp.ext().last_kernel().startswith("gemm_tq2f_"), bp.ext().last_kernel()
+    assert bp.ext().last_kernel().startswith("gemm_tq2f4_"), bp.ext().last_kernel()
     want = np.concatenate([c_gemm(x[a:b], None, packed[0][e], scales[0][e].astype(np.float32), K, GROUP, "tq2")
                            for e, (a, b) in enumerate(zip(offsets[:-1], offsets[1:]))])
     rel = np.linalg.norm(got.cpu().numpy() - want) / np.linalg.norm(want)
@@ -815,10 +815,10 @@ def test_tq2_gemm_float32_scales(bp, act, tq2_gemm_kernel):
     """What the reference's wrappers hand the kernel (`w_scale.float()`, boilerplate/kernels/ternary_cuda.py:95-97);
     also with one scale per 256 weights and an odd number of them per row."""
     got, want, kern = _run(bp, "tq2", 3, 80, 2304, [21, 0, 50], act, terms=2, seed=31, scale_dtype="f32")
-    assert kern.startswith(tq2_gemm_kernel if act == "bf16" else "gemm_tq2_i8"), kern
+    assert kern.startswith(tq2_gemm_kernel + ("bf16" if act == "bf16" else "i8")), kern
     _check(got, want)
     got, want, kern = _run(bp, "tq2", 2, 528, 2304, [19, 33], act, terms=2, seed=32, scale_dtype="f32", group=256)
-    assert kern.startswith(tq2_gemm_kernel if act == "bf16" else "gemm_tq2_i8"), kern
+    assert kern.startswith(tq2_gemm_kernel + ("bf16" if act == "bf16" else "i8")), kern
     _check(got, want)
 
 
@@ -838,7 +838,7 @@ def test_tq2_gemm_over_converted_activations_is_the_default_for_large_prefill(bp
     offsets = torch.arange(0, E * rows + 1, rows, device="cuda", dtype=torch.int64)
     offsets[3] -= 13  # ragged tiles on both sides
     got = bp.grouped_ternary_gemm(x, None, offsets, pk, sc, K, GROUP, "tq2", max_rows=rows + 13)
-    assert bp.ext().last_kernel() == "gemm_tq2f_bf16", bp.ext().last_kernel()
+    assert bp.ext().last_kernel() == "gemm_tq2f4_bf16", bp.ext().last_kernel()
     lib = bp.ext().lib
     assert lib.bp_grouped_gemm_workspace_bytes(_lib.BP_BF16, E * rows, N, K, E, 2, rows + 13) > 0
     assert lib.bp_grouped_gemm_workspace_bytes(_lib.BP_I8, E * rows, N, K, E, 2, rows + 13) == 0
@@ -874,7 +874,7 @@ def test_tq2_gemm_over_converted_activations_is_the_default_for_large_prefill(bp
 def test_tq2_gemm_scales_from_global_memory_and_other_scale_dtypes(bp, tq2_gemm_kernel):
     """K = 10240: 256 rows x 80 groups of scales do not fit beside the bf16 kernel's two activation tiles; bf16 scales; float32 scales."""
     got, want, kern = _run(bp, "tq2", 2, 64, 10240, [33, 18], "bf16", seed=21)
-    assert kern == ("gemm_tq2_bf16_gs" if tq2_gemm_kernel == "gemm_tq2_" else "gemm_tq2f_bf16"), kern
+    assert kern == ("gemm_tq2_bf16_gs" if tq2_gemm_kernel == "gemm_tq2_" else "gemm_tq2f4_bf16"), kern
     _check(got, want)
     got, want, kern = _run(bp, "tq2", 2, 64, 2048, [18, 40], "bf16", seed=22, scale_dtype=np.float32)  # bf16 scales
     assert kern.startswith(tq2_gemm_kernel), kern
@@ -980,7 +980,7 @@ def test_group_256(bp, act, fmt, K, counts, prefix):
 # --------------------------------------------------------------------------- activations that are not finite
 @pytest.mark.parametrize("fmt,counts,prefix", [
     ("tq1", [1, 1], "fp4_tq1_t1"), ("tq1", [1, 1], "fp4_tq1_t1_cw"), ("tq1", [2, 2], "fp4_tq1_m2_cw"), ("tq1", [4, 3], "fp4_tq1_m4"), ("tq1", [20, 12], "gemm_tq1"),
-    ("tq2", [1, 1], "mfma_tq2"), ("tq2", [1, 1], "fp4_tq2_t1_ks"), ("tq2", [9, 16], "mfma_tq2"), ("tq2", [40, 33], "gemm_tq2_"), ("tq2", [40, 33], "gemm_tq2f_"),
+    ("tq2", [1, 1], "mfma_tq2"), ("tq2", [1, 1], "fp4_tq2_t1_ks"), ("tq2", [9, 16], "mfma_tq2"), ("tq2", [40, 33], "gemm_tq2_"), ("tq2", [40, 33], "gemm_tq2f4_"),
 ])
 def test_non_finite_activations_never_give_finite_wrong_values(bp, tune, fmt, counts, prefix):
     """The reference's CPU kernel skips zero weights (boilerplate/kernels/csrc/boilerplate_cpu.cpp:70-77), so a NaN or an
@@ -988,7 +988,7 @@ def test_non_finite_activations_never_give_finite_wrong_values(bp, tune, fmt, co
     zeros too (0 x Inf = NaN) or scale whole blocks: they may make more outputs of that token non-finite, but every
     output the reference makes non-finite must be non-finite here, and tokens without such an activation are untouched."""
     E, N, K = 2, 64, 2048
-    if prefix == "gemm_tq2f_":
+    if prefix == "gemm_tq2f4_":
         tune("BP_TUNE_TQ2G", "fp4")
     if prefix.endswith("_cw"):
         tune("BP_TUNE_TQ1", "chunk")
