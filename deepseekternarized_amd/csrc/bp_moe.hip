@@ -31,6 +31,48 @@ namespace {
 
 constexpr int TILE_ROWS = 32;  // token tile of k_gemm_tq1 / k_gemm_tq2
 
+// (expert, first row) of every token tile of `tile_rows` rows, in expert order; count[0] = their number: a second list beside the sort's, for
+// layers whose two products run over tiles of different sizes. One workgroup; experts in chunks of 1024 with a running total.
+__global__ __launch_bounds__(1024) void k_tile_list(int32_t* __restrict__ tiles, int32_t* __restrict__ count, const int64_t* __restrict__ offsets,
+                                                    int64_t E, int64_t T, int64_t cap, int tile_rows) {
+  __shared__ int part[16];
+  __shared__ int carry;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x == 0) carry = 0;
+  __syncthreads();
+  for (int64_t base = 0; base < E; base += 1024) {
+    const int64_t e = base + threadIdx.x;
+    int64_t o0 = 0, rows = 0;
+    if (e < E) {
+      o0 = clamp_i64(offsets[e], 0, T);
+      const int64_t o1 = clamp_i64(offsets[e + 1], 0, T);
+      rows = o1 > o0 ? o1 - o0 : 0;
+    }
+    const int mine = (int)((rows + tile_rows - 1) / tile_rows);
+    int incl = mine;  // inclusive prefix sum within the wave
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += up;
+    }
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    int before = carry;
+    for (int w = 0; w < wave; ++w) before += part[w];
+    int64_t at = before + incl - mine;
+    for (int j = 0; j < mine; ++j, ++at) {
+      if (at < cap) {
+        tiles[2 * at] = (int32_t)e;
+        tiles[2 * at + 1] = (int32_t)(o0 + (int64_t)j * tile_rows);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 1023) carry = before + incl;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) count[0] = carry < cap ? carry : (int)cap;
+}
+
 // The row gather xg[r] = x[order[r] / k] (rows of 16-byte pieces).
 __global__ __launch_bounds__(256) void k_gather16(u32x4* __restrict__ xg, const u32x4* __restrict__ x, const int64_t* __restrict__ order, int64_t n,
                                                   int64_t k, int64_t T, int64_t row16) {
@@ -126,10 +168,15 @@ __global__ __launch_bounds__(ROUTE_SMALL_THREADS) void k_route_small(int64_t* __
   }
 }
 
-// Layers whose two GEMMs run on the kernel for token tiles of 64 (32 for TQ1).
+// A product of N output rows of a TQ2 layer with bf16 activations: on fp8 pieces where it would be as a grouped call (f4_pays_bf16; launches
+// sized by the tokens with few rows per expert stay on the 16-token tiles). The two products of a layer are held to it one by one: the
+// one below stays on bf16 matrix instructions, which sum more exactly.
+bool f4_product(int64_t T, int64_t n, int64_t N, int64_t E) { return f4_pays_bf16(n, N) && (T > 64 || n > 8 * E || tuning().tq2g == 'f'); }
+
+// Layers whose GEMMs run on the kernel for token tiles of 64 (32 for TQ1).
 // TQ2, int8: from 16 rows per expert on average. Whole layer on it / on the 32-token tiles, us: 2048 / 1024 (hidden / intermediate), 64
 // experts, 16 rows each 73 / 82, 50 rows 112 / 146; 4096 / 2048, 64 experts, 12 rows 164 / 163, 37 rows 203 / 305; 384 experts, 6 rows
-// 733 / 739, 19 rows 750 / 920, 62 rows 1350 / 2194. bf16: where one of the two products alone would (f4_pays_bf16).
+// 733 / 739, 19 rows 750 / 920, 62 rows 1350 / 2194. bf16: layers of which a product does (f4_product).
 // TQ1, int8: from 129 routed rows, where all experts together have 512 workgroups (two to a CU) or there are more than 64 tokens (the old
 // kernels' grids are bounded by the tokens up to there). Whole layer, us: 4096 / 2048, 64 experts of 6, 16 tokens 194 / 181, 32 205 / 316, 64
 // 204 / 221, 251 241 / 372, 1500 765 / 1274; 384 experts, 400 tokens 1038 / 1188, 2000 1357 / 2033; 2048 / 1024, 64 experts of 8, 16 tokens
@@ -143,7 +190,7 @@ bool moe_f4(int act, int fmt, int64_t T, int64_t n, int64_t H, int64_t I, int64_
   if (fmt == BP_TQ1 && tuning().f4q >= 0) return n >= tuning().f4q;
   if (fmt == BP_TQ1) return act == BP_I8 ? n > 128 && (T > 64 || E * I >= 512 * 128) : n >= (n_terms == 1 ? 16 : 44) * E;
   if (act == BP_I8) return n >= (tuning().f4 >= 0 ? tuning().f4 : 16) * E;
-  return rewritten || f4_pays_bf16(n, 2 * I) || f4_pays_bf16(n, H);  // (a TQ1 layer that isn't rewritten runs on fp8 pieces as well)
+  return rewritten || f4_product(T, n, 2 * I, E) || f4_product(T, n, H, E);  // (a TQ1 layer that isn't rewritten runs on fp8 pieces as well)
 }
 
 // TQ1 layers whose weights are rewritten as TQ2 ones first (k_tq1_to_tq2, 0.45 bytes of traffic per weight), in memory that the caller
@@ -179,6 +226,7 @@ struct Plan {
   int32_t* sort_ws;
   int32_t* tiles;
   int32_t* tile_count;
+  int32_t* tiles64;  // ... of 64 rows and their number, where `tiles` holds those of 32 for the other product
   void* xg;       // gathered rows, bf16 [T k, H]
   int8_t* q;      // int8 activations of the wider of the two GEMM inputs
   float* q_scale;
@@ -202,6 +250,7 @@ Plan plan(void* workspace, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k
   p.tile_cap = (n + TILE_ROWS - 1) / TILE_ROWS + E;
   p.tiles = (int32_t*)c.take(8 * (size_t)p.tile_cap);
   p.tile_count = (int32_t*)c.take(4);
+  p.tiles64 = (int32_t*)c.take(act == BP_BF16 ? 8 * (size_t)((n + F4_TOK - 1) / F4_TOK + E) + 4 : 0);
   p.xg = c.take(2 * (size_t)n * H);
   p.q = (int8_t*)c.take(act == BP_I8 ? (size_t)n * (H > I ? H : I) : 0);
   p.q_scale = (float*)c.take(act == BP_I8 ? 4 * (size_t)n : 0);
@@ -323,12 +372,13 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     }
     fuse = gemm_tiles_supported(a) && gemm_tq2f_applies(a) == BP_OK;
   }
-  // TQ2 over token tiles of 64, either activation type: the conversion passes gather (int8: the token rows are quantised once) and
+  // Token tiles of 64 (TQ1: 32), either activation type: the conversion passes gather (int8: the token rows are quantised once) and
   // quantise h; gate | up applies SwiGLU and the down projection writes bf16 rows. A down projection that the kernel does not take runs
-  // elsewhere, unless it would need the list of 32-row tiles.
+  // elsewhere, unless it would need the list of 32-row tiles. TQ2 with bf16 activations: each product by its own line, with two lists.
   GemmArgs f4_gu, f4_down;
   const int f4_tok = fmt == BP_TQ1 ? F4_TOK1 : F4_TOK;
-  bool f4 = false, f4_both = false;
+  const bool f4_each = act == BP_BF16 && fmt == BP_TQ2 && !rewritten;
+  bool f4 = false, f4_first = false, f4_second = false, two_lists = false;  // (of gate | up and down; any of them)
   const bool f4_glu = tuning().glu != 'n', f4_gather = f4_glu && tuning().glu != 'g';
   if (moe_f4(act, fmt, T, n, H, I, E, n_terms, rewritten) && pieces && aligned16 && kernel_policy() != 1 && (f4_gather || act == BP_BF16)) {
     memset(&f4_gu, 0, sizeof(f4_gu));
@@ -355,10 +405,19 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     d.out16 = f4_glu ? (uint16_t*)p.y : nullptr;
     GemmArgs probe = d;  // (mfma_supports knows the product's own activation type)
     probe.x_dtype = act;
-    f4_both = mfma_supports(probe) && gemm_f4_applies(d) == BP_OK;
-    f4 = mfma_supports(a) && gemm_f4_applies(a) == BP_OK && (f4_both || !gemm_tiles_supported(probe));
+    f4_first = mfma_supports(a) && gemm_f4_applies(a) == BP_OK && (!f4_each || f4_product(T, n, 2 * I, E));
+    f4_second = mfma_supports(probe) && gemm_f4_applies(d) == BP_OK && (!f4_each || f4_product(T, n, H, E));
+    if (!f4_each && (!f4_first || (!f4_second && gemm_tiles_supported(probe)))) f4_first = f4_second = false;
+    f4 = f4_first || f4_second;
+    two_lists = f4_each && tiles && f4_first != f4_second;
+    if (two_lists) {
+      a.tiles = d.tiles = p.tiles64;
+      a.tile_count = d.tile_count = p.tiles64 + 2 * a.tile_cap;
+    }
   }
-  const int64_t row16 = (f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4) ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
+  const bool f4_reads = f4_first && f4_gather;  // gate | up reads its rows through `order`
+  const int list_rows = f4 && !two_lists ? f4_tok : TILE_ROWS;
+  const int64_t row16 = f4_reads || (fuse && fused.x_index) || (quant_in && !f4) ? 0 : H / 8;  // (no rows to copy where they are read through `order`)
   // A few routed rows in one launch: up to 256 where it gathers, which the sort doesn't, and up to 64 else (every thread reads all ids: 4 us for
   // 6 rows, 12 for 192, where k_sort takes 5.4 for 384; its histograms grow with the experts. 64 experts of 4096 / 2048, TQ1 bf16, 32 tokens x 6: 198.8 -> 193.5 us).
   const bool small = n <= (row16 || E > 512 ? ROUTE_SMALL_N : 64) && (((uintptr_t)x | (uintptr_t)p.xg) & 15) == 0;
@@ -367,12 +426,12 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
     g = g < 1 ? 1 : (g > 256 ? 256 : g);
     hipLaunchKernelGGL(k_route_small, dim3((unsigned)g), dim3(ROUTE_SMALL_THREADS), 0, s, p.order, p.offsets, p.inv, experts, (int)n, E, bad,
                        (u32x4*)p.xg, (const u32x4*)x, (int)k, T, row16, tiles || f4 ? p.tiles : nullptr, p.tile_count,
-                       p.tile_cap, f4 ? f4_tok : TILE_ROWS);
+                       p.tile_cap, list_rows);
     if ((rc = check_launch("route_small")) != BP_OK) return rc;
   } else {
-    const SortTiles list = {tiles || f4 ? p.tiles : nullptr, p.tile_count, p.tile_cap, f4 ? f4_tok : TILE_ROWS};
+    const SortTiles list = {tiles || f4 ? p.tiles : nullptr, p.tile_count, p.tile_cap, list_rows};
     if ((rc = sort_with_inverse(p.order, p.offsets, p.inv, experts, n, E, p.sort_ws, bad, s, list)) != BP_OK) return rc;
-    if ((f4 && f4_gather) || (fuse && fused.x_index) || (quant_in && !f4)) {
+    if (f4_reads || (fuse && fused.x_index) || (quant_in && !f4)) {
       // (no routed copy of the activations: the gate | up launch's conversion pass reads them through `order`)
     } else if (aligned16) {
       int64_t g = (n * (H / 8) + 255) / 256;
@@ -438,13 +497,19 @@ static int moe_layer(bool v4, void* out, int out_dtype, float limit, const void*
   };
   if (f4) {
     if (act == BP_I8 && (rc = bp_quant_act_int8(p.q, p.q_scale, x, BP_BF16, T, H, s)) != BP_OK) return rc;
-    if ((rc = launch_gemm_f4(f4_gu, s, rewritten)) != BP_OK) return rc;
-    if (!f4_glu) rc = v4 ? bp_swiglu_v4(p.h, p.gu, p.gu + I, (const float*)weights, p.order, n, limit, n, I, 2 * I, s) : bp_swiglu_bf16(p.h, p.gu, p.gu + I, n, I, 2 * I, s);
+    if (two_lists) {
+      hipLaunchKernelGGL(k_tile_list, dim3(1), dim3(1024), 0, s, p.tiles64, p.tiles64 + 2 * f4_gu.tile_cap, p.offsets, E, n, f4_gu.tile_cap, F4_TOK);
+      if ((rc = check_launch("tile_list")) != BP_OK) return rc;
+    }
+    rc = f4_first ? launch_gemm_f4(f4_gu, s, rewritten) : gemm(p.gu, p.xg, gate_up_packed, gate_up_scale, 2 * I, H, tiles, nullptr, false);
+    if (rc != BP_OK) return rc;
+    const bool glu_done = f4_first && f4_glu;
+    if (!glu_done) rc = v4 ? bp_swiglu_v4(p.h, p.gu, p.gu + I, (const float*)weights, p.order, n, limit, n, I, 2 * I, s) : bp_swiglu_bf16(p.h, p.gu, p.gu + I, n, I, 2 * I, s);
     if (rc != BP_OK) return rc;
     bool y16 = f4_glu;
-    rc = f4_both ? launch_gemm_f4(f4_down, s, rewritten) : gemm(p.y, p.h, down_packed, down_scale, H, I, false, &y16, false);
+    rc = f4_second ? launch_gemm_f4(f4_down, s, rewritten) : gemm(p.y, p.h, down_packed, down_scale, H, I, two_lists, &y16, false);
     if (rc != BP_OK) return rc;
-    if (f4_glu) note_kernel_suffix(f4_gather ? "+glu+gather" : "+glu");
+    if (glu_done) note_kernel_suffix(f4_gather ? "+glu+gather" : "+glu");
     if (y16) note_kernel_suffix("+y16");
     if (v4) return moe_combine_v4(out, out_dtype, p.y, y16, p.inv, experts, T, k, H, s);
     return moe_combine(out, p.y, y16, p.inv, weights, experts, T, k, H, s);

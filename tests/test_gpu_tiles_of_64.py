@@ -81,10 +81,10 @@ def test_bf16_pieces_keep_what_the_matrix_instruction_sums(tune, spread):
 
 
 # TQ1 layers either side of the lines from which their weights are rewritten as TQ2 ones: the same trits in either format are the same
-# layer to the bit (int8: exact group sums; bf16: the same kernel). Rows that start at any byte; two terms; groups of 256.
+# layer to the bit (int8: exact group sums; bf16: the same kernel, on which BP_TUNE_TQ2G=fp4 puts the TQ2 layer's down projection too). Rows that start at any byte; two terms; groups of 256.
 @pytest.mark.parametrize("act,T,E,k,terms,group,H,I", [("int8", 383, 16, 2, 1, 128, 1280, 1024), ("int8", 384, 16, 2, 1, 128, 1280, 1024), ("int8", 300, 8, 3, 2, 128, 1024, 1792),
                                                        ("int8", 400, 8, 2, 1, 256, 2048, 2560), ("bf16", 3100, 8, 2, 2, 128, 1024, 1280)])
-def test_tq1_layers_rewritten_as_tq2(act, T, E, k, terms, group, H, I):
+def test_tq1_layers_rewritten_as_tq2(tune, act, T, E, k, terms, group, H, I):
     import deepseekternarized_amd as bp
     from deepseekternarized_amd.moe import TernaryMoE
 
@@ -104,6 +104,8 @@ def test_tq1_layers_rewritten_as_tq2(act, T, E, k, terms, group, H, I):
     logits = 1.5 * torch.randn(T, E, device="cuda", generator=gen)
     got = {}
     for fmt in gate:
+        if act == "bf16" and fmt == "tq2":
+            tune("BP_TUNE_TQ2G", "fp4")
         moe = TernaryMoE(gate[fmt], up[fmt], down[fmt], H, I, k, fmt, group, act=act)
         got[fmt] = moe(x, logits)
         rewritten = bp.ext().last_kernel().startswith("gemm_tq1_as_tq2f4")
@@ -142,6 +144,28 @@ def test_tq1_layers_by_the_byte_table(tune, act, T, E, k, terms, group, H, I, sd
         tune("BP_TUNE_F4Q", "1000000000")
         ref = TernaryMoE(*packed("tq1"), H, I, k, "tq1", group, act=act)(x, logits)
     assert torch.isfinite(got.float()).all() and torch.equal(got, ref), bp.ext().last_kernel()
+
+
+# TQ2 layers with bf16 activations whose intermediate size is not half the hidden one: each product by its own line (768 tiles of 32 x 512), so
+# that a layer between the two has one of them on the pieces and the other one on bf16 matrix instructions, over a tile list each. As
+# grouped calls the products have the same lines, kernels and order of additions: the same bits.
+@pytest.mark.parametrize("T,H,I,first,second", [(1015, 2048, 1536, False, False), (1030, 2048, 1536, True, False), (1530, 2048, 1536, True, True),
+                                                (1015, 3072, 1024, False, False), (1030, 3072, 1024, False, True), (1530, 3072, 1024, True, True)])
+@pytest.mark.parametrize("terms", [1, 2])
+def test_bf16_layers_decide_per_product(tune, T, H, I, first, second, terms):
+    from deepseekternarized_amd import ext
+    from deepseekternarized_amd.moe import TernaryMoE
+
+    gen = torch.Generator(device="cuda").manual_seed(27)
+    E, k = 8, 4
+    moe = TernaryMoE(_terms(E, I, H, terms, gen), _terms(E, I, H, terms, gen), _terms(E, H, I, terms, gen), H, I, k, "tq2", 128)
+    x = torch.randn(T, H, device="cuda", generator=gen).bfloat16()
+    logits = torch.randn(T, E, device="cuda", generator=gen)
+    logits[:, 5] = -40.0  # an expert without rows
+    got = moe(x, logits)
+    name = ext().last_kernel()
+    assert name.startswith("gemm_tq2f4_bf16" if second else "gemm_tq2_bf16") and ("+glu+gather" in name) == first, name
+    assert torch.isfinite(got.float()).all() and torch.equal(got, moe.composed(x, logits)), name
 
 
 # The tile list that the sort makes: one workgroup over more experts than it has threads, one over the whole list at 257 and 4095 rows, the
