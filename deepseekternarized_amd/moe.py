@@ -108,15 +108,19 @@ class TernaryMoE:
 
     def _workspace(self, tokens: int, device, full: int = 0) -> torch.Tensor:
         """The layer's workspace. ``full``: the bytes with which the library would also rewrite a TQ1 layer's weights; room for these
-        is taken for the one call, since a layer doesn't hold on to it between calls."""
+        is taken for the one call, since a layer doesn't hold on to it between calls. The library runs the layer without it as well: so it
+        does where the device has no such room left, and under capture, whose graph would keep the room in its pool for good."""
         e = _need_ext(self.down[0][0])
         ws = getattr(self, "_ws", None)
         if 0 < full and ws is not None and ws.numel() >= full and ws.device == device:
             return ws
         need = int(e.lib.bp_moe_layer_workspace_bytes(tokens, self.hidden, self.inter, self.n_experts, self.top_k,
                                                       _lib.BP_I8 if self.act == "int8" else _lib.BP_BF16, _fmt_code(self.fmt)))
-        if full > need:
-            return torch.empty(full, dtype=torch.uint8, device=device)
+        if full > need and not torch.cuda.is_current_stream_capturing():
+            try:
+                return torch.empty(full, dtype=torch.uint8, device=device)
+            except torch.cuda.OutOfMemoryError:
+                pass
         device = torch.device(device)
         if device.index is None:  # torch.device("cuda") != torch.device("cuda:0"): compare devices with their index
             device = torch.device(device.type, torch.cuda.current_device())

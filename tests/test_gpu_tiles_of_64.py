@@ -114,6 +114,44 @@ def test_tq1_layers_rewritten_as_tq2(tune, act, T, E, k, terms, group, H, I):
     assert torch.isfinite(got["tq1"].float()).all() and torch.equal(got["tq1"], got["tq2"])
 
 
+def test_tq1_layers_run_without_room_for_rewritten_weights(monkeypatch):
+    """The rewriting's memory is optional: a device without it, and a capture (whose graph would keep it), run the layer on its TQ1
+    weights - the same exact group sums, so the same bits."""
+    import deepseekternarized_amd as bp
+    from deepseekternarized_amd import moe as module
+
+    gen = torch.Generator(device="cuda").manual_seed(28)
+    H, I, E, k, T = 1024, 1024, 8, 2, 400
+
+    def terms(N, K):
+        trits = torch.randint(-1, 2, (E * N, K), dtype=torch.int8, device="cuda", generator=gen)
+        return [(bp.pack(trits, "tq1").view(E, N, -1), (0.02 * torch.rand(E, N, K // 128, device="cuda", generator=gen)).half())]
+
+    layer = module.TernaryMoE(terms(I, H), terms(I, H), terms(H, I), H, I, k, "tq1", 128, act="int8")
+    x = torch.randn(T, H, device="cuda", generator=gen).bfloat16()
+    logits = torch.randn(T, E, device="cuda", generator=gen)
+    got = layer(x, logits)
+    assert bp.ext().last_kernel().startswith("gemm_tq1_as_tq2f4_i8"), bp.ext().last_kernel()
+    need = bp.ext().lib.bp_moe_layer_workspace_bytes(T, H, I, E, k, 0, 1)
+
+    class Full:  # torch on a device with room for the layer's own workspace only
+        def __getattr__(self, name):
+            return getattr(torch, name)
+
+        def empty(self, *size, **kw):
+            if size[0] == need or kw.get("dtype") != torch.uint8:
+                return torch.empty(*size, **kw)
+            raise torch.cuda.OutOfMemoryError("no room")
+
+    run = layer.graphed(T)
+    assert torch.equal(run(x, logits), got) and torch.equal(run(x, logits), got)
+    assert bp.ext().last_kernel().startswith("gemm_tq1f4_i8"), bp.ext().last_kernel()
+    assert run.workspace.numel() == need
+    monkeypatch.setattr(module, "torch", Full())
+    assert torch.equal(layer(x, logits), got)
+    assert bp.ext().last_kernel().startswith("gemm_tq1f4_i8"), bp.ext().last_kernel()
+
+
 # TQ1 layers on that kernel as they are, by the byte table: tiles of 32 tokens, rows that start at any byte, windows of an odd count, two
 # terms, groups of 256, scales of 32 bits (bf16 layers of these keep the kernel without pieces); either side of its lines. int8 (exact group sums): the bits of the same trits' TQ2 layer on the
 # kernels over tiles of 32; bf16: of the kernel for 16 x 16 x 128 pieces, whose pieces and order of additions are the same.
