@@ -312,7 +312,7 @@ extern "C" int bp_ternary_linear(void* out, int out_dtype, const void* x, int x_
       a = b;
     }
   }
-  if (p.f4 && a.stage && g_policy != 1) {
+  if (p.f4 && a.fmt == BP_TQ2 && a.stage && g_policy != 1) {  // (TQ1 weights that could not be rewritten stay on their kernels)
     GemmArgs w = a;
     w.x_dtype = BP_BF16;
     w.quant = 1;

@@ -48,6 +48,25 @@ def test_linear_call_equals_its_steps(T, fmt, act, xdt, N, K, group, terms):
         assert torch.equal(lin(x, out_dtype), _steps(x, same, K, group, same_fmt, act, out_dtype)), out_dtype
 
 
+def test_weights_that_cannot_be_rewritten_stay_on_their_kernels():
+    """TQ1 scales that start 4 bytes into a 16-byte line, which the TQ2 kernels don't read: the TQ1 kernels take the linear as it is, at a size
+    that a rewritten one takes to the tiles of 64 - the same exact group sums."""
+    import deepseekternarized_amd as bp
+
+    T, N, K = 1100, 4096, 1024
+    (w,), gen = _weights("tq1", N, K, 128, 1, torch.float16)
+    x = torch.randn(T, K, device="cuda", generator=gen).bfloat16()
+    room = torch.empty(w.scale.numel() + 2, dtype=torch.float16, device="cuda")
+    scale = room[2:].view(w.scale.shape)
+    scale.copy_(w.scale)
+    assert scale.data_ptr() % 16 == 4
+    want = bp.TernaryLinear([w], K, "tq1", 128)(x, torch.float32)
+    assert bp.ext().last_kernel() == "gemm_tq2f4_i8"
+    got = bp.TernaryLinear([bp.PackedTerm(w.packed, scale)], K, "tq1", 128)(x, torch.float32)
+    assert bp.ext().last_kernel() == "gemm_tq1_i8", bp.ext().last_kernel()
+    assert torch.isfinite(got).all() and torch.equal(got, want)
+
+
 def test_linear_call_with_leading_dimensions():
     import deepseekternarized_amd as bp
 
