@@ -176,7 +176,13 @@ bool f4_product(int64_t T, int64_t n, int64_t N, int64_t E) { return f4_pays_bf1
 // Layers whose GEMMs run on the kernel for token tiles of 64 (32 for TQ1).
 // TQ2, int8: from 16 rows per expert on average. Whole layer on it / on the 32-token tiles, us: 2048 / 1024 (hidden / intermediate), 64
 // experts, 16 rows each 73 / 82, 50 rows 112 / 146; 4096 / 2048, 64 experts, 12 rows 164 / 163, 37 rows 203 / 305; 384 experts, 6 rows
-// 733 / 739, 19 rows 750 / 920, 62 rows 1350 / 2194. bf16: layers of which a product does (f4_product).
+// 733 / 739, 19 rows 750 / 920, 62 rows 1350 / 2194. Few experts leave its larger workgroups short of the device: with at most 1024 output
+// columns of gate and up it takes over where the 32-token kernel needs more than one workgroup per CU (by the average rows: half a tile
+// per expert is padding), with more from 128 rows on; up to 64 tokens, where the other kernels' launches are sized by the tokens, where all experts
+// together have 384 blocks of 128 columns. On it / off it: 2048 / 1024, 8 experts, 300 rows 64 / 54, 800 rows 65 / 59, 1200 rows 70 / 84; 16 experts,
+// 600 rows 66 / 56, 900 rows 67 / 79; 4096 / 2048, 4 experts, 66 rows 73 / 61, 160 rows 86 / 102; 2048 / 1280, 2 experts, 66 rows 65 / 52, 200 rows
+// 66 / 63; 64 tokens: 7168 / 2048, 4 experts 112 / 76, 8 experts (256 rows) 112 / 86, 16 experts (512) 117 / 133; 2048 / 1024, 32 experts (512) 63 / 59;
+// 2816 / 1536, 32 experts (512) 81 / 88; 2048 / 1024, 64 experts (1024) 81 / 91. bf16: layers of which a product does (f4_product).
 // TQ1, int8: from 129 routed rows, where all experts together have 512 workgroups (two to a CU) or there are more than 64 tokens (the old
 // kernels' grids are bounded by the tokens up to there). Whole layer, us: 4096 / 2048, 64 experts of 6, 16 tokens 194 / 181, 32 205 / 316, 64
 // 204 / 221, 251 241 / 372, 1500 765 / 1274; 384 experts, 400 tokens 1038 / 1188, 2000 1357 / 2033; 2048 / 1024, 64 experts of 8, 16 tokens
@@ -189,7 +195,12 @@ bool moe_f4(int act, int fmt, int64_t T, int64_t n, int64_t H, int64_t I, int64_
   if (tuning().tq2g == 'b') return false;
   if (fmt == BP_TQ1 && tuning().f4q >= 0) return n >= tuning().f4q;
   if (fmt == BP_TQ1) return act == BP_I8 ? n > 128 && (T > 64 || E * I >= 512 * 128) : n >= (n_terms == 1 ? 16 : 44) * E;
-  if (act == BP_I8) return n >= (tuning().f4 >= 0 ? tuning().f4 : 16) * E;
+  if (act == BP_I8) {
+    if (tuning().f4 >= 0) return n >= tuning().f4 * E;
+    if (rewritten || n < 16 * E) return rewritten;
+    if (T <= 64) return E * I >= 384 * 128;
+    return (I > 1024 && n >= 128) || (n + 16 * E) * ((2 * I + 255) / 256) > 280 * 32;
+  }
   return rewritten || f4_product(T, n, 2 * I, E) || f4_product(T, n, H, E);  // (a TQ1 layer that isn't rewritten runs on fp8 pieces as well)
 }
 

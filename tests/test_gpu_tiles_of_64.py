@@ -13,10 +13,12 @@ def _terms(E, N, K, terms, gen, sdt=torch.float16, group=128):
              (0.02 * torch.rand(E, N, -(-K // group), device="cuda", generator=gen)).to(sdt)) for _ in range(terms)]
 
 
-# int8 layers either side of the line of 16 rows per expert on average; up to 256 routed rows (preparation and tile list in one launch)
-# and more; against the kernels over tiles of 32, whose exact group sums are scaled and added in the same order
-@pytest.mark.parametrize("pattern,T,E,k,terms,I,wide", [("standard", 127, 16, 2, 1, 1040, False), ("standard", 128, 16, 2, 1, 1040, True), ("v4", 70, 8, 2, 2, 1024, True),
-                                                        ("standard", 333, 16, 3, 2, 1280, True)])
+# int8 layers either side of the lines: 16 rows per expert on average; 128 rows; with 1024 columns 280 tiles of 32 rows x 256 gate | up rows; up to 64
+# tokens 384 blocks of 128 columns. Up to 256 routed rows (preparation and tile list in one launch) and more; against the kernels over tiles of 32, whose exact group sums are scaled and added in the same order
+@pytest.mark.parametrize("pattern,T,E,k,terms,I,wide", [("standard", 127, 16, 2, 1, 1040, False), ("standard", 128, 16, 2, 1, 1040, True), ("v4", 70, 8, 2, 2, 1280, True),
+                                                        ("standard", 333, 16, 3, 2, 1280, True), ("standard", 127, 4, 1, 1, 1280, False), ("standard", 128, 4, 1, 1, 1280, True),
+                                                        ("standard", 432, 16, 2, 1, 1024, False), ("v4", 433, 16, 2, 1, 1024, True), ("standard", 64, 47, 12, 1, 1024, False),
+                                                        ("standard", 64, 48, 12, 1, 1024, True), ("standard", 64, 8, 4, 2, 1280, False)])
 def test_int8_layers_from_sixteen_rows_per_expert(tune, pattern, T, E, k, terms, I, wide):
     import deepseekternarized_amd as bp
     from deepseekternarized_amd.moe import TernaryMoE
