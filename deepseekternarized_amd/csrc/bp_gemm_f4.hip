@@ -1,5 +1,5 @@
 // Grouped GEMM over token tiles of 64 rows (TQ2) or 32 (TQ1) on v_mfma_scale_f32_32x32x64_f8f6f4: ternary weights as fp4, activations
-// as two exact pieces, bf16 ones in fp8 and int8 ones in fp6, converted beforehand.
+// as two pieces, int8 ones in fp6 (exact) and bf16 ones in fp8 (exact down to 2^-9 of a block's largest), converted beforehand.
 //
 // Contract as everywhere (boilerplate/kernels/ternary_cuda.py:52-64, boilerplate/kernels/csrc/ternary_cuda_kernel.cu:44-99):
 // out[t, n] += sum_g scale[n, g] * sum_{k in g} x[t, k] * trit[n, k] over the groups in ascending order and the stacked terms, in float32.

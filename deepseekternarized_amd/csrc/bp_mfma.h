@@ -39,7 +39,7 @@ BP_LAUNCHER(launch_gemm_tq2, (const GemmArgs& a, hipStream_t s), (a, s))
 int launch_gemm_tq2f(const GemmArgs& a, hipStream_t s);
 int gemm_tq2f_applies(const GemmArgs& a);  // TQ1: BP_OK where launch_gemm_tq2f takes the call (nothing is launched)
 // bp_gemm_f4.hip: TQ2 over token tiles of 64, TQ1 over tiles of 32, weights as fp4, bf16 activations (or int8 ones, or bf16 ones to be quantised:
-// GemmArgs::quant) as two exact pieces. With a tile list (GemmArgs::tiles, entries of that many rows): max_rows is that.
+// GemmArgs::quant) as two pieces. With a tile list (GemmArgs::tiles, entries of that many rows): max_rows is that.
 constexpr int F4_TOK = 64, F4_TOK1 = 32;  // (TQ2, TQ1)
 int launch_gemm_f4(const GemmArgs& a, hipStream_t s, bool rewritten = false);  // rewritten: of TQ1 weights (named so)
 int gemm_f4_applies(const GemmArgs& a);  // BP_OK where launch_gemm_f4 takes the call (nothing is launched)
@@ -97,7 +97,9 @@ typedef __attribute__((address_space(3))) unsigned short lds_u16;
 
 // Weights and scales are read with raw buffer loads: a wave-uniform descriptor (base, byte range) in
 // scalar registers, a 32-bit lane offset and a scalar step offset, so a load needs no vector address
-// arithmetic, and a read past the range returns zeros instead of touching memory.
+// arithmetic, and a read past the range returns zeros instead of touching memory. The range check counts the lane and the scalar offset
+// together, dword by dword, also where the scalar offset alone lies past the range (measured inside one allocation: a range of 4096 bytes,
+// scalar offsets up to 900,000): rows past a tensor's end may be named by either.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, int64_t bytes) {
   const int n = bytes > 0x7fffffff ? 0x7fffffff : (int)bytes;
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, n, 0x00020000);

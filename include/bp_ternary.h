@@ -95,7 +95,7 @@ int bp_ternary_grouped_gemm(float* out, const void* x, int x_dtype, const float*
  * runs on them as well: the activations are split into a bf16 pair x = hi + lo (exact for fp16, to 2^-17 |x| for float32)
  * and both products are added into out. Without one they run on the general kernel. */
 size_t bp_grouped_gemm_workspace_bytes(int x_dtype, int64_t T, int64_t N, int64_t K, int64_t E, int fmt, int64_t max_rows);
-/* The same for int8 activations and TQ2: the workspace of the kernel for token tiles of 128 rows (large dense calls, and
+/* The same for int8 activations and TQ2: the workspace of the kernel for token tiles of 64 rows (large dense calls, and
  * grouped ones with at least 112 rows per expert on average), 0 where the call's sizes and number of terms mean that
  * bp_ternary_grouped_gemm_ws would not use one (beside them it needs the alignments that the tuned kernels need). */
 size_t bp_grouped_gemm_int8_workspace_bytes(int64_t T, int64_t N, int64_t K, int64_t group, int64_t E, int fmt, int n_terms, int64_t max_rows);

@@ -56,11 +56,11 @@ def tune(monkeypatch):
     _lib.load().bp_reload_tuning()
 
 
-# token tiles of 128: a full one and a remainder of 1, 2, 63, 64, 65 or 127 rows, experts without rows; K of an odd number of
+# token tiles of 64: full ones and a remainder of 1, 2, 16, 17, 44 or 63 rows, experts without rows; K of an odd number of
 # 256-wide windows and of one scale per 256; 16 rows past a whole row block of 256
 @pytest.mark.parametrize("counts", [(130,), (129, 0, 63), (192, 65, 127, 128), (16, 17, 300)])
 @pytest.mark.parametrize("N,K,group,terms,sdt", [(256, 1024, 128, 1, torch.float16), (272, 1280, 128, 2, torch.bfloat16), (528, 2048, 256, 1, torch.float32)])
-def test_int8_tiles_of_128(tune, counts, N, K, group, terms, sdt):
+def test_int8_tiles_of_64(tune, counts, N, K, group, terms, sdt):
     import deepseekternarized_amd as bp
 
     tune("BP_TUNE_TQ2G", "f")
@@ -70,12 +70,11 @@ def test_int8_tiles_of_128(tune, counts, N, K, group, terms, sdt):
     assert bp.ext().last_kernel() == "gemm_tq2f4_i8"
 
 
-# the same with eight waves of 256 rows per workgroup: rows whose scales leave room for one workgroup per CU - one term from K = 3584
-# on, two from 1792, three always -, an odd number of windows, one scale per 256, remainders of 1, 63, 65 and 127 rows
+# longer rows and more terms, an odd number of windows, one scale per 256, remainders of 1 and 63 rows
 @pytest.mark.parametrize("counts", [(129, 0, 63), (193, 65, 255)])
 @pytest.mark.parametrize("N,K,group,terms,sdt", [(272, 3584, 128, 1, torch.float16), (528, 4352, 128, 1, torch.float32), (256, 2048, 128, 2, torch.bfloat16),
                                                  (272, 2304, 128, 2, torch.float16), (528, 4096, 256, 1, torch.float16), (272, 1280, 128, 3, torch.float32)])
-def test_int8_tiles_of_128_with_eight_waves(tune, counts, N, K, group, terms, sdt):
+def test_int8_tiles_of_64_with_long_rows_and_terms(tune, counts, N, K, group, terms, sdt):
     import deepseekternarized_amd as bp
 
     tune("BP_TUNE_TQ2G", "f")
@@ -117,10 +116,10 @@ def test_linear_quantises_in_the_conversion_pass(tune, T, K, scale, out_dtype):
 
 @pytest.mark.parametrize("pattern,T,E,k,terms,H", [("standard", 1100, 8, 1, 1, 1024), ("standard", 700, 16, 4, 2, 1024), ("v4", 520, 4, 2, 1, 1024),
                                                    ("standard", 1100, 8, 1, 1, 4096), ("standard", 700, 4, 3, 2, 2048), ("v4", 520, 4, 2, 1, 4096)])
-def test_int8_layer_on_tiles_of_128(tune, pattern, T, E, k, terms, H):
-    """The layer on the 128-token kernel against the same layer as separate launches (standard), or on the 32-token kernel (v4):
+def test_int8_layer_on_tiles_of_64(tune, pattern, T, E, k, terms, H):
+    """The layer on the 64-token kernel against the same layer as separate launches (standard), or on the 32-token kernel (v4):
     the same rounding points over float32 sums that differ in order, so a few bf16 roundings and int8 steps fall otherwise.
-    H = 4096, and 2048 in two terms: the gate | up launch, with SwiGLU and the gather, on eight waves."""
+    H = 4096, and 2048 in two terms: long rows in the gate | up launch, which applies SwiGLU and gathers."""
     import deepseekternarized_amd as bp
     from deepseekternarized_amd.moe import TernaryMoE
 

@@ -16,7 +16,8 @@ def lib():
     return _lib.load()
 
 
-# one expert: 96 tokens, 128 blocks as four waves, 192 as eight (two terms from K = 1792, three always); several: 112 rows each and 384 blocks;
+# (lines of the kernel over tiles of 128 that k_gemm_f4 replaced) one expert: 96 tokens, 128 blocks, 192 with scales that leave room for one workgroup
+# per CU (two terms from K = 1792, three always); several: 112 rows each and 384 blocks;
 # scales that do not fit (K = 7168 in two terms), a group and row counts that the kernel does not take: no workspace
 @pytest.mark.parametrize("T,N,K,group,E,fmt,terms,asks", [
     (2048, 2048, 2048, 128, 1, TQ2, 1, True), (1920, 2048, 2048, 128, 1, TQ2, 1, False), (2048, 2048, 2048, 128, 1, TQ2, 2, False), (3072, 2048, 2048, 128, 1, TQ2, 2, True),
